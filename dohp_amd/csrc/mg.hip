@@ -9,8 +9,9 @@
 // (again 27-point), smoothing is a Jacobi-preconditioned Chebyshev polynomial on
 // [lo * lmax, hi * lmax] of D^{-1} A, the coarsest level (at most a few hundred nodes) is solved
 // with its explicit inverse.  The V-cycle works on symmetric half stencils (see
-// half_residual_kernel).  Pre- and post-smoothers are the same polynomial, so the V-cycle is
+// half_row).  Pre- and post-smoothers are the same polynomial, so the V-cycle is
 // a symmetric operator and serves as a CG preconditioner.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -125,35 +126,203 @@ __global__ void stencil_mult_kernel(Box b, const T *__restrict__ A, const T *__r
 // diagonal and the 13 upper neighbours, H[s - 13][r] for s = 13..26; the entry of a lower
 // neighbour is the upper entry stored at that neighbour's row.  The product reads 14 coefficient
 // streams instead of 27 (the shifted reads of the lower half hit the caches).
-template <typename T>
-__global__ void __launch_bounds__(256) half_residual_kernel(Box bx, const T *__restrict__ H, const T *__restrict__ b,
-                                                            const T *__restrict__ x, T *__restrict__ r)
+//
+// Sweeps (products with the half stencil).  A workgroup of 64 x BY threads takes NR planes of 64 x BY rows and stages
+// the iterate on their neighbourhood (NR + 2 planes, BY + 2 rows, 66 columns, zero outside the box) in LDS: a row then
+// issues its 27 coefficient loads and 2 to 5 staged ones instead of 54.  What bounds the row-per-thread form without
+// staging is the vector memory path, not the bytes: at 191^3 rows in FP64 it takes 281 us whatever the shape of the
+// block (and the bytes it fetches), 202 us if the iterate is not loaded; staged, 215 us with 64 x 4 rows of one plane,
+// 204 us with two planes (2.7 instead of 4.6 staged loads per row) and 200 us with 64 x 8 rows of two planes, 4.7 TB/s
+// on the 17 values a row cannot do without (a large copy reaches 4.9).  239^3: 561 -> 438, 416, 410 us.
+template <int BY, int NR>
+struct SweepTile {
+  static constexpr int TX = kBX + 2, TY = BY + 2, N = (NR + 2) * TY * TX, NT = kBX * BY, IT = (N + NT - 1) / NT;
+};
+// Levels take the 64 x 8 x 2 tile where it leaves at least four workgroups per compute unit (1024: from about 90^3
+// rows), the 64 x 4 x 1 tile below (47^3: 144 workgroups against 564).
+inline bool sweep_big(const Box &b)
 {
-  const long n = bx.n();
-  int I, J, K;
-  long i;
-  if (!box_index(bx, I, J, K, i)) return;
+  return (long)((b.nz + kBX - 1) / kBX) * ((b.ny + 7) / 8) * ((b.nx + 1) / 2) >= 1024;
+}
+
+// Fills the tile of the block at (I0, J0, K0) with load(g), g the row of the tile entry (every load unconditional:
+// entries outside the box load row 0 and are zero).  Ends with a barrier.
+template <int BY, int NR, typename T, typename Load>
+__device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0, int tid, T *tile, Load load)
+{
+  using S = SweepTile<BY, NR>;
   const long sy = bx.nz, sx = (long)bx.ny * bx.nz;
-  // unconditional loads at clamped indices, dropped by selects (see stencil_mult_kernel)
-  T acc = H[i] * x[i];
+  T v[S::IT];
+#pragma unroll
+  for (int u = 0; u < S::IT; u++) {
+    const int t = min(tid + u * S::NT, S::N - 1);
+    const int p = t / (S::TY * S::TX), rem = t - p * (S::TY * S::TX), jj = rem / S::TX, kk = rem - jj * S::TX;
+    const int gi = I0 + p - 1, gj = J0 + jj - 1, gk = K0 + kk - 1;
+    const bool in = inside(bx, gi, gj, gk);
+    const T y = load(in ? gi * sx + gj * sy + gk : 0L);
+    v[u] = in ? y : T(0);
+  }
+#pragma unroll
+  for (int u = 0; u < S::IT; u++)
+    if (tid + u * S::NT < S::N) tile[tid + u * S::NT] = v[u];
+  __syncthreads();
+}
+
+// Row i = (I, J, K) of the product, on plane q of the block's tile; tj, tk its row and column there.
+template <int BY, typename T>
+__device__ __forceinline__ T half_row(const Box &bx, const T *__restrict__ H, const T *tile, int q, int tj, int tk,
+                                      int I, int J, int K, long i)
+{
+  constexpr int TX = SweepTile<BY, 1>::TX, TY = SweepTile<BY, 1>::TY;
+  const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz;
+  T acc = H[i] * tile[((q + 1) * TY + tj) * TX + tk];
 #pragma unroll
   for (int s = 14; s < 27; s++) {
     const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
     const long off = di * sx + dj * sy + dk;
-    const bool up = inside(bx, I + di, J + dj, K + dk), lo = inside(bx, I - di, J - dj, K - dk);
-    const long iu = up ? i + off : i, il = lo ? i - off : i;
-    const T vu = H[(s - 13) * n + i] * x[iu], vl = H[(s - 13) * n + il] * x[il];
-    acc += up ? vu : T(0);
-    acc += lo ? vl : T(0);
+    // (a neighbour outside the box is zero in the tile; its lower coefficient is read at whatever row i - off is)
+    const long il = i - off >= 0 ? i - off : i;
+    acc += H[(s - 13) * n + i] * tile[((q + 1 + di) * TY + tj + dj) * TX + tk + dk];
+    acc += H[(s - 13) * n + il] * tile[((q + 1 - di) * TY + tj - dj) * TX + tk - dk];
   }
-  r[i] = (b ? b[i] : T(0)) - acc;
+  return acc;
+}
+
+// SW_RESID: out = b - A x (b may be null).  SW_CHEB: one Chebyshev step of the smoother, out of place (Jacobi needs the
+// old iterate at the neighbours): dn = a d + c D^-1 (b - A x), out = x + dn; d is read when a != 0 and written when
+// keep_d.  The _FIRST forms start from the first step's iterate x1 = c1 D^-1 b, formed in the staging: SW_FIRST_CHEB
+// takes the second step from it, SW_FIRST_RESID stores it in x1 and its residual in out.
+enum { SW_RESID, SW_CHEB, SW_FIRST_CHEB, SW_FIRST_RESID };
+template <typename T, int MODE, int BY, int NR>
+__global__ void __launch_bounds__(kBX *BY) half_sweep_kernel(Box bx, const T *__restrict__ H,
+                                                             const T *__restrict__ dinv, const T *__restrict__ b,
+                                                             const T *__restrict__ x, T *__restrict__ out,
+                                                             T *__restrict__ d, T *__restrict__ x1, T a, T c, T c1,
+                                                             int keep_d)
+{
+  using S = SweepTile<BY, NR>;
+  constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID;
+  __shared__ T tile[S::N];
+  const int I0 = blockIdx.z * NR, J0 = blockIdx.y * BY, K0 = blockIdx.x * kBX;
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g) {
+    if constexpr (FIRST) return c1 * dinv[g] * b[g];
+    else return x[g];
+  });
+  const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
+  if (K >= bx.nz || J >= bx.ny) return;
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int I = I0 + q;
+    if (NR > 1 && I >= bx.nx) break;
+    const long i = ((long)I * bx.ny + J) * bx.nz + K;
+    const T ax = half_row<BY, T>(bx, H, tile, q, tj, tk, I, J, K, i);
+    const T r = (MODE != SW_RESID || b ? b[i] : T(0)) - ax;
+    const T xi = tile[((q + 1) * S::TY + tj) * S::TX + tk];
+    if constexpr (MODE == SW_RESID) {
+      out[i] = r;
+    } else if constexpr (MODE == SW_FIRST_RESID) {
+      x1[i] = xi;
+      out[i] = r;
+    } else {
+      const T dn = (MODE == SW_FIRST_CHEB ? a * xi : a == T(0) ? T(0) : a * d[i]) + c * dinv[i] * r;
+      if (keep_d) d[i] = dn;
+      out[i] = xi + dn;
+    }
+  }
+}
+
+template <typename T, int MODE>
+void sweep(const Box &bx, const T *H, const T *dinv, const T *b, const T *x, T *out, T *d, T *x1, T a, T c, T c1,
+           int keep_d, hipStream_t st)
+{
+  const unsigned gx = (bx.nz + kBX - 1) / kBX;
+  if (sweep_big(bx))
+    hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 8, 2>), dim3(gx, (bx.ny + 7) / 8, (bx.nx + 1) / 2), dim3(kBX, 8), 0,
+                       st, bx, H, dinv, b, x, out, d, x1, a, c, c1, keep_d);
+  else
+    hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 4, 1>), dim3(gx, (bx.ny + 3) / 4, bx.nx), dim3(kBX, 4), 0, st, bx,
+                       H, dinv, b, x, out, d, x1, a, c, c1, keep_d);
 }
 
 // r = b - A x (b may be null) on a level.
 template <typename T>
 void residual(const Box &bx, const T *H, const T *b, const T *x, T *r, hipStream_t st)
 {
-  hipLaunchKernelGGL(half_residual_kernel<T>, box_grid(bx), box_block(), 0, st, bx, H, b, x, r);
+  sweep<T, SW_RESID>(bx, H, nullptr, b, x, r, nullptr, nullptr, T(0), T(0), T(0), 0, st);
+}
+
+// Power iterations for the largest eigenvalue of D^-1 A, on all smoothed levels at once: an iteration is one launch
+// over the blocks of every level (the coarse ones ride along with the finest), w = D^-1 A (v / ||v||) with the scaling
+// applied in the staging and the sums of squares of w reduced per block, and one that sums each level's block sums in
+// order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3 rows and their coarse
+// levels, 15 iterations, 6.5 -> 3.8 ms (4.4 TB/s on the 17 values a row cannot do without).
+constexpr int kMaxLevels = 16, kPowerThreads = kBX * 8;
+struct PowerLevel {
+  Box bx;
+  const double *H, *dinv;
+  double *v[2], *part;
+  unsigned first, gx, gy;  // first block of the level, its tiles along K and J
+  int blocks, big;         // number of blocks; 64 x 8 x 2 tiles, else 64 x 8 x 1
+};
+struct PowerArgs {
+  PowerLevel l[kMaxLevels];
+  int nl;
+};
+
+// Sum over the workgroup in a fixed order (within each wavefront, then over the wavefronts); the result is valid in
+// thread 0.  sh: one entry per wavefront.
+template <int NT>
+__device__ __forceinline__ double block_sum(double s, int t, double *sh)
+{
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+  if ((t & 63) == 0) sh[t >> 6] = s;
+  __syncthreads();
+  double r = 0;
+  if (t == 0)
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) r += sh[w];
+  return r;
+}
+
+template <int NR>
+__device__ __forceinline__ double power_rows(const PowerLevel &l, unsigned blk, double inv, const double *v, double *w,
+                                             double *tile)
+{
+  using S = SweepTile<8, NR>;
+  const Box &bx = l.bx;
+  const unsigned tx = blk % l.gx, rest = blk / l.gx, ty = rest % l.gy, tz = rest / l.gy;
+  const int I0 = tz * NR, J0 = ty * 8, K0 = tx * kBX, lx = threadIdx.x & (kBX - 1), ly = threadIdx.x / kBX;
+  stage_tile<8, NR>(bx, I0, J0, K0, threadIdx.x, tile, [&](long g) { return inv * v[g]; });
+  const int J = J0 + ly, K = K0 + lx;
+  double s = 0;
+  if (K < bx.nz && J < bx.ny) {
+#pragma unroll
+    for (int q = 0; q < NR; q++) {
+      const int I = I0 + q;
+      if (NR > 1 && I >= bx.nx) break;
+      const long i = ((long)I * bx.ny + J) * bx.nz + K;
+      const double y = l.dinv[i] * half_row<8, double>(bx, l.H, tile, q, ly + 1, lx + 1, I, J, K, i);
+      w[i] = y;
+      s += y * y;
+    }
+  }
+  return s;
+}
+
+__global__ void __launch_bounds__(kPowerThreads) power_step_kernel(PowerArgs g, int from,
+                                                                   const double *__restrict__ inv)
+{
+  __shared__ double tile[SweepTile<8, 2>::N];
+  __shared__ double sh[kPowerThreads / 64];
+  int k = 0;
+  while (k + 1 < g.nl && blockIdx.x >= g.l[k + 1].first) k++;
+  const PowerLevel &l = g.l[k];
+  const unsigned blk = blockIdx.x - l.first;
+  const double s = l.big ? power_rows<2>(l, blk, inv[k], l.v[from], l.v[1 - from], tile)
+                         : power_rows<1>(l, blk, inv[k], l.v[from], l.v[1 - from], tile);
+  const double t = block_sum<kPowerThreads>(s, threadIdx.x, sh);
+  if (threadIdx.x == 0) l.part[blk] = t;
 }
 
 // FP16 coefficients of the FP32 V-cycle.  With the row scales s_i = sqrt(a_ii) (FP32), a level keeps the 13 upper
@@ -325,18 +494,6 @@ __global__ void diag_inv_kernel(long n, const T *__restrict__ A, T *__restrict__
   if (r < n) dinv[r] = T(1) / A[13 * n + r];
 }
 
-// Chebyshev step: d = a d + c dinv r;  x += d   (first step: a = 0)
-template <typename T>
-__global__ void cheb_step_kernel(long n, T a, T c, const T *__restrict__ dinv, const T *__restrict__ r,
-                                 T *__restrict__ d, T *__restrict__ x, int first_sets_x)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const T dn = (a == T(0) ? T(0) : a * d[i]) + c * dinv[i] * r[i];
-  d[i] = dn;
-  x[i] = first_sets_x ? dn : x[i] + dn;
-}
-
 // 1-D prolongation weights of fine index f onto coarse indices (at most two).
 __device__ __forceinline__ int parents(int f, int nc, int (&c)[2], double (&w)[2])
 {
@@ -390,32 +547,9 @@ __device__ __forceinline__ void parents2(int f, int nc, int (&c)[2], float (&w)[
   w[1] = m > 1 ? (float)ww[1] : 0.f;
 }
 
-// xout = xin + P xc (out of place: the FP16 V-cycle's iterate alternates between two buffers)
-__global__ void prolong_kernel(Box f, Box c, const float *__restrict__ xc, const float *__restrict__ xin,
-                               float *__restrict__ xout)
-{
-  int I, J, K;
-  long F;
-  if (!box_index(f, I, J, K, F)) return;
-  int ci[2], cj[2], ck[2];
-  float wi[2], wj[2], wk[2];
-  parents2(I, c.nx, ci, wi);
-  parents2(J, c.ny, cj, wj);
-  parents2(K, c.nz, ck, wk);
-  float acc = 0;
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int d = 0; d < 2; d++)
-        acc += (wi[a] * wj[b] * wk[d]) * xc[((long)ci[a] * c.ny + cj[b]) * c.nz + ck[d]];
-  xout[F] = xin[F] + acc;
-}
-
-// xf += P xc
+// xout = xin + P xc (xout may be xin: the smoothers' iterate alternates between two buffers)
 template <typename T>
-__global__ void prolong_add_kernel(Box f, Box c, const T *__restrict__ xc, T *__restrict__ xf)
+__global__ void prolong_kernel(Box f, Box c, const T *__restrict__ xc, const T *xin, T *xout)
 {
   int I, J, K;
   long F;
@@ -433,7 +567,7 @@ __global__ void prolong_add_kernel(Box f, Box c, const T *__restrict__ xc, T *__
 #pragma unroll
       for (int d = 0; d < 2; d++)
         acc += T(wi[a] * wj[b] * wk[d]) * xc[((long)ci[a] * c.ny + cj[b]) * c.nz + ck[d]];
-  xf[F] += acc;
+  xout[F] = xin[F] + acc;
 }
 
 // 1-D prolongation weight of the coarse node at offset t (in -1..1) from coarse node c at the fine node at offset e
@@ -526,55 +660,43 @@ __global__ void to_f32(long n, const double *__restrict__ a, float *__restrict__
   if (i < n) b[i] = (float)a[i];
 }
 
-__global__ void sumsq_kernel(long n, const double *__restrict__ a, double *__restrict__ part)
+// Start vectors of the power iteration: a counter-based hash (splitmix64) of the row, uniform in [0.25, 1.25), with
+// the sums of squares of 256 blocks per level (blockIdx.y).
+__global__ void __launch_bounds__(256) power_start_kernel(PowerArgs g)
 {
-  __shared__ double sh[256];
+  __shared__ double sh[4];
+  const PowerLevel &l = g.l[blockIdx.y];
+  const long n = l.bx.n();
   double s = 0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) s += a[i] * a[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    uint64_t z = (uint64_t)i + 0x9E3779B97F4A7C15ULL;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
+    z ^= z >> 31;
+    const double v = (double)(z >> 11) * (1.0 / 9007199254740992.0) + 0.25;
+    l.v[0][i] = v;
+    s += v * v;
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  const double t = block_sum<256>(s, threadIdx.x, sh);
+  if (threadIdx.x == 0) l.part[blockIdx.x] = t;
 }
 
-// Start vector of the power iteration: a counter-based hash (splitmix64) of the row, uniform in [0.25, 1.25).
-__global__ void power_start_kernel(long n, double *__restrict__ v)
+// ||v|| and 1 / ||v|| of every level (blockIdx.x) from its block sums, taken in order: the 256 of the start vector, or
+// one per block of the level.
+__global__ void __launch_bounds__(1024) power_norm_kernel(PowerArgs g, int start, double *__restrict__ norm,
+                                                          double *__restrict__ inv)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint64_t z = (uint64_t)i + 0x9E3779B97F4A7C15ULL;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-  z ^= z >> 31;
-  v[i] = (double)(z >> 11) * (1.0 / 9007199254740992.0) + 0.25;
-}
-
-// v = w / ||w||, with ||w||^2 the sum of sumsq_kernel's 256 partial sums taken in order (the same sum on every
-// block, no host round trip); block 0 also stores ||w|| (norm may be null).  v may be w.
-__global__ void normalize_kernel(long n, const double *__restrict__ part, const double *w, double *v,
-                                 double *__restrict__ norm)
-{
-  __shared__ double inv;
+  __shared__ double sh[16];
+  const PowerLevel &l = g.l[blockIdx.x];
+  const int m = start ? 256 : l.blocks;
+  double s = 0;
+  for (int k = threadIdx.x; k < m; k += 1024) s += l.part[k];
+  const double t = block_sum<1024>(s, threadIdx.x, sh);
   if (threadIdx.x == 0) {
-    double t = 0;
-    for (int k = 0; k < 256; k++) t += part[k];
     const double nw = sqrt(t);
-    inv = 1.0 / nw;
-    if (blockIdx.x == 0 && norm) *norm = nw;
+    norm[blockIdx.x] = nw;
+    inv[blockIdx.x] = 1.0 / nw;
   }
-  __syncthreads();
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = inv * w[i];
-}
-
-__global__ void scale_kernel(long n, double s, const double *__restrict__ dinv, const double *__restrict__ a,
-                             double *__restrict__ b)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = s * (dinv ? dinv[i] : 1.0) * a[i];
 }
 
 inline dim3 grid_of(long n) { return dim3((unsigned)((n + 255) / 256)); }
@@ -649,7 +771,7 @@ struct _p_dohpMG {
   int coeff16 = 1;  // the FP32 V-cycle reads the FP16 coefficients
   DevBuf<double> cinv64;
   DevBuf<float> cinv32;
-  DevBuf<double> part;  // the power iteration's 256 partial sums and last norm
+  DevBuf<double> part;  // the power iterations' norms and block sums
   // V-cycles replayed as HIP graphs: the coarse levels' kernels run for a few microseconds each, less than their
   // launch costs the host, so the eager V-cycle leaves the GPU waiting; a graph is captured (on a private stream)
   // per precision for the vectors it was applied to and replayed while they stay the same.
@@ -678,26 +800,50 @@ struct _p_dohpMG {
 
 namespace {
 
-// lmax of D^-1 A on a level by power iteration, in the level's work vectors (free outside a V-cycle).
-dErr estimate_lmax(MGLevel &lv, DevBuf<double> &part, hipStream_t st, int its)
+// lmax of D^-1 A on every smoothed level by power iteration, in the levels' work vectors (free outside a V-cycle).  The
+// iterations stay on the device: one read of the last norms at the end.
+dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
 {
-  DevBuf<double> &v = lv.r64, &w = lv.d64;
-  hipLaunchKernelGGL(power_start_kernel, grid_of(lv.n), dim3(256), 0, st, lv.n, v.ptr);
-  // the iterations stay on the device: one read of the last norm at the end
-  hipLaunchKernelGGL(sumsq_kernel, dim3(256), dim3(256), 0, st, lv.n, v.ptr, part.ptr);
-  hipLaunchKernelGGL(normalize_kernel, grid_of(lv.n), dim3(256), 0, st, lv.n, part.ptr, v.ptr, v.ptr, nullptr);
+  const int nl = (int)mg->L.size() - 1;
+  if (nl == 0) return 0;
+  DOHP_CHECK(nl <= kMaxLevels, dohpERR_ARG, "multigrid: too many levels");
+  PowerArgs g{};
+  g.nl = nl;
+  unsigned blocks = 0;
+  size_t parts = 2 * kMaxLevels;  // norms and their inverses, then the levels' block sums
+  for (int k = 0; k < nl; k++) {
+    MGLevel &lv = mg->L[k];
+    PowerLevel &l = g.l[k];
+    l.bx = lv.box;
+    l.H = lv.H64.ptr;
+    l.dinv = lv.dinv64.ptr;
+    l.v[0] = lv.r64.ptr;
+    l.v[1] = lv.d64.ptr;
+    l.big = sweep_big(lv.box);
+    l.gx = (lv.box.nz + kBX - 1) / kBX;
+    l.gy = (lv.box.ny + 7) / 8;
+    l.blocks = (int)(l.gx * l.gy * (l.big ? (lv.box.nx + 1) / 2 : lv.box.nx));
+    l.first = blocks;
+    blocks += l.blocks;
+    parts += std::max(256, l.blocks);
+  }
+  if (!mg->part.holds(parts)) DOHP_CALL(mg->part.alloc(parts));
+  double *norm = mg->part.ptr, *inv = norm + kMaxLevels, *at = inv + kMaxLevels;
+  for (int k = 0; k < nl; k++) {
+    g.l[k].part = at;
+    at += std::max(256, g.l[k].blocks);
+  }
+  hipLaunchKernelGGL(power_start_kernel, dim3(256, nl), dim3(256), 0, st, g);
+  hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 1, norm, inv);
   for (int k = 0; k < its; k++) {
-    residual<double>(lv.box, lv.H64.ptr, nullptr, v.ptr, w.ptr, st);  // w = -A v
-    hipLaunchKernelGGL(scale_kernel, grid_of(lv.n), dim3(256), 0, st, lv.n, -1.0, lv.dinv64.ptr, w.ptr, w.ptr);
-    hipLaunchKernelGGL(sumsq_kernel, dim3(256), dim3(256), 0, st, lv.n, w.ptr, part.ptr);
-    hipLaunchKernelGGL(normalize_kernel, grid_of(lv.n), dim3(256), 0, st, lv.n, part.ptr, w.ptr, v.ptr,
-                       part.ptr + 256);
+    hipLaunchKernelGGL(power_step_kernel, dim3(blocks), dim3(kPowerThreads), 0, st, g, k & 1, inv);
+    hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 0, norm, inv);
   }
   DOHP_HIP(hipGetLastError());
-  double nw = 0;
-  if (its > 0) DOHP_HIP(hipMemcpyAsync(&nw, part.ptr + 256, sizeof(double), hipMemcpyDeviceToHost, st));
+  double h[kMaxLevels] = {};
+  DOHP_HIP(hipMemcpyAsync(h, norm, sizeof(double) * nl, hipMemcpyDeviceToHost, st));
   DOHP_HIP(hipStreamSynchronize(st));
-  lv.lmax = nw;
+  for (int k = 0; k < nl; k++) mg->L[k].lmax = h[k];
   return 0;
 }
 
@@ -765,28 +911,75 @@ struct LvPtr<float> {
   static const float *cinv(const _p_dohpMG *m) { return m->cinv32.ptr; }
 };
 
-// x <- x + p(D^-1 A) D^-1 (b - A x), Chebyshev of the given degree on [lo, hi] * lmax.
+// Coefficients of the Chebyshev smoother of the given degree on [lo, hi] * lmax: step k (from 0) is
+// d = a_k d + c_k D^-1 (b - A x), x += d (a_0 = 0).
+struct ChebCoeffs {
+  double theta, delta, sigma, rho;
+  ChebCoeffs(const _p_dohpMG *mg, const MGLevel &lv)
+  {
+    const double lmin = mg->lo * lv.lmax, lmax = mg->hi * lv.lmax;
+    theta = 0.5 * (lmax + lmin);
+    delta = 0.5 * (lmax - lmin);
+    sigma = theta / delta;
+    rho = 1.0 / sigma;
+  }
+  void step(int k, double &a, double &c)
+  {
+    a = 0.0;
+    c = 1.0 / theta;
+    if (k == 0) return;
+    const double rho_new = 1.0 / (2.0 * sigma - rho);
+    a = rho_new * rho;
+    c = 2.0 * rho_new / delta;
+    rho = rho_new;
+  }
+};
+
+// The V-cycle at level l.  The smoothers' steps move the iterate between x and the level's residual vector: the first
+// two pre-smoothing steps from zero are one sweep (at degree 1 the first step and the residual are), and the
+// prolongation writes into the buffer from which the post-smoother's steps end in x.
 template <typename T>
-void smooth(const _p_dohpMG *mg, MGLevel &lv, const T *b, T *x, bool zero_init, hipStream_t st)
+void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
 {
   using P = LvPtr<T>;
-  const double lmin = mg->lo * lv.lmax, lmaxs = mg->hi * lv.lmax;
-  const double theta = 0.5 * (lmaxs + lmin), delta = 0.5 * (lmaxs - lmin), sigma = theta / delta;
-  double rho = 1.0 / sigma;
-  T *r = P::r(lv), *d = P::d(lv);
-  const dim3 g = grid_of(lv.n);
-  if (zero_init)
-    hipLaunchKernelGGL(cheb_step_kernel<T>, g, dim3(256), 0, st, lv.n, T(0), (T)(1.0 / theta), P::dinv(lv), b, d, x, 1);
-  else {
-    residual<T>(lv.box, P::A(lv), b, x, r, st);
-    hipLaunchKernelGGL(cheb_step_kernel<T>, g, dim3(256), 0, st, lv.n, T(0), (T)(1.0 / theta), P::dinv(lv), r, d, x, 0);
+  MGLevel &lv = mg->L[l];
+  if (l + 1 == mg->L.size()) {
+    hipLaunchKernelGGL(dense_mv_kernel<T>, dim3((unsigned)((lv.n + 3) / 4)), dim3(256), 0, st, (int)lv.n,
+                       P::cinv(mg), b, x);
+    return;
   }
-  for (int k = 1; k < mg->degree; k++) {
-    residual<T>(lv.box, P::A(lv), b, x, r, st);
-    const double rho_new = 1.0 / (2.0 * sigma - rho);
-    hipLaunchKernelGGL(cheb_step_kernel<T>, g, dim3(256), 0, st, lv.n, (T)(rho_new * rho), (T)(2.0 * rho_new / delta),
-                       P::dinv(lv), r, d, x, 0);
-    rho = rho_new;
+  MGLevel &cv = mg->L[l + 1];
+  const T *H = P::A(lv), *dinv = P::dinv(lv);
+  T *d = P::d(lv), *cur = x, *other = P::r(lv);
+  double a, c, c1;
+  ChebCoeffs pre(mg, lv);
+  pre.step(0, a, c1);
+  if (mg->degree == 1) {
+    sweep<T, SW_FIRST_RESID>(lv.box, H, dinv, b, nullptr, other, nullptr, cur, T(0), T(0), (T)c1, 0, st);
+  } else {
+    for (int k = 1; k < mg->degree; k++) {
+      pre.step(k, a, c);
+      const int keep_d = k + 1 < mg->degree;
+      if (k == 1) {
+        sweep<T, SW_FIRST_CHEB>(lv.box, H, dinv, b, nullptr, cur, d, nullptr, (T)a, (T)c, (T)c1, keep_d, st);
+      } else {
+        sweep<T, SW_CHEB>(lv.box, H, dinv, b, cur, other, d, nullptr, (T)a, (T)c, T(0), keep_d, st);
+        std::swap(cur, other);
+      }
+    }
+    residual<T>(lv.box, H, b, cur, other, st);
+  }
+  hipLaunchKernelGGL(restrict_kernel<T>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, P::b(cv));
+  vcycle<T>(mg, l + 1, P::b(cv), P::x(cv), st);
+  T *start = mg->degree % 2 == 0 ? x : P::r(lv);
+  hipLaunchKernelGGL(prolong_kernel<T>, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, P::x(cv), cur, start);
+  cur = start;
+  other = start == x ? P::r(lv) : x;
+  ChebCoeffs post(mg, lv);
+  for (int k = 0; k < mg->degree; k++) {
+    post.step(k, a, c);
+    sweep<T, SW_CHEB>(lv.box, H, dinv, b, cur, other, d, nullptr, (T)a, (T)c, T(0), k + 1 < mg->degree, st);
+    std::swap(cur, other);
   }
 }
 
@@ -837,29 +1030,11 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
                      cv.b32.ptr);
   vcycle16(mg, l + 1, cv.b32.ptr, cv.x32.ptr, st);
   float *other = cur == x ? lv.t32.ptr : x;
-  hipLaunchKernelGGL(prolong_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, cv.x32.ptr, cur, other);
+  hipLaunchKernelGGL(prolong_kernel<float>, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, cv.x32.ptr, cur,
+                     other);
   cur = smooth16(mg, lv, b, other, cur, false, st);
   if (cur != x)  // (not reached: the moves are even)
     (void)hipMemcpyAsync(x, cur, sizeof(float) * lv.n, hipMemcpyDeviceToDevice, st);
-}
-
-template <typename T>
-void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
-{
-  using P = LvPtr<T>;
-  MGLevel &lv = mg->L[l];
-  if (l + 1 == mg->L.size()) {
-    hipLaunchKernelGGL(dense_mv_kernel<T>, dim3((unsigned)((lv.n + 3) / 4)), dim3(256), 0, st, (int)lv.n,
-                       P::cinv(mg), b, x);
-    return;
-  }
-  MGLevel &cv = mg->L[l + 1];
-  smooth<T>(mg, lv, b, x, true, st);
-  residual<T>(lv.box, P::A(lv), b, x, P::r(lv), st);
-  hipLaunchKernelGGL(restrict_kernel<T>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, P::r(lv), P::b(cv));
-  vcycle<T>(mg, l + 1, P::b(cv), P::x(cv), st);
-  hipLaunchKernelGGL(prolong_add_kernel<T>, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, P::x(cv), x);
-  smooth<T>(mg, lv, b, x, false, st);
 }
 
 }  // namespace
@@ -885,8 +1060,8 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
                          lv.dg16.ptr, lv.sc16.ptr);
     hipLaunchKernelGGL(diag_inv_kernel<double>, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.dinv64.ptr);
     hipLaunchKernelGGL(to_f32<float>, grid_of(n), dim3(256), 0, st, n, lv.dinv64.ptr, lv.dinv32.ptr);
-    if (l + 1 < mg->L.size()) DOHP_CALL(estimate_lmax(lv, mg->part, st, 15));
   }
+  DOHP_CALL(estimate_lmax(mg, st, 15));
   std::vector<double> inv;
   DOHP_CALL(coarse_inverse(mg->L.back(), st, inv));
   mg->ncoarse = (int)mg->L.back().n;
@@ -911,7 +1086,7 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
   _p_dohpMG *mg = new _p_dohpMG;
   mg->degree = smooth_degree > 0 ? smooth_degree : 2;
   const long nmax = max_coarse > 0 ? max_coarse : 512;
-  dErr err = mg->part.alloc(257);
+  dErr err = 0;
   {
     MGLevel lv;
     lv.box = Box{q1->box[0], q1->box[1], q1->box[2]};
