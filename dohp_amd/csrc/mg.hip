@@ -145,8 +145,8 @@ inline bool sweep_big(const Box &b)
   return (long)((b.nz + kBX - 1) / kBX) * ((b.ny + 7) / 8) * ((b.nx + 1) / 2) >= 1024;
 }
 
-// Fills the tile of the block at (I0, J0, K0) with load(g), g the row of the tile entry (every load unconditional:
-// entries outside the box load row 0 and are zero).  Ends with a barrier.
+// Fills the tile of the block at (I0, J0, K0) with load(g, gi, gj, gk), g the row of the tile entry at (gi, gj, gk)
+// (every load unconditional: entries outside the box load row 0 and are zero).  Ends with a barrier.
 template <int BY, int NR, typename T, typename Load>
 __device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0, int tid, T *tile, Load load)
 {
@@ -159,13 +159,56 @@ __device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0
     const int p = t / (S::TY * S::TX), rem = t - p * (S::TY * S::TX), jj = rem / S::TX, kk = rem - jj * S::TX;
     const int gi = I0 + p - 1, gj = J0 + jj - 1, gk = K0 + kk - 1;
     const bool in = inside(bx, gi, gj, gk);
-    const T y = load(in ? gi * sx + gj * sy + gk : 0L);
+    const T y = load(in ? gi * sx + gj * sy + gk : 0L, gi, gj, gk);
     v[u] = in ? y : T(0);
   }
 #pragma unroll
   for (int u = 0; u < S::IT; u++)
     if (tid + u * S::NT < S::N) tile[tid + u * S::NT] = v[u];
   __syncthreads();
+}
+
+// Coarse correction of a block's tile: the coarse nodes that interpolate to the tile's fine ones, staged in LDS (zero
+// outside the coarse box).  Fine index f has the coarse parents f/2 - 1 and f/2 with weight 1/2 if it is even and
+// (f-1)/2 if it is odd; with I0, J0, K0 the block's first fine row, the parents of I0 - 1 .. I0 + NR start at
+// I0/2 - 1.  A prolongation of its own (read and write the iterate, 8 coarse loads per row) took 78 us at 239^3 rows in
+// FP32, as much as half a smoothing step.
+template <int BY, int NR>
+struct CoarseTile {
+  static constexpr int X = kBX / 2 + 2, Y = BY / 2 + 2, Z = 3, N = X * Y * Z, NT = kBX * BY, IT = (N + NT - 1) / NT;
+  static_assert(NR <= 2 && BY % 2 == 0, "three coarse planes cover the tile");
+};
+template <int BY, int NR, typename T>
+__device__ __forceinline__ void stage_coarse(const Box &cb, const T *__restrict__ xc, int I0, int J0, int K0, int tid,
+                                             T *ct)
+{
+  using C = CoarseTile<BY, NR>;
+  T v[C::IT];
+#pragma unroll
+  for (int u = 0; u < C::IT; u++) {
+    const int t = min(tid + u * C::NT, C::N - 1);
+    const int p = t / (C::Y * C::X), rem = t - p * (C::Y * C::X), jj = rem / C::X, kk = rem - jj * C::X;
+    const int ci = (I0 >> 1) - 1 + p, cj = (J0 >> 1) - 1 + jj, ck = (K0 >> 1) - 1 + kk;
+    const bool in = inside(cb, ci, cj, ck);
+    const T y = xc[in ? ((long)ci * cb.ny + cj) * cb.nz + ck : 0L];
+    v[u] = in ? y : T(0);
+  }
+#pragma unroll
+  for (int u = 0; u < C::IT; u++)
+    if (tid + u * C::NT < C::N) ct[tid + u * C::NT] = v[u];
+  __syncthreads();
+}
+// The correction at fine node (gi, gj, gk) of the tile.
+template <int BY, int NR, typename T>
+__device__ __forceinline__ T coarse_value(const T *ct, int I0, int J0, int K0, int gi, int gj, int gk)
+{
+  using C = CoarseTile<BY, NR>;
+  const int i1 = (gi >> 1) - (I0 >> 1) + 1, j1 = (gj >> 1) - (J0 >> 1) + 1, k1 = (gk >> 1) - (K0 >> 1) + 1;
+  const int i0 = i1 - 1 + (gi & 1), j0 = j1 - 1 + (gj & 1), k0 = k1 - 1 + (gk & 1);  // odd: the one parent twice
+  const T *a = ct + i0 * C::Y * C::X, *b = ct + i1 * C::Y * C::X;
+  const int r0 = j0 * C::X, r1 = j1 * C::X;
+  return T(0.125) * (((a[r0 + k0] + a[r0 + k1]) + (a[r1 + k0] + a[r1 + k1])) +
+                     ((b[r0 + k0] + b[r0 + k1]) + (b[r1 + k0] + b[r1 + k1])));
 }
 
 // Row i = (I, J, K) of the product, on plane q of the block's tile; tj, tk its row and column there.
@@ -191,21 +234,25 @@ __device__ __forceinline__ T half_row(const Box &bx, const T *__restrict__ H, co
 // SW_RESID: out = b - A x (b may be null).  SW_CHEB: one Chebyshev step of the smoother, out of place (Jacobi needs the
 // old iterate at the neighbours): dn = a d + c D^-1 (b - A x), out = x + dn; d is read when a != 0 and written when
 // keep_d.  The _FIRST forms start from the first step's iterate x1 = c1 D^-1 b, formed in the staging: SW_FIRST_CHEB
-// takes the second step from it, SW_FIRST_RESID stores it in x1 and its residual in out.
-enum { SW_RESID, SW_CHEB, SW_FIRST_CHEB, SW_FIRST_RESID };
+// takes the second step from it, SW_FIRST_RESID stores it in x1 and its residual in out.  SW_PRO_CHEB takes its step
+// from x + P xc, the iterate with the coarse correction.
+enum { SW_RESID, SW_CHEB, SW_FIRST_CHEB, SW_FIRST_RESID, SW_PRO_CHEB };
 template <typename T, int MODE, int BY, int NR>
 __global__ void __launch_bounds__(kBX *BY) half_sweep_kernel(Box bx, const T *__restrict__ H,
                                                              const T *__restrict__ dinv, const T *__restrict__ b,
                                                              const T *__restrict__ x, T *__restrict__ out,
                                                              T *__restrict__ d, T *__restrict__ x1, T a, T c, T c1,
-                                                             int keep_d)
+                                                             int keep_d, Box cb, const T *__restrict__ xc)
 {
   using S = SweepTile<BY, NR>;
-  constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID;
+  constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID, PRO = MODE == SW_PRO_CHEB;
   __shared__ T tile[S::N];
+  __shared__ T ct[PRO ? CoarseTile<BY, NR>::N : 1];
   const int I0 = blockIdx.z * NR, J0 = blockIdx.y * BY, K0 = blockIdx.x * kBX;
-  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g) {
+  if constexpr (PRO) stage_coarse<BY, NR>(cb, xc, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, ct);
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int gi, int gj, int gk) {
     if constexpr (FIRST) return c1 * dinv[g] * b[g];
+    else if constexpr (PRO) return x[g] + coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
     else return x[g];
   });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
@@ -233,15 +280,15 @@ __global__ void __launch_bounds__(kBX *BY) half_sweep_kernel(Box bx, const T *__
 
 template <typename T, int MODE>
 void sweep(const Box &bx, const T *H, const T *dinv, const T *b, const T *x, T *out, T *d, T *x1, T a, T c, T c1,
-           int keep_d, hipStream_t st)
+           int keep_d, hipStream_t st, const Box &cb = Box{}, const T *xc = nullptr)
 {
   const unsigned gx = (bx.nz + kBX - 1) / kBX;
   if (sweep_big(bx))
     hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 8, 2>), dim3(gx, (bx.ny + 7) / 8, (bx.nx + 1) / 2), dim3(kBX, 8), 0,
-                       st, bx, H, dinv, b, x, out, d, x1, a, c, c1, keep_d);
+                       st, bx, H, dinv, b, x, out, d, x1, a, c, c1, keep_d, cb, xc);
   else
     hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 4, 1>), dim3(gx, (bx.ny + 3) / 4, bx.nx), dim3(kBX, 4), 0, st, bx,
-                       H, dinv, b, x, out, d, x1, a, c, c1, keep_d);
+                       H, dinv, b, x, out, d, x1, a, c, c1, keep_d, cb, xc);
 }
 
 // r = b - A x (b may be null) on a level.
@@ -293,7 +340,7 @@ __device__ __forceinline__ double power_rows(const PowerLevel &l, unsigned blk, 
   const Box &bx = l.bx;
   const unsigned tx = blk % l.gx, rest = blk / l.gx, ty = rest % l.gy, tz = rest / l.gy;
   const int I0 = tz * NR, J0 = ty * 8, K0 = tx * kBX, lx = threadIdx.x & (kBX - 1), ly = threadIdx.x / kBX;
-  stage_tile<8, NR>(bx, I0, J0, K0, threadIdx.x, tile, [&](long g) { return inv * v[g]; });
+  stage_tile<8, NR>(bx, I0, J0, K0, threadIdx.x, tile, [&](long g, int, int, int) { return inv * v[g]; });
   const int J = J0 + ly, K = K0 + lx;
   double s = 0;
   if (K < bx.nz && J < bx.ny) {
@@ -329,8 +376,9 @@ __global__ void __launch_bounds__(kPowerThreads) power_step_kernel(PowerArgs g, 
 // off-diagonals as h_ij = fp16(a_ij / (s_i s_j)) (|h_ij| <= 1 for a symmetric positive definite matrix) and, in FP32,
 // the diagonal d_i = a_ii + sum_j (a_ij - s_i s_j h_ij) over all 26 neighbours: the rounding of the off-diagonals
 // moves into the diagonal, so every row sum (and with it the near-null space of constants, on which the
-// preconditioner's quality rests) is that of the FP64 matrix.  A row then reads 28 + 8 bytes of coefficients
-// (the 13 off-diagonals padded to 7 pairs) instead of 56.
+// preconditioner's quality rests) is that of the FP64 matrix.  The V-cycle's sweeps work in the scaled variables
+// y = s x, b' = b / s, in which row i reads b'_i - e_i y_i - sum_j h_ij y_j with e_i = d_i / s_i^2: 28 + 4 bytes of
+// coefficients (the 13 off-diagonals padded to 7 pairs) instead of 56, and one load per neighbour.
 __device__ __forceinline__ _Float16 coeff16(double a, float si, float sj)
 {
   return (_Float16)(float)(a / ((double)si * (double)sj));
@@ -338,7 +386,8 @@ __device__ __forceinline__ _Float16 coeff16(double a, float si, float sj)
 
 __global__ void __launch_bounds__(256) half16_setup_kernel(Box bx, const double *__restrict__ A,
                                                            _Float16 *__restrict__ H, float *__restrict__ dg,
-                                                           float *__restrict__ sc)
+                                                           float *__restrict__ sc, float *__restrict__ eg,
+                                                           float *__restrict__ fg, int scaled_in)
 {
   const long n = bx.n();
   int I, J, K;
@@ -368,52 +417,28 @@ __global__ void __launch_bounds__(256) half16_setup_kernel(Box bx, const double 
     }
   }
   H[6 * 2 * n + 2 * i + 1] = 0;  // (the pad of the last pair)
-  dg[i] = (float)(A[13 * n + i] + comp);
+  const double dd = A[13 * n + i] + comp, s1 = (double)si;
+  dg[i] = (float)dd;
   sc[i] = si;
+  eg[i] = (float)(dd / (s1 * s1));
+  fg[i] = (float)((scaled_in ? s1 * s1 : s1) / dd);  // y = c f b is the first smoothing step from b' or (finest) b
 }
 
-// The FP16 products stage the scaled iterate s x of their block's neighbourhood in LDS: planes I-1..I+1, rows
-// J0-1..J0+kBY, columns K0-1..K0+kBX (zero outside the box), loaded once by the block (every load unconditional, at a
-// clamped index) instead of 26 loads of x and 26 of s per row; each row then reads its neighbours from the tile.
-constexpr int kTX = kBX + 2, kTY = kBY + 2, kTile = 3 * kTY * kTX, kTileIt = (kTile + kBX * kBY - 1) / (kBX * kBY);
-__device__ __forceinline__ void stage_scaled(const Box &bx, const float *__restrict__ sc, const float *__restrict__ x,
-                                             float *tile)
-{
-  const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
-  const long sy = bx.nz, sx = (long)bx.ny * bx.nz;
-  const int tid = threadIdx.y * kBX + threadIdx.x;
-  float v[kTileIt];
-#pragma unroll
-  for (int u = 0; u < kTileIt; u++) {
-    const int t = min(tid + u * kBX * kBY, kTile - 1);
-    const int p = t / (kTY * kTX), rem = t - p * (kTY * kTX), jj = rem / kTX, kk = rem - jj * kTX;
-    const int gi = I + p - 1, gj = J0 + jj - 1, gk = K0 + kk - 1;
-    const bool in = inside(bx, gi, gj, gk);
-    const long g = in ? gi * sx + gj * sy + gk : 0;
-    const float y = sc[g] * x[g];
-    v[u] = in ? y : 0.f;
-  }
-#pragma unroll
-  for (int u = 0; u < kTileIt; u++)
-    if (tid + u * kBX * kBY < kTile) tile[tid + u * kBX * kBY] = v[u];
-  __syncthreads();
-}
-
-// sum_j h_ij s_j x_j over the 26 neighbours of row i (the thread's row of the block), from the staged tile.  The
-// coefficients are stored as pairs of directions per row ([7][n] dwords, directions 14 + 2j and 15 + 2j, the last
-// pair padded): a row reads its 13 upper ones with 7 dword loads, and each lower one (the upper one of the lower
-// neighbour's row) with one, instead of 26 two-byte loads.  A neighbour outside the box has a zero tile entry; its
-// coefficient is read at a clamped index.
+// sum_j h_ij y_j over the 26 neighbours of row i, on plane q of the block's staged tile.  The coefficients are stored as
+// pairs of directions per row ([7][n] dwords, directions 14 + 2j and 15 + 2j, the last pair padded): a row reads its 13
+// upper ones with 7 dword loads, and each lower one (the upper one of the lower neighbour's row) with one, instead of
+// 26 two-byte loads.  A neighbour outside the box has a zero tile entry; its coefficient is read at a clamped index.
 __device__ __forceinline__ float half16_value(unsigned pair, int hi)
 {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(hi ? pair >> 16 : pair & 0xffffu));
 }
-__device__ __forceinline__ float half16_tile_row(const Box &bx, const _Float16 *__restrict__ H, const float *tile,
-                                                 long i)
+template <int BY>
+__device__ __forceinline__ float half16_row(const Box &bx, const _Float16 *__restrict__ H, const float *tile, int q,
+                                            int tj, int tk, long i)
 {
+  constexpr int TX = SweepTile<BY, 1>::TX, TY = SweepTile<BY, 1>::TY;
   const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz;
   const unsigned *__restrict__ H2 = (const unsigned *)H;
-  const int tj = threadIdx.y + 1, tk = threadIdx.x + 1;
   unsigned up[7];
 #pragma unroll
   for (int j = 0; j < 7; j++) up[j] = H2[j * n + i];
@@ -422,58 +447,81 @@ __device__ __forceinline__ float half16_tile_row(const Box &bx, const _Float16 *
   for (int s = 14; s < 27; s++) {
     const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
     const long off = di * sx + dj * sy + dk;
-    const long il = i - off >= 0 && i - off < n ? i - off : i;
+    const long il = i - off >= 0 ? i - off : i;
     const float hu = half16_value(up[(s - 14) >> 1], (s - 14) & 1);
     const float hl = half16_value(H2[((s - 14) >> 1) * n + il], (s - 14) & 1);
-    acc += hu * tile[((1 + di) * kTY + tj + dj) * kTX + tk + dk];
-    acc += hl * tile[((1 - di) * kTY + tj - dj) * kTX + tk - dk];
+    acc += hu * tile[((q + 1 + di) * TY + tj + dj) * TX + tk + dk];
+    acc += hl * tile[((q + 1 - di) * TY + tj - dj) * TX + tk - dk];
   }
   return acc;
 }
 
+// r = b - A x on the FP16 coefficients, in the caller's (unscaled) variables.
 __global__ void __launch_bounds__(256) half16_residual_kernel(Box bx, const _Float16 *__restrict__ H,
                                                               const float *__restrict__ dg, const float *__restrict__ sc,
                                                               const float *__restrict__ b, const float *__restrict__ x,
                                                               float *__restrict__ r)
 {
-  __shared__ float tile[kTile];
-  stage_scaled(bx, sc, x, tile);
-  int I, J, K;
-  long i;
-  if (!box_index(bx, I, J, K, i)) return;
-  const float ax = dg[i] * x[i] + sc[i] * half16_tile_row(bx, H, tile, i);
+  __shared__ float tile[SweepTile<kBY, 1>::N];
+  const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
+  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int, int, int) { return sc[g] * x[g]; });
+  const int J = J0 + threadIdx.y, K = K0 + threadIdx.x;
+  if (K >= bx.nz || J >= bx.ny) return;
+  const long i = ((long)I * bx.ny + J) * bx.nz + K;
+  const float ax = dg[i] * x[i] + sc[i] * half16_row<kBY>(bx, H, tile, 0, threadIdx.y + 1, threadIdx.x + 1, i);
   r[i] = (b ? b[i] : 0.f) - ax;
 }
 
-// One Chebyshev step of the smoother on the FP16 coefficients, out of place (Jacobi needs the old iterate at the
-// neighbours): dn = a d + c (b - A xin) / d_ii, xout = xin + dn; d is read when a != 0 and written when keep_d.
-__global__ void __launch_bounds__(256) half16_cheb_kernel(Box bx, const _Float16 *__restrict__ H,
-                                                          const float *__restrict__ dg, const float *__restrict__ sc,
-                                                          const float *__restrict__ b, const float *__restrict__ xin,
-                                                          float *__restrict__ xout, float *__restrict__ d, float a,
-                                                          float c, int keep_d)
+// The V-cycle's sweeps on the FP16 coefficients, in the scaled variables; the modes are half_sweep_kernel's.  The
+// residuals leave unscaled (the restriction works on them), and so does the last step of a level (unscale: x = y / s).
+// On the finest level b is the caller's (raw) in the _FIRST forms, which store b' = b / s in bs for the later sweeps.
+// 48 bytes a row instead of 56 and one staged load per neighbour instead of two (s and x): at 239^3 rows a smoothing step
+// 215 -> 165 us, and the first step and the pass that wrote it (55 us) are part of the second one.
+template <int MODE, int BY, int NR>
+__global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, const _Float16 *__restrict__ H,
+                                                               const float *__restrict__ e, const float *__restrict__ f,
+                                                               const float *__restrict__ s, const float *__restrict__ b,
+                                                               const float *__restrict__ y, float *__restrict__ out,
+                                                               float *__restrict__ d, float *__restrict__ y1,
+                                                               float *__restrict__ bs, float a, float c, float c1,
+                                                               int keep_d, int raw, int unscale, Box cb,
+                                                               const float *__restrict__ xc)
 {
-  __shared__ float tile[kTile];
-  stage_scaled(bx, sc, xin, tile);
-  int I, J, K;
-  long i;
-  if (!box_index(bx, I, J, K, i)) return;
-  const float xi = xin[i];
-  const float r = b[i] - (dg[i] * xi + sc[i] * half16_tile_row(bx, H, tile, i));
-  const float dn = (a != 0.f ? a * d[i] : 0.f) + c * r / dg[i];
-  if (keep_d) d[i] = dn;
-  xout[i] = xi + dn;
-}
-
-// First step from a zero iterate: x = d = c b / d_ii.
-__global__ void half16_cheb_first_kernel(long n, float c, const float *__restrict__ dg, const float *__restrict__ b,
-                                         float *__restrict__ x, float *__restrict__ d, int keep_d)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float dn = c * b[i] / dg[i];
-  if (keep_d) d[i] = dn;
-  x[i] = dn;
+  using S = SweepTile<BY, NR>;
+  constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID, PRO = MODE == SW_PRO_CHEB;
+  __shared__ float tile[S::N];
+  __shared__ float ct[PRO ? CoarseTile<BY, NR>::N : 1];
+  const int I0 = blockIdx.z * NR, J0 = blockIdx.y * BY, K0 = blockIdx.x * kBX;
+  if constexpr (PRO) stage_coarse<BY, NR>(cb, xc, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, ct);
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int gi, int gj, int gk) {
+    if constexpr (FIRST) return c1 * f[g] * b[g];
+    else if constexpr (PRO) return y[g] + s[g] * coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
+    else return y[g];
+  });
+  const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
+  if (K >= bx.nz || J >= bx.ny) return;
+#pragma unroll
+  for (int q = 0; q < NR; q++) {
+    const int I = I0 + q;
+    if (NR > 1 && I >= bx.nx) break;
+    const long i = ((long)I * bx.ny + J) * bx.nz + K;
+    const float ay = half16_row<BY>(bx, H, tile, q, tj, tk, i);
+    const float yi = tile[((q + 1) * S::TY + tj) * S::TX + tk], ei = e[i];
+    float bi = b[i];
+    if (FIRST && raw) {
+      bi /= s[i];
+      bs[i] = bi;
+    }
+    const float r = bi - (ei * yi + ay);
+    if constexpr (MODE == SW_RESID || MODE == SW_FIRST_RESID) {
+      if constexpr (FIRST) y1[i] = yi;
+      out[i] = s[i] * r;
+    } else {
+      const float dn = (MODE == SW_FIRST_CHEB ? a * yi : a != 0.f ? a * d[i] : 0.f) + c * r / ei;
+      if (keep_d) d[i] = dn;
+      out[i] = unscale ? (yi + dn) / s[i] : yi + dn;
+    }
+  }
 }
 
 __global__ void half_from_full_kernel(long n, const double *__restrict__ A, double *__restrict__ H,
@@ -494,24 +542,9 @@ __global__ void diag_inv_kernel(long n, const T *__restrict__ A, T *__restrict__
   if (r < n) dinv[r] = T(1) / A[13 * n + r];
 }
 
-// 1-D prolongation weights of fine index f onto coarse indices (at most two).
-__device__ __forceinline__ int parents(int f, int nc, int (&c)[2], double (&w)[2])
-{
-  if (f & 1) {
-    c[0] = (f - 1) >> 1;
-    w[0] = 1.0;
-    return c[0] < nc ? 1 : 0;
-  }
-  int m = 0;
-  const int lo = (f >> 1) - 1, hi = f >> 1;
-  if (lo >= 0 && lo < nc) { c[m] = lo; w[m] = 0.5; m++; }
-  if (hi >= 0 && hi < nc) { c[m] = hi; w[m] = 0.5; m++; }
-  return m;
-}
-
-// bc = P^T rf
+// bc = P^T rf, divided by the coarse level's row scales s (null: not)
 template <typename T>
-__global__ void restrict_kernel(Box f, Box c, const T *__restrict__ rf, T *__restrict__ bc)
+__global__ void restrict_kernel(Box f, Box c, const T *__restrict__ rf, T *__restrict__ bc, const T *__restrict__ s)
 {
   int I, J, K;
   long C;
@@ -531,43 +564,7 @@ __global__ void restrict_kernel(Box f, Box c, const T *__restrict__ rf, T *__res
         const T v = w * rf[in ? base + a * sx + b * sy + d : base];  // unconditional load, dropped by a select
         acc += in ? v : T(0);
       }
-  bc[C] = acc;
-}
-
-// The two coarse parents of fine index f in one direction with their weights; a missing parent has weight 0 and
-// index 0, so that prolongations load unconditionally (nc >= 1).
-__device__ __forceinline__ void parents2(int f, int nc, int (&c)[2], float (&w)[2])
-{
-  int cc[2];
-  double ww[2];
-  const int m = parents(f, nc, cc, ww);
-  c[0] = m > 0 ? cc[0] : 0;
-  w[0] = m > 0 ? (float)ww[0] : 0.f;
-  c[1] = m > 1 ? cc[1] : 0;
-  w[1] = m > 1 ? (float)ww[1] : 0.f;
-}
-
-// xout = xin + P xc (xout may be xin: the smoothers' iterate alternates between two buffers)
-template <typename T>
-__global__ void prolong_kernel(Box f, Box c, const T *__restrict__ xc, const T *xin, T *xout)
-{
-  int I, J, K;
-  long F;
-  if (!box_index(f, I, J, K, F)) return;
-  int ci[2], cj[2], ck[2];
-  float wi[2], wj[2], wk[2];  // 0, 1/2 or 1: their products are exact in either precision
-  parents2(I, c.nx, ci, wi);
-  parents2(J, c.ny, cj, wj);
-  parents2(K, c.nz, ck, wk);
-  T acc = 0;
-#pragma unroll
-  for (int a = 0; a < 2; a++)
-#pragma unroll
-    for (int b = 0; b < 2; b++)
-#pragma unroll
-      for (int d = 0; d < 2; d++)
-        acc += T(wi[a] * wj[b] * wk[d]) * xc[((long)ci[a] * c.ny + cj[b]) * c.nz + ck[d]];
-  xout[F] = xin[F] + acc;
+  bc[C] = s ? acc / s[C] : acc;
 }
 
 // 1-D prolongation weight of the coarse node at offset t (in -1..1) from coarse node c at the fine node at offset e
@@ -758,8 +755,10 @@ struct MGLevel {
   const double *A64 = nullptr;  // full 27-point stencil (finest level: the Q1 matrix's own)
   DevBuf<double> own64, H64, dinv64, b64, x64, r64, d64;  // H: symmetric half stencil [14][n]
   DevBuf<float> H32, dinv32, b32, x32, r32, d32;
-  DevBuf<_Float16> H16;        // FP16 upper off-diagonals, pairs of directions per row [7][n][2] (half16_tile_row)
-  DevBuf<float> dg16, sc16, t32;  // their diagonal and row scales; the second iterate buffer of the FP16 V-cycle
+  DevBuf<_Float16> H16;        // FP16 upper off-diagonals, pairs of directions per row [7][n][2] (half16_row)
+  DevBuf<float> dg16, sc16;    // their diagonal d and row scales s
+  DevBuf<float> e16, f16;      // d / s^2; the first smoothing step's factor (half16_setup_kernel)
+  DevBuf<float> t32;           // finest level: the scaled right-hand side
   double lmax = 0;
 };
 
@@ -935,9 +934,9 @@ struct ChebCoeffs {
   }
 };
 
-// The V-cycle at level l.  The smoothers' steps move the iterate between x and the level's residual vector: the first
-// two pre-smoothing steps from zero are one sweep (at degree 1 the first step and the residual are), and the
-// prolongation writes into the buffer from which the post-smoother's steps end in x.
+// The V-cycle at level l.  The first two pre-smoothing steps from zero are one sweep (at degree 1 the first step and the
+// residual are), and the first post-smoothing step takes the prolongation.  Every later step moves the iterate between x
+// and the level's residual vector; it starts where the moves end in x.
 template <typename T>
 void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
 {
@@ -951,6 +950,7 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
   MGLevel &cv = mg->L[l + 1];
   const T *H = P::A(lv), *dinv = P::dinv(lv);
   T *d = P::d(lv), *cur = x, *other = P::r(lv);
+  if (mg->degree == 1) std::swap(cur, other);
   double a, c, c1;
   ChebCoeffs pre(mg, lv);
   pre.step(0, a, c1);
@@ -969,51 +969,42 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
     }
     residual<T>(lv.box, H, b, cur, other, st);
   }
-  hipLaunchKernelGGL(restrict_kernel<T>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, P::b(cv));
+  hipLaunchKernelGGL(restrict_kernel<T>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, P::b(cv),
+                     nullptr);
   vcycle<T>(mg, l + 1, P::b(cv), P::x(cv), st);
-  T *start = mg->degree % 2 == 0 ? x : P::r(lv);
-  hipLaunchKernelGGL(prolong_kernel<T>, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, P::x(cv), cur, start);
-  cur = start;
-  other = start == x ? P::r(lv) : x;
   ChebCoeffs post(mg, lv);
   for (int k = 0; k < mg->degree; k++) {
     post.step(k, a, c);
-    sweep<T, SW_CHEB>(lv.box, H, dinv, b, cur, other, d, nullptr, (T)a, (T)c, T(0), k + 1 < mg->degree, st);
+    const int keep_d = k + 1 < mg->degree;
+    if (k == 0)
+      sweep<T, SW_PRO_CHEB>(lv.box, H, dinv, b, cur, other, d, nullptr, (T)a, (T)c, T(0), keep_d, st, cv.box, P::x(cv));
+    else
+      sweep<T, SW_CHEB>(lv.box, H, dinv, b, cur, other, d, nullptr, (T)a, (T)c, T(0), keep_d, st);
     std::swap(cur, other);
   }
 }
 
-// The FP32 smoother on the FP16 coefficients: Chebyshev steps alternate the iterate between cur and other (zero_init:
-// cur is first set from b).  Returns the buffer that holds the result.
-float *smooth16(const _p_dohpMG *mg, MGLevel &lv, const float *b, float *cur, float *other, bool zero_init,
-                hipStream_t st)
+// The tile of the FP16 sweeps: two planes of 64 x 4 rows from 8 million rows on, where the level's 48 bytes a row
+// (384 MB) stream from HBM and the fewer staged loads show (239^3: 162 against 166 us, 207^3: 115 against 118), one plane
+// below, where the level lives in the 256 MB cache (191^3: 78 against 82 us, 95^3: 15.0 against 15.6).
+template <int MODE>
+void sweep16(const MGLevel &lv, const float *b, const float *y, float *out, float *y1, double a, double c, double c1,
+             int keep_d, int raw, int unscale, hipStream_t st, const Box &cb = Box{}, const float *xc = nullptr)
 {
-  const double lmin = mg->lo * lv.lmax, lmaxs = mg->hi * lv.lmax;
-  const double theta = 0.5 * (lmaxs + lmin), delta = 0.5 * (lmaxs - lmin), sigma = theta / delta;
-  double rho = 1.0 / sigma;
-  const int keep_d = mg->degree > 1;
-  if (zero_init) {
-    hipLaunchKernelGGL(half16_cheb_first_kernel, grid_of(lv.n), dim3(256), 0, st, lv.n, (float)(1.0 / theta),
-                       lv.dg16.ptr, b, cur, lv.d32.ptr, keep_d);
-  } else {
-    hipLaunchKernelGGL(half16_cheb_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.H16.ptr, lv.dg16.ptr,
-                       lv.sc16.ptr, b, cur, other, lv.d32.ptr, 0.f, (float)(1.0 / theta), keep_d);
-    std::swap(cur, other);
-  }
-  for (int k = 1; k < mg->degree; k++) {
-    const double rho_new = 1.0 / (2.0 * sigma - rho);
-    hipLaunchKernelGGL(half16_cheb_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.H16.ptr, lv.dg16.ptr,
-                       lv.sc16.ptr, b, cur, other, lv.d32.ptr, (float)(rho_new * rho), (float)(2.0 * rho_new / delta),
-                       keep_d);
-    std::swap(cur, other);
-    rho = rho_new;
-  }
-  return cur;
+  const Box &bx = lv.box;
+  const unsigned gx = (bx.nz + kBX - 1) / kBX, gy = (bx.ny + 3) / 4;
+  if (lv.n >= 8000000)
+    hipLaunchKernelGGL((half16_sweep_kernel<MODE, 4, 2>), dim3(gx, gy, (bx.nx + 1) / 2), dim3(kBX, 4), 0, st, bx,
+                       lv.H16.ptr, lv.e16.ptr, lv.f16.ptr, lv.sc16.ptr, b, y, out, lv.d32.ptr, y1, lv.t32.ptr,
+                       (float)a, (float)c, (float)c1, keep_d, raw, unscale, cb, xc);
+  else
+    hipLaunchKernelGGL((half16_sweep_kernel<MODE, 4, 1>), dim3(gx, gy, bx.nx), dim3(kBX, 4), 0, st, bx, lv.H16.ptr,
+                       lv.e16.ptr, lv.f16.ptr, lv.sc16.ptr, b, y, out, lv.d32.ptr, y1, lv.t32.ptr, (float)a, (float)c,
+                       (float)c1, keep_d, raw, unscale, cb, xc);
 }
 
-// FP32 V-cycle on the FP16 coefficients.  The iterate alternates between x and the level's second buffer: the
-// pre-smoother's steps, the prolongation and the post-smoother's steps make an even number of moves, so the result
-// ends in x.
+// FP32 V-cycle on the FP16 coefficients, in the scaled variables: b is b' on the coarse levels (the restriction scales
+// it) and the caller's on the finest; the result x is unscaled on every level.  Steps and buffers as in vcycle.
 void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
 {
   MGLevel &lv = mg->L[l];
@@ -1023,18 +1014,41 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
     return;
   }
   MGLevel &cv = mg->L[l + 1];
-  float *cur = smooth16(mg, lv, b, x, lv.t32.ptr, true, st);
-  hipLaunchKernelGGL(half16_residual_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.H16.ptr, lv.dg16.ptr,
-                     lv.sc16.ptr, b, cur, lv.r32.ptr);
-  hipLaunchKernelGGL(restrict_kernel<float>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, lv.r32.ptr,
-                     cv.b32.ptr);
+  const int raw = l == 0;
+  const float *bs = raw ? lv.t32.ptr : b;
+  float *cur = x, *other = lv.r32.ptr;
+  if (mg->degree == 1) std::swap(cur, other);
+  double a, c, c1;
+  ChebCoeffs pre(mg, lv);
+  pre.step(0, a, c1);
+  if (mg->degree == 1) {
+    sweep16<SW_FIRST_RESID>(lv, b, nullptr, other, cur, 0, 0, c1, 0, raw, 0, st);
+  } else {
+    for (int k = 1; k < mg->degree; k++) {
+      pre.step(k, a, c);
+      const int keep_d = k + 1 < mg->degree;
+      if (k == 1) {
+        sweep16<SW_FIRST_CHEB>(lv, b, nullptr, cur, nullptr, a, c, c1, keep_d, raw, 0, st);
+      } else {
+        sweep16<SW_CHEB>(lv, bs, cur, other, nullptr, a, c, 0, keep_d, 0, 0, st);
+        std::swap(cur, other);
+      }
+    }
+    sweep16<SW_RESID>(lv, bs, cur, other, nullptr, 0, 0, 0, 0, 0, 0, st);
+  }
+  hipLaunchKernelGGL(restrict_kernel<float>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, cv.b32.ptr,
+                     l + 2 < mg->L.size() ? cv.sc16.ptr : nullptr);
   vcycle16(mg, l + 1, cv.b32.ptr, cv.x32.ptr, st);
-  float *other = cur == x ? lv.t32.ptr : x;
-  hipLaunchKernelGGL(prolong_kernel<float>, box_grid(lv.box), box_block(), 0, st, lv.box, cv.box, cv.x32.ptr, cur,
-                     other);
-  cur = smooth16(mg, lv, b, other, cur, false, st);
-  if (cur != x)  // (not reached: the moves are even)
-    (void)hipMemcpyAsync(x, cur, sizeof(float) * lv.n, hipMemcpyDeviceToDevice, st);
+  ChebCoeffs post(mg, lv);
+  for (int k = 0; k < mg->degree; k++) {
+    post.step(k, a, c);
+    const int last = k + 1 == mg->degree;
+    if (k == 0)
+      sweep16<SW_PRO_CHEB>(lv, bs, cur, other, nullptr, a, c, 0, !last, 0, last, st, cv.box, cv.x32.ptr);
+    else
+      sweep16<SW_CHEB>(lv, bs, cur, other, nullptr, a, c, 0, !last, 0, last, st);
+    std::swap(cur, other);
+  }
 }
 
 }  // namespace
@@ -1057,7 +1071,7 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
     hipLaunchKernelGGL(half_from_full_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.H64.ptr, lv.H32.ptr);
     if (l + 1 < mg->L.size())
       hipLaunchKernelGGL(half16_setup_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.A64, lv.H16.ptr,
-                         lv.dg16.ptr, lv.sc16.ptr);
+                         lv.dg16.ptr, lv.sc16.ptr, lv.e16.ptr, lv.f16.ptr, l > 0);
     hipLaunchKernelGGL(diag_inv_kernel<double>, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.dinv64.ptr);
     hipLaunchKernelGGL(to_f32<float>, grid_of(n), dim3(256), 0, st, n, lv.dinv64.ptr, lv.dinv32.ptr);
   }
@@ -1125,7 +1139,9 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
     if (!err && l + 1 < mg->L.size()) err = lv.H16.alloc(14 * n);
     if (!err && l + 1 < mg->L.size()) err = lv.dg16.alloc(n);
     if (!err && l + 1 < mg->L.size()) err = lv.sc16.alloc(n);
-    if (!err && l + 1 < mg->L.size()) err = lv.t32.alloc(n);
+    if (!err && l + 1 < mg->L.size()) err = lv.e16.alloc(n);
+    if (!err && l + 1 < mg->L.size()) err = lv.f16.alloc(n);
+    if (!err && l == 0 && mg->L.size() > 1) err = lv.t32.alloc(n);
   }
   if (!err) err = mg_fill(mg, st);
   if (err) {
