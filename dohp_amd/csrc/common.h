@@ -204,6 +204,11 @@ extern "C" dErr dohpEllipFunctionState_Private(dohpEllip op, const double *u, hi
 // y = J x without the entry points' non-finite check (no wait for the stream): the library's solvers.
 dErr dohpEllipMatMult_Private(dohpEllip op, const double *x, double *y, hipStream_t st);
 dErr dohpEllipMatMult_Private(dohpEllip op, const float *x, float *y, hipStream_t st);
+// y += J x, unchecked, for a y that the caller has cleared (either scatter).
+dErr dohpEllipMatMultAdd_Private(dohpEllip op, const double *x, double *y, hipStream_t st);
+dErr dohpEllipMatMultAdd_Private(dohpEllip op, const float *x, float *y, hipStream_t st);
+// Eight pinned doubles of the operator (host and device address) that its solver's kernels write scalars to.
+dErr dohpEllipPinned_Private(dohpEllip op, double **host, double **dev);
 // The operator's pool of solver work vectors.
 dohp::Pool *dohpEllipPool_Private(dohpEllip op);
 

@@ -407,6 +407,7 @@ struct _p_dohpEllip {
   // vector or the state); the checked entry points clear it, wait for their stream and read it back
   DevBuf<int> nanflag;
   int *nan_host = nullptr;  // pinned
+  double *scal_host = nullptr;  // pinned: scalars of the solves on this operator
   int checks = 1;
   const float *q1_cscale = nullptr;  // learned sub-cell derivative scales of later Q1 assemblies (caller's array)
   // host tables
@@ -414,6 +415,7 @@ struct _p_dohpEllip {
   ~_p_dohpEllip()
   {
     if (nan_host) (void)hipHostFree(nan_host);
+    if (scal_host) (void)hipHostFree(scal_host);
   }
 };
 
@@ -752,6 +754,11 @@ extern "C" dErr dohpEllipCreate(dohpFS fs, const dohpEllipParam *prm, dohpEllip 
     set_error("pinned allocation failed");
     err = dohpERR_OOM;
   }
+  if (!err && hipHostMalloc((void **)&op->scal_host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    op->scal_host = nullptr;
+    set_error("pinned allocation failed");
+    err = dohpERR_OOM;
+  }
   if (err) {
     delete op;
     return err;
@@ -1006,6 +1013,23 @@ dErr dohpEllipMatMult_Private(dohpEllip op, const float *x, float *y, hipStream_
 {
   DOHP_CALL(zero(y, op->fs->nowned, st));
   return apply_add(op, x, y, st);
+}
+dErr dohpEllipMatMultAdd_Private(dohpEllip op, const double *x, double *y, hipStream_t st)
+{
+  return apply_add(op, x, y, st);
+}
+dErr dohpEllipMatMultAdd_Private(dohpEllip op, const float *x, float *y, hipStream_t st)
+{
+  return apply_add(op, x, y, st);
+}
+
+dErr dohpEllipPinned_Private(dohpEllip op, double **host, double **dev)
+{
+  *host = op->scal_host;
+  void *p = nullptr;
+  DOHP_HIP(hipHostGetDevicePointer(&p, op->scal_host, 0));
+  *dev = (double *)p;
+  return 0;
 }
 
 extern "C" dErr dohpEllipShellMatMult(dohpEllip op, const double *x, double *y, void *stream)

@@ -25,7 +25,7 @@ extern "C" dErr dohpEllipGetQ1Context_Private(dohpEllip op, dohpFS *fs, dohpElli
 
 namespace {
 
-constexpr int kRedBlocks = 1024;
+constexpr int kRedBlocks = 2048;  // blocks of a reduction (one partial sum each): eight per compute unit
 
 template <typename T>
 __global__ void dot_partial_kernel(long n, const T *__restrict__ a, const T *__restrict__ b, double *__restrict__ part)
@@ -100,10 +100,135 @@ __global__ void promote_add_kernel(long n, double s, const float *__restrict__ y
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] += s * (double)y[i];
 }
-__global__ void promote_kernel(long n, const float *__restrict__ y, double *__restrict__ x)
+
+// ---- CG's vector work, fused.  An iteration's scalars stay on the device: a kernel that needs one sums the partial
+// sums that the previous kernel left (kRedBlocks of them, in a fixed order, once per workgroup), and only ||r||^2 goes to
+// the host, which reads it while the preconditioner already runs.  Per iteration (FP64 CG, FP32 preconditioner) 58 bytes
+// a row in four launches and one wait instead of 96 in eleven launches and four waits.
+__device__ __forceinline__ double sum_block(double s, double *sh)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = (double)y[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  const double r = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  __syncthreads();
+  return r;
+}
+__device__ __forceinline__ double sum_partials(const double *__restrict__ part, double *sh)
+{
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < kRedBlocks / 256; i++) s += part[i * 256 + threadIdx.x];
+  return sum_block(s, sh);
+}
+
+// r = b - q (and its FP32 copy if lr is not null), partial sums of b.b and r.r
+template <typename T>
+__global__ void __launch_bounds__(256) krylov_init_kernel(long n, const T *__restrict__ b, const T *__restrict__ q,
+                                                          T *__restrict__ r, float *__restrict__ lr,
+                                                          double *__restrict__ part_bb, double *__restrict__ part_rr)
+{
+  __shared__ double sh[4];
+  double sb = 0.0, sr = 0.0;
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    const T bi = b[i], ri = bi - q[i];
+    r[i] = ri;
+    if (lr) lr[i] = (float)ri;
+    sb += (double)bi * (double)bi;
+    sr += (double)ri * (double)ri;
+  }
+  const double tb = sum_block(sb, sh), tr = sum_block(sr, sh);
+  if (threadIdx.x == 0) {
+    part_bb[blockIdx.x] = tb;
+    part_rr[blockIdx.x] = tr;
+  }
+}
+
+// host[j] = sum of the j-th array of partial sums (host: pinned memory, read by the host after the kernel has ended)
+__global__ void __launch_bounds__(256) krylov_read_kernel(const double *__restrict__ part, int m,
+                                                          double *__restrict__ host)
+{
+  __shared__ double sh[4];
+  for (int j = 0; j < m; j++) {
+    const double t = sum_partials(part + (long)j * kRedBlocks, sh);
+    if (threadIdx.x == 0) host[j] = t;
+  }
+}
+
+// alpha = rz / p.q;  x += alpha p;  r -= alpha q (and its FP32 copy), partial sums of r.r
+template <typename T>
+__global__ void __launch_bounds__(256) krylov_update_kernel(long n, const double *__restrict__ part_pq,
+                                                            const double *__restrict__ rz, double *__restrict__ alpha,
+                                                            const T *__restrict__ p, const T *__restrict__ q,
+                                                            T *__restrict__ x, T *__restrict__ r,
+                                                            float *__restrict__ lr, double *__restrict__ part_rr)
+{
+  __shared__ double sh[4];
+  const double al = rz[0] / sum_partials(part_pq, sh);
+  const T a = (T)al;
+  double s = 0.0;
+#pragma unroll 2
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    x[i] = a * p[i] + x[i];
+    const T ri = -a * q[i] + r[i];
+    r[i] = ri;
+    if (lr) lr[i] = (float)ri;
+    s += (double)ri * (double)ri;
+  }
+  const double t = sum_block(s, sh);
+  if (threadIdx.x == 0) {
+    part_rr[blockIdx.x] = t;
+    if (blockIdx.x == 0) alpha[0] = al;
+  }
+}
+
+// partial sums of r.z and, if q is not null, of z.q
+template <typename T, typename Z>
+__global__ void __launch_bounds__(256) krylov_zdots_kernel(long n, const T *__restrict__ r, const Z *__restrict__ z,
+                                                           const T *__restrict__ q, double *__restrict__ part_rz,
+                                                           double *__restrict__ part_zq)
+{
+  __shared__ double sh[4];
+  double s0 = 0.0, s1 = 0.0;
+#pragma unroll 2
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    const double zi = (double)z[i];
+    s0 += (double)r[i] * zi;
+    if (q) s1 += zi * (double)q[i];
+  }
+  const double t0 = sum_block(s0, sh), t1 = sum_block(s1, sh);
+  if (threadIdx.x == 0) {
+    part_rz[blockIdx.x] = t0;
+    part_zq[blockIdx.x] = t1;
+  }
+}
+
+// rz_new = r.z;  p = z + beta p with beta = rz_new / rz (mode KB_STANDARD), -alpha z.q / rz (KB_FLEXIBLE) or 0
+// (KB_FIRST: p = z, p is not read);  q = 0 for the operator's scatter
+enum { KB_FIRST, KB_STANDARD, KB_FLEXIBLE };
+template <typename T, typename Z>
+__global__ void __launch_bounds__(256) krylov_direction_kernel(long n, int mode, const double *__restrict__ part_rz,
+                                                               const double *__restrict__ part_zq,
+                                                               const double *__restrict__ rz,
+                                                               double *__restrict__ rz_new,
+                                                               const double *__restrict__ alpha,
+                                                               const Z *__restrict__ z, T *__restrict__ p,
+                                                               T *__restrict__ q)
+{
+  __shared__ double sh[4];
+  const double rzn = sum_partials(part_rz, sh);
+  double beta = 0.0;
+  if (mode == KB_STANDARD) beta = rzn / rz[0];
+  if (mode == KB_FLEXIBLE) beta = -alpha[0] * sum_partials(part_zq, sh) / rz[0];
+  const T be = (T)beta;
+#pragma unroll 2
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += 256L * gridDim.x) {
+    const T zi = (T)z[i];
+    p[i] = mode == KB_FIRST ? zi : zi + be * p[i];
+    q[i] = T(0);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) rz_new[0] = rzn;
 }
 
 inline dim3 grid(long n) { return dim3((n + 255) / 256); }
@@ -113,6 +238,16 @@ struct Ctx {
   long n;
   Pool *pool;  // the operator's: every work vector of a solve comes from it
   PoolBuf<double> part, res;
+  double *host = nullptr;  // pinned scalars of the operator, and their device address
+  double *host_dev = nullptr;
+};
+
+struct Event {
+  hipEvent_t e = nullptr;
+  ~Event()
+  {
+    if (e) (void)hipEventDestroy(e);
+  }
 };
 
 template <typename T>
@@ -139,11 +274,13 @@ struct Ops;
 template <>
 struct Ops<double> {
   static dErr A(dohpEllip op, const double *x, double *y, hipStream_t s) { return dohpEllipMatMult_Private(op, x, y, s); }
+  static dErr A_add(dohpEllip op, const double *x, double *y, hipStream_t s) { return dohpEllipMatMultAdd_Private(op, x, y, s); }
   static dErr Q(dohpMat m, const double *x, double *y, hipStream_t s) { return dohpMatMult(m, x, y, s); }
 };
 template <>
 struct Ops<float> {
   static dErr A(dohpEllip op, const float *x, float *y, hipStream_t s) { return dohpEllipMatMult_Private(op, x, y, s); }
+  static dErr A_add(dohpEllip op, const float *x, float *y, hipStream_t s) { return dohpEllipMatMultAdd_Private(op, x, y, s); }
   static dErr Q(dohpMat m, const float *x, float *y, hipStream_t s) { return dohpMatMultF32(m, x, y, s); }
 };
 
@@ -155,6 +292,12 @@ struct Cheb {
   double lmin, lmax;
   int degree;
   PoolBuf<T> res, d, w;
+  dErr alloc(Ctx &c)
+  {
+    DOHP_CALL(res.alloc(*c.pool, c.n));
+    DOHP_CALL(d.alloc(*c.pool, c.n));
+    return w.alloc(*c.pool, c.n);
+  }
   dErr apply(Ctx &c, const T *r, T *z)
   {
     const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin), sigma = theta / delta;
@@ -186,8 +329,7 @@ __global__ void scale2_kernel(long n, const double *__restrict__ s, const void *
 }
 
 // Preconditioner of one precision: Jacobi-Chebyshev on the Q1 matrix, or a multigrid V-cycle on
-// it, optionally corrected by learned node weights, z = S M(S r).  An FP64 preconditioner may hand
-// the work to an FP32 one (low): r is rounded to FP32, z comes back exactly.
+// it, optionally corrected by learned node weights, z = S M(S r).
 template <typename T>
 struct Prec {
   Cheb<T> *cheb = nullptr;
@@ -196,8 +338,6 @@ struct Prec {
   const double *s = nullptr;  // learned node weights, or null
   T *tmp = nullptr;
   bool learned_on = false;
-  Prec<float> *low = nullptr;
-  float *lr = nullptr, *lz = nullptr;
   dErr apply(Ctx &c, const T *r, T *z);
 };
 template <typename T>
@@ -209,15 +349,6 @@ dErr mg_apply<float>(dohpMG mg, const float *r, float *z, hipStream_t st) { retu
 template <typename T>
 dErr Prec<T>::apply(Ctx &c, const T *r, T *z)
 {
-  if constexpr (sizeof(T) == 8) {
-    if (low) {
-      hipLaunchKernelGGL(demote_kernel, grid(c.n), dim3(256), 0, c.st, c.n, 1.0, r, lr);
-      DOHP_CALL(low->apply(c, lr, lz));
-      hipLaunchKernelGGL(promote_kernel, grid(c.n), dim3(256), 0, c.st, c.n, lz, z);
-      DOHP_HIP(hipGetLastError());
-      return 0;
-    }
-  }
   if (!mg) return cheb->apply(c, r, z);
   if (mg_fb && !learned_on) return mg_apply<T>(mg_fb, r, z, c.st);
   if (!(s && learned_on)) return mg_apply<T>(mg, r, z, c.st);
@@ -273,51 +404,79 @@ dErr estimate_lmax(Ctx &c, dohpMat q1, const double *dinv, int its, double *lmax
 // dot product), equal to the usual z_{k+1}.r_{k+1} / z_k.r_k when the preconditioner is symmetric and exact, and
 // robust when it is not: an FP32 V-cycle inside FP64 CG is symmetric only to FP32 rounding, which on the reference
 // arithmetic's matrix at 48^3, p = 6 sometimes doubled the iteration count (91 -> 193).
-template <typename T>
-dErr pcg(Ctx &c, dohpEllip op, Prec<T> &M, Budget &bud, const T *b, T *x, double rtol, int max_it, int *its,
+// The preconditioner works on Z vectors: with Z = float inside FP64 CG, r is rounded to FP32 and z used exactly.
+// The preconditioner of the next iteration is launched before ||r|| is known while the last known ||r|| is more than
+// four times the tolerance (the wait is hidden behind it; were it the last iteration, one application is for nothing).
+template <typename T, typename Z>
+dErr pcg(Ctx &c, dohpEllip op, Prec<Z> &M, Budget &bud, const T *b, T *x, double rtol, int max_it, int *its,
          double *rnorm, double *bnorm, T *snap = nullptr, int nsnap = 0, int every = 0, int *nsnapped = nullptr,
          bool flexible = false)
 {
-  PoolBuf<T> r, z, p, q;
+  constexpr bool LOW = sizeof(Z) < sizeof(T);
+  PoolBuf<T> r, p, q;
+  PoolBuf<Z> z, lr;
+  PoolBuf<double> part, sc;
   DOHP_CALL(r.alloc(*c.pool, c.n));
-  DOHP_CALL(z.alloc(*c.pool, c.n));
   DOHP_CALL(p.alloc(*c.pool, c.n));
   DOHP_CALL(q.alloc(*c.pool, c.n));
+  DOHP_CALL(z.alloc(*c.pool, c.n));
+  if (LOW) DOHP_CALL(lr.alloc(*c.pool, c.n));
+  DOHP_CALL(part.alloc(*c.pool, 4 * kRedBlocks));
+  DOHP_CALL(sc.alloc(*c.pool, 3));
+  double *part_pq = part.ptr, *part_rr = part_pq + kRedBlocks, *part_rz = part_rr + kRedBlocks,
+         *part_zq = part_rz + kRedBlocks, *alpha = sc.ptr + 2;
+  const dim3 red(kRedBlocks), bs(256);
+  float *lrp = LOW ? (float *)lr.ptr : nullptr;
+  Event ev;
+  DOHP_HIP(hipEventCreateWithFlags(&ev.e, hipEventDisableTiming));
   DOHP_CALL(Ops<T>::A(op, x, q.ptr, c.st));
-  DOHP_HIP(hipMemcpyAsync(r.ptr, b, sizeof(T) * c.n, hipMemcpyDeviceToDevice, c.st));
-  DOHP_CALL(axpby<T>(c, T(-1), q.ptr, T(1), r.ptr));
-  double bb, rr;
-  DOHP_CALL(dot(c, b, b, &bb));
-  DOHP_CALL(dot(c, r.ptr, r.ptr, &rr));
+  hipLaunchKernelGGL(krylov_init_kernel<T>, red, bs, 0, c.st, c.n, b, q.ptr, r.ptr, lrp, part_pq, part_rr);
+  hipLaunchKernelGGL(krylov_read_kernel, dim3(1), bs, 0, c.st, part_pq, 2, c.host_dev);
+  DOHP_HIP(hipStreamSynchronize(c.st));
+  const double bb = c.host[0];
+  double rr = c.host[1];
   *bnorm = std::sqrt(bb);
   DOHP_CHECK(std::isfinite(bb) && std::isfinite(rr), dohpERR_NAN, "PCG: non-finite right-hand side or initial residual");
   const double tol = rtol * std::sqrt(bb);
   int k = 0, ns = 0;
-  double rz = 0, alpha = 0;
   bool restart = false;
+  auto switches = [&](int used) { return M.learned_on && bud.fallback_its > 0 && used >= bud.fallback_its; };
   auto precondition = [&]() -> dErr {
-    bool &learned_on = M.low ? M.low->learned_on : M.learned_on;
-    if (learned_on && bud.fallback_its > 0 && bud.used >= bud.fallback_its) {
-      learned_on = false;
+    if (switches(bud.used)) {
+      M.learned_on = false;
       bud.fell_back = 1;
       restart = true;
     }
-    return M.apply(c, r.ptr, z.ptr);
+    if constexpr (LOW) return M.apply(c, lr.ptr, z.ptr);
+    else return M.apply(c, r.ptr, z.ptr);
   };
-  if (std::sqrt(rr) > tol) {
+  // p and r.z of the next iteration from z (k counts the slots of r.z, which alternate)
+  auto direction = [&](int mode) -> dErr {
+    const T *qz = mode == KB_FLEXIBLE ? q.ptr : nullptr;
+    hipLaunchKernelGGL((krylov_zdots_kernel<T, Z>), red, bs, 0, c.st, c.n, r.ptr, z.ptr, qz, part_rz, part_zq);
+    hipLaunchKernelGGL((krylov_direction_kernel<T, Z>), red, bs, 0, c.st, c.n, mode, part_rz, part_zq,
+                       sc.ptr + ((k + 1) & 1), sc.ptr + (k & 1), alpha, z.ptr, p.ptr, q.ptr);
+    DOHP_HIP(hipGetLastError());
+    return 0;
+  };
+  if (std::sqrt(rr) > tol && max_it > 0) {
     DOHP_CALL(precondition());
     restart = false;
-    DOHP_HIP(hipMemcpyAsync(p.ptr, z.ptr, sizeof(T) * c.n, hipMemcpyDeviceToDevice, c.st));
-    DOHP_CALL(dot(c, r.ptr, z.ptr, &rz));
+    DOHP_CALL(direction(KB_FIRST));
   }
   while (std::sqrt(rr) > tol && k < max_it) {
-    DOHP_CALL(Ops<T>::A(op, p.ptr, q.ptr, c.st));
-    double pq;
-    DOHP_CALL(dot(c, p.ptr, q.ptr, &pq));
-    alpha = rz / pq;
-    DOHP_CALL(axpby<T>(c, (T)alpha, p.ptr, T(1), x));
-    DOHP_CALL(axpby<T>(c, (T)-alpha, q.ptr, T(1), r.ptr));
-    DOHP_CALL(dot(c, r.ptr, r.ptr, &rr));
+    DOHP_CALL(Ops<T>::A_add(op, p.ptr, q.ptr, c.st));  // (q is zero)
+    hipLaunchKernelGGL(dot_partial_kernel<T>, red, bs, 0, c.st, c.n, p.ptr, q.ptr, part_pq);
+    hipLaunchKernelGGL(krylov_update_kernel<T>, red, bs, 0, c.st, c.n, part_pq, sc.ptr + (k & 1), alpha, p.ptr, q.ptr, x,
+                       r.ptr, lrp, part_rr);
+    hipLaunchKernelGGL(krylov_read_kernel, dim3(1), bs, 0, c.st, part_rr, 1, c.host_dev);
+    DOHP_HIP(hipGetLastError());
+    DOHP_HIP(hipEventRecord(ev.e, c.st));
+    const bool ahead = std::sqrt(rr) > 4 * tol && k + 1 < max_it && !switches(bud.used + 1);
+    if (ahead) DOHP_CALL(precondition());
+    DOHP_HIP(hipEventSynchronize(ev.e));
+    rr = c.host[0];
+    if (!std::isfinite(rr)) DOHP_HIP(hipStreamSynchronize(c.st));  // (the work vectors go back to the pool)
     DOHP_CHECK(std::isfinite(rr), dohpERR_NAN, "PCG: non-finite residual at iteration " + std::to_string(k + 1));
     k++;
     bud.used++;
@@ -325,23 +484,11 @@ dErr pcg(Ctx &c, dohpEllip op, Prec<T> &M, Budget &bud, const T *b, T *x, double
       DOHP_HIP(hipMemcpyAsync(snap + (long)ns * c.n, x, sizeof(T) * c.n, hipMemcpyDeviceToDevice, c.st));
       ns++;
     }
-    if (std::sqrt(rr) <= tol) break;
-    DOHP_CALL(precondition());
-    double rz_new;
-    DOHP_CALL(dot(c, r.ptr, z.ptr, &rz_new));
-    if (restart) {  // the preconditioner changed: new Krylov sequence from here
-      DOHP_HIP(hipMemcpyAsync(p.ptr, z.ptr, sizeof(T) * c.n, hipMemcpyDeviceToDevice, c.st));
-      restart = false;
-    } else {
-      double beta = rz_new / rz;
-      if (flexible) {
-        double zq;
-        DOHP_CALL(dot(c, z.ptr, q.ptr, &zq));
-        beta = -alpha * zq / rz;
-      }
-      DOHP_CALL(axpby<T>(c, T(1), z.ptr, (T)beta, p.ptr));
-    }
-    rz = rz_new;
+    if (std::sqrt(rr) <= tol || k >= max_it) break;
+    if (!ahead) DOHP_CALL(precondition());
+    // (a preconditioner that changed starts a new Krylov sequence)
+    DOHP_CALL(direction(restart ? KB_FIRST : flexible ? KB_FLEXIBLE : KB_STANDARD));
+    restart = false;
   }
   *its = k;
   *rnorm = std::sqrt(rr);
@@ -386,16 +533,19 @@ dErr solve_impl(dohpEllip op, dohpMat q1, dohpMLP mlp, const double *b, double *
   c.pool = dohpEllipPool_Private(op);
   DOHP_CALL(c.part.alloc(*c.pool, kRedBlocks));
   DOHP_CALL(c.res.alloc(*c.pool, 1));
+  DOHP_CALL(dohpEllipPinned_Private(op, &c.host, &c.host_dev));
   *stats = dohpSolveStats{};
   // Jacobi scaling and, for the one-level preconditioner, the Chebyshev interval
   // [lmax/ratio, 1.05 lmax] of D^{-1} A_q1
   PoolBuf<double> diag, dinv;
   PoolBuf<float> dinv32;
-  DOHP_CALL(diag.alloc(*c.pool, c.n));
-  DOHP_CALL(dinv.alloc(*c.pool, c.n));
-  DOHP_CALL(dinv32.alloc(*c.pool, c.n));
-  DOHP_CALL(dohpMatGetDiagonal(q1, diag.ptr, c.st));
-  hipLaunchKernelGGL(inv_kernel, grid(c.n), dim3(256), 0, c.st, c.n, diag.ptr, dinv.ptr, dinv32.ptr);
+  if (opts->pc == 0 || mlp) {
+    DOHP_CALL(diag.alloc(*c.pool, c.n));
+    DOHP_CALL(dinv.alloc(*c.pool, c.n));
+    DOHP_CALL(dinv32.alloc(*c.pool, c.n));
+    DOHP_CALL(dohpMatGetDiagonal(q1, diag.ptr, c.st));
+    hipLaunchKernelGGL(inv_kernel, grid(c.n), dim3(256), 0, c.st, c.n, diag.ptr, dinv.ptr, dinv32.ptr);
+  }
   double lmax = 1.0;
   if (opts->pc == 0) {
     DOHP_CALL(estimate_lmax(c, q1, dinv.ptr, opts->eig_its > 0 ? opts->eig_its : 20, &lmax));
@@ -443,9 +593,7 @@ dErr solve_impl(dohpEllip op, dohpMat q1, dohpMLP mlp, const double *b, double *
   stats->setup_seconds = std::chrono::duration<double>(t_setup - t0).count();
   if (opts->mixed == 2) {  // FP64 PCG, preconditioner in FP32
     Cheb<float> C32{q1, dinv32.ptr, lmin, lmax, degree};
-    DOHP_CALL(C32.res.alloc(*c.pool, c.n));
-    DOHP_CALL(C32.d.alloc(*c.pool, c.n));
-    DOHP_CALL(C32.w.alloc(*c.pool, c.n));
+    if (opts->pc == 0) DOHP_CALL(C32.alloc(c));
     Prec<float> M32;
     M32.cheb = &C32;
     M32.mg = mgh.mg;
@@ -453,26 +601,17 @@ dErr solve_impl(dohpEllip op, dohpMat q1, dohpMLP mlp, const double *b, double *
     M32.s = wts.ptr;
     M32.tmp = tmp32.ptr;
     M32.learned_on = mlp != nullptr || q1fb != nullptr;
-    PoolBuf<float> lr, lz;
-    DOHP_CALL(lr.alloc(*c.pool, c.n));
-    DOHP_CALL(lz.alloc(*c.pool, c.n));
-    Prec<double> M;
-    M.low = &M32;
-    M.lr = lr.ptr;
-    M.lz = lz.ptr;
     int its;
     double rn, bn;
-    DOHP_CALL(pcg<double>(c, op, M, bud, b, x, opts->rtol, opts->max_it, &its, &rn, &bn, snap, nsnap, every, nsnapped,
-                          true));
+    DOHP_CALL((pcg<double, float>(c, op, M32, bud, b, x, opts->rtol, opts->max_it, &its, &rn, &bn, snap, nsnap, every,
+                                  nsnapped, true)));
     stats->inner_its = its;
     stats->outer_its = 1;
     stats->rnorm = rn;
     stats->bnorm = bn;
   } else if (!opts->mixed) {
     Cheb<double> C64{q1, dinv.ptr, lmin, lmax, degree};
-    DOHP_CALL(C64.res.alloc(*c.pool, c.n));
-    DOHP_CALL(C64.d.alloc(*c.pool, c.n));
-    DOHP_CALL(C64.w.alloc(*c.pool, c.n));
+    if (opts->pc == 0) DOHP_CALL(C64.alloc(c));
     Prec<double> M;
     M.cheb = &C64;
     M.mg = mgh.mg;
@@ -482,16 +621,15 @@ dErr solve_impl(dohpEllip op, dohpMat q1, dohpMLP mlp, const double *b, double *
     M.learned_on = mlp != nullptr || q1fb != nullptr;
     int its;
     double rn, bn;
-    DOHP_CALL(pcg<double>(c, op, M, bud, b, x, opts->rtol, opts->max_it, &its, &rn, &bn, snap, nsnap, every, nsnapped));
+    DOHP_CALL((pcg<double, double>(c, op, M, bud, b, x, opts->rtol, opts->max_it, &its, &rn, &bn, snap, nsnap, every,
+                                   nsnapped)));
     stats->inner_its = its;
     stats->outer_its = 1;
     stats->rnorm = rn;
     stats->bnorm = bn;
   } else {
     Cheb<float> C32{q1, dinv32.ptr, lmin, lmax, degree};
-    DOHP_CALL(C32.res.alloc(*c.pool, c.n));
-    DOHP_CALL(C32.d.alloc(*c.pool, c.n));
-    DOHP_CALL(C32.w.alloc(*c.pool, c.n));
+    if (opts->pc == 0) DOHP_CALL(C32.alloc(c));
     Prec<float> M;
     M.cheb = &C32;
     M.mg = mgh.mg;
@@ -528,7 +666,7 @@ dErr solve_impl(dohpEllip op, dohpMat q1, dohpMLP mlp, const double *b, double *
       // the last sweep needs only the reduction that is left to reach rtol ||b||
       const double need = 0.5 * opts->rtol * stats->bnorm / stats->rnorm;
       const double irtol = std::max(opts->inner_rtol, need);
-      DOHP_CALL(pcg<float>(c, op, M, bud, r32.ptr, e32.ptr, irtol, opts->max_it, &its, &rn, &bn));
+      DOHP_CALL((pcg<float, float>(c, op, M, bud, r32.ptr, e32.ptr, irtol, opts->max_it, &its, &rn, &bn)));
       inner_total += its;
       hipLaunchKernelGGL(promote_add_kernel, grid(c.n), dim3(256), 0, c.st, c.n, stats->rnorm, e32.ptr, x);
       outer++;
