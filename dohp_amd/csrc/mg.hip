@@ -384,42 +384,65 @@ __device__ __forceinline__ _Float16 coeff16(double a, float si, float sj)
   return (_Float16)(float)(a / ((double)si * (double)sj));
 }
 
-__global__ void __launch_bounds__(256) half16_setup_kernel(Box bx, const double *__restrict__ A,
-                                                           _Float16 *__restrict__ H, float *__restrict__ dg,
-                                                           float *__restrict__ sc, float *__restrict__ eg,
-                                                           float *__restrict__ fg, int scaled_in)
+// Row scales and inverse diagonals of a level from its 27-point stencil.
+__global__ void diag_kernel(long n, const double *__restrict__ A, double *__restrict__ dinv, float *__restrict__ dinv32,
+                            float *__restrict__ sc)
 {
-  const long n = bx.n();
-  int I, J, K;
-  long i;
-  if (!box_index(bx, I, J, K, i)) return;
-  const long sy = bx.nz, sx = (long)bx.ny * bx.nz;
-  const float si = (float)sqrt(A[13 * n + i]);
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double a = A[13 * n + i], r = 1.0 / a;
+  dinv[i] = r;
+  dinv32[i] = (float)r;
+  if (sc) sc[i] = (float)sqrt(a);
+}
+
+// The half stencil of a level in FP64 (H, null where the level's own stencil serves), FP32 and FP16 in one pass over its
+// 27-point stencil A: a row's 13 upper entries are read once for all three, the row scales of its neighbours come from
+// a staged tile, and its lower neighbours' entries (which those rows round) are read for the diagonal's compensation.
+// 112 bytes read and 112 + 56 + 48 written per row and 27 FP64 divisions: 191^3 rows 0.95 -> 0.63 ms against a copy of the half
+// stencil and an FP16 pass that took 52 square roots per row.
+__global__ void __launch_bounds__(256) half_setup_kernel(Box bx, const double *__restrict__ A, double *__restrict__ H,
+                                                         float *__restrict__ H32, _Float16 *__restrict__ H16,
+                                                         float *__restrict__ dg, const float *__restrict__ sc,
+                                                         float *__restrict__ eg, float *__restrict__ fg, int scaled_in)
+{
+  using S = SweepTile<kBY, 1>;
+  __shared__ float tile[S::N];
+  const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
+  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile,
+                     [&](long g, int, int, int) { return sc[g]; });
+  const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
+  if (K >= bx.nz || J >= bx.ny) return;
+  const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz, i = ((long)I * bx.ny + J) * bx.nz + K;
+  const float si = tile[(S::TY + tj) * S::TX + tk];
+  const double aii = A[13 * n + i];
+  if (H) H[i] = aii;
+  H32[i] = (float)aii;
   double comp = 0;
-#pragma unroll 1
+  unsigned pair = 0;
+#pragma unroll
   for (int s = 14; s < 27; s++) {
     const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
     const long off = di * sx + dj * sy + dk;
-    _Float16 h = 0;
-    if (I + di >= 0 && I + di < bx.nx && J + dj >= 0 && J + dj < bx.ny && K + dk >= 0 && K + dk < bx.nz) {
-      const float sj = (float)sqrt(A[13 * n + i + off]);
-      const double a = A[s * n + i];
-      h = coeff16(a, si, sj);
-      comp += a - (double)si * (double)sj * (double)h;
-    }
-    H[((s - 14) >> 1) * 2 * n + 2 * i + ((s - 14) & 1)] = h;
-    if (I - di >= 0 && I - di < bx.nx && J - dj >= 0 && J - dj < bx.ny && K - dk >= 0 && K - dk < bx.nz) {
-      // the lower neighbour's entry is its upper one, rounded as that row rounds it
-      const float sj = (float)sqrt(A[13 * n + i - off]);
-      const double a = A[s * n + i - off];
-      const _Float16 hl = coeff16(a, sj, si);
-      comp += a - (double)sj * (double)si * (double)hl;
-    }
+    const bool up = inside(bx, I + di, J + dj, K + dk), lo = inside(bx, I - di, J - dj, K - dk);
+    const double a = A[s * n + i], al = A[s * n + (lo ? i - off : i)];
+    if (H) H[(s - 13) * n + i] = a;
+    H32[(s - 13) * n + i] = (float)a;
+    const float sj = up ? tile[((1 + di) * S::TY + tj + dj) * S::TX + tk + dk] : 1.f;
+    const float sl = lo ? tile[((1 - di) * S::TY + tj - dj) * S::TX + tk - dk] : 1.f;
+    const _Float16 h = up ? coeff16(a, si, sj) : (_Float16)0;
+    if (up) comp += a - (double)si * (double)sj * (double)h;
+    // the lower neighbour's entry is its upper one, rounded as that row rounds it
+    if (lo) comp += al - (double)sl * (double)si * (double)coeff16(al, sl, si);
+    const unsigned bits = __builtin_bit_cast(unsigned short, h);
+    if ((s - 14) & 1)
+      ((unsigned *)H16)[((s - 14) >> 1) * n + i] = pair | bits << 16;
+    else
+      pair = bits;
   }
-  H[6 * 2 * n + 2 * i + 1] = 0;  // (the pad of the last pair)
-  const double dd = A[13 * n + i] + comp, s1 = (double)si;
+  ((unsigned *)H16)[6 * n + i] = pair;  // (the last pair is padded)
+  const double dd = aii + comp, s1 = (double)si;
   dg[i] = (float)dd;
-  sc[i] = si;
   eg[i] = (float)(dd / (s1 * s1));
   fg[i] = (float)((scaled_in ? s1 * s1 : s1) / dd);  // y = c f b is the first smoothing step from b' or (finest) b
 }
@@ -524,22 +547,16 @@ __global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, const _Fl
   }
 }
 
+// The half stencil alone (the coarsest level, which is solved directly).
 __global__ void half_from_full_kernel(long n, const double *__restrict__ A, double *__restrict__ H,
                                       float *__restrict__ H32)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   for (int s = 13; s < 27; s++) {
-    H[(s - 13) * n + i] = A[s * n + i];
+    if (H) H[(s - 13) * n + i] = A[s * n + i];
     H32[(s - 13) * n + i] = (float)A[s * n + i];
   }
-}
-
-template <typename T>
-__global__ void diag_inv_kernel(long n, const T *__restrict__ A, T *__restrict__ dinv)
-{
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < n) dinv[r] = T(1) / A[13 * n + r];
 }
 
 // bc = P^T rf, divided by the coarse level's row scales s (null: not)
@@ -574,67 +591,154 @@ __host__ __device__ constexpr double pweight(int e, int t)
   return e == 2 * t ? 1.0 : (e - 2 * t == 1 || e - 2 * t == -1) ? 0.5 : 0.0;
 }
 
-// Ac = P^T Af P, one thread per coarse row (FP64).  Row C gathers over the 27 fine nodes f of its prolongation's
-// support (weight P[f][C]) and their 27 stencil entries A[f][g].  The weights factor by direction: with f at offsets
-// (a, b, d) from C's own fine node and g = f + (si, sj, sk), P[f][C] P[g][C + t] = X(a, si, ti) Y(b, sj, tj)
-// Z(d, sk, tk).  The x part (a, si) is a loop; inside it the 81 (b, d, sj, sk) terms have compile-time y and z weights
+// Ac = P^T Af P (FP64).  Row C gathers over the 27 fine nodes f of its prolongation's support (weight P[f][C]) and
+// their 27 stencil entries A[f][g].  The weights factor by direction: with f at offsets (a, b, d) from C's own fine node
+// and g = f + (si, sj, sk), P[f][C] P[g][C + t] = X(a, si, ti) Y(b, sj, tj) Z(d, sk, tk).  A workgroup takes 64 rows;
+// each of its nine wavefronts takes one x part (a, si): the 81 (b, d, sj, sk) terms have compile-time y and z weights
 // and are summed into 3 x 3 partial sums in registers (every load unconditional: a support node outside the fine box
-// reads entry 0 with weight 0), which then meet the three x weights.  Entries toward coarse nodes outside the box are
-// zero, as the assembly leaves them on the finest level.
-__global__ void __launch_bounds__(256) rap_kernel(Box f, Box c, const double *__restrict__ Af, double *__restrict__ Ac)
+// reads entry 0 with weight 0).  The partial sums meet the x weights through LDS, three of the 27 entries per wavefront.
+// With one thread per row the nine parts followed one another, 729 loads at 13 wavefronts per SIMD in all: latency
+// bound, 1.90 ms at 95^3 coarse rows and 0.11 ms at 5^3; this takes 0.84 and 0.01 ms.  Entries toward coarse nodes
+// outside the box are zero, as the assembly leaves them on the finest level.
+__global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, const double *__restrict__ Af, double *__restrict__ Ac)
 {
-  const long C = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long nc = c.n(), nf = f.n();
-  if (C >= nc) return;
+  __shared__ double part[9][9][64];  // [x part][3 x 3 sum][row]
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, a = w / 3 - 1, si = w % 3 - 1;
+  const long nc = c.n(), nf = f.n(), C = (long)blockIdx.x * 64 + lane;
   int I, J, K;
-  unrank(c, C, I, J, K);
-  double acc[27];
-#pragma unroll
-  for (int t = 0; t < 27; t++) acc[t] = 0.0;
+  unrank(c, C < nc ? C : nc - 1, I, J, K);
   const long sy = f.nz, sx = (long)f.ny * f.nz;
-#pragma unroll 1
-  for (int a = -1; a <= 1; a++) {
-    const int fi = 2 * I + 1 + a;  // >= 0
-    if (fi >= f.nx) continue;
-#pragma unroll 1
-    for (int si = -1; si <= 1; si++) {
-      double T[9];
+  const int fi = 2 * I + 1 + a;  // >= 0
+  double T[9];
 #pragma unroll
-      for (int u = 0; u < 9; u++) T[u] = 0.0;
+  for (int u = 0; u < 9; u++) T[u] = 0.0;
 #pragma unroll
-      for (int b = -1; b <= 1; b++)
+  for (int b = -1; b <= 1; b++)
 #pragma unroll
-        for (int d = -1; d <= 1; d++) {
-          const int fj = 2 * J + 1 + b, fk = 2 * K + 1 + d;
-          const bool in = fj < f.ny && fk < f.nz;
-          const long fr = in ? fi * sx + fj * sy + fk : 0;
-          const double w = in ? pweight(b, 0) * pweight(d, 0) : 0.0;
+    for (int d = -1; d <= 1; d++) {
+      const int fj = 2 * J + 1 + b, fk = 2 * K + 1 + d;
+      const bool in = fi < f.nx && fj < f.ny && fk < f.nz;
+      const long fr = in ? fi * sx + fj * sy + fk : 0;
+      const double w0 = in ? pweight(b, 0) * pweight(d, 0) : 0.0;
 #pragma unroll
-          for (int sj = -1; sj <= 1; sj++)
+      for (int sj = -1; sj <= 1; sj++)
 #pragma unroll
-            for (int sk = -1; sk <= 1; sk++) {
-              const double v = w * Af[((si + 1) * 9 + (sj + 1) * 3 + (sk + 1)) * nf + fr];
+        for (int sk = -1; sk <= 1; sk++) {
+          const double v = w0 * Af[((si + 1) * 9 + (sj + 1) * 3 + (sk + 1)) * nf + fr];
 #pragma unroll
-              for (int tj = -1; tj <= 1; tj++)
+          for (int tj = -1; tj <= 1; tj++)
 #pragma unroll
-                for (int tk = -1; tk <= 1; tk++) {
-                  const double q = pweight(b + sj, tj) * pweight(d + sk, tk);
-                  if (q != 0.0) T[(tj + 1) * 3 + (tk + 1)] = fma(v, q, T[(tj + 1) * 3 + (tk + 1)]);
-                }
+            for (int tk = -1; tk <= 1; tk++) {
+              const double q = pweight(b + sj, tj) * pweight(d + sk, tk);
+              if (q != 0.0) T[(tj + 1) * 3 + (tk + 1)] = fma(v, q, T[(tj + 1) * 3 + (tk + 1)]);
             }
         }
-      const double wa = pweight(a, 0);
-#pragma unroll
-      for (int ti = -1; ti <= 1; ti++) {
-        const double x = wa * pweight(a + si, ti);
-#pragma unroll
-        for (int u = 0; u < 9; u++) acc[(ti + 1) * 9 + u] = fma(x, T[u], acc[(ti + 1) * 9 + u]);
-      }
     }
-  }
 #pragma unroll
-  for (int t = 0; t < 27; t++)
-    Ac[t * nc + C] = inside(c, I + t / 9 - 1, J + (t / 3) % 3 - 1, K + t % 3 - 1) ? acc[t] : 0.0;
+  for (int u = 0; u < 9; u++) part[w][u][lane] = T[u];
+  __syncthreads();
+  if (C >= nc) return;
+#pragma unroll
+  for (int o = 0; o < 3; o++) {  // entry t = 9 o + w: x offset o - 1
+    const int t = 9 * o + w;
+    double acc = 0.0;
+#pragma unroll
+    for (int aa = -1; aa <= 1; aa++)
+#pragma unroll
+      for (int ss = -1; ss <= 1; ss++)
+        acc = fma(pweight(aa, 0) * pweight(aa + ss, o - 1), part[(aa + 1) * 3 + ss + 1][w][lane], acc);
+    Ac[t * nc + C] = inside(c, I + o - 1, J + w / 3 - 1, K + w % 3 - 1) ? acc : 0.0;
+  }
+}
+
+// Explicit inverse of the (symmetric positive definite) coarsest matrix, in place, by Gauss-Jordan elimination on
+// 32 x 32 blocks without pivoting.  A step k takes two launches: the panel kernel inverts the diagonal block (every
+// workgroup for itself, in LDS), forms its part of R = D A_k: and copies its part of the block column A_:k; the update
+// kernel writes A_ij -= A_ik R_j, R in block row k, -A_ik D in block column k and D itself: 31 us a
+// step.  A hierarchy's whole set-up at 47 x 47 x 47 rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343
+// 13.4 -> 0.72 ms, at 65^3 over 512 46 -> 0.94 ms: scalar host code between two copies did the elimination before.
+constexpr int kCB = 32;
+__global__ void dense_fill_kernel(Box b, const double *__restrict__ st, double *__restrict__ A)
+{
+  const long n = b.n(), t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * n) return;
+  const long r = t / n;
+  int I, J, K, I2, J2, K2;
+  unrank(b, r, I, J, K);
+  unrank(b, t - r * n, I2, J2, K2);
+  const int di = I2 - I, dj = J2 - J, dk = K2 - K;
+  const bool in = di >= -1 && di <= 1 && dj >= -1 && dj <= 1 && dk >= -1 && dk <= 1;
+  A[t] = in ? st[((di + 1) * 9 + (dj + 1) * 3 + (dk + 1)) * n + r] : 0.0;
+}
+
+__global__ void __launch_bounds__(256) dense_panel_kernel(int n, int k0, const double *__restrict__ A,
+                                                          double *__restrict__ R, double *__restrict__ Cc,
+                                                          double *__restrict__ D, double *__restrict__ bad)
+{
+  __shared__ double d[kCB][kCB + 1];
+  const int t = threadIdx.x, m = min(kCB, n - k0);
+  for (int q = t; q < kCB * kCB; q += 256) {
+    const int r = q / kCB, c = q % kCB;
+    d[r][c] = r < m && c < m ? A[(long)(k0 + r) * n + k0 + c] : r == c ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  const int c = t % kCB, r0 = t / kCB;  // this thread's column and rows r0, r0 + 8, ...
+  for (int p = 0; p < m; p++) {
+    const double piv = d[p][p];
+    if (t == 0 && blockIdx.x == 0 && !(piv > 0.0)) *bad = 1.0;
+    const double ip = 1.0 / piv, rowc = (c == p ? 1.0 : d[p][c]) * ip;
+    double colr[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) colr[u] = d[r0 + 8 * u][p];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int r = r0 + 8 * u;
+      d[r][c] = r == p ? rowc : (c == p ? 0.0 : d[r][c]) - colr[u] * rowc;
+    }
+    __syncthreads();
+  }
+  if (blockIdx.x == 0)
+    for (int q = t; q < kCB * kCB; q += 256) D[q] = d[q / kCB][q % kCB];
+  // columns (of R) and rows (of the copied panel) j0 .. j0 + 31 of this workgroup
+  const int j0 = blockIdx.x * kCB, j = j0 + c;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + 8 * u;
+    if (j < n && r < m) {
+      double s = 0.0;
+      for (int q = 0; q < m; q++) s += d[r][q] * A[(long)(k0 + q) * n + j];
+      R[(long)r * n + j] = s;
+    }
+    if (j0 + r < n && c < m) Cc[(long)(j0 + r) * kCB + c] = A[(long)(j0 + r) * n + k0 + c];
+  }
+}
+
+__global__ void __launch_bounds__(256) dense_update_kernel(int n, int k0, double *__restrict__ A,
+                                                           const double *__restrict__ R,
+                                                           const double *__restrict__ Cc,
+                                                           const double *__restrict__ D)
+{
+  __shared__ double cs[kCB][kCB + 1], rs[kCB][kCB + 1];
+  const int t = threadIdx.x, m = min(kCB, n - k0), i0 = blockIdx.y * kCB, j0 = blockIdx.x * kCB, c = t % kCB, r0 = t / kCB;
+  const bool row = i0 == k0, col = j0 == k0;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + 8 * u;
+    cs[r][c] = i0 + r < n && c < m ? Cc[(long)(i0 + r) * kCB + c] : 0.0;
+    rs[r][c] = r < m && j0 + c < n ? (col ? D[r * kCB + c] : R[(long)r * n + j0 + c]) : 0.0;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + 8 * u;
+    if (i0 + r >= n || j0 + c >= n) continue;
+    double *a = &A[(long)(i0 + r) * n + j0 + c];
+    double s = 0.0;
+    if (!row)
+      for (int q = 0; q < m; q++) s += cs[r][q] * rs[q][c];
+    *a = row ? rs[r][c] : (col ? 0.0 : *a) - s;
+  }
 }
 
 // x = Ainv b, one wavefront per row (lanes stride the row, then a butterfly reduction).
@@ -650,7 +754,12 @@ __global__ void dense_mv_kernel(int n, const T *__restrict__ Ainv, const T *__re
   if (lane == 0) x[r] = acc;
 }
 
-template <typename T>
+__global__ void zero_kernel(long n, double *__restrict__ a)
+{
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) a[i] = 0.0;
+}
+
 __global__ void to_f32(long n, const double *__restrict__ a, float *__restrict__ b)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -753,7 +862,8 @@ struct MGLevel {
   Box box{};
   long n = 0;
   const double *A64 = nullptr;  // full 27-point stencil (finest level: the Q1 matrix's own)
-  DevBuf<double> own64, H64, dinv64, b64, x64, r64, d64;  // H: symmetric half stencil [14][n]
+  const double *H = nullptr;    // symmetric half stencil [14][n]: H64 on the finest level, part of own64 below
+  DevBuf<double> own64, H64, dinv64, b64, x64, r64, d64;
   DevBuf<float> H32, dinv32, b32, x32, r32, d32;
   DevBuf<_Float16> H16;        // FP16 upper off-diagonals, pairs of directions per row [7][n][2] (half16_row)
   DevBuf<float> dg16, sc16;    // their diagonal d and row scales s
@@ -770,7 +880,8 @@ struct _p_dohpMG {
   int coeff16 = 1;  // the FP32 V-cycle reads the FP16 coefficients
   DevBuf<double> cinv64;
   DevBuf<float> cinv32;
-  DevBuf<double> part;  // the power iterations' norms and block sums
+  DevBuf<double> part;   // the power iterations' norms and block sums
+  DevBuf<double> cwork;  // the coarsest inverse's panels
   // V-cycles replayed as HIP graphs: the coarse levels' kernels run for a few microseconds each, less than their
   // launch costs the host, so the eager V-cycle leaves the GPU waiting; a graph is captured (on a private stream)
   // per precision for the vectors it was applied to and replayed while they stay the same.
@@ -800,7 +911,7 @@ struct _p_dohpMG {
 namespace {
 
 // lmax of D^-1 A on every smoothed level by power iteration, in the levels' work vectors (free outside a V-cycle).  The
-// iterations stay on the device: one read of the last norms at the end.
+// iterations stay on the device and leave the last norms at the start of mg->part.
 dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
 {
   const int nl = (int)mg->L.size() - 1;
@@ -814,7 +925,7 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     MGLevel &lv = mg->L[k];
     PowerLevel &l = g.l[k];
     l.bx = lv.box;
-    l.H = lv.H64.ptr;
+    l.H = lv.H;
     l.dinv = lv.dinv64.ptr;
     l.v[0] = lv.r64.ptr;
     l.v[1] = lv.d64.ptr;
@@ -839,51 +950,29 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 0, norm, inv);
   }
   DOHP_HIP(hipGetLastError());
-  double h[kMaxLevels] = {};
-  DOHP_HIP(hipMemcpyAsync(h, norm, sizeof(double) * nl, hipMemcpyDeviceToHost, st));
-  DOHP_HIP(hipStreamSynchronize(st));
-  for (int k = 0; k < nl; k++) mg->L[k].lmax = h[k];
   return 0;
 }
 
-// Explicit inverse of the (symmetric positive definite) coarsest matrix by Gauss-Jordan, host FP64.
-dErr coarse_inverse(const MGLevel &lv, hipStream_t st, std::vector<double> &inv)
+// Inverse of the coarsest matrix, FP64 and FP32, on the device; work[0] is set to 1 if a pivot is not positive.
+dErr coarse_inverse(_p_dohpMG *mg, hipStream_t st)
 {
-  const long n = lv.n;
-  DOHP_CHECK(n <= 4096, dohpERR_ARG, "multigrid: the coarsest level is too large for a direct solve");
-  std::vector<double> S(27 * n);
-  DOHP_HIP(hipMemcpyAsync(S.data(), lv.A64, sizeof(double) * 27 * n, hipMemcpyDeviceToHost, st));
-  DOHP_HIP(hipStreamSynchronize(st));
-  std::vector<double> A(n * n, 0.0);
-  const Box b = lv.box;
-  for (long r = 0; r < n; r++) {
-    const int I = (int)(r / ((long)b.ny * b.nz)), J = (int)((r / b.nz) % b.ny), K = (int)(r % b.nz);
-    for (int s = 0; s < 27; s++) {
-      const int i2 = I + s / 9 - 1, j2 = J + (s / 3) % 3 - 1, k2 = K + s % 3 - 1;
-      if (i2 < 0 || i2 >= b.nx || j2 < 0 || j2 >= b.ny || k2 < 0 || k2 >= b.nz) continue;
-      A[r * n + ((long)i2 * b.ny + j2) * b.nz + k2] += S[s * n + r];
-    }
+  const MGLevel &lv = mg->L.back();
+  const int n = (int)lv.n;
+  DOHP_CHECK(lv.n <= 4096, dohpERR_ARG, "multigrid: the coarsest level is too large for a direct solve");
+  const size_t nn = (size_t)n * n, nw = 1 + kCB * kCB + 2 * (size_t)kCB * n;
+  if (!mg->cinv64.holds(nn)) DOHP_CALL(mg->cinv64.alloc(nn));
+  if (!mg->cinv32.holds(nn)) DOHP_CALL(mg->cinv32.alloc(nn));
+  if (!mg->cwork.holds(nw)) DOHP_CALL(mg->cwork.alloc(nw));
+  double *A = mg->cinv64.ptr, *bad = mg->cwork.ptr, *D = bad + 1, *R = D + kCB * kCB, *Cc = R + (size_t)kCB * n;
+  const unsigned nb = (unsigned)((n + kCB - 1) / kCB);
+  hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, st, 1L, bad);
+  hipLaunchKernelGGL(dense_fill_kernel, grid_of((long)nn), dim3(256), 0, st, lv.box, lv.A64, A);
+  for (int k0 = 0; k0 < n; k0 += kCB) {
+    hipLaunchKernelGGL(dense_panel_kernel, dim3(nb), dim3(256), 0, st, n, k0, A, R, Cc, D, bad);
+    hipLaunchKernelGGL(dense_update_kernel, dim3(nb, nb), dim3(256), 0, st, n, k0, A, R, Cc, D);
   }
-  inv.assign(n * n, 0.0);
-  for (long i = 0; i < n; i++) inv[i * n + i] = 1.0;
-  for (long k = 0; k < n; k++) {
-    const double piv = A[k * n + k];
-    DOHP_CHECK(piv > 0.0, dohpERR_GENERIC, "multigrid: coarsest matrix is not positive definite");
-    const double ip = 1.0 / piv;
-    for (long j = 0; j < n; j++) {
-      A[k * n + j] *= ip;
-      inv[k * n + j] *= ip;
-    }
-    for (long i = 0; i < n; i++) {
-      if (i == k) continue;
-      const double f = A[i * n + k];
-      if (f == 0.0) continue;
-      for (long j = 0; j < n; j++) {
-        A[i * n + j] -= f * A[k * n + j];
-        inv[i * n + j] -= f * inv[k * n + j];
-      }
-    }
-  }
+  hipLaunchKernelGGL(to_f32, grid_of((long)nn), dim3(256), 0, st, (long)nn, A, mg->cinv32.ptr);
+  DOHP_HIP(hipGetLastError());
   return 0;
 }
 
@@ -891,7 +980,7 @@ template <typename T>
 struct LvPtr;
 template <>
 struct LvPtr<double> {
-  static const double *A(const MGLevel &l) { return l.H64.ptr; }
+  static const double *A(const MGLevel &l) { return l.H; }
   static const double *dinv(const MGLevel &l) { return l.dinv64.ptr; }
   static double *b(MGLevel &l) { return l.b64.ptr; }
   static double *x(MGLevel &l) { return l.x64.ptr; }
@@ -1063,29 +1152,36 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
   for (size_t l = 1; l < mg->L.size(); l++) {
     const MGLevel &f = mg->L[l - 1];
     MGLevel &c = mg->L[l];
-    hipLaunchKernelGGL(rap_kernel, grid_of(c.n), dim3(256), 0, st, f.box, c.box, f.A64, c.own64.ptr);
+    hipLaunchKernelGGL(rap_kernel, dim3((unsigned)((c.n + 63) / 64)), dim3(576), 0, st, f.box, c.box, f.A64,
+                       c.own64.ptr);
   }
   for (size_t l = 0; l < mg->L.size(); l++) {
     MGLevel &lv = mg->L[l];
     const long n = lv.n;
-    hipLaunchKernelGGL(half_from_full_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.H64.ptr, lv.H32.ptr);
-    if (l + 1 < mg->L.size())
-      hipLaunchKernelGGL(half16_setup_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.A64, lv.H16.ptr,
-                         lv.dg16.ptr, lv.sc16.ptr, lv.e16.ptr, lv.f16.ptr, l > 0);
-    hipLaunchKernelGGL(diag_inv_kernel<double>, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.dinv64.ptr);
-    hipLaunchKernelGGL(to_f32<float>, grid_of(n), dim3(256), 0, st, n, lv.dinv64.ptr, lv.dinv32.ptr);
+    const bool smoothed = l + 1 < mg->L.size();
+    hipLaunchKernelGGL(diag_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.dinv64.ptr, lv.dinv32.ptr,
+                       smoothed ? lv.sc16.ptr : nullptr);
+    if (smoothed)
+      hipLaunchKernelGGL(half_setup_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.A64, lv.H64.ptr,
+                         lv.H32.ptr, lv.H16.ptr, lv.dg16.ptr, lv.sc16.ptr, lv.e16.ptr, lv.f16.ptr, l > 0);
+    else
+      hipLaunchKernelGGL(half_from_full_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.H64.ptr, lv.H32.ptr);
+    lv.H = lv.H64.ptr ? lv.H64.ptr : lv.A64 + 13 * n;
   }
   DOHP_CALL(estimate_lmax(mg, st, 15));
-  std::vector<double> inv;
-  DOHP_CALL(coarse_inverse(mg->L.back(), st, inv));
-  mg->ncoarse = (int)mg->L.back().n;
-  DOHP_CALL(mg->cinv64.upload(inv.data(), inv.size()));
-  std::vector<float> inv32(inv.begin(), inv.end());
-  DOHP_CALL(mg->cinv32.upload(inv32.data(), inv32.size()));
+  DOHP_CALL(coarse_inverse(mg, st));
+  // one read of the eigenvalue estimates and the inverse's flag
+  const size_t nl = mg->L.size() - 1;
+  double h[kMaxLevels + 1] = {};
+  if (nl) DOHP_HIP(hipMemcpyAsync(h, mg->part.ptr, sizeof(double) * nl, hipMemcpyDeviceToHost, st));
+  DOHP_HIP(hipMemcpyAsync(h + kMaxLevels, mg->cwork.ptr, sizeof(double), hipMemcpyDeviceToHost, st));
   if (hipStreamSynchronize(st) != hipSuccess) {
     set_error("multigrid setup failed");
     return dohpERR_HIP;
   }
+  for (size_t l = 0; l < nl; l++) mg->L[l].lmax = h[l];
+  DOHP_CHECK(h[kMaxLevels] == 0.0, dohpERR_GENERIC, "multigrid: coarsest matrix is not positive definite");
+  mg->ncoarse = (int)mg->L.back().n;
   return 0;
 }
 
@@ -1126,7 +1222,7 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
     const long n = lv.n;
     err = lv.dinv64.alloc(n);
     if (!err) err = lv.dinv32.alloc(n);
-    if (!err) err = lv.H64.alloc(14 * n);
+    if (!err && l == 0) err = lv.H64.alloc(14 * n);  // (the matrix may be refilled or freed before the hierarchy)
     if (!err) err = lv.H32.alloc(14 * n);
     if (!err) err = lv.r64.alloc(n);
     if (!err) err = lv.d64.alloc(n);
@@ -1264,7 +1360,7 @@ extern "C" dErr dohpMGResidual(dohpMG mg, int level, const double *b, const doub
   DOHP_CHECK(mg && level >= 0 && level < (int)mg->L.size(), dohpERR_ARG, "no such multigrid level");
   DOHP_CHECK(x && r, dohpERR_ARG, "null argument");
   const MGLevel &lv = mg->L[level];
-  residual<double>(lv.box, lv.H64.ptr, b, x, r, (hipStream_t)stream);
+  residual<double>(lv.box, lv.H, b, x, r, (hipStream_t)stream);
   DOHP_HIP(hipGetLastError());
   return 0;
 }

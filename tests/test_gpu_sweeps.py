@@ -129,3 +129,21 @@ def test_vcycle_matches_plain_fp64(C, M, p, mask, degree):
             torch.cuda.synchronize()
             assert float(torch.linalg.norm(z32.double() - ref)) <= tol * float(torch.linalg.norm(ref)), fp16
     assert torch.equal(r32, r.float())
+
+
+# One level: the V-cycle is the explicit inverse.  Sizes on both sides of the elimination's 32-row blocks and the largest
+# default coarsest level; well-conditioned Q1 matrices: 512 roundings of 1.1e-16 times a condition number below 1e3.
+@pytest.mark.parametrize("M", [(2, 2, 2), (2, 2, 32), (3, 5, 5), (4, 12, 2), (5, 5, 5), (6, 14, 2), (9, 9, 9)])
+def test_direct_coarse_solve(C, M):
+    n = (M[0] - 1) * (M[1] - 1) * (M[2] - 1)
+    print(f"coarse inverse n={n}", flush=True)
+    op, q1, mg, L = setup(C, M, 1, 7, 2)
+    assert mg.nlevels == 1 and mg.ncoarse == n == q1.nrows
+    A = q1.to_scipy().toarray()
+    r = torch.as_tensor(np.sin(1.0 + np.arange(n)), device="cuda")
+    ref = np.linalg.solve(A, r.cpu().numpy())
+    z, z32 = torch.zeros_like(r), torch.zeros(n, dtype=torch.float32, device="cuda")
+    mg.apply(r, z)
+    mg.apply_f32(r.float(), z32)
+    assert np.linalg.norm(z.cpu().numpy() - ref) <= 1e-11 * np.linalg.norm(ref)
+    assert np.linalg.norm(z32.cpu().numpy() - ref) <= 1e-4 * np.linalg.norm(ref)
