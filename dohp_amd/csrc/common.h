@@ -233,7 +233,9 @@ struct _p_dohpMat {
   int scaled = 0;     // assembled with learned per-sub-cell derivative scales
   bool csr_stale = false;  // block-space matrix: CSR values and FP32 stencil not yet derived from the stencil form
   bool mg_stale = false;   // refilled since the cached hierarchy was computed (refreshed in place on its next use)
-  dohp::DevBuf<double> q1tab;  // the assembly kernel's 1-D tables
+  dohp::DevBuf<double> q1tab;   // the assembly kernel's 1-D tables, of degree q1tab_degree
+  int q1tab_degree = 0;
+  dohp::DevBuf<double> q1ring;  // sub-cell matrices of a few layers (the assembly's workspace)
   ~_p_dohpMat() { dohpMGDestroy(&mg); }
 };
 // Sets the box of a block-space matrix and allocates its stencil form (*box = false: not a box, CSR only).

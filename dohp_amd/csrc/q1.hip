@@ -11,16 +11,18 @@
 //   * u, grad u and the weights are taken at the correct patch points.
 // dohpEllipSetQ1Mode(op, 1) assembles the corrected matrix instead (the Q1 finite-element stiffness of
 // the GLL sub-mesh): sub-cell derivatives +-1/h and the inverse Jacobian at each patch point.
-// The 8x8 sub-cell matrices are added into a CSR matrix over owned nodes (Dirichlet rows and
-// columns are dropped, src/fs/interface/fsbuild.c:31-34).  One thread per sub-cell, in eight launches by the parity
-// of the sub-cell's lattice position: sub-cells of one colour share no node, so the blocks are added without atomics
-// in a fixed order and the matrix is bitwise reproducible.
+// The 8x8 sub-cell matrices are added over owned nodes only (Dirichlet rows and columns are dropped,
+// src/fs/interface/fsbuild.c:31-34).  One kernel forms the sub-cell matrices of a few layers of elements, one thread per
+// sub-cell, and a second adds them up, one thread per row of the 27-point stencil: every sum is taken in a fixed order, so
+// the matrix is bitwise reproducible, and every entry is written once.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "common.h"
+#include "element.h"
 
 using namespace dohp;
 
@@ -29,28 +31,10 @@ namespace {
 
 constexpr int kMaxP = 10;  // degree limit of the sub-cell kernel (n <= 11)
 
-struct Q1Tab {
-  int p, n, nq;                     // degree, nodes per direction, sparse points per direction (2p)
-  int corrected;                    // 1: sub-cell derivatives +-1/h and the inverse Jacobian at the point
-  double hsub[kMaxP];               // GLL sub-interval widths (element-reference coordinates)
-  double zq[2 * kMaxP], wq[2 * kMaxP];
-  double Bs[2 * kMaxP][kMaxP + 1];  // GLL basis at the sparse points
-  double Ds[2 * kMaxP][kMaxP + 1];  // its derivative
-};
-
 struct Q1Phys {
   double p, eps2, lambda;
-  int has_k;
+  int has_k, qpow;     // qpow: 4 (p-2)/2 when it is an integer in [-8, 8], else 99 (powe)
   int M1, M2, Ly, Lz;  // block extents: elements, and node lattice (the state is in lattice order)
-};
-
-// One colour of the sub-cell lattice: sub-cells whose global lattice position (e_d p + a_d) has parity c_d in every
-// direction d share no node, so a launch over one colour adds its blocks without atomics; the eight colours in
-// turn give a fixed summation order (the assembled matrix is bitwise reproducible).
-struct CellColor {
-  int c[3];    // parity per direction
-  int cnt[3];  // sub-cells of this colour per direction
-  __host__ __device__ long n() const { return (long)cnt[0] * cnt[1] * cnt[2]; }
 };
 
 __device__ inline void jac_at(const double (&X)[8][3], double x0, double x1, double x2, double (&J)[3][3])
@@ -91,223 +75,352 @@ __device__ inline double invert3(const double (&a)[3][3], double (&b)[3][3])
   return det;
 }
 
-__device__ inline int find_col(const int *__restrict__ col, int lo, int hi, int c)
-{
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (col[mid] < c) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
 // position of entry (r, c) of a symmetric 8x8 block in its row-major upper triangle
 __host__ __device__ constexpr int sym_index(int r, int c)
 {
   return r <= c ? r * 8 - r * (r - 1) / 2 + (c - r) : c * 8 - c * (c - 1) / 2 + (r - c);
 }
 
-// pow and exp out of line: their registers do not constrain the allocation of the sub-cell block
-__device__ __noinline__ double q1_pow(double x, double e) { return pow(x, e); }
+// row and column of entry t of that triangle
+__host__ __device__ constexpr int sym_row(int t)
+{
+  int r = 0;
+  while (t >= sym_index(r, 7) + 1) r++;
+  return r;
+}
+__host__ __device__ constexpr int sym_col(int t) { return sym_row(t) + t - sym_index(sym_row(t), sym_row(t)); }
+
+template <typename F, int... I>
+__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F f)
+{
+  (f(std::integral_constant<int, I>()), ...);
+}
+
+// exp out of line: its registers do not constrain the allocation of the sub-cell block
 __device__ __noinline__ double q1_exp(double x) { return exp(x); }
 
-// Sub-cell kernel of the embedded-Q1 assembly for n = N nodes per direction, one thread per GLL sub-cell: the
-// 1-D tables sit in device memory (zq, wq, hsub, Bs, Ds at tab, read through the caches), the state's values at the
-// sub-cell's 8 points accumulate over the element's x planes (no per-thread copies of tables or partial sums),
-// the points' data waits in LDS and the 8x8 block in registers.
-template <int N>
-__global__ void __launch_bounds__(128) q1_cell_kernel(int nelem, const int *__restrict__ enodes,
-                                                     const int *__restrict__ everts, const double *__restrict__ vxyz,
-                                                     const double *__restrict__ kv, const double *__restrict__ ustate,
-                                                     long nowned, const int *__restrict__ rowptr,
-                                                     const int *__restrict__ colidx, double *__restrict__ val,
-                                                     double *__restrict__ st, int corrected,
-                                                     const double *__restrict__ tab, Q1Phys ph,
-                                                     const float *__restrict__ cscale, CellColor col)
+// Elements per workgroup and LDS (doubles per element: the state contracted along z, then along z and y; the node values
+// share the latter's space) of the sub-cell kernel.
+constexpr int q1_lds_z(int N) { return 2 * N * N * 2 * (N - 1); }
+constexpr int q1_lds_y(int N) { return 3 * N * 4 * (N - 1) * (N - 1); }
+constexpr int q1_epb(int N)
 {
-  constexpr int P = N - 1, NP3 = P * P * P, NQ = 2 * P;
-  // per thread: u and the reference gradient at the 8 points
-  __shared__ double PD[32][128];
-  const double *zq = tab, *wq = tab + NQ, *hsub = tab + 2 * NQ, *Bs = tab + 2 * NQ + P, *Ds = Bs + NQ * N;
-  const int lt = threadIdx.x;
-  const long t = (long)blockIdx.x * blockDim.x + lt;
-  if (t >= col.n()) return;
-  // sub-cell of this colour: global lattice position G_d = c_d + 2 t_d, element e_d = G_d / p, sub-cell G_d % p
-  const int t2 = (int)(t % col.cnt[2]), t1 = (int)((t / col.cnt[2]) % col.cnt[1]), t0 = (int)(t / ((long)col.cnt[1] * col.cnt[2]));
-  const int G0 = col.c[0] + 2 * t0, G1 = col.c[1] + 2 * t1, G2 = col.c[2] + 2 * t2;
-  const long e0 = G0 / P, e1 = G1 / P, e2 = G2 / P;
-  const int pa = G0 - (int)e0 * P, pb = G1 - (int)e1 * P, pc = G2 - (int)e2 * P;
-  const long e = (e0 * ph.M1 + e1) * ph.M2 + e2;
-  const int pidx = (pa * P + pb) * P + pc;
-  const long tid = e * NP3 + pidx;  // the sub-cell's index (learned scales)
-  (void)nelem;
-  const int *ev = everts + e * 8;
-  const long lat0 = ((e0 * P) * ph.Ly + e1 * P) * ph.Lz + e2 * P;
-  {
-    const double *bz0 = Bs + (2 * pc) * N, *bz1 = bz0 + N, *dz0 = Ds + (2 * pc) * N, *dz1 = dz0 + N;
-    const double *by0 = Bs + (2 * pb) * N, *by1 = by0 + N, *dy0 = Ds + (2 * pb) * N, *dy1 = dy0 + N;
-    const double *bx0 = Bs + (2 * pa) * N, *bx1 = bx0 + N, *dx0 = Ds + (2 * pa) * N, *dx1 = dx0 + N;
-    double PU[8], PG0[8], PG1[8], PG2[8];
+  const int P3 = (N - 1) * (N - 1) * (N - 1), want = P3 >= 216 ? 1 : P3 == 1 ? 128 : 256 / P3;
+  const int fit = 8000 / (q1_lds_z(N) + q1_lds_y(N));
+  return want < fit ? want : fit < 1 ? 1 : fit;
+}
+constexpr int q1_threads(int) { return 256; }
+
+// The value of the other lane of an even-odd pair.
+__device__ __forceinline__ double pair_swap(double v)
+{
+  const long b = __builtin_bit_cast(long, v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xF, 0xF, true);  // quad_perm [1, 0, 3, 2]
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, ((long)hi << 32) | (unsigned)lo);
+}
+
+// Trilinear map of an element as polynomials in the reference coordinates: column m of the Jacobian is bilinear in the
+// other two coordinates, G[m][0..3] = constant, first, second, product; k is trilinear, Gk[8] (bit 2: x0, 1: x1, 0: x2).
+struct Q1Geo {
+  double G[3][4][3], Gk[8];
+};
+__device__ inline void q1_geo(const double *__restrict__ vxyz, const double *__restrict__ kv, const int *ev, int t,
+                              Q1Geo &g)
+{
+  if (t < 9) {  // column m, component d
+    const int m = t / 3, d = t % 3, sm = m == 0 ? 4 : m == 1 ? 2 : 1, s1 = m == 0 ? 2 : 4, s2 = m == 2 ? 2 : 1;
+    double S[2][2];
+    for (int i = 0; i < 2; i++)
+      for (int j = 0; j < 2; j++)
+        S[i][j] = 0.5 * (vxyz[3 * (long)ev[sm + i * s1 + j * s2] + d] - vxyz[3 * (long)ev[i * s1 + j * s2] + d]);
+    g.G[m][0][d] = 0.25 * ((S[0][0] + S[0][1]) + (S[1][0] + S[1][1]));
+    g.G[m][1][d] = 0.25 * ((S[1][0] + S[1][1]) - (S[0][0] + S[0][1]));
+    g.G[m][2][d] = 0.25 * ((S[0][1] + S[1][1]) - (S[0][0] + S[1][0]));
+    g.G[m][3][d] = 0.25 * ((S[1][1] - S[0][1]) - (S[1][0] - S[0][0]));
+  } else if (t < 17 && kv) {
+    const int c = t - 9;
+    double s = 0;
+    for (int v = 0; v < 8; v++) s += __builtin_popcount(c & ~v) & 1 ? -kv[ev[v]] : kv[ev[v]];
+    g.Gk[c] = 0.125 * s;
+  }
+}
+// Rows J[m] = dX/dx_m of the Jacobian's transpose at (x0, x1, x2); its inverse rows c[m] = grad x_m and determinant.
+__device__ __forceinline__ double q1_inverse(const Q1Geo &g, double x0, double x1, double x2, double (&c)[3][3])
+{
+  double J[3][3];
+  const double a[3] = {x1, x0, x0}, b[3] = {x2, x2, x1};
 #pragma unroll
-    for (int q = 0; q < 8; q++) PU[q] = PG0[q] = PG1[q] = PG2[q] = 0.0;
-    // the state enters the block only through eta(grad u) and s (p != 2) and lambda e^u: for the linear operator
-    // (p = 2, lambda = 0) eta = 1 and s = 0 whatever the state, and its interpolation is skipped
-    const int na = ustate && (ph.p != 2.0 || ph.lambda != 0.0) ? N : 0;
-#pragma unroll 1
-    for (int a = 0; a < na; a++) {
-      double Y[2][2][3];  // [jj][kk][BB | DB | BD]
+  for (int m = 0; m < 3; m++)
 #pragma unroll
-      for (int jj = 0; jj < 2; jj++)
+    for (int d = 0; d < 3; d++)
+      J[m][d] = (g.G[m][0][d] + a[m] * g.G[m][1][d]) + b[m] * (g.G[m][2][d] + a[m] * g.G[m][3][d]);
+  cross3(J[1], J[2], c[0]);
+  cross3(J[2], J[0], c[1]);
+  cross3(J[0], J[1], c[2]);
+  const double det = J[0][0] * c[0][0] + J[0][1] * c[0][1] + J[0][2] * c[0][2], id = recip(det);
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++) Y[jj][kk][0] = Y[jj][kk][1] = Y[jj][kk][2] = 0.0;
-#pragma unroll 1
+  for (int m = 0; m < 3; m++)
+#pragma unroll
+    for (int d = 0; d < 3; d++) c[m][d] *= id;
+  return det;
+}
+
+// Sub-cell matrices of `nel` elements from element `first` on, two threads per GLL sub-cell, n = N nodes per direction:
+// the 36 upper entries K[sym_index] of sub-cell (G0, G1, G2) of the block's sub-cell lattice go to
+// KC[entry * ring + ((G0 % slots) * (M1 p) + G1) * (M2 p) + G2], ring = slots * M1 p * M2 p.
+//  - The state's values and reference gradient at the (2p)^3 points of an element are formed by contractions along z and
+//    y in LDS, shared by its sub-cells, and along x per sub-cell: about 360 multiply-adds per sub-cell at p = 6 where each
+//    sub-cell contracted the whole element's state for itself (1,700).
+//  - The integrand at a point is g_r . M g_c with the basis gradients g, which are products of one-dimensional factors
+//    (-+1 or the two interpolation weights), and one symmetric M, so the sum over the 2 x 2 x 2 points is contracted one
+//    direction at a time: 14 sums over the first direction, 31 over the second, then the 36 entries: about 900 operations
+//    against 36 x 8 x 8 and the gradients.
+//  - A pair of lanes shares a sub-cell, one for each point of the last direction, and exchanges halves of the entries at
+//    the end: one thread with the entries and all partial sums live needs 360 registers (one wavefront per SIMD).
+//  - Four wavefronts a workgroup in two rounds at 249 registers: two workgroups per compute unit, so one's contractions
+//    overlap the other's points (seven wavefronts in one round: 190 us a pass of 663,000 sub-cells against 148).
+// Eight coloured launches that added 64 entries per sub-cell into the stencil, and its clearing, took 6.2 ms at 32^3
+// elements, p = 6 (7.1 M sub-cells); this and the gather below take 2.3 ms (1.5 and 0.7).
+template <int N, bool LAM>
+__global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per_eu(2))) q1_cell_kernel(long first, long nel, int slots,
+                                                                const int *__restrict__ everts,
+                                                                const double *__restrict__ vxyz,
+                                                                const double *__restrict__ kv,
+                                                                const double *__restrict__ ustate, int corrected,
+                                                                const double *__restrict__ tab, Q1Phys ph,
+                                                                const float *__restrict__ cscale,
+                                                                double *__restrict__ KC)
+{
+  constexpr int P = N - 1, NP3 = P * P * P, NQ = 2 * P, NN = N * N, EPB = q1_epb(N), NT = q1_threads(N);
+  constexpr int LZ = q1_lds_z(N), LY = q1_lds_y(N);
+  extern __shared__ double lds[];  // [EPB][LZ], [EPB][LY] (with a state)
+  __shared__ Q1Geo geo[EPB];
+  __shared__ double tb[2 * NQ + P + 2 * NQ * N];  // zq, wq, hsub, B, D
+  const double *zq = tb, *wq = tb + NQ, *hsub = tb + 2 * NQ, *Bs = tb + 2 * NQ + P, *Ds = Bs + NQ * N;
+  const int tid = threadIdx.x;
+  const long e0 = first + (long)blockIdx.x * EPB;
+  const int ne = (int)min((long)EPB, first + nel - e0);
+  for (int t = tid; t < 2 * NQ + P + 2 * NQ * N; t += NT) tb[t] = tab[t];
+  for (int t = tid; t < ne * 17; t += NT) q1_geo(vxyz, ph.has_k ? kv : nullptr, everts + (e0 + t / 17) * 8, t % 17, geo[t / 17]);
+  // the state enters the block only through eta(grad u) and s (p != 2) and lambda e^u: for the linear operator
+  // (p = 2, lambda = 0) eta = 1 and s = 0 whatever the state, and its interpolation is skipped
+  const bool has_u = ustate && (ph.p != 2.0 || LAM);
+  double *Z = lds, *Y = lds + EPB * LZ;
+  if (has_u) {
+    for (int t = tid; t < ne * NN * N; t += NT) {
+      const int l = t / (NN * N), r = t - l * NN * N, a = r / NN, b = (r / N) % N, c = r % N;
+      const long e = e0 + l, ex = e / ((long)ph.M1 * ph.M2), ey = (e / ph.M2) % ph.M1, ez = e % ph.M2;
+      Y[l * LY + r] = ustate[((ex * P + a) * ph.Ly + ey * P + b) * ph.Lz + ez * P + c];
+    }
+    __syncthreads();
+    for (int t = tid; t < ne * NN * NQ; t += NT) {  // along z: values, derivatives
+      const int l = t / (NN * NQ), r = t - l * NN * NQ, ab = r / NQ, q = r - ab * NQ;
+      double v = 0, d = 0;
+#pragma unroll
+      for (int c = 0; c < N; c++) {
+        const double u = Y[l * LY + ab * N + c];
+        v += Bs[q * N + c] * u;
+        d += Ds[q * N + c] * u;
+      }
+      Z[l * LZ + r] = v;
+      Z[l * LZ + NN * NQ + r] = d;
+    }
+    __syncthreads();
+    for (int t = tid; t < ne * N * NQ * NQ; t += NT) {  // along y: (B, B), (D, B), (B, D) in (y, z)
+      const int l = t / (N * NQ * NQ), r = t - l * N * NQ * NQ, a = r / (NQ * NQ), q = r - a * NQ * NQ, qj = q / NQ,
+                qk = q - qj * NQ;
+      const double *z = Z + l * LZ + a * N * NQ + qk;
+      double bb = 0, db = 0, bd = 0;
+#pragma unroll
       for (int b = 0; b < N; b++) {
-        const double *ucol = ustate + lat0 + ((long)a * ph.Ly + b) * ph.Lz;
-        double s00 = 0, s01 = 0, s10 = 0, s11 = 0;  // [kk][B | D]
-#pragma unroll
-        for (int c = 0; c < N; c++) {
-          const double uv = ucol[c];
-          s00 += bz0[c] * uv;
-          s01 += dz0[c] * uv;
-          s10 += bz1[c] * uv;
-          s11 += dz1[c] * uv;
-        }
-        const double B[2] = {by0[b], by1[b]}, D[2] = {dy0[b], dy1[b]};
-#pragma unroll
-        for (int jj = 0; jj < 2; jj++) {
-          Y[jj][0][0] += B[jj] * s00;
-          Y[jj][0][1] += D[jj] * s00;
-          Y[jj][0][2] += B[jj] * s01;
-          Y[jj][1][0] += B[jj] * s10;
-          Y[jj][1][1] += D[jj] * s10;
-          Y[jj][1][2] += B[jj] * s11;
-        }
+        const double v = z[b * NQ], d = z[NN * NQ + b * NQ];
+        bb += Bs[qj * N + b] * v;
+        db += Ds[qj * N + b] * v;
+        bd += Bs[qj * N + b] * d;
       }
-      const double Bx[2] = {bx0[a], bx1[a]}, Dx[2] = {dx0[a], dx1[a]};
+      double *y = Y + l * LY + r;
+      y[0] = bb;
+      y[N * NQ * NQ] = db;
+      y[2 * N * NQ * NQ] = bd;
+    }
+  }
+  __syncthreads();
+  constexpr double WI[2] = {0.78867513459481287, 0.21132486540518713};  // basis values at a sub-cell's two points
+  for (int item = tid; item < 2 * ne * NP3; item += NT) {
+    // pairs of lanes walk (a, b, element, c): runs of consecutive sub-cells along z over neighbouring elements
+    const int t = item >> 1, kk = item & 1, ab = t / (ne * P), rest = t - ab * ne * P, l = rest / P,
+              pc = rest - l * P, pa = ab / P, pb = ab - pa * P;
+    const long e = e0 + l;
+    const int pidx = ab * P + pc;
+    // sub-cell derivative scale per reference direction: 1 (the reference's), 1/h (corrected), times the learned
+    // per-sub-cell factors when given
+    double sx = corrected ? 1.0 / hsub[pa] : 1.0, sy = corrected ? 1.0 / hsub[pb] : 1.0,
+           sz = corrected ? 1.0 / hsub[pc] : 1.0;
+    if (cscale) {
+      const float *s = cscale + 3 * (e * NP3 + pidx);
+      sx *= (double)s[0];
+      sy *= (double)s[1];
+      sz *= (double)s[2];
+    }
+    // sums over the first two directions: 00 [r1 c1], 01 [x][y], 02 [x][r1 c1], 11 [r0 c0], 22 [r0 c0][r1 c1],
+    // 12 [r0 c0][y], and the Bratu term's [r0 c0][r1 c1]; a pair (0 0), (0 1), (1 1) is indexed 0, 1, 2
+    double B00[3] = {0, 0, 0}, B01[2][2] = {{0, 0}, {0, 0}}, B02[2][3] = {{0, 0, 0}, {0, 0, 0}}, B11[3] = {0, 0, 0},
+           B22[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, B12[3][2] = {{0, 0}, {0, 0}, {0, 0}},
+           BL[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const int ii = q >> 2, jj = (q >> 1) & 1, kk = q & 1;
-        PU[q] += Bx[ii] * Y[jj][kk][0];
-        PG0[q] += Dx[ii] * Y[jj][kk][0];
-        PG1[q] += Bx[ii] * Y[jj][kk][1];
-        PG2[q] += Bx[ii] * Y[jj][kk][2];
+    for (int pt = 0; pt < 4; pt++) {
+      const int ii = pt & 1, jj = pt >> 1, qi = 2 * pa + ii, qj = 2 * pb + jj, qk = 2 * pc + kk;
+      {
+        double U = 0, G0 = 0, G1 = 0, G2 = 0;
+        if (has_u) {
+          const double *y = Y + l * LY + qj * NQ + qk, *bx = Bs + qi * N, *dx = Ds + qi * N;
+#pragma unroll
+          for (int a = 0; a < N; a++) {
+            const double y0 = y[a * NQ * NQ], y1 = y[(N + a) * NQ * NQ], y2 = y[(2 * N + a) * NQ * NQ];
+            if (LAM) U += bx[a] * y0;
+            G0 += dx[a] * y0;
+            G1 += bx[a] * y1;
+            G2 += bx[a] * y2;
+          }
+        }
+        int lg = l;  // the element's polynomials are read here, not kept in registers over the loops
+        asm volatile("" : "+v"(lg));
+        const Q1Geo &g = geo[lg];
+        const double x0 = zq[qi], x1 = zq[qj], x2 = zq[qk];
+        double Ji[3][3], cj[3][3];
+        const double det = q1_inverse(g, x0, x1, x2, Ji);
+        const double w = wq[qi] * wq[qj] * wq[qk] * det;
+        double kq = 1.0;
+        if (ph.has_k)
+          kq = ((g.Gk[0] + x2 * g.Gk[1]) + x1 * (g.Gk[2] + x2 * g.Gk[3])) +
+               x0 * ((g.Gk[4] + x2 * g.Gk[5]) + x1 * (g.Gk[6] + x2 * g.Gk[7]));
+        if (corrected) {  // the inverse Jacobian at the point itself
+#pragma unroll
+          for (int m = 0; m < 3; m++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) cj[m][d] = Ji[m][d];
+        } else {  // element-natural point pidx*8+q, decoded on the (2p)^3 sparse lattice
+          const int qe = pidx * 8 + ii * 4 + jj * 2 + kk;
+          q1_inverse(g, zq[qe / (NQ * NQ)], zq[(qe / NQ) % NQ], zq[qe % NQ], cj);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          cj[0][d] *= sx;
+          cj[1][d] *= sy;
+          cj[2][d] *= sz;
+        }
+        // EllipPointwiseComputeStore (ellip.c:333-343) with the coefficient factor
+        double etaw = w * kq, sm[3] = {0, 0, 0};
+        if (has_u) {
+          double Du[3];
+#pragma unroll
+          for (int d = 0; d < 3; d++) Du[d] = G0 * Ji[0][d] + G1 * Ji[1][d] + G2 * Ji[2][d];
+          const double espg = ph.eps2 + 0.5 * (Du[0] * Du[0] + Du[1] * Du[1] + Du[2] * Du[2]);
+          const double ex = (ph.p - 2) / 2, eta = powe(espg, ex, ph.qpow);
+          const double smdc = sqrt_pos(-ex * eta * recip(espg)) * sqrt_pos(kq);
+#pragma unroll
+          for (int d = 0; d < 3; d++) sm[d] = smdc * Du[d];
+          etaw *= eta;
+        }
+        // EllipPointwiseJacobian (ellip.c:369-377): g_r . M g_c, M_mn = eta w c_m . c_n - w (s . c_m)(s . c_n)
+        double tm[3], M[3][3];
+#pragma unroll
+        for (int m = 0; m < 3; m++) tm[m] = sm[0] * cj[m][0] + sm[1] * cj[m][1] + sm[2] * cj[m][2];
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+#pragma unroll
+          for (int n = m; n < 3; n++)
+            M[m][n] = etaw * (cj[m][0] * cj[n][0] + cj[m][1] * cj[n][1] + cj[m][2] * cj[n][2]) - w * tm[m] * tm[n];
+        const double u[2] = {WI[ii], WI[1 - ii]}, v[2] = {WI[jj], WI[1 - jj]};
+        const double f[3] = {u[0] * u[0], u[0] * u[1], u[1] * u[1]}, g2[3] = {v[0] * v[0], v[0] * v[1], v[1] * v[1]};
+        double lw = 0;
+        if constexpr (LAM) lw = -w * (ph.lambda * q1_exp(U));
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          B00[c] += g2[c] * M[0][0];
+          B11[c] += f[c] * M[1][1];
+#pragma unroll
+          for (int d = 0; d < 2; d++) {
+            B02[d][c] += (u[d] * g2[c]) * M[0][2];
+            B12[c][d] += (f[c] * v[d]) * M[1][2];
+          }
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            B22[c][d] += (f[c] * g2[d]) * M[2][2];
+            if (LAM) BL[c][d] += (f[c] * g2[d]) * lw;
+          }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+          for (int d = 0; d < 2; d++) B01[c][d] += (u[c] * v[d]) * M[0][1];
       }
+      __builtin_amdgcn_sched_barrier(0);  // (points one after another: fewer registers)
     }
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      PD[q][lt] = PU[q];
-      PD[8 + q][lt] = PG0[q];
-      PD[16 + q][lt] = PG1[q];
-      PD[24 + q][lt] = PG2[q];
-    }
+    const double h[2] = {kk ? WI[1] : WI[0], kk ? WI[0] : WI[1]};
+    const auto entry = [&](auto T) {  // this point's share of entry T
+      constexpr int r = sym_row(decltype(T)::value), c = sym_col(decltype(T)::value);
+      constexpr int r0 = r >> 2, r1 = (r >> 1) & 1, r2 = r & 1, c0 = c >> 2, c1 = (c >> 1) & 1, c2 = c & 1;
+      constexpr int x = r0 + c0, y = r1 + c1;  // pair indices
+      const auto sg = [](int i, int j) { return i == j ? 1.0 : -1.0; };
+      double in = sg(r0, c0) * B00[y] + sg(r1, c1) * B11[x] + (sg(r0, c1) * B01[c0][r1] + sg(r1, c0) * B01[r0][c1]);
+      if (LAM) in += BL[x][y];
+      return h[r2] * h[c2] * in + sg(r2, c2) * B22[x][y] +
+             h[r2] * (sg(r0, c2) * B02[c0][y] + sg(r1, c2) * B12[x][c1]) +
+             h[c2] * (sg(r2, c0) * B02[r0][y] + sg(r2, c1) * B12[x][r1]);
+    };
+    const int ex = (int)(e / ((long)ph.M1 * ph.M2)), ey = (int)((e / ph.M2) % ph.M1), ez = (int)(e % ph.M2);
+    const long G1 = (long)ph.M1 * P, G2 = (long)ph.M2 * P, ring = slots * G1 * G2;
+    double *out = KC + (kk ? 18 * ring : 0) + ((long)((ex * P + pa) % slots) * G1 + ey * P + pb) * G2 + ez * P + pc;
+    // lane 0 of the pair stores the first 18 entries, lane 1 the others, each with the other lane's point added
+    static_for(std::make_integer_sequence<int, 18>(), [&](auto T) {
+      constexpr int i = decltype(T)::value;
+      const double k0 = entry(std::integral_constant<int, i>()), k1 = entry(std::integral_constant<int, 18 + i>());
+      out[i * ring] = (kk ? k1 : k0) + pair_swap(kk ? k0 : k1);
+      __builtin_amdgcn_sched_barrier(0);  // (entries are formed one after another: fewer registers)
+    });
   }
-  const double i1[2][2] = {{0.78867513459481287, 0.21132486540518713}, {0.21132486540518713, 0.78867513459481287}};
-  const double d1[2][2] = {{-1., 1.}, {-1., 1.}};
-  // sub-cell derivative scale per reference direction: 1 (the reference's), 1/h (corrected), times the learned
-  // per-sub-cell factors when given
-  double sx = corrected ? 1.0 / hsub[pa] : 1.0, sy = corrected ? 1.0 / hsub[pb] : 1.0,
-         sz = corrected ? 1.0 / hsub[pc] : 1.0;
-  if (cscale) {
-    sx *= (double)cscale[3 * tid];
-    sy *= (double)cscale[3 * tid + 1];
-    sz *= (double)cscale[3 * tid + 2];
-  }
-  // the block is symmetric (EllipPointwiseJacobian below gives K[r][c] = -w lambda e^u I_r I_c + eta w D_r.D_c
-  // - w (s.D_r)(s.D_c)): its upper triangle, row-major, is accumulated
-  double K[36];
-#pragma unroll
-  for (int t = 0; t < 36; t++) K[t] = 0.0;
-#pragma unroll 1
-  for (int q = 0; q < 8; q++) {
-    const int ii = q >> 2, jj = (q >> 1) & 1, kk = q & 1;
-    const int qi = 2 * pa + ii, qj = 2 * pb + jj, qk = 2 * pc + kk;
-    double X[8][3];  // (read here, through the caches, so that they are not live in the block's accumulation)
-    for (int t = 0; t < 8; t++)
-      for (int d = 0; d < 3; d++) X[t][d] = vxyz[3 * (long)ev[t] + d];
-    double J[3][3], Ji[3][3], cj[3][3];
-    jac_at(X, zq[qi], zq[qj], zq[qk], J);
-    const double det = invert3(J, Ji);
-    const double w = wq[qi] * wq[qj] * wq[qk] * det;
-    const double g0 = PD[8 + q][lt], g1 = PD[16 + q][lt], g2 = PD[24 + q][lt];
-    double Du[3];
-    for (int d = 0; d < 3; d++) Du[d] = g0 * Ji[0][d] + g1 * Ji[1][d] + g2 * Ji[2][d];
-    double kq = 0;
-    {
-      const double f0[2] = {0.5 * (1 - zq[qi]), 0.5 * (1 + zq[qi])};
-      const double f1[2] = {0.5 * (1 - zq[qj]), 0.5 * (1 + zq[qj])};
-      const double f2[2] = {0.5 * (1 - zq[qk]), 0.5 * (1 + zq[qk])};
-      for (int t = 0; t < 8; t++) kq += (ph.has_k ? kv[ev[t]] : 1.0) * f0[t >> 2] * f1[(t >> 1) & 1] * f2[t & 1];
-    }
-    if (corrected) {  // the inverse Jacobian at the point itself
-      for (int r = 0; r < 3; r++)
-        for (int d = 0; d < 3; d++) cj[r][d] = Ji[r][d];
-    } else {  // element-natural point pidx*8+q, decoded on the (2p)^3 sparse lattice
-      const int qe = pidx * 8 + q;
-      const int ei = qe / (NQ * NQ), ej = (qe / NQ) % NQ, ek = qe % NQ;
-      double J2[3][3];
-      jac_at(X, zq[ei], zq[ej], zq[ek], J2);
-      invert3(J2, cj);
-    }
-    // EllipPointwiseComputeStore (ellip.c:333-343) with the coefficient factor
-    const double gamma = 0.5 * (Du[0] * Du[0] + Du[1] * Du[1] + Du[2] * Du[2]);
-    const double espg = ph.eps2 + gamma;
-    double eta = q1_pow(espg, (ph.p - 2) / 2);
-    const double smdc = sqrt(-((ph.p - 2) / 2) * eta / espg) * sqrt(kq);
-    eta *= kq;
-    const double smd[3] = {smdc * Du[0], smdc * Du[1], smdc * Du[2]};
-    const double lexp = ph.lambda != 0 ? ph.lambda * q1_exp(PD[q][lt]) : 0.0;
-    double I8[8], D8[8][3];
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      const int a0 = b >> 2, a1 = (b >> 1) & 1, a2 = b & 1;
-      const double dX = sx * d1[ii][a0] * i1[jj][a1] * i1[kk][a2];
-      const double dY = sy * i1[ii][a0] * d1[jj][a1] * i1[kk][a2];
-      const double dZ = sz * i1[ii][a0] * i1[jj][a1] * d1[kk][a2];
-      I8[b] = i1[ii][a0] * i1[jj][a1] * i1[kk][a2];
-#pragma unroll
-      for (int d = 0; d < 3; d++) D8[b][d] = dX * cj[0][d] + dY * cj[1][d] + dZ * cj[2][d];
-    }
-    // EllipPointwiseJacobian (ellip.c:369-377) on basis function c, tested against basis function r:
-    // v_c = -w lambda e^u I_c, Dv_c = eta w D_c - w (s.D_c) s
-    const double etaw = eta * w, lw = -w * lexp;
-    double sd[8];
-#pragma unroll
-    for (int b = 0; b < 8; b++) sd[b] = smd[0] * D8[b][0] + smd[1] * D8[b][1] + smd[2] * D8[b][2];
-#pragma unroll
-    for (int r = 0, t = 0; r < 8; r++)
-#pragma unroll
-      for (int c = r; c < 8; c++, t++)
-        K[t] += I8[r] * (lw * I8[c]) + etaw * (D8[r][0] * D8[c][0] + D8[r][1] * D8[c][1] + D8[r][2] * D8[c][2]) -
-                w * sd[r] * sd[c];
-  }
-  const int *en = &enodes[e * N * N * N];
-  int gidx[8];
-#pragma unroll
-  for (int b = 0; b < 8; b++) {
-    const int a0 = b >> 2, a1 = (b >> 1) & 1, a2 = b & 1;
-    gidx[b] = en[((pa + a0) * N + pb + a1) * N + pc + a2];
-  }
+}
+
+// Rows of the 27-point stencil st[27][n] on node planes plane0 .. of the lattice, from the sub-cell matrices of the
+// sub-cells around them: a thread adds the diagonal and the 13 upper entries of its row (36 values, each sub-cell entry
+// read once) and also stores each upper entry as the lower one of that neighbour's row; entries toward nodes that are not
+// owned are zero.  I0, J0, K0: first owned node of the lattice; G: sub-cells per direction.
+__global__ void __launch_bounds__(256) q1_gather_kernel(int plane0, int slots, int I0, int J0, int K0, int nx, int ny,
+                                                        int nz, int G0, int G1, int G2, const double *__restrict__ KC,
+                                                        double *__restrict__ st)
+{
+  const int K = blockIdx.x * 64 + threadIdx.x, J = blockIdx.y * 4 + threadIdx.y, I = plane0 + blockIdx.z - I0;
+  if (K >= nz || J >= ny || I < 0 || I >= nx) return;
+  const long n = (long)nx * ny * nz, i = ((long)I * ny + J) * nz + K, ring = (long)slots * G1 * G2;
+  // sub-cell (node - r) for each corner r of it that this node is (clamped: one outside the block adds nothing)
+  long cell[8];
+  bool has[8];
 #pragma unroll
   for (int r = 0; r < 8; r++) {
-    const int gr = gidx[r];
-    if (gr >= nowned) continue;
-    if (st) {  // stencil form [27][rows]: the entry's slot is the lattice offset from the row node
+    const int a = I + I0 - (r >> 2), b = J + J0 - ((r >> 1) & 1), c = K + K0 - (r & 1);
+    has[r] = a >= 0 && a < G0 && b >= 0 && b < G1 && c >= 0 && c < G2;
+    cell[r] = has[r] ? ((long)(a % slots) * G1 + b) * G2 + c : 0;
+  }
 #pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int gc = gidx[c];
-        if (gc >= nowned) continue;
-        const int sl = ((c >> 2) - (r >> 2) + 1) * 9 + (((c >> 1) & 1) - ((r >> 1) & 1) + 1) * 3 + ((c & 1) - (r & 1) + 1);
-        st[sl * nowned + gr] += K[sym_index(r, c)];  // (no other sub-cell of this colour holds the entry)
-      }
-    } else {
-      const int lo = rowptr[gr], hi = rowptr[gr + 1];
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int gc = gidx[c];
-        if (gc >= nowned) continue;
-        val[find_col(colidx, lo, hi, gc)] += K[sym_index(r, c)];
-      }
+  for (int s = 0; s < 27; s++) {
+    const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
+    const bool in = I + di >= 0 && I + di < nx && J + dj >= 0 && J + dj < ny && K + dk >= 0 && K + dk < nz;
+    if (s < 13) {  // written by the lower neighbour's row, or zero
+      if (!in) st[s * n + i] = 0.0;
+      continue;
     }
+    double v = 0.0;
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      const int c0 = (r >> 2) + di, c1 = ((r >> 1) & 1) + dj, c2 = (r & 1) + dk;
+      if (c0 < 0 || c0 > 1 || c1 < 0 || c1 > 1 || c2 < 0 || c2 > 1) continue;
+      const double k = KC[sym_index(r, c0 * 4 + c1 * 2 + c2) * ring + cell[r]];
+      v += has[r] ? k : 0.0;
+    }
+    st[s * n + i] = in ? v : 0.0;
+    if (s > 13 && in) st[(26 - s) * n + i + ((long)di * ny + dj) * nz + dk] = v;
   }
 }
 
@@ -333,22 +446,10 @@ __global__ void csr_diag_kernel(long nrows, const int *__restrict__ rowptr, cons
   d[r] = s;
 }
 
-__global__ void to_f32_kernel(const double *__restrict__ a, float *__restrict__ b, long n)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) b[i] = (float)a[i];
-}
-
 __global__ void copy_f64_kernel(const double *__restrict__ a, double *__restrict__ b, long n)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) b[i] = a[i];
-}
-
-__global__ void zero_f64_kernel(double *__restrict__ a, long n)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = 0.0;
 }
 
 // GLL node a of the element from the sub-interval widths.
@@ -607,6 +708,34 @@ static dErr build_pattern(dohpFS fs, _p_dohpMat *A)
   return 0;
 }
 
+namespace {
+
+// Ring of sub-cell matrices of an assembly: as many layers of elements per pass as keep it in the 256 MB cache, so that
+// the gather does not read them from HBM (32^3 elements, p = 6: 96 MB 2.61 ms, 192 MB 2.31, 512 MB 2.64, one pass 3.02).
+constexpr size_t kQ1RingBytes = (size_t)192 << 20;
+
+template <typename F>
+dErr q1_dispatch(int n, F f)
+{
+  switch (n) {
+  case 2: f(std::integral_constant<int, 2>()); break;
+  case 3: f(std::integral_constant<int, 3>()); break;
+  case 4: f(std::integral_constant<int, 4>()); break;
+  case 5: f(std::integral_constant<int, 5>()); break;
+  case 6: f(std::integral_constant<int, 6>()); break;
+  case 7: f(std::integral_constant<int, 7>()); break;
+  case 8: f(std::integral_constant<int, 8>()); break;
+  case 9: f(std::integral_constant<int, 9>()); break;
+  case 10: f(std::integral_constant<int, 10>()); break;
+  case 11: f(std::integral_constant<int, 11>()); break;
+  default: set_error("embedded-Q1 assembly supports degree 1..10"); return dohpERR_ARG;
+  }
+  DOHP_HIP(hipGetLastError());
+  return 0;
+}
+
+}  // namespace
+
 extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out, void *stream)
 {
   DOHP_CHECK(op && out, dohpERR_ARG, "null argument");
@@ -631,91 +760,73 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
     }
     *out = A;
   }
-  Q1Tab tb;
-  tb.p = fs->p;
-  tb.n = fs->n;
-  tb.corrected = q1mode;
   A->corrected = q1mode;
   A->scaled = cscale != nullptr;
-  {
-    double zg[kMaxN], wg[kMaxN];
+  if (A->q1tab_degree != fs->p) {  // 1-D tables of the degree: zq, wq (2p each), hsub (p), Bs, Ds (2p x n each)
+    double zg[kMaxN], wg[kMaxN], zq[2 * kMaxP], wq[2 * kMaxP];
     gauss_lobatto(fs->n, zg, wg);
-    for (int i = 0; i < fs->p; i++) tb.hsub[i] = zg[i + 1] - zg[i];
+    int nq;
+    DOHP_CALL(dohpTensorRule(dQUADRATURE_METHOD_SPARSE, dGAUSS_LEGENDRE, 2 * fs->p, &nq, zq, wq));
+    std::vector<double> Bs(nq * fs->n), Ds(nq * fs->n), tab(zq, zq + nq);
+    DOHP_CALL(dohpTensorBasis(fs->n, nq, zq, Bs.data(), Ds.data(), nullptr, nullptr));
+    tab.insert(tab.end(), wq, wq + nq);
+    for (int i = 0; i < fs->p; i++) tab.push_back(zg[i + 1] - zg[i]);
+    tab.insert(tab.end(), Bs.begin(), Bs.end());
+    tab.insert(tab.end(), Ds.begin(), Ds.end());
+    A->q1tab_degree = 0;
+    DOHP_CALL(A->q1tab.upload(tab.data(), tab.size()));
+    A->q1tab_degree = fs->p;
   }
-  int nq;
-  DOHP_CALL(dohpTensorRule(dQUADRATURE_METHOD_SPARSE, dGAUSS_LEGENDRE, 2 * fs->p, &nq, tb.zq, tb.wq));
-  tb.nq = nq;
-  std::vector<double> Bs(nq * fs->n), Ds(nq * fs->n);
-  DOHP_CALL(dohpTensorBasis(fs->n, nq, tb.zq, Bs.data(), Ds.data(), nullptr, nullptr));
-  for (int q = 0; q < nq; q++)
-    for (int a = 0; a < fs->n; a++) {
-      tb.Bs[q][a] = Bs[q * fs->n + a];
-      tb.Ds[q][a] = Ds[q * fs->n + a];
-    }
-  Q1Phys ph{prm.p, prm.epsilon * prm.epsilon, prm.lambda, kvert != nullptr, fs->M[1], fs->M[2],
+  const double q4 = 2.0 * (prm.p - 2.0);
+  Q1Phys ph{prm.p, prm.epsilon * prm.epsilon, prm.lambda, kvert != nullptr,
+            q4 == std::floor(q4) && std::fabs(q4) <= 8.0 ? (int)q4 : 99, fs->M[1], fs->M[2],
             fs->p * fs->M[1] + 1, fs->p * fs->M[2] + 1};
-  const long nt = (long)fs->nelem * fs->p * fs->p * fs->p;
-  // On a block space the owned nodes form a box and the matrix is a 27-point stencil: the sub-cells add into the
-  // stencil form directly (at computed slots, colour by colour), and the CSR values are read back from it.
+  // On a block space the owned nodes form a box and the matrix is a 27-point stencil (without owned nodes there is
+  // nothing to assemble); the CSR values are read back from it on demand.
   bool box = false;
   DOHP_CALL(dohpMatPrepareStencil_Private(A, fs, &box, st));
-  if (box) {
-    hipLaunchKernelGGL(zero_f64_kernel, dim3((27 * A->nrows + 255) / 256), dim3(256), 0, st, A->st64.ptr,
-                       27 * A->nrows);
-  } else {
-    hipLaunchKernelGGL(zero_f64_kernel, dim3((A->nnz + 255) / 256), dim3(256), 0, st, A->val.ptr, A->nnz);
+  A->csr_stale = box;
+  if (!box) return 0;
+  // Layers of elements per pass: the sub-cell matrices of a pass (288 bytes per sub-cell) and of the layer of sub-cells
+  // before it are kept in a ring of layers.
+  const int G[3] = {fs->M[0] * fs->p, fs->M[1] * fs->p, fs->M[2] * fs->p};
+  const size_t layer = (size_t)G[1] * G[2] * 36;
+  int lx = (int)std::min<size_t>(fs->M[0], std::max<size_t>(1, kQ1RingBytes / (8 * layer * fs->p)));
+  int slots = 0;
+  for (;; lx = (lx + 1) / 2) {
+    slots = lx * fs->p + 1;
+    if (A->q1ring.n >= slots * layer) break;
+    const dErr err = A->q1ring.alloc(slots * layer);
+    if (!err) break;
+    if (err != dohpERR_OOM || lx == 1) return err;
   }
-  {  // 1-D tables for the kernel: zq, wq (2p each), hsub (p), Bs, Ds (2p x n each)
-    const int nq2 = tb.nq, pp = tb.p, nn = tb.n;
-    std::vector<double> tab;
-    tab.insert(tab.end(), tb.zq, tb.zq + nq2);
-    tab.insert(tab.end(), tb.wq, tb.wq + nq2);
-    tab.insert(tab.end(), tb.hsub, tb.hsub + pp);
-    for (int q = 0; q < nq2; q++) tab.insert(tab.end(), tb.Bs[q], tb.Bs[q] + nn);
-    for (int q = 0; q < nq2; q++) tab.insert(tab.end(), tb.Ds[q], tb.Ds[q] + nn);
-    if (!A->q1tab.holds(tab.size())) DOHP_CALL(A->q1tab.alloc(tab.size()));
-    DOHP_HIP(hipMemcpyAsync(A->q1tab.ptr, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice, st));
-    DOHP_HIP(hipStreamSynchronize(st));  // the host vector goes out of scope
+  const int m = fs->dirichlet_mask, I0 = m & 1, K0 = (m >> 2) & 1;
+  const dim3 gg((A->box[2] + 63) / 64, (A->box[1] + 3) / 4);
+  for (int x0 = 0; x0 < fs->M[0]; x0 += lx) {
+    const int x1 = std::min(fs->M[0], x0 + lx);
+    const long first = (long)x0 * fs->M[1] * fs->M[2], nel = (long)(x1 - x0) * fs->M[1] * fs->M[2];
+    DOHP_CALL(q1_dispatch(fs->n, [&](auto NN) {
+      constexpr int N = decltype(NN)::value;
+      const bool has_u = state && (prm.p != 2.0 || prm.lambda != 0.0);
+      const size_t lds = has_u ? sizeof(double) * q1_epb(N) * (q1_lds_z(N) + q1_lds_y(N)) : 0;
+      const dim3 grid((unsigned)((nel + q1_epb(N) - 1) / q1_epb(N)));
+      auto go = [&](auto kernel) {
+        if (lds > 65536)
+          (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipLaunchKernelGGL(kernel, grid, dim3(q1_threads(N)), lds, st, first, nel, slots, fs->d_elem_verts.ptr,
+                           fs->d_vcoords.ptr, kvert, state, q1mode, A->q1tab.ptr, ph, cscale, A->q1ring.ptr);
+      };
+      if (prm.lambda != 0.0)
+        go(q1_cell_kernel<N, true>);
+      else
+        go(q1_cell_kernel<N, false>);
+    }));
+    // node planes whose sub-cells are all there: up to the pass's last layer of sub-cells, and the block's last plane
+    const int p0 = x0 * fs->p, p1 = x1 == fs->M[0] ? G[0] + 1 : x1 * fs->p;
+    hipLaunchKernelGGL(q1_gather_kernel, dim3(gg.x, gg.y, p1 - p0), dim3(64, 4), 0, st, p0, slots, I0, I0, K0, A->box[0],
+                       A->box[1], A->box[2], G[0], G[1], G[2], A->q1ring.ptr, A->st64.ptr);
+    DOHP_HIP(hipGetLastError());
   }
-  (void)nt;
-  double *stp = box ? A->st64.ptr : nullptr;
-  for (int color = 0; color < 8; color++) {
-  CellColor cc;
-  for (int d = 0; d < 3; d++) {
-    cc.c[d] = (color >> (2 - d)) & 1;
-    const int G = fs->M[d] * fs->p;  // sub-cells per direction
-    cc.cnt[d] = G > cc.c[d] ? (G - cc.c[d] + 1) / 2 : 0;
-  }
-  if (cc.n() == 0) continue;
-  const dim3 grid((unsigned)((cc.n() + 127) / 128));
-  switch (fs->n) {
-#define DOHP_CASE(NN)                                                                                              \
-  case NN:                                                                                                         \
-    hipLaunchKernelGGL(q1_cell_kernel<NN>, grid, dim3(128), 0, st, fs->nelem, fs->d_elem_nodes.ptr,               \
-                       fs->d_elem_verts.ptr, fs->d_vcoords.ptr, kvert, state, fs->nowned, A->rowptr.ptr, A->col.ptr, \
-                       A->val.ptr, stp, tb.corrected, A->q1tab.ptr, ph, cscale, cc);                              \
-    break;
-    DOHP_CASE(2)
-    DOHP_CASE(3)
-    DOHP_CASE(4)
-    DOHP_CASE(5)
-    DOHP_CASE(6)
-    DOHP_CASE(7)
-    DOHP_CASE(8)
-    DOHP_CASE(9)
-    DOHP_CASE(10)
-    DOHP_CASE(11)
-#undef DOHP_CASE
-  default: set_error("embedded-Q1 assembly supports degree 1..10"); return dohpERR_ARG;
-  }
-  DOHP_HIP(hipGetLastError());
-  }
-  if (box) {  // the multigrid and the FP64 product read the stencil form; the CSR values follow on demand
-    A->csr_stale = true;
-    return 0;
-  }
-  hipLaunchKernelGGL(to_f32_kernel, dim3((A->nnz + 255) / 256), dim3(256), 0, st, A->val.ptr, A->val32.ptr, A->nnz);
-  DOHP_HIP(hipGetLastError());
   return 0;
 }
 
@@ -793,30 +904,6 @@ extern "C" dErr dohpMatDestroy(dohpMat *A)
 }
 
 // ------------------------------------------------------ learned sub-cell scales of the embedded-Q1 matrix
-
-namespace {
-
-template <typename F>
-dErr q1_dispatch(int n, F f)
-{
-  switch (n) {
-  case 2: f(std::integral_constant<int, 2>()); break;
-  case 3: f(std::integral_constant<int, 3>()); break;
-  case 4: f(std::integral_constant<int, 4>()); break;
-  case 5: f(std::integral_constant<int, 5>()); break;
-  case 6: f(std::integral_constant<int, 6>()); break;
-  case 7: f(std::integral_constant<int, 7>()); break;
-  case 8: f(std::integral_constant<int, 8>()); break;
-  case 9: f(std::integral_constant<int, 9>()); break;
-  case 10: f(std::integral_constant<int, 10>()); break;
-  case 11: f(std::integral_constant<int, 11>()); break;
-  default: set_error("embedded-Q1 assembly supports degree 1..10"); return dohpERR_ARG;
-  }
-  DOHP_HIP(hipGetLastError());
-  return 0;
-}
-
-}  // namespace
 
 extern "C" dErr dohpQ1CellCount(dohpEllip op, long *ncell)
 {
