@@ -366,8 +366,7 @@ def efs_apply_hex_batched(P, rcoord, nelem, jinv, D, x, y, amode, imode=INSERT_V
 
 
 def efs_apply_hex_batched_noalloc(P, rcoord, nelem, jinv, D, x, y, amode, imode=INSERT_VALUES, stream=None):
-    """dEFSApplyHexBatched without device allocation (tables staged in the library's per-GPU array); returns
-    without waiting for the stream."""
+    """dEFSApplyHexBatched without device allocation; returns without waiting for the stream."""
     rc, rcp = _np(rcoord)
     check(_lib.dEFSApplyHexBatchedNoAlloc(P, rc.size, rcp, nelem, _ptr(jinv), D, _ptr(x), _ptr(y), amode, imode,
                                           _stream(stream)))

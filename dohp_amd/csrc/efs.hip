@@ -1,10 +1,8 @@
 // Batched dEFSApply for isotropic tensor-product hexahedra (dEFSApply_Tensor_Hex,
 // src/jacobi/impls/tensor/efstopo.c:368-423, with TensorMult_Hex_nounroll,
 // src/jacobi/impls/tensor/inlinetmulthex.h:19-100, and the geometry mappings of
-// efstopo.c:518-623).  One workgroup per element; each 1-D contraction is one pass over
-// an LDS tile, components of a block size D > 1 are processed one at a time.
+// efstopo.c:518-623).
 #include <algorithm>
-#include <mutex>
 #include <vector>
 
 #include "common.h"
@@ -13,107 +11,193 @@ using namespace dohp;
 
 namespace {
 
-// dst (dims nout) = A applied along `dim` of src (dims nin).  A is [nout][nin] row-major
-// (leading dimension lda) or, when trans, [nin][nout] read transposed.
-__device__ void contract(const double *A, bool trans, int lda, int dim, const int nin[3], const int nout[3],
-                         const double *src, double *dst)
+constexpr int kEfsMaxP = 12;
+constexpr int kEfsTab = 2 * kEfsMaxP * kEfsMaxP;  // B and D, [out][in] each
+
+// Arguments of one launch, tables included (2.4 KB of kernel arguments, read as scalars: no device copy of the tables, so
+// calls need no allocation and do not share anything).  a: length of the contracted lines, b: length of the results.
+struct EfsArgs {
+  int b, D, dc, nelem, epb, add;
+  const double *jinv, *in;
+  double *out;
+  double tab[kEfsTab];
+};
+enum { EFS_INTERP, EFS_GRAD, EFS_GRAD_T };
+
+__host__ __device__ constexpr int odd(int n) { return n | 1; }
+// LDS of one element with dc components (doubles): region 0, then region 1 (see efs_kernel).
+__host__ __device__ constexpr int efs_r0(int mode, int a, int b, int dc)
 {
-  const int total = nout[0] * nout[1] * nout[2];
-  for (int t = threadIdx.x; t < total; t += blockDim.x) {
-    int o[3] = {t / (nout[1] * nout[2]), (t / nout[2]) % nout[1], t % nout[2]};
-    const int od = o[dim];
-    double s = 0.0;
-    for (int i = 0; i < nin[dim]; i++) {
-      o[dim] = i;
-      const double a = trans ? A[i * lda + od] : A[od * lda + i];
-      s += a * src[(o[0] * nin[1] + o[1]) * nin[2] + o[2]];
-    }
-    dst[t] = s;
-  }
-  __syncthreads();
+  const int pz = odd(b * dc), pa = odd(a * dc), x = a * a * pa;
+  if (mode == EFS_GRAD_T) return 3 * b * a * pa > b * b * b * dc ? 3 * b * a * pa : b * b * b * dc;
+  const int y = (mode == EFS_GRAD ? 3 : 1) * a * b * pz;
+  return x > y ? x : y;
+}
+__host__ __device__ constexpr int efs_r1(int mode, int a, int b, int dc)
+{
+  return mode == EFS_GRAD_T ? 2 * b * b * odd(a * dc) : (mode == EFS_GRAD ? 2 : 1) * a * a * odd(b * dc);
 }
 
-// Three passes (dim 0, 1, 2) from an (a,a,a) tile to a (b,b,b) tile; result lands in w0.
-__device__ void tensor3(const double *A0, const double *A1, const double *A2, bool trans, int lda, int a, int b,
-                        double *w0, double *w1)
+// out(q) = sum_m M[q][m] in[m] for a line held in registers; the row of M is uniform over the workgroup
+template <int A>
+__device__ __forceinline__ double row_dot(const double *M, int q, const double (&in)[A])
 {
-  const int s0[3] = {a, a, a}, s1[3] = {b, a, a}, s2[3] = {b, b, a}, s3[3] = {b, b, b};
-  contract(A0, trans, lda, 0, s0, s1, w0, w1);
-  contract(A1, trans, lda, 1, s1, s2, w1, w0);
-  contract(A2, trans, lda, 2, s2, s3, w0, w1);
-  const int n = b * b * b;
-  for (int t = threadIdx.x; t < n; t += blockDim.x) w0[t] = w1[t];
-  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int m = 0; m < A; m++) s = fma(M[q * A + m], in[m], s);
+  return s;
 }
 
-__global__ void efs_apply_kernel(int P, int Q, const double *__restrict__ tab, const double *__restrict__ jinv, int D,
-                                 const double *__restrict__ in, double *__restrict__ out, int amode, int imode)
+// A workgroup takes epb elements, dc components at a time.  Values keep the reference's order [i][j][k][d] in LDS; every
+// pass contracts one index of one line per thread, the line in registers and the table row as scalar operands, so an
+// element's tables are read once per line and no value is read from LDS more than once per pass.  The gradient shares
+// its partial products (8 line passes instead of 9 full contractions of three):
+//   forward:  along k: B x, D x;  along j: B, D of the first, B of the second;  along i: D, B, B, straight to the output
+//   transpose: along i: the mapped fluxes, straight from the input, D^T, B^T, B^T;  along j: B^T + D^T, B^T;  along k.
+// Rows of lines along k have an odd pitch (bank conflicts at even lengths).  What bounds it is the bytes: input, inverse
+// Jacobians and output once each.  8192 elements, P = Q = 7, D = 1, gradient with inverse Jacobians (292 MB): 221 -> 65 us
+// (4.5 TB/s) against three full contractions per component out of LDS with the output updated once per direction; 1500
+// elements, P = 4, Q = 5, D = 3, transposed gradient (29 MB): 28.0 -> 9.2 us.
+template <int A, int MODE, bool ONE>
+__global__ void __launch_bounds__(256) efs_kernel(EfsArgs g)
 {
-  extern __shared__ double sm[];
-  const int M = P > Q ? P : Q, M3 = M * M * M;
-  double *sB = sm, *sD = sm + Q * P, *w0 = sD + Q * P, *w1 = w0 + M3, *acc = w1 + M3;
-  for (int t = threadIdx.x; t < 2 * Q * P; t += blockDim.x) sm[t] = tab[t];
-  __syncthreads();
-  const long e = blockIdx.x;
-  const int P3 = P * P * P, Q3 = Q * Q * Q;
-  const bool add = imode == dADD_VALUES;
-  switch (amode) {
-  case dAPPLY_INTERP:
-  case dAPPLY_INTERP_TRANSPOSE: {
-    const bool tr = amode == dAPPLY_INTERP_TRANSPOSE;
-    const int a = tr ? Q : P, b = tr ? P : Q, a3 = a * a * a, b3 = b * b * b;
-    const double *x = in + e * a3 * D;
-    double *y = out + e * b3 * D;
-    for (int d = 0; d < D; d++) {
-      for (int t = threadIdx.x; t < a3; t += blockDim.x) w0[t] = x[t * D + d];
+  extern __shared__ double lds[];
+  constexpr int AA = A * A, A3 = AA * A;
+  const int tid = threadIdx.x, b = g.b, D = ONE ? 1 : g.D, bb = b * b, b3 = bb * b;
+  const long e0 = (long)blockIdx.x * g.epb;
+  const int ne = (int)min((long)g.epb, g.nelem - e0);
+  const double *B = g.tab, *Dm = g.tab + b * A;
+  for (int d0 = 0; d0 < D; d0 += g.dc) {
+    const int dc = ONE ? 1 : min(g.dc, D - d0), aw = A * dc, bw = b * dc;
+    const int pa = odd(aw), pb = odd(bw), s0 = efs_r0(MODE, A, b, dc), s1 = efs_r1(MODE, A, b, dc);
+    double *R0 = lds, *R1 = lds + ne * s0;
+    if constexpr (MODE != EFS_GRAD_T) {
+      constexpr int NZ = MODE == EFS_GRAD ? 2 : 1, NY = MODE == EFS_GRAD ? 3 : 1;
+      const int sz = AA * pb, sy = A * b * pb;
+      for (int t = tid; t < ne * AA * aw; t += 256) {
+        const int l = t / (AA * aw), t2 = t - l * AA * aw, r = t2 / aw, c = t2 - r * aw, k = ONE ? c : c / dc;
+        R0[l * s0 + r * pa + c] = g.in[((e0 + l) * A3 + r * A + k) * D + d0 + (c - k * dc)];
+      }
       __syncthreads();
-      tensor3(sB, sB, sB, tr, P, a, b, w0, w1);
-      for (int t = threadIdx.x; t < b3; t += blockDim.x) y[t * D + d] = add ? y[t * D + d] + w0[t] : w0[t];
+      for (int t = tid; t < ne * AA * dc; t += 256) {  // along k
+        const int l = t / (AA * dc), t2 = t - l * AA * dc, r = ONE ? t2 : t2 / dc, d = t2 - r * dc;
+        double v[A];
+#pragma unroll
+        for (int m = 0; m < A; m++) v[m] = R0[l * s0 + r * pa + m * dc + d];
+        double *o = &R1[l * s1 + r * pb + d];
+        for (int q = 0; q < b; q++) {
+          o[q * dc] = row_dot<A>(B, q, v);
+          if (NZ > 1) o[sz + q * dc] = row_dot<A>(Dm, q, v);
+        }
+      }
       __syncthreads();
-    }
-  } break;
-  case dAPPLY_GRAD: {
-    const double *x = in + e * P3 * D;
-    double *y = out + e * Q3 * D * 3;
-    const double *J = jinv ? jinv + e * Q3 * 9 : nullptr;
-    for (int d = 0; d < D; d++) {
-      for (int c = 0; c < 3; c++) {  // df_c = (D (x) B (x) B) x, etc.: three full contractions
-        for (int t = threadIdx.x; t < P3; t += blockDim.x) w0[t] = x[t * D + d];
-        __syncthreads();
-        tensor3(c == 0 ? sD : sB, c == 1 ? sD : sB, c == 2 ? sD : sB, false, P, P, Q, w0, w1);
-        for (int q = threadIdx.x; q < Q3; q += blockDim.x) {
-          const double df = w0[q];
-          for (int ee = 0; ee < 3; ee++) {
-            const double v = J ? df * J[q * 9 + c * 3 + ee] : (ee == c ? df : 0.0);
-            double *dst = &y[(q * D + d) * 3 + ee];
-            if (c == 0 && !add) *dst = v;
-            else if (J || ee == c) *dst += v;
+      for (int t = tid; t < ne * A * bw; t += 256) {  // along j
+        const int l = t / (A * bw), t2 = t - l * A * bw, i = t2 / bw, c = t2 - i * bw;
+        const double *z = &R1[l * s1 + i * A * pb + c];
+        double *o = &R0[l * s0 + i * b * pb + c];
+        double v[A], w[NZ > 1 ? A : 1];
+#pragma unroll
+        for (int m = 0; m < A; m++) {
+          v[m] = z[m * pb];
+          if constexpr (NZ > 1) w[m] = z[sz + m * pb];
+        }
+        for (int q = 0; q < b; q++) {
+          o[q * pb] = row_dot<A>(B, q, v);
+          if constexpr (NZ > 1) {
+            o[sy + q * pb] = row_dot<A>(Dm, q, v);
+            o[2 * sy + q * pb] = row_dot<A>(B, q, w);
           }
         }
-        __syncthreads();
       }
-    }
-  } break;
-  case dAPPLY_GRAD_TRANSPOSE: {
-    const double *x = in + e * Q3 * D * 3;
-    double *y = out + e * P3 * D;
-    const double *J = jinv + e * Q3 * 9;
-    for (int d = 0; d < D; d++) {
-      for (int t = threadIdx.x; t < P3; t += blockDim.x) acc[t] = add ? y[t * D + d] : 0.0;
-      for (int c = 0; c < 3; c++) {  // df_c[q] = sum_e jinv[q][c][e] x[q][d][e], then (D^T|B^T)^3
-        for (int q = threadIdx.x; q < Q3; q += blockDim.x) {
-          const double *u = &x[(q * D + d) * 3];
-          w0[q] = u[0] * J[q * 9 + c * 3 + 0] + u[1] * J[q * 9 + c * 3 + 1] + u[2] * J[q * 9 + c * 3 + 2];
-        }
-        __syncthreads();
-        tensor3(c == 0 ? sD : sB, c == 1 ? sD : sB, c == 2 ? sD : sB, true, P, Q, P, w0, w1);
-        for (int t = threadIdx.x; t < P3; t += blockDim.x) acc[t] += w0[t];
-        __syncthreads();
-      }
-      for (int t = threadIdx.x; t < P3; t += blockDim.x) y[t * D + d] = acc[t];
       __syncthreads();
+      for (int t = tid; t < ne * b * bw; t += 256) {  // along i
+        const int l = t / (b * bw), t2 = t - l * b * bw, j = t2 / bw, c = t2 - j * bw, k = ONE ? c : c / dc;
+        const double *y = &R0[l * s0 + j * pb + c];
+        double v[NY][A];
+#pragma unroll
+        for (int m = 0; m < A; m++)
+#pragma unroll
+          for (int n = 0; n < NY; n++) v[n][m] = y[n * sy + m * b * pb];
+        const long pt0 = (e0 + l) * b3 + j * b + k;
+        const int d = d0 + (c - k * dc);
+        for (int q = 0; q < b; q++) {
+          const long pt = pt0 + q * bb;
+          if constexpr (MODE == EFS_INTERP) {
+            const double r = row_dot<A>(B, q, v[0]);
+            double *o = &g.out[pt * D + d];
+            *o = g.add ? *o + r : r;
+          } else {
+            const double f0 = row_dot<A>(Dm, q, v[0]), f1 = row_dot<A>(B, q, v[1]), f2 = row_dot<A>(B, q, v[2]);
+            double r[3] = {f0, f1, f2};
+            if (g.jinv) {
+              const double *J = g.jinv + pt * 9;
+#pragma unroll
+              for (int e = 0; e < 3; e++) r[e] = f0 * J[e] + f1 * J[3 + e] + f2 * J[6 + e];
+            }
+            double *o = &g.out[(pt * D + d) * 3];
+#pragma unroll
+            for (int e = 0; e < 3; e++) o[e] = g.add ? o[e] + r[e] : r[e];
+          }
+        }
+      }
+    } else {
+      const int sx = b * A * pa, sy = bb * pa;
+      for (int t = tid; t < ne * A * aw; t += 256) {  // along i
+        const int l = t / (A * aw), t2 = t - l * A * aw, j = t2 / aw, c = t2 - j * aw, k = ONE ? c : c / dc;
+        const long pt0 = (e0 + l) * A3 + j * A + k;
+        const int d = d0 + (c - k * dc);
+        double f[3][A];
+#pragma unroll
+        for (int m = 0; m < A; m++) {
+          const long pt = pt0 + m * AA;
+          const double *u = &g.in[(pt * D + d) * 3], *J = g.jinv + pt * 9;
+          const double u0 = u[0], u1 = u[1], u2 = u[2];
+#pragma unroll
+          for (int n = 0; n < 3; n++) f[n][m] = u0 * J[n * 3] + u1 * J[n * 3 + 1] + u2 * J[n * 3 + 2];
+        }
+        double *o = &R0[l * s0 + j * pa + c];
+        for (int q = 0; q < b; q++) {
+          o[q * A * pa] = row_dot<A>(Dm, q, f[0]);
+          o[sx + q * A * pa] = row_dot<A>(B, q, f[1]);
+          o[2 * sx + q * A * pa] = row_dot<A>(B, q, f[2]);
+        }
+      }
+      __syncthreads();
+      for (int t = tid; t < ne * b * aw; t += 256) {  // along j
+        const int l = t / (b * aw), t2 = t - l * b * aw, i = t2 / aw, c = t2 - i * aw;
+        const double *x = &R0[l * s0 + i * A * pa + c];
+        double v[3][A];
+#pragma unroll
+        for (int m = 0; m < A; m++)
+#pragma unroll
+          for (int n = 0; n < 3; n++) v[n][m] = x[n * sx + m * pa];
+        double *o = &R1[l * s1 + i * b * pa + c];
+        for (int q = 0; q < b; q++) {
+          o[q * pa] = row_dot<A>(B, q, v[0]) + row_dot<A>(Dm, q, v[1]);
+          o[sy + q * pa] = row_dot<A>(B, q, v[2]);
+        }
+      }
+      __syncthreads();
+      for (int t = tid; t < ne * bb * dc; t += 256) {  // along k
+        const int l = t / (bb * dc), t2 = t - l * bb * dc, r = ONE ? t2 : t2 / dc, d = t2 - r * dc;
+        const double *y = &R1[l * s1 + r * pa + d];
+        double v[2][A];
+#pragma unroll
+        for (int m = 0; m < A; m++)
+#pragma unroll
+          for (int n = 0; n < 2; n++) v[n][m] = y[n * sy + m * dc];
+        double *o = &R0[l * s0 + r * bw + d];
+        for (int q = 0; q < b; q++) o[q * dc] = row_dot<A>(B, q, v[0]) + row_dot<A>(Dm, q, v[1]);
+      }
+      __syncthreads();
+      for (int t = tid; t < ne * bb * bw; t += 256) {
+        const int l = t / (bb * bw), t2 = t - l * bb * bw, r = ONE ? t2 : t2 / dc;
+        double *o = &g.out[((e0 + l) * b3 + r) * D + d0 + (t2 - r * dc)];
+        const double v = R0[l * s0 + t2];
+        *o = g.add ? *o + v : v;
+      }
     }
-  } break;
+    if (d0 + g.dc < D) __syncthreads();  // the next components overwrite the regions
   }
 }
 
@@ -183,9 +267,6 @@ extern "C" dErr dRuleComputePhysicalBatched(int Q, const double *weight, int nel
 
 namespace {
 
-constexpr int kEfsMaxP = 12;
-constexpr int kEfsTab = 2 * kEfsMaxP * kEfsMaxP;  // B and D, [Q][P] each
-
 dErr efs_check(int P, int Q, int nelem, const double *rcoord, const double *jinv, int D, const double *in,
                double *out, int amode, int imode)
 {
@@ -200,47 +281,71 @@ dErr efs_check(int P, int Q, int nelem, const double *rcoord, const double *jinv
   return 0;
 }
 
-dErr efs_launch(int P, int Q, const double *dtab, int nelem, const double *jinv, int D, const double *in, double *out,
-                int amode, int imode, hipStream_t st)
+template <int A, int MODE>
+dErr efs_launch(const EfsArgs &g, size_t lds, hipStream_t st)
 {
-  const int M = std::max(P, Q), M3 = M * M * M;
-  const size_t shmem = sizeof(double) * (2 * Q * P + 3 * M3);
-  hipLaunchKernelGGL(efs_apply_kernel, dim3(nelem), dim3(256), shmem, st, P, Q, dtab, jinv, D, in, out, amode,
-                     imode);
+  const auto kernel = g.D == 1 ? efs_kernel<A, MODE, true> : efs_kernel<A, MODE, false>;
+  if (lds > 65536)
+    DOHP_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((g.nelem + g.epb - 1) / g.epb)), dim3(256), lds, st, g);
   DOHP_HIP(hipGetLastError());
   return 0;
 }
 
-// The 1-D tables of the allocation-free entry point: one copy per GPU, written by a kernel that takes them by
-// value (no copy from host memory), read by the apply kernel that follows on the same stream.
-static __device__ __align__(256) double scratch[kEfsTab];
-
-struct EfsTab {
-  double v[kEfsTab];
-};
-
-__global__ void efs_store_tab_kernel(EfsTab t, int n, double *__restrict__ dst)
+template <int MODE>
+dErr efs_dispatch(int a, const EfsArgs &g, size_t lds, hipStream_t st)
 {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = t.v[i];
+  switch (a) {
+#define DOHP_CASE(AA) \
+  case AA: return efs_launch<AA, MODE>(g, lds, st);
+    DOHP_CASE(1)
+    DOHP_CASE(2)
+    DOHP_CASE(3)
+    DOHP_CASE(4)
+    DOHP_CASE(5)
+    DOHP_CASE(6)
+    DOHP_CASE(7)
+    DOHP_CASE(8)
+    DOHP_CASE(9)
+    DOHP_CASE(10)
+    DOHP_CASE(11)
+    DOHP_CASE(12)
+#undef DOHP_CASE
+  }
+  return dohpERR_ARG;  // (not reached: P and Q are checked)
 }
 
-// Device address of `scratch` on the current device, looked up once per device (the host-side name of a
-// __device__ array is not its device address).
-dErr efs_scratch(double **ptr)
+// Lays out one launch.  All components of an element at once while they fit in 64 KB of LDS (the gradients' largest
+// element, P = Q = 12, takes 75 KB for one); as many elements as give every thread of the longest pass a line, at most
+// 40 KB (four workgroups per compute unit) and leaving at least four workgroups per compute unit.
+dErr efs_apply(int P, int Q, const double *rcoord, int nelem, const double *jinv, int D, const double *in, double *out,
+               int amode, int imode, hipStream_t st)
 {
-  static std::mutex mu;
-  static double *addr[64] = {};
-  int dev = 0;
-  DOHP_HIP(hipGetDevice(&dev));
-  DOHP_CHECK(dev >= 0 && dev < 64, dohpERR_ARG, "device index out of range");
-  std::lock_guard<std::mutex> lock(mu);
-  if (!addr[dev]) {
-    void *p = nullptr;
-    DOHP_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    addr[dev] = (double *)p;
-  }
-  *ptr = addr[dev];
-  return 0;
+  const bool tr = amode == dAPPLY_INTERP_TRANSPOSE || amode == dAPPLY_GRAD_TRANSPOSE;
+  const int mode = amode == dAPPLY_GRAD ? EFS_GRAD : amode == dAPPLY_GRAD_TRANSPOSE ? EFS_GRAD_T : EFS_INTERP;
+  const int a = tr ? Q : P, b = tr ? P : Q, m = std::max(a, b);
+  EfsArgs g;
+  double t[kEfsTab];
+  DOHP_CALL(dohpTensorBasis(P, Q, rcoord, t, t + Q * P, nullptr, nullptr));
+  for (int o = 0; o < 2; o++)
+    for (int q = 0; q < b; q++)
+      for (int i = 0; i < a; i++) g.tab[(o * b + q) * a + i] = t[o * Q * P + (tr ? i * P + q : q * P + i)];
+  const auto bytes = [&](int dc) { return sizeof(double) * (efs_r0(mode, a, b, dc) + efs_r1(mode, a, b, dc)); };
+  g.b = b;
+  g.D = D;
+  g.dc = std::min(D, 64);
+  while (g.dc > 1 && bytes(g.dc) > 65536) g.dc--;
+  const int lines = m * m * g.dc;
+  g.epb = std::max(1, std::min({256 / lines, (int)(40960 / bytes(g.dc)), nelem / 1024}));
+  g.nelem = nelem;
+  g.add = imode == dADD_VALUES;
+  g.jinv = jinv;
+  g.in = in;
+  g.out = out;
+  const size_t lds = g.epb * bytes(g.dc);
+  if (mode == EFS_INTERP) return efs_dispatch<EFS_INTERP>(a, g, lds, st);
+  if (mode == EFS_GRAD) return efs_dispatch<EFS_GRAD>(a, g, lds, st);
+  return efs_dispatch<EFS_GRAD_T>(a, g, lds, st);
 }
 
 }  // namespace
@@ -250,13 +355,9 @@ extern "C" dErr dEFSApplyHexBatched(int P, int Q, const double *rcoord, int nele
 {
   DOHP_CALL(efs_check(P, Q, nelem, rcoord, jinv, D, in, out, amode, imode));
   if (nelem == 0) return 0;
-  std::vector<double> tab(2 * Q * P);
-  DOHP_CALL(dohpTensorBasis(P, Q, rcoord, tab.data(), tab.data() + Q * P, nullptr, nullptr));
-  DevBuf<double> dtab;
-  DOHP_CALL(dtab.upload(tab.data(), tab.size()));
   hipStream_t st = (hipStream_t)stream;
-  DOHP_CALL(efs_launch(P, Q, dtab.ptr, nelem, jinv, D, in, out, amode, imode, st));
-  DOHP_HIP(hipStreamSynchronize(st));  // dtab is freed on return
+  DOHP_CALL(efs_apply(P, Q, rcoord, nelem, jinv, D, in, out, amode, imode, st));
+  DOHP_HIP(hipStreamSynchronize(st));  // (the results are there when the call returns)
   return 0;
 }
 
@@ -264,14 +365,6 @@ extern "C" dErr dEFSApplyHexBatchedNoAlloc(int P, int Q, const double *rcoord, i
                                            const double *in, double *out, int amode, int imode, void *stream)
 {
   DOHP_CALL(efs_check(P, Q, nelem, rcoord, jinv, D, in, out, amode, imode));
-  DOHP_CHECK(2 * Q * P <= kEfsTab, dohpERR_ARG, "dEFSApplyHexBatchedNoAlloc: tables exceed the 2*12*12 staging area");
   if (nelem == 0) return 0;
-  double *dtab = nullptr;
-  DOHP_CALL(efs_scratch(&dtab));
-  EfsTab t;  // host stack: B and D of the rule, passed to the device by value
-  DOHP_CALL(dohpTensorBasis(P, Q, rcoord, t.v, t.v + Q * P, nullptr, nullptr));
-  hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(efs_store_tab_kernel, dim3(1), dim3(256), 0, st, t, 2 * Q * P, dtab);
-  DOHP_HIP(hipGetLastError());
-  return efs_launch(P, Q, dtab, nelem, jinv, D, in, out, amode, imode, st);
+  return efs_apply(P, Q, rcoord, nelem, jinv, D, in, out, amode, imode, (hipStream_t)stream);
 }

@@ -63,11 +63,10 @@ dErr dEFSApplyHexBatched(int P, int Q, const double *rcoord_host, int nelem, con
                          const double *in_dev, double *out_dev, int amode, int imode, void *stream);
 
 /* No counterpart in the reference.  dEFSApplyHexBatched without any device allocation or wait, for callers
- * that cannot allocate (code under HIP graph capture, tight loops applying elements the way the reference's
+ * that cannot allocate or wait (code under HIP graph capture, tight loops applying elements the way the reference's
  * per-element dEFSApply call sites do).  Same arguments, results and errors as dEFSApplyHexBatched (it shares its
- * kernel); P, Q <= 12.  The B and D tables (2 Q P <= 288 doubles) are staged in a 2.3 KB device array of the
- * library, one per GPU, held until the process ends: calls that overlap on one GPU (several streams or host
- * threads) race on it. */
+ * kernel); P, Q <= 12.  The B and D tables travel with the launch: calls on several streams or host threads share
+ * nothing. */
 dErr dEFSApplyHexBatchedNoAlloc(int P, int Q, const double *rcoord_host, int nelem, const double *jinv_dev, int D,
                                 const double *in_dev, double *out_dev, int amode, int imode, void *stream);
 
