@@ -206,7 +206,7 @@ __attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <=
 #undef DOHP_SCATTER
 #undef DOHP_BATCH_HOOK
 #undef DOHP_ELEM
-  if (bad) atomicOr(nanflag, 1);
+  if (bad) *nanflag = 1;
 }
 
 // Persistent form of the kernel (one wavefront per workgroup, atomic scatter): each workgroup
@@ -354,7 +354,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
 #undef DOHP_ELEM
     __syncthreads();  // the next batch overwrites the tiles
   }
-  if (bad) atomicOr(nanflag, 1);
+  if (bad) *nanflag = 1;
 }
 
 template <typename T>
@@ -365,17 +365,17 @@ __global__ void zero_kernel(T *__restrict__ y, long n)
 }
 
 // Linearization state in lattice order (closure order for a space from element maps, lat2clo = null): owned
-// values from u, Dirichlet values from the cache.
+// values from u, Dirichlet values from the cache.  If f is not null it also gets its first value on every owned node:
+// the forcing term, or zero.
 __global__ void lattice_state_kernel(const double *__restrict__ u, const double *__restrict__ dcache,
                                      const int *__restrict__ lat2clo, long nowned, long nlat, double *__restrict__ st,
-                                     float *__restrict__ st32)
+                                     const double *__restrict__ forcing, double *__restrict__ f)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nlat) return;
   const long c = lat2clo ? lat2clo[i] : i;
-  const double v = c < nowned ? u[c] : dcache[c - nowned];
-  st[i] = v;
-  st32[i] = (float)v;
+  st[i] = c < nowned ? u[c] : dcache[c - nowned];
+  if (f && c < nowned) f[c] = forcing ? forcing[c] : 0.0;
 }
 
 }  // namespace
@@ -403,10 +403,14 @@ struct _p_dohpEllip {
   DevBuf<double> forcing;                     // assembled forcing term -(f, phi) on the owned nodes
   bool has_forcing = false;
   DevBuf<float> state32, tab32;
-  // set by the element kernels when a scattered contribution is not finite (a NaN or Inf in the input
-  // vector or the state); the checked entry points clear it, wait for their stream and read it back
+  bool state32_ok = false;  // state32 is the rounded state (formed by the first FP32 application that reads it)
+  // Set by the element kernels when a scattered contribution is not finite (a NaN or Inf in the input vector or the
+  // state).  The checked entry points clear a flag in pinned host memory, launch with it, wait for their stream and read
+  // it: no clearing kernel and no copy.  Unchecked launches set a flag on the device that nobody reads, so that one still
+  // in flight cannot touch a later checked call's.
   DevBuf<int> nanflag;
-  int *nan_host = nullptr;  // pinned
+  int *nan_host = nullptr, *nan_dev = nullptr;  // pinned, and its device address
+  int *flag = nullptr;                          // the flag of the launches now: nan_dev inside a checked call
   double *scal_host = nullptr;  // pinned: scalars of the solves on this operator
   int checks = 1;
   const float *q1_cscale = nullptr;  // learned sub-cell derivative scales of later Q1 assemblies (caller's array)
@@ -477,7 +481,7 @@ void launch_shape(const _p_dohpEllip *op, const T *ust, const T *x, T *y, hipStr
     const long ne = fs->nelem;
     hipLaunchKernelGGL((ellip_kernel<N, T, MODE, EPB, MF>), dim3((ne + EPB - 1) / EPB), block, 0, st, nullptr, ne,
                        box_map(fs), enodes, everts, fs->d_vcoords.ptr, op->kvert.ptr, ust, x, y, fs->nowned, 1,
-                       gtab<T>(op), op->wphi.ptr, ph, op->nanflag.ptr);
+                       gtab<T>(op), op->wphi.ptr, ph, op->flag);
   } else {
     for (int col = 0; col < fs->ncolor; col++) {
       const long ne = fs->color_off[col + 1] - fs->color_off[col];
@@ -485,7 +489,7 @@ void launch_shape(const _p_dohpEllip *op, const T *ust, const T *x, T *y, hipStr
       hipLaunchKernelGGL((ellip_kernel<N, T, MODE, EPB, MF>), dim3((ne + EPB - 1) / EPB), block, 0, st,
                          fs->d_color_elems.ptr + fs->color_off[col], ne, box_map(fs), enodes, everts,
                          fs->d_vcoords.ptr, op->kvert.ptr, ust, x, y, fs->nowned, 0, gtab<T>(op), op->wphi.ptr, ph,
-                         op->nanflag.ptr);
+                         op->flag);
     }
   }
 }
@@ -512,7 +516,7 @@ dErr launch_persistent(const _p_dohpEllip *op, const T *ust, const T *x, T *y, h
   grid = std::max(8L, grid - grid % 8);
   hipLaunchKernelGGL((ellip_persistent_kernel<N, T, MODE, EPB>), dim3((unsigned)grid), dim3(threads), 0, st, nbatch,
                      (long)fs->nelem, box_map(fs), fs->d_vcoords.ptr, op->kvert.ptr, ust, x, y, fs->nowned,
-                     gtab<T>(op), op->wphi.ptr, ph, op->nanflag.ptr);
+                     gtab<T>(op), op->wphi.ptr, ph, op->flag);
   return 0;
 }
 
@@ -748,12 +752,13 @@ extern "C" dErr dohpEllipCreate(dohpFS fs, const dohpEllipParam *prm, dohpEllip 
   if (!err) err = op->state.alloc(fs->nclosure);
   if (!err) err = op->state32.alloc(fs->nclosure);
   if (!err) err = op->nanflag.alloc(1);
-  if (!err && hipMemset(op->nanflag.ptr, 0, sizeof(int)) != hipSuccess) err = dohpERR_HIP;
+  op->flag = op->nanflag.ptr;
   if (!err && hipHostMalloc((void **)&op->nan_host, sizeof(int), hipHostMallocDefault) != hipSuccess) {
     op->nan_host = nullptr;
     set_error("pinned allocation failed");
     err = dohpERR_OOM;
   }
+  if (!err && hipHostGetDevicePointer((void **)&op->nan_dev, op->nan_host, 0) != hipSuccess) err = dohpERR_HIP;
   if (!err && hipHostMalloc((void **)&op->scal_host, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
     op->scal_host = nullptr;
     set_error("pinned allocation failed");
@@ -823,34 +828,41 @@ extern "C" dErr dohpEllipSetCoefficient(dohpEllip op, const double *kvert)
 
 namespace {
 
-// Checked form of an entry point (checks on): clears the non-finite flag, runs f, waits for the stream
+// Checked form of an entry point (checks on): clears the host's non-finite flag, runs f, waits for the stream
 // and reports a non-finite value met by the element kernels.  Checks off: f alone, asynchronous.
 template <typename F>
 dErr checked(_p_dohpEllip *op, hipStream_t st, const char *what, F f)
 {
   if (!op->checks) return f();
-  DOHP_CALL(zero(op->nanflag.ptr, 1L, st));
-  DOHP_CALL(f());
-  DOHP_HIP(hipMemcpyAsync(op->nan_host, op->nanflag.ptr, sizeof(int), hipMemcpyDeviceToHost, st));
+  *op->nan_host = 0;
+  op->flag = op->nan_dev;
+  const dErr err = f();
+  op->flag = op->nanflag.ptr;
+  if (err) return err;
   DOHP_HIP(hipStreamSynchronize(st));
-  DOHP_CHECK(*op->nan_host == 0, dohpERR_NAN,
+  DOHP_CHECK(*(volatile int *)op->nan_host == 0, dohpERR_NAN,
              std::string(what) + ": non-finite value met on the device (NaN or Inf in the input vector or the state)");
+  return 0;
+}
+
+// Records u as the linearization state; f (may be null) gets the forcing term or zero.
+dErr set_state(_p_dohpEllip *op, const double *u, double *f, hipStream_t st)
+{
+  const dohpFS fs = op->fs;
+  hipLaunchKernelGGL(lattice_state_kernel, dim3((fs->nclosure + 255) / 256), dim3(256), 0, st, u, fs->d_dcache.ptr,
+                     fs->d_lat2clo.ptr, fs->nowned, fs->nclosure, op->state.ptr, op->has_forcing ? op->forcing.ptr : nullptr,
+                     f);
+  op->has_state = true;
+  op->state32_ok = false;
+  drop_qd(op);
+  DOHP_HIP(hipGetLastError());
   return 0;
 }
 
 dErr ellip_function(_p_dohpEllip *op, const double *u, double *f, hipStream_t st)
 {
-  const dohpFS fs = op->fs;
-  hipLaunchKernelGGL(lattice_state_kernel, dim3((fs->nclosure + 255) / 256), dim3(256), 0, st, u, fs->d_dcache.ptr,
-                     fs->d_lat2clo.ptr, fs->nowned, fs->nclosure, op->state.ptr, op->state32.ptr);
-  op->has_state = true;
-  drop_qd(op);
-  if (op->prm.exact >= 0) {  // y = forcing term, then the state's terms are added
-    if (!op->has_forcing) DOHP_CALL(assemble_forcing(op, st));
-    DOHP_HIP(hipMemcpyAsync(f, op->forcing.ptr, sizeof(double) * fs->nowned, hipMemcpyDeviceToDevice, st));
-  } else {
-    DOHP_CALL(zero(f, fs->nowned, st));
-  }
+  if (op->prm.exact >= 0 && !op->has_forcing) DOHP_CALL(assemble_forcing(op, st));
+  DOHP_CALL(set_state(op, u, f, st));
   return launch<double, MODE_FUN>(op, op->state.ptr, nullptr, f, st);
 }
 
@@ -872,13 +884,7 @@ extern "C" dErr dohpEllipSetChecks(dohpEllip op, int mode)
 
 extern "C" dErr dohpEllipFunctionState_Private(dohpEllip op, const double *u, hipStream_t st)
 {
-  const dohpFS fs = op->fs;
-  hipLaunchKernelGGL(lattice_state_kernel, dim3((fs->nclosure + 255) / 256), dim3(256), 0, st, u, fs->d_dcache.ptr,
-                     fs->d_lat2clo.ptr, fs->nowned, fs->nclosure, op->state.ptr, op->state32.ptr);
-  op->has_state = true;
-  drop_qd(op);
-  DOHP_HIP(hipGetLastError());
-  return 0;
+  return set_state(op, u, nullptr, st);
 }
 
 dohp::Pool *dohpEllipPool_Private(dohpEllip op) { return &op->pool; }
@@ -930,10 +936,26 @@ struct Prec<float> {
   static const float *state(const _p_dohpEllip *op) { return op->state32.ptr; }
 };
 
+// The FP32 state, rounded once per linearization (in a captured graph: by every replay, and by the next eager
+// application, since the capture itself runs nothing).
+dErr ensure_state32(_p_dohpEllip *op, hipStream_t st)
+{
+  if (op->state32_ok) return 0;
+  const long n = op->fs->nclosure;
+  hipLaunchKernelGGL(round_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, op->state.ptr,
+                     op->state32.ptr, n);
+  DOHP_HIP(hipGetLastError());
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  DOHP_HIP(hipStreamIsCapturing(st, &cap));
+  op->state32_ok = cap == hipStreamCaptureStatusNone;
+  return 0;
+}
+
 template <typename T>
 dErr apply_recomputed(_p_dohpEllip *op, const T *x, T *y, hipStream_t st)
 {
   if (is_linear(op)) return launch<T, MODE_LIN>(op, nullptr, x, y, st);
+  if (sizeof(T) == 4) DOHP_CALL(ensure_state32(op, st));
   return launch<T, MODE_JAC>(op, Prec<T>::state(op), x, y, st);
 }
 
