@@ -145,26 +145,83 @@ inline bool sweep_big(const Box &b)
   return (long)((b.nz + kBX - 1) / kBX) * ((b.ny + 7) / 8) * ((b.nx + 1) / 2) >= 1024;
 }
 
-// Fills the tile of the block at (I0, J0, K0) with load(g, gi, gj, gk), g the row of the tile entry at (gi, gj, gk)
-// (every load unconditional: entries outside the box load row 0 and are zero).  Ends with a barrier.
+// Workgroups and the eight L2 caches.  Consecutive workgroups go to the XCDs in turn, so tiles in natural order share
+// none of the lines that they have in common: the FP16 sweeps fetched 2.2 times the bytes of a row (1.18 GB at 239^3),
+// the Galerkin product 3.7 times, and ran at the rate of that traffic.  A box's lines are therefore split into eight
+// parts along J, one per XCD (blockIdx.x & 7), each traversed x, y, z in order, so that a part's last plane is still in
+// its L2 (191^3: 36 k entries of 112 bytes a plane over eight caches of 4 MB).  At 239^3 the FP16 sweeps fetch 0.63 GB and
+// take 158 to 195 instead of 170 to 221 us, the Galerkin product 1.37 instead of 1.62 ms, the half stencils 1.10 instead
+// of 1.44 ms; a power iteration at 191^3 231 instead of 244 us.  Boxes with fewer than two tiles of lines per part are not
+// split (47^3, all of it in every L2: no difference).
+struct Split {
+  int lg, lines;  // log2 of the number of parts, lines of a part
+  __device__ __forceinline__ int j0(unsigned bx, unsigned by, int BY) const
+  {
+    return (int)(bx & ((1u << lg) - 1)) * lines + (int)by * BY;
+  }
+  __device__ __forceinline__ int k0(unsigned bx) const { return (int)(bx >> lg) * kBX; }
+  __device__ __forceinline__ int j1(unsigned bx, int ny) const
+  {
+    return min(ny, ((int)(bx & ((1u << lg) - 1)) + 1) * lines);
+  }
+};
+inline Split split_of(const Box &b, int BY)
+{
+  const int l = (b.ny + 15) / 16 * 2;  // (even: the coarse tiles start at half the first line)
+  return l >= 2 * BY ? Split{3, l} : Split{0, b.ny};
+}
+inline dim3 split_grid(const Box &b, const Split &s, int BY, int NR)
+{
+  return dim3((unsigned)((b.nz + kBX - 1) / kBX) << s.lg, (unsigned)((s.lines + BY - 1) / BY),
+              (unsigned)((b.nx + NR - 1) / NR));
+}
+
+// Entry `row` (the workgroup's part of the row number) + i (the thread's) of an array: a scalar base and a 32-bit offset,
+// so that the streams of a row share one address register.  With 64-bit row numbers per thread and stream the addresses
+// of a row were half of the vector instructions of a sweep (285 a row in the FP16 one, now 152).
+template <typename T>
+__device__ __forceinline__ const T &at(const T *p, long row, unsigned i)
+{
+  return *(const T *)((const char *)(p + row) + i * (unsigned)sizeof(T));
+}
+template <typename T>
+__device__ __forceinline__ T &at(T *p, long row, unsigned i)
+{
+  return *(T *)((char *)(p + row) + i * (unsigned)sizeof(T));
+}
+
+// Fills the tile of the block at (I0, J0, K0) with load(row, i, gi, gj, gk), row + i the row of the tile entry at
+// (gi, gj, gk) (every load unconditional: entries outside the box load a row inside it and are zero).  A wavefront takes
+// whole lines of 64 columns, whose line numbers are scalars; the two columns beside them go to the first threads.  Ends
+// with a barrier.
 template <int BY, int NR, typename T, typename Load>
 __device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0, int tid, T *tile, Load load)
 {
   using S = SweepTile<BY, NR>;
+  constexpr int L = (NR + 2) * S::TY, IT = (L + BY - 1) / BY;
+  static_assert(2 * L <= S::NT, "one halo entry per thread");
   const long sy = bx.nz, sx = (long)bx.ny * bx.nz;
-  T v[S::IT];
+  const int lane = tid & (kBX - 1), w = __builtin_amdgcn_readfirstlane(tid / kBX);
+  const bool ink = K0 + lane < bx.nz;
+  const unsigned kl = ink ? lane : 0;
+  T v[IT], h = T(0);
 #pragma unroll
-  for (int u = 0; u < S::IT; u++) {
-    const int t = min(tid + u * S::NT, S::N - 1);
-    const int p = t / (S::TY * S::TX), rem = t - p * (S::TY * S::TX), jj = rem / S::TX, kk = rem - jj * S::TX;
-    const int gi = I0 + p - 1, gj = J0 + jj - 1, gk = K0 + kk - 1;
+  for (int u = 0; u < IT; u++) {
+    const int l = min(w + u * BY, L - 1), gi = I0 + l / S::TY - 1, gj = J0 + l % S::TY - 1;
+    const bool in = gi >= 0 && gi < bx.nx && gj >= 0 && gj < bx.ny;
+    const T y = load(in ? gi * sx + gj * sy + K0 : (long)K0, kl, gi, gj, K0 + lane);
+    v[u] = in && ink ? y : T(0);
+  }
+  if (tid < 2 * L) {
+    const int l = tid >> 1, gi = I0 + l / S::TY - 1, gj = J0 + l % S::TY - 1, gk = tid & 1 ? K0 + kBX : K0 - 1;
     const bool in = inside(bx, gi, gj, gk);
-    const T y = load(in ? gi * sx + gj * sy + gk : 0L, gi, gj, gk);
-    v[u] = in ? y : T(0);
+    const T y = load(in ? gi * sx + gj * sy + gk : 0L, 0u, gi, gj, gk);
+    h = in ? y : T(0);
   }
 #pragma unroll
-  for (int u = 0; u < S::IT; u++)
-    if (tid + u * S::NT < S::N) tile[tid + u * S::NT] = v[u];
+  for (int u = 0; u < IT; u++)
+    if (w + u * BY < L) tile[(w + u * BY) * S::TX + 1 + lane] = v[u];
+  if (tid < 2 * L) tile[(tid >> 1) * S::TX + (tid & 1 ? kBX + 1 : 0)] = h;
   __syncthreads();
 }
 
@@ -211,22 +268,22 @@ __device__ __forceinline__ T coarse_value(const T *ct, int I0, int J0, int K0, i
                      ((b[r0 + k0] + b[r0 + k1]) + (b[r1 + k0] + b[r1 + k1])));
 }
 
-// Row i = (I, J, K) of the product, on plane q of the block's tile; tj, tk its row and column there.
+// Row `row` + i of the product, on plane q of the block's tile; tj, tk its row and column there.  A neighbour outside the
+// box is zero in the tile; its lower coefficient is read at whatever entry lies there (the stream of direction s starts
+// (s - 13) n entries into H, further than the direction reaches back).
 template <int BY, typename T>
 __device__ __forceinline__ T half_row(const Box &bx, const T *__restrict__ H, const T *tile, int q, int tj, int tk,
-                                      int I, int J, int K, long i)
+                                      long row, unsigned i)
 {
   constexpr int TX = SweepTile<BY, 1>::TX, TY = SweepTile<BY, 1>::TY;
   const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz;
-  T acc = H[i] * tile[((q + 1) * TY + tj) * TX + tk];
+  T acc = at(H, row, i) * tile[((q + 1) * TY + tj) * TX + tk];
 #pragma unroll
   for (int s = 14; s < 27; s++) {
     const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
     const long off = di * sx + dj * sy + dk;
-    // (a neighbour outside the box is zero in the tile; its lower coefficient is read at whatever row i - off is)
-    const long il = i - off >= 0 ? i - off : i;
-    acc += H[(s - 13) * n + i] * tile[((q + 1 + di) * TY + tj + dj) * TX + tk + dk];
-    acc += H[(s - 13) * n + il] * tile[((q + 1 - di) * TY + tj - dj) * TX + tk - dk];
+    acc += at(H, (s - 13) * n + row, i) * tile[((q + 1 + di) * TY + tj + dj) * TX + tk + dk];
+    acc += at(H, (s - 13) * n + row - off, i) * tile[((q + 1 - di) * TY + tj - dj) * TX + tk - dk];
   }
   return acc;
 }
@@ -238,7 +295,7 @@ __device__ __forceinline__ T half_row(const Box &bx, const T *__restrict__ H, co
 // from x + P xc, the iterate with the coarse correction.
 enum { SW_RESID, SW_CHEB, SW_FIRST_CHEB, SW_FIRST_RESID, SW_PRO_CHEB };
 template <typename T, int MODE, int BY, int NR>
-__global__ void __launch_bounds__(kBX *BY) half_sweep_kernel(Box bx, const T *__restrict__ H,
+__global__ void __launch_bounds__(kBX *BY, 4) half_sweep_kernel(Box bx, Split sp, const T *__restrict__ H,
                                                              const T *__restrict__ dinv, const T *__restrict__ b,
                                                              const T *__restrict__ x, T *__restrict__ out,
                                                              T *__restrict__ d, T *__restrict__ x1, T a, T c, T c1,
@@ -248,32 +305,35 @@ __global__ void __launch_bounds__(kBX *BY) half_sweep_kernel(Box bx, const T *__
   constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID, PRO = MODE == SW_PRO_CHEB;
   __shared__ T tile[S::N];
   __shared__ T ct[PRO ? CoarseTile<BY, NR>::N : 1];
-  const int I0 = blockIdx.z * NR, J0 = blockIdx.y * BY, K0 = blockIdx.x * kBX;
+  const int I0 = blockIdx.z * NR, J0 = sp.j0(blockIdx.x, blockIdx.y, BY), K0 = sp.k0(blockIdx.x);
+  const int J1 = sp.j1(blockIdx.x, bx.ny);
+  if (J0 >= J1) return;
   if constexpr (PRO) stage_coarse<BY, NR>(cb, xc, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, ct);
-  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int gi, int gj, int gk) {
-    if constexpr (FIRST) return c1 * dinv[g] * b[g];
-    else if constexpr (PRO) return x[g] + coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
-    else return x[g];
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, unsigned i, int gi, int gj, int gk) {
+    if constexpr (FIRST) return c1 * at(dinv, g, i) * at(b, g, i);
+    else if constexpr (PRO) return at(x, g, i) + coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
+    else return at(x, g, i);
   });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
-  if (K >= bx.nz || J >= bx.ny) return;
+  if (K >= bx.nz || J >= J1) return;
+  const unsigned i = threadIdx.y * (unsigned)bx.nz + threadIdx.x;
 #pragma unroll
   for (int q = 0; q < NR; q++) {
     const int I = I0 + q;
     if (NR > 1 && I >= bx.nx) break;
-    const long i = ((long)I * bx.ny + J) * bx.nz + K;
-    const T ax = half_row<BY, T>(bx, H, tile, q, tj, tk, I, J, K, i);
-    const T r = (MODE != SW_RESID || b ? b[i] : T(0)) - ax;
+    const long row = ((long)I * bx.ny + J0) * bx.nz + K0;
+    const T ax = half_row<BY, T>(bx, H, tile, q, tj, tk, row, i);
+    const T r = (MODE != SW_RESID || b ? at(b, row, i) : T(0)) - ax;
     const T xi = tile[((q + 1) * S::TY + tj) * S::TX + tk];
     if constexpr (MODE == SW_RESID) {
-      out[i] = r;
+      at(out, row, i) = r;
     } else if constexpr (MODE == SW_FIRST_RESID) {
-      x1[i] = xi;
-      out[i] = r;
+      at(x1, row, i) = xi;
+      at(out, row, i) = r;
     } else {
-      const T dn = (MODE == SW_FIRST_CHEB ? a * xi : a == T(0) ? T(0) : a * d[i]) + c * dinv[i] * r;
-      if (keep_d) d[i] = dn;
-      out[i] = xi + dn;
+      const T dn = (MODE == SW_FIRST_CHEB ? a * xi : a == T(0) ? T(0) : a * at(d, row, i)) + c * at(dinv, row, i) * r;
+      if (keep_d) at(d, row, i) = dn;
+      at(out, row, i) = xi + dn;
     }
   }
 }
@@ -282,13 +342,15 @@ template <typename T, int MODE>
 void sweep(const Box &bx, const T *H, const T *dinv, const T *b, const T *x, T *out, T *d, T *x1, T a, T c, T c1,
            int keep_d, hipStream_t st, const Box &cb = Box{}, const T *xc = nullptr)
 {
-  const unsigned gx = (bx.nz + kBX - 1) / kBX;
+  const auto launch = [&](auto kernel, int BY, int NR) {
+    const Split sp = split_of(bx, BY);
+    hipLaunchKernelGGL(kernel, split_grid(bx, sp, BY, NR), dim3(kBX, BY), 0, st, bx, sp, H, dinv, b, x, out, d, x1, a,
+                       c, c1, keep_d, cb, xc);
+  };
   if (sweep_big(bx))
-    hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 8, 2>), dim3(gx, (bx.ny + 7) / 8, (bx.nx + 1) / 2), dim3(kBX, 8), 0,
-                       st, bx, H, dinv, b, x, out, d, x1, a, c, c1, keep_d, cb, xc);
+    launch(half_sweep_kernel<T, MODE, 8, 2>, 8, 2);
   else
-    hipLaunchKernelGGL((half_sweep_kernel<T, MODE, 4, 1>), dim3(gx, (bx.ny + 3) / 4, bx.nx), dim3(kBX, 4), 0, st, bx,
-                       H, dinv, b, x, out, d, x1, a, c, c1, keep_d, cb, xc);
+    launch(half_sweep_kernel<T, MODE, 4, 1>, 4, 1);
 }
 
 // r = b - A x (b may be null) on a level.
@@ -302,13 +364,14 @@ void residual(const Box &bx, const T *H, const T *b, const T *x, T *r, hipStream
 // over the blocks of every level (the coarse ones ride along with the finest), w = D^-1 A (v / ||v||) with the scaling
 // applied in the staging and the sums of squares of w reduced per block, and one that sums each level's block sums in
 // order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3 rows and their coarse
-// levels, 15 iterations, 6.5 -> 3.8 ms (4.4 TB/s on the 17 values a row cannot do without).
+// levels, 15 iterations, 6.5 -> 3.5 ms (4.7 TB/s on the 17 values a row cannot do without).
 constexpr int kMaxLevels = 16, kPowerThreads = kBX * 8;
 struct PowerLevel {
   Box bx;
   const double *H, *dinv;
   double *v[2], *part;
-  unsigned first, gx, gy;  // first block of the level, its tiles along K and J
+  Split sp;
+  unsigned first, gx, gy;  // first block of the level (a multiple of eight), its grid along x and y
   int blocks, big;         // number of blocks; 64 x 8 x 2 tiles, else 64 x 8 x 1
 };
 struct PowerArgs {
@@ -339,18 +402,21 @@ __device__ __forceinline__ double power_rows(const PowerLevel &l, unsigned blk, 
   using S = SweepTile<8, NR>;
   const Box &bx = l.bx;
   const unsigned tx = blk % l.gx, rest = blk / l.gx, ty = rest % l.gy, tz = rest / l.gy;
-  const int I0 = tz * NR, J0 = ty * 8, K0 = tx * kBX, lx = threadIdx.x & (kBX - 1), ly = threadIdx.x / kBX;
-  stage_tile<8, NR>(bx, I0, J0, K0, threadIdx.x, tile, [&](long g, int, int, int) { return inv * v[g]; });
+  const int I0 = tz * NR, J0 = l.sp.j0(tx, ty, 8), J1 = l.sp.j1(tx, bx.ny), K0 = l.sp.k0(tx);
+  const int lx = threadIdx.x & (kBX - 1), ly = threadIdx.x / kBX;
+  if (J0 >= J1) return 0.0;
+  stage_tile<8, NR>(bx, I0, J0, K0, threadIdx.x, tile, [&](long g, unsigned i, int, int, int) { return inv * at(v, g, i); });
   const int J = J0 + ly, K = K0 + lx;
+  const unsigned i = ly * (unsigned)bx.nz + lx;
   double s = 0;
-  if (K < bx.nz && J < bx.ny) {
+  if (K < bx.nz && J < J1) {
 #pragma unroll
     for (int q = 0; q < NR; q++) {
       const int I = I0 + q;
       if (NR > 1 && I >= bx.nx) break;
-      const long i = ((long)I * bx.ny + J) * bx.nz + K;
-      const double y = l.dinv[i] * half_row<8, double>(bx, l.H, tile, q, ly + 1, lx + 1, I, J, K, i);
-      w[i] = y;
+      const long row = ((long)I * bx.ny + J0) * bx.nz + K0;
+      const double y = at(l.dinv, row, i) * half_row<8, double>(bx, l.H, tile, q, ly + 1, lx + 1, row, i);
+      at(w, row, i) = y;
       s += y * y;
     }
   }
@@ -366,6 +432,7 @@ __global__ void __launch_bounds__(kPowerThreads) power_step_kernel(PowerArgs g, 
   while (k + 1 < g.nl && blockIdx.x >= g.l[k + 1].first) k++;
   const PowerLevel &l = g.l[k];
   const unsigned blk = blockIdx.x - l.first;
+  if (blk >= (unsigned)l.blocks) return;  // (the next level starts at a multiple of eight)
   const double s = l.big ? power_rows<2>(l, blk, inv[k], l.v[from], l.v[1 - from], tile)
                          : power_rows<1>(l, blk, inv[k], l.v[from], l.v[1 - from], tile);
   const double t = block_sum<kPowerThreads>(s, threadIdx.x, sh);
@@ -399,20 +466,22 @@ __global__ void diag_kernel(long n, const double *__restrict__ A, double *__rest
 // The half stencil of a level in FP64 (H, null where the level's own stencil serves), FP32 and FP16 in one pass over its
 // 27-point stencil A: a row's 13 upper entries are read once for all three, the row scales of its neighbours come from
 // a staged tile, and its lower neighbours' entries (which those rows round) are read for the diagonal's compensation.
-// 112 bytes read and 112 + 56 + 48 written per row and 27 FP64 divisions: 191^3 rows 0.95 -> 0.63 ms against a copy of the half
+// 112 bytes read and 112 + 56 + 48 written per row and 27 FP64 divisions: 191^3 rows 0.95 -> 0.51 ms against a copy of the half
 // stencil and an FP16 pass that took 52 square roots per row.
-__global__ void __launch_bounds__(256) half_setup_kernel(Box bx, const double *__restrict__ A, double *__restrict__ H,
+__global__ void __launch_bounds__(256) half_setup_kernel(Box bx, Split sp, const double *__restrict__ A, double *__restrict__ H,
                                                          float *__restrict__ H32, _Float16 *__restrict__ H16,
                                                          float *__restrict__ dg, const float *__restrict__ sc,
                                                          float *__restrict__ eg, float *__restrict__ fg, int scaled_in)
 {
   using S = SweepTile<kBY, 1>;
   __shared__ float tile[S::N];
-  const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
+  const int I = blockIdx.z, J0 = sp.j0(blockIdx.x, blockIdx.y, kBY), J1 = sp.j1(blockIdx.x, bx.ny);
+  const int K0 = sp.k0(blockIdx.x);
+  if (J0 >= J1) return;
   stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile,
-                     [&](long g, int, int, int) { return sc[g]; });
+                     [&](long g, unsigned i, int, int, int) { return at(sc, g, i); });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
-  if (K >= bx.nz || J >= bx.ny) return;
+  if (K >= bx.nz || J >= J1) return;
   const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz, i = ((long)I * bx.ny + J) * bx.nz + K;
   const float si = tile[(S::TY + tj) * S::TX + tk];
   const double aii = A[13 * n + i];
@@ -450,29 +519,31 @@ __global__ void __launch_bounds__(256) half_setup_kernel(Box bx, const double *_
 // sum_j h_ij y_j over the 26 neighbours of row i, on plane q of the block's staged tile.  The coefficients are stored as
 // pairs of directions per row ([7][n] dwords, directions 14 + 2j and 15 + 2j, the last pair padded): a row reads its 13
 // upper ones with 7 dword loads, and each lower one (the upper one of the lower neighbour's row) with one, instead of
-// 26 two-byte loads.  A neighbour outside the box has a zero tile entry; its coefficient is read at a clamped index.
+// 26 two-byte loads.  A neighbour outside the box has a zero tile entry; its coefficient is read at whatever entry lies
+// there: only the first pair reaches back past the start of H, from the box's first row (direction 14, row0) and first
+// line (direction 15, line0), which read on instead.
 __device__ __forceinline__ float half16_value(unsigned pair, int hi)
 {
   return (float)__builtin_bit_cast(_Float16, (unsigned short)(hi ? pair >> 16 : pair & 0xffffu));
 }
 template <int BY>
 __device__ __forceinline__ float half16_row(const Box &bx, const _Float16 *__restrict__ H, const float *tile, int q,
-                                            int tj, int tk, long i)
+                                            int tj, int tk, long row, unsigned i, bool line0, bool row0)
 {
   constexpr int TX = SweepTile<BY, 1>::TX, TY = SweepTile<BY, 1>::TY;
   const long n = bx.n(), sy = bx.nz, sx = (long)bx.ny * bx.nz;
   const unsigned *__restrict__ H2 = (const unsigned *)H;
+  const unsigned i14 = row0 ? i + 1 : i, i15 = line0 ? i + (unsigned)bx.nz : i;
   unsigned up[7];
 #pragma unroll
-  for (int j = 0; j < 7; j++) up[j] = H2[j * n + i];
+  for (int j = 0; j < 7; j++) up[j] = at(H2, j * n + row, i);
   float acc = 0;
 #pragma unroll
   for (int s = 14; s < 27; s++) {
-    const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1;
+    const int di = s / 9 - 1, dj = (s / 3) % 3 - 1, dk = s % 3 - 1, j = (s - 14) >> 1;
     const long off = di * sx + dj * sy + dk;
-    const long il = i - off >= 0 ? i - off : i;
-    const float hu = half16_value(up[(s - 14) >> 1], (s - 14) & 1);
-    const float hl = half16_value(H2[((s - 14) >> 1) * n + il], (s - 14) & 1);
+    const float hu = half16_value(up[j], (s - 14) & 1);
+    const float hl = half16_value(at(H2, j * n + row - off, s == 14 ? i14 : s == 15 ? i15 : i), (s - 14) & 1);
     acc += hu * tile[((q + 1 + di) * TY + tj + dj) * TX + tk + dk];
     acc += hl * tile[((q + 1 - di) * TY + tj - dj) * TX + tk - dk];
   }
@@ -487,21 +558,24 @@ __global__ void __launch_bounds__(256) half16_residual_kernel(Box bx, const _Flo
 {
   __shared__ float tile[SweepTile<kBY, 1>::N];
   const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
-  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int, int, int) { return sc[g] * x[g]; });
+  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, unsigned i, int, int, int) { return at(sc, g, i) * at(x, g, i); });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x;
   if (K >= bx.nz || J >= bx.ny) return;
-  const long i = ((long)I * bx.ny + J) * bx.nz + K;
-  const float ax = dg[i] * x[i] + sc[i] * half16_row<kBY>(bx, H, tile, 0, threadIdx.y + 1, threadIdx.x + 1, i);
-  r[i] = (b ? b[i] : 0.f) - ax;
+  const long row = ((long)I * bx.ny + J0) * bx.nz + K0;
+  const unsigned i = threadIdx.y * (unsigned)bx.nz + threadIdx.x;
+  const float ax = at(dg, row, i) * at(x, row, i) +
+                   at(sc, row, i) * half16_row<kBY>(bx, H, tile, 0, threadIdx.y + 1, threadIdx.x + 1, row, i,
+                                                    I == 0 && J == 0, I == 0 && J == 0 && K == 0);
+  at(r, row, i) = (b ? at(b, row, i) : 0.f) - ax;
 }
 
 // The V-cycle's sweeps on the FP16 coefficients, in the scaled variables; the modes are half_sweep_kernel's.  The
 // residuals leave unscaled (the restriction works on them), and so does the last step of a level (unscale: x = y / s).
 // On the finest level b is the caller's (raw) in the _FIRST forms, which store b' = b / s in bs for the later sweeps.
 // 48 bytes a row instead of 56 and one staged load per neighbour instead of two (s and x): at 239^3 rows a smoothing step
-// 215 -> 165 us, and the first step and the pass that wrote it (55 us) are part of the second one.
+// 215 -> 174 us, and the first step and the pass that wrote it (55 us) are part of the second one.
 template <int MODE, int BY, int NR>
-__global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, const _Float16 *__restrict__ H,
+__global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, Split sp, const _Float16 *__restrict__ H,
                                                                const float *__restrict__ e, const float *__restrict__ f,
                                                                const float *__restrict__ s, const float *__restrict__ b,
                                                                const float *__restrict__ y, float *__restrict__ out,
@@ -514,35 +588,38 @@ __global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, const _Fl
   constexpr bool FIRST = MODE == SW_FIRST_CHEB || MODE == SW_FIRST_RESID, PRO = MODE == SW_PRO_CHEB;
   __shared__ float tile[S::N];
   __shared__ float ct[PRO ? CoarseTile<BY, NR>::N : 1];
-  const int I0 = blockIdx.z * NR, J0 = blockIdx.y * BY, K0 = blockIdx.x * kBX;
+  const int I0 = blockIdx.z * NR, J0 = sp.j0(blockIdx.x, blockIdx.y, BY), K0 = sp.k0(blockIdx.x);
+  const int J1 = sp.j1(blockIdx.x, bx.ny);
+  if (J0 >= J1) return;
   if constexpr (PRO) stage_coarse<BY, NR>(cb, xc, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, ct);
-  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, int gi, int gj, int gk) {
-    if constexpr (FIRST) return c1 * f[g] * b[g];
-    else if constexpr (PRO) return y[g] + s[g] * coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
-    else return y[g];
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, unsigned i, int gi, int gj, int gk) {
+    if constexpr (FIRST) return c1 * at(f, g, i) * at(b, g, i);
+    else if constexpr (PRO) return at(y, g, i) + at(s, g, i) * coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
+    else return at(y, g, i);
   });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x, tj = threadIdx.y + 1, tk = threadIdx.x + 1;
-  if (K >= bx.nz || J >= bx.ny) return;
+  if (K >= bx.nz || J >= J1) return;
+  const unsigned i = threadIdx.y * (unsigned)bx.nz + threadIdx.x;
 #pragma unroll
   for (int q = 0; q < NR; q++) {
     const int I = I0 + q;
     if (NR > 1 && I >= bx.nx) break;
-    const long i = ((long)I * bx.ny + J) * bx.nz + K;
-    const float ay = half16_row<BY>(bx, H, tile, q, tj, tk, i);
-    const float yi = tile[((q + 1) * S::TY + tj) * S::TX + tk], ei = e[i];
-    float bi = b[i];
+    const long row = ((long)I * bx.ny + J0) * bx.nz + K0;
+    const float ay = half16_row<BY>(bx, H, tile, q, tj, tk, row, i, I == 0 && J == 0, I == 0 && J == 0 && K == 0);
+    const float yi = tile[((q + 1) * S::TY + tj) * S::TX + tk], ei = at(e, row, i);
+    float bi = at(b, row, i);
     if (FIRST && raw) {
-      bi /= s[i];
-      bs[i] = bi;
+      bi /= at(s, row, i);
+      at(bs, row, i) = bi;
     }
     const float r = bi - (ei * yi + ay);
     if constexpr (MODE == SW_RESID || MODE == SW_FIRST_RESID) {
-      if constexpr (FIRST) y1[i] = yi;
-      out[i] = s[i] * r;
+      if constexpr (FIRST) at(y1, row, i) = yi;
+      at(out, row, i) = at(s, row, i) * r;
     } else {
-      const float dn = (MODE == SW_FIRST_CHEB ? a * yi : a != 0.f ? a * d[i] : 0.f) + c * r / ei;
-      if (keep_d) d[i] = dn;
-      out[i] = unscale ? (yi + dn) / s[i] : yi + dn;
+      const float dn = (MODE == SW_FIRST_CHEB ? a * yi : a != 0.f ? a * at(d, row, i) : 0.f) + c * r / ei;
+      if (keep_d) at(d, row, i) = dn;
+      at(out, row, i) = unscale ? (yi + dn) / at(s, row, i) : yi + dn;
     }
   }
 }
@@ -598,15 +675,19 @@ __host__ __device__ constexpr double pweight(int e, int t)
 // and are summed into 3 x 3 partial sums in registers (every load unconditional: a support node outside the fine box
 // reads entry 0 with weight 0).  The partial sums meet the x weights through LDS, three of the 27 entries per wavefront.
 // With one thread per row the nine parts followed one another, 729 loads at 13 wavefronts per SIMD in all: latency
-// bound, 1.90 ms at 95^3 coarse rows and 0.11 ms at 5^3; this takes 0.84 and 0.01 ms.  Entries toward coarse nodes
+// bound, 1.90 ms at 95^3 coarse rows and 0.11 ms at 5^3; this takes 0.71 and 0.01 ms.  Entries toward coarse nodes
 // outside the box are zero, as the assembly leaves them on the finest level.
-__global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, const double *__restrict__ Af, double *__restrict__ Ac)
+__global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const double *__restrict__ Af, double *__restrict__ Ac)
 {
-  __shared__ double part[9][9][64];  // [x part][3 x 3 sum][row]
+  __shared__ double psum[9][9][64];  // [x part][3 x 3 sum][row]
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, a = w / 3 - 1, si = w % 3 - 1;
-  const long nc = c.n(), nf = f.n(), C = (long)blockIdx.x * 64 + lane;
-  int I, J, K;
-  unrank(c, C < nc ? C : nc - 1, I, J, K);
+  const long nc = c.n(), nf = f.n();
+  // a part's lines of one plane are one run of rows
+  const int xcd = blockIdx.x & 7, jp = xcd * part, lines = min(part, c.ny - jp), o0 = (int)(blockIdx.x >> 3) * 64 + lane;
+  if (lines <= 0 || (int)(blockIdx.x >> 3) * 64 >= lines * c.nz) return;
+  const bool valid = o0 < lines * c.nz;
+  const int o = valid ? o0 : 0, I = blockIdx.y, J = jp + o / c.nz, K = o % c.nz;
+  const long C = ((long)I * c.ny + J) * c.nz + K;
   const long sy = f.nz, sx = (long)f.ny * f.nz;
   const int fi = 2 * I + 1 + a;  // >= 0
   double T[9];
@@ -635,19 +716,19 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, const double *__
         }
     }
 #pragma unroll
-  for (int u = 0; u < 9; u++) part[w][u][lane] = T[u];
+  for (int u = 0; u < 9; u++) psum[w][u][lane] = T[u];
   __syncthreads();
-  if (C >= nc) return;
+  if (!valid) return;
 #pragma unroll
-  for (int o = 0; o < 3; o++) {  // entry t = 9 o + w: x offset o - 1
-    const int t = 9 * o + w;
+  for (int x = 0; x < 3; x++) {  // entry t = 9 x + w: x offset x - 1
+    const int t = 9 * x + w;
     double acc = 0.0;
 #pragma unroll
     for (int aa = -1; aa <= 1; aa++)
 #pragma unroll
       for (int ss = -1; ss <= 1; ss++)
-        acc = fma(pweight(aa, 0) * pweight(aa + ss, o - 1), part[(aa + 1) * 3 + ss + 1][w][lane], acc);
-    Ac[t * nc + C] = inside(c, I + o - 1, J + w / 3 - 1, K + w % 3 - 1) ? acc : 0.0;
+        acc = fma(pweight(aa, 0) * pweight(aa + ss, x - 1), psum[(aa + 1) * 3 + ss + 1][w][lane], acc);
+    Ac[t * nc + C] = inside(c, I + x - 1, J + w / 3 - 1, K + w % 3 - 1) ? acc : 0.0;
   }
 }
 
@@ -930,11 +1011,13 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     l.v[0] = lv.r64.ptr;
     l.v[1] = lv.d64.ptr;
     l.big = sweep_big(lv.box);
-    l.gx = (lv.box.nz + kBX - 1) / kBX;
-    l.gy = (lv.box.ny + 7) / 8;
-    l.blocks = (int)(l.gx * l.gy * (l.big ? (lv.box.nx + 1) / 2 : lv.box.nx));
+    l.sp = split_of(lv.box, 8);
+    const dim3 grid = split_grid(lv.box, l.sp, 8, l.big ? 2 : 1);
+    l.gx = grid.x;
+    l.gy = grid.y;
+    l.blocks = (int)(grid.x * grid.y * grid.z);
     l.first = blocks;
-    blocks += l.blocks;
+    blocks += (l.blocks + 7) / 8 * 8;
     parts += std::max(256, l.blocks);
   }
   if (!mg->part.holds(parts)) DOHP_CALL(mg->part.alloc(parts));
@@ -1081,15 +1164,16 @@ void sweep16(const MGLevel &lv, const float *b, const float *y, float *out, floa
              int keep_d, int raw, int unscale, hipStream_t st, const Box &cb = Box{}, const float *xc = nullptr)
 {
   const Box &bx = lv.box;
-  const unsigned gx = (bx.nz + kBX - 1) / kBX, gy = (bx.ny + 3) / 4;
+  const auto launch = [&](auto kernel, int BY, int NR) {
+    const Split sp = split_of(bx, BY);
+    hipLaunchKernelGGL(kernel, split_grid(bx, sp, BY, NR), dim3(kBX, BY), 0, st, bx, sp, lv.H16.ptr, lv.e16.ptr,
+                       lv.f16.ptr, lv.sc16.ptr, b, y, out, lv.d32.ptr, y1, lv.t32.ptr, (float)a, (float)c, (float)c1,
+                       keep_d, raw, unscale, cb, xc);
+  };
   if (lv.n >= 8000000)
-    hipLaunchKernelGGL((half16_sweep_kernel<MODE, 4, 2>), dim3(gx, gy, (bx.nx + 1) / 2), dim3(kBX, 4), 0, st, bx,
-                       lv.H16.ptr, lv.e16.ptr, lv.f16.ptr, lv.sc16.ptr, b, y, out, lv.d32.ptr, y1, lv.t32.ptr,
-                       (float)a, (float)c, (float)c1, keep_d, raw, unscale, cb, xc);
+    launch(half16_sweep_kernel<MODE, 4, 2>, 4, 2);
   else
-    hipLaunchKernelGGL((half16_sweep_kernel<MODE, 4, 1>), dim3(gx, gy, bx.nx), dim3(kBX, 4), 0, st, bx, lv.H16.ptr,
-                       lv.e16.ptr, lv.f16.ptr, lv.sc16.ptr, b, y, out, lv.d32.ptr, y1, lv.t32.ptr, (float)a, (float)c,
-                       (float)c1, keep_d, raw, unscale, cb, xc);
+    launch(half16_sweep_kernel<MODE, 4, 1>, 4, 1);
 }
 
 // FP32 V-cycle on the FP16 coefficients, in the scaled variables: b is b' on the coarse levels (the restriction scales
@@ -1152,8 +1236,9 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
   for (size_t l = 1; l < mg->L.size(); l++) {
     const MGLevel &f = mg->L[l - 1];
     MGLevel &c = mg->L[l];
-    hipLaunchKernelGGL(rap_kernel, dim3((unsigned)((c.n + 63) / 64)), dim3(576), 0, st, f.box, c.box, f.A64,
-                       c.own64.ptr);
+    const int part = (c.box.ny + 7) / 8;
+    hipLaunchKernelGGL(rap_kernel, dim3(8u * (unsigned)(((long)part * c.box.nz + 63) / 64), (unsigned)c.box.nx),
+                       dim3(576), 0, st, f.box, c.box, part, f.A64, c.own64.ptr);
   }
   for (size_t l = 0; l < mg->L.size(); l++) {
     MGLevel &lv = mg->L[l];
@@ -1161,11 +1246,13 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
     const bool smoothed = l + 1 < mg->L.size();
     hipLaunchKernelGGL(diag_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.dinv64.ptr, lv.dinv32.ptr,
                        smoothed ? lv.sc16.ptr : nullptr);
-    if (smoothed)
-      hipLaunchKernelGGL(half_setup_kernel, box_grid(lv.box), box_block(), 0, st, lv.box, lv.A64, lv.H64.ptr,
-                         lv.H32.ptr, lv.H16.ptr, lv.dg16.ptr, lv.sc16.ptr, lv.e16.ptr, lv.f16.ptr, l > 0);
-    else
+    if (smoothed) {
+      const Split sp = split_of(lv.box, kBY);
+      hipLaunchKernelGGL(half_setup_kernel, split_grid(lv.box, sp, kBY, 1), box_block(), 0, st, lv.box, sp, lv.A64,
+                         lv.H64.ptr, lv.H32.ptr, lv.H16.ptr, lv.dg16.ptr, lv.sc16.ptr, lv.e16.ptr, lv.f16.ptr, l > 0);
+    } else {
       hipLaunchKernelGGL(half_from_full_kernel, grid_of(n), dim3(256), 0, st, n, lv.A64, lv.H64.ptr, lv.H32.ptr);
+    }
     lv.H = lv.H64.ptr ? lv.H64.ptr : lv.A64 + 13 * n;
   }
   DOHP_CALL(estimate_lmax(mg, st, 15));
