@@ -101,3 +101,35 @@ def test_captured_and_concurrent_calls(C):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ref), k
+
+
+def test_physical_flags_do_not_outlive_their_call(C):
+    """A negative or non-finite determinant is that call's error alone, from several threads and streams at once."""
+    import threading
+
+    w = np.array([5 / 9, 8 / 9, 5 / 9])
+    out = []
+
+    def calls(kind):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            jac = (torch.eye(3, dtype=torch.float64, device="cuda") * 0.5).expand(700, 3, 3, 3, 3, 3).contiguous()
+            if kind == 1:
+                jac[699, 2, 2, 2, 0, 0] = -0.5
+            elif kind == 2:
+                jac[0, 0, 0, 0, 0, 0] = float("nan")
+            jinv, jw = torch.zeros_like(jac), torch.zeros(jac.shape[:4], dtype=torch.float64, device="cuda")
+            st.synchronize()
+            for _ in range(20):
+                try:
+                    C.rule_compute_physical_batched(w, 700, jac, jinv, jw)
+                    out.append((kind, "ok"))
+                except C.DohpError as e:
+                    out.append((kind, "negative" if "egative" in str(e) else "finite" if "finite" in str(e) else str(e)))
+
+    threads = [threading.Thread(target=calls, args=(k % 3,)) for k in range(12)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(out) == 240 and set(out) == {(0, "ok"), (1, "negative"), (2, "finite")}
