@@ -200,7 +200,7 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ tab, int op, cons
   }
 }
 
-// Element tiles [i][j][k] (k fastest, the reference's node order).  A thread (a, b) of an
+// Element tiles [i][j][k] (k fastest, the reference's node order; lines of n values at a pitch of line_pitch(n)).  A thread (a, b) of an
 // element owns one line per phase: a z line (i, j) = (a, b), a y line (i, k) = (a, b) or an
 // x line (j, k) = (a, b).  No register value crosses from one phase to the next, so any one-to-one
 // assignment of lines to threads within a phase is valid.  At n = 7 the y lines are dealt out as
@@ -210,11 +210,24 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ tab, int op, cons
 // residual and recomputing kernels at degree 6 run 1.3-1.9 % faster).  At the other orders no
 // permutation of this kind measured faster, and (a, b) is kept.
 enum { DIR_X = 0, DIR_Y = 1, DIR_Z = 2 };
+// At n = 4 a line of the tile is followed by an unused slot: at a pitch of 4 the 16 lanes of an element start on a
+// quarter of the banks in the z phase (conflicts a third of the compute units' cycles; A x at degree 3, 250 k elements
+// 185 -> 177 us, the residual 255 -> 250).  At the other even orders the larger tiles cost more than the conflicts (n = 6:
+// A x 154 -> 187 us; the batched mixed orders 393 -> 485).  Point t (i n^2 + j n + k, over all elements of the workgroup)
+// is at tile_slot(t).
+constexpr int line_pitch(int N) { return N == 4 ? 5 : N; }
+constexpr int tile_len(int N) { return N * N * line_pitch(N); }
+template <int N>
+__device__ __forceinline__ int tile_slot(int t)
+{
+  return line_pitch(N) == N ? t : t + t / N;
+}
 template <int N, int DIR>
 __device__ __forceinline__ int line_at(int a, int b, int s)
 {
   if constexpr (DIR == DIR_Y && N == 7) return (b * N + s) * N + (a == 0 ? 0 : N - a);
-  return DIR == DIR_Z ? (a * N + b) * N + s : DIR == DIR_Y ? (a * N + s) * N + b : (s * N + a) * N + b;
+  constexpr int P = line_pitch(N);
+  return DIR == DIR_Z ? (a * N + b) * P + s : DIR == DIR_Y ? (a * N + s) * P + b : (s * N + a) * P + b;
 }
 template <int N, int DIR, typename T>
 __device__ __forceinline__ void ld_line(const T *tile, int a, int b, T (&v)[N])
@@ -366,7 +379,7 @@ __device__ __forceinline__ void mfma_lines(const T *__restrict__ frag, const T *
                                            int own, int lane)
 {
   static_assert(N <= kMfmaMaxN, "the line pass holds at most 8 points per field");
-  constexpr int STR = DIR == DIR_Z ? 1 : DIR == DIR_Y ? N : N * N, KS = 2 * NIN;
+  constexpr int STR = DIR == DIR_Z ? 1 : DIR == DIR_Y ? line_pitch(N) : N * line_pitch(N), KS = 2 * NIN;
   typedef typename Mfma16<T>::acc acc;
   const int kq = lane >> 4;
   T op[KS];
@@ -399,7 +412,7 @@ template <int N, typename T>
 __device__ __forceinline__ void forward_mfma(const T *tab, const T *frag, T *TA, T *TGX, T *TGY, int le, int a,
                                              int b, T (&q)[N], T (&gx)[N], T (&gy)[N], T (&gz)[N])
 {
-  const int lane = threadIdx.x & 63, e0 = le * N * N * N;
+  const int lane = threadIdx.x & 63, e0 = le * tile_len(N);
   const int bz = e0 + line_at<N, DIR_Z>(a, b, 0), by = e0 + line_at<N, DIR_Y>(a, b, 0),
             bx = e0 + line_at<N, DIR_X>(a, b, 0);
   mfma_lines<N, DIR_Z, T, 1, 1>(frag + MF_B, TA, TA, TA, TA, bz, lane);
@@ -423,7 +436,7 @@ __device__ __forceinline__ void backward_mfma(const T *tab, const T *frag, T *TA
                                               int b, const T (&v)[N], const T (&d0)[N], const T (&d1)[N],
                                               const T (&d2)[N])
 {
-  const int lane = threadIdx.x & 63, e0 = le * N * N * N;
+  const int lane = threadIdx.x & 63, e0 = le * tile_len(N);
   const int bz = e0 + line_at<N, DIR_Z>(a, b, 0), by = e0 + line_at<N, DIR_Y>(a, b, 0),
             bx = e0 + line_at<N, DIR_X>(a, b, 0);
   T w[N];

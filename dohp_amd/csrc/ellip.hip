@@ -84,7 +84,7 @@ __attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <=
                 "matrix-core passes: n <= 8, one line per thread, modes that scatter");
   constexpr int NN = N * N, N3 = NN * N, NT = MF ? 256 : wg_threads(N, EPB), NS = (EPB * N3 + NT - 1) / NT;
   constexpr int ET = EPB + (MF ? 1 : 0);  // element tiles (the pad tile last)
-  __shared__ T TA[ET * N3], TGX[ET * N3], TGY[ET * N3];
+  __shared__ T TA[ET * tile_len(N)], TGX[ET * tile_len(N)], TGY[ET * tile_len(N)];
   __shared__ int IDX[EPB * N3];
   __shared__ double VX[ET * 8 * 4];
   __shared__ int EB[ET * 4];  // per element slot: first lattice point, 1 if the slot holds an element
@@ -180,7 +180,7 @@ __attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <=
       if (t < EPB * N3) {
         const T v = own[s] >= 0 ? xv[s] : T(0), u = lat[s] >= 0 ? uv[s] : T(0);
         IDX[t] = own[s];
-        TA[t] = STATE_FIRST ? u : v;
+        TA[tile_slot<N>(t)] = STATE_FIRST ? u : v;
         if (MODE == MODE_JAC) pre2[s] = STATE_FIRST ? v : u;
       }
     }
@@ -227,7 +227,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
   constexpr bool PREFETCH_VALUES = MODE != MODE_JAC || sizeof(T) == 4;
   constexpr bool GATHER_X = MODE == MODE_LIN || MODE == MODE_JQD;  // else the state
   constexpr bool PREFETCH_STATE = MODE == MODE_JAC && PREFETCH_VALUES;
-  __shared__ T TA[EPB * N3], TGX[EPB * N3], TGY[EPB * N3];
+  __shared__ T TA[EPB * tile_len(N)], TGX[EPB * tile_len(N)], TGY[EPB * tile_len(N)];
   __shared__ int IDX[EPB * N3];
   __shared__ double VX[EPB * 8 * 4];
   const int tid = threadIdx.x;
@@ -299,7 +299,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
         const int t = s * NT + tid;
         if (t < EPB * N3) {
           IDX[t] = pidx[s];
-          TA[t] = pval[s];
+          TA[tile_slot<N>(t)] = pval[s];
         }
       }
     }
@@ -322,7 +322,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
         if (t < EPB * N3) {
           IDX[t] = own;
           const T xv = own >= 0 ? xdir[own] : T(0), uv = lat >= 0 ? ustate[lat] : T(0);
-          TA[t] = jac_state_first<N, T>() ? uv : xv;
+          TA[tile_slot<N>(t)] = jac_state_first<N, T>() ? uv : xv;
           pre2[s] = jac_state_first<N, T>() ? xv : uv;
         }
       }
