@@ -624,6 +624,327 @@ __global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, Split sp,
   }
 }
 
+// Two sweeps in one pass over the coefficients.  A sweep reads 112 (FP64) or 28 bytes of coefficients per row for one
+// product and runs at the rate of memory, so two of them that follow each other are taken together: a workgroup owns a
+// column of the box, lines x columns of its (J, K) face, and marches along I.  On plane i it takes the first sweep,
+// y1 = S1 (A v0), and with it finishes the second one, S2 (A y1), on plane i - 1.  Symmetry lets a plane's coefficients be
+// read once: the product of row (i, j, k) with its lower neighbours is summed while their plane is at hand, as the part
+// that the plane below adds to plane i (p1 for the first product, p2 for the second).
+//  - A thread owns one (j, k); the face has two rows and columns more on each side than the workgroup's output (its
+//    first product is valid one row inside, its second two).
+//  - LDS holds the coefficients of the current plane (written by their owners, read by the neighbours above them), v0 on
+//    planes i and i + 1, and y1 on plane i.  The next plane's coefficients and the vectors of the one after it are
+//    loaded into registers a plane ahead.
+//  - Faces: one workgroup per compute unit.  FP16 coefficients: 1024 threads, 64 columns wide (32: 252 instead of 221 us
+//    at 239^3).  FP64: 768 threads, whose 168 registers hold a plane ahead (1024 threads: 128, and 176 bytes spilled; 915
+//    us a pair of power iterations at 191^3 against 256), 48 columns (32: 269 us).
+// 239^3 rows, FP16: both pre-smoothing steps and the residual 221 us against 353 in two sweeps, both post-smoothing steps
+// 235 against 370.  191^3, FP64: two power iterations 256 us against 462, pre-smoothing 264 against 392, post-smoothing
+// 295 against 476.
+// PAIR_POWER: w = (D^-1 A)^2 (v / ||v||) and its sum of squares.  PAIR_PRE: the first two smoothing steps from zero and
+// their residual.  PAIR_POST: prolongation and the last two smoothing steps.
+enum { PAIR_POWER, PAIR_PRE, PAIR_POST };
+constexpr int kPairPad = 80;  // LDS entries around the face: border threads read past it, values that nothing uses
+constexpr int kPairSlots = 256;
+template <typename T>
+constexpr int pair_threads()
+{
+  return sizeof(T) == 8 ? 768 : 1024;
+}
+template <typename T>
+constexpr int pair_width()
+{
+  return sizeof(T) == 8 ? 48 : 64;
+}
+static_assert(kPairPad > pair_width<float>() + 5, "a border thread reads one line and one column away");
+struct PairTiles {
+  int tk, tj, nk, nj, ni, chunk;  // columns and lines of a face, workgroups along K, J and I, planes of one
+  int blocks() const { return nk * nj * ni; }
+};
+// Levels that take pairs.  Below, a face's border and the few planes of a chunk cost more than the second read of the
+// coefficients, which then comes from the 256 MB cache: V-cycles of 79^3 rows take 153 us with pairs against 151 (FP64) and
+// 126 against 116 (FP16), of 89^3 159 against 211 and 126 against 122, of 99^3 134 against 148 (FP16).
+template <typename T>
+inline bool pair_level(const Box &b)
+{
+  return b.n() >= (sizeof(T) == 8 ? 600000 : 800000);
+}
+// Faces as wide as the box divides into at most 64 columns, and as many chunks along I as fill `slots` workgroups.
+template <typename T>
+PairTiles pair_tiles(const Box &b, int slots)
+{
+  PairTiles g;
+  g.nk = (b.nz + pair_width<T>() - 1) / pair_width<T>();
+  g.tk = (b.nz + g.nk - 1) / g.nk + 4;
+  g.tj = std::min(pair_threads<T>() / g.tk, b.ny + 4);
+  g.nj = (b.ny + g.tj - 5) / (g.tj - 4);
+  const int ni = std::max(1, std::min(slots / (g.nk * g.nj), b.nx / 8));
+  g.chunk = (b.nx + ni - 1) / ni;
+  g.ni = (b.nx + g.chunk - 1) / g.chunk;
+  return g;
+}
+
+template <typename T>
+struct PairCoeffs;
+template <>
+struct PairCoeffs<double> {  // h[0]: diagonal
+  typedef double E;
+  static constexpr int kRegs = 14;
+  double h[14];
+  __device__ __forceinline__ void load(const void *H, long n, long row, unsigned i)
+  {
+#pragma unroll
+    for (int j = 0; j < 14; j++) h[j] = at((const double *)H, j * n + row, i);
+  }
+  static constexpr int kPlanes = 22;  // directions 14..17, and 18..26 of two planes in turn
+  static __device__ __forceinline__ int plane(int s, int par)
+  {
+    return (s < 18 ? s - 14 : 4 + 9 * par + s - 18) * pair_threads<double>();
+  }
+  __device__ __forceinline__ void store(double *hs, int t, int par) const
+  {
+#pragma unroll
+    for (int s = 14; s < 27; s++) hs[plane(s, par) + t] = h[s - 13];
+  }
+  __device__ __forceinline__ double up(int s) const { return h[s - 13]; }
+  static __device__ __forceinline__ double lo(const double *hs, int s, int t, int par) { return hs[plane(s, par) + t]; }
+  // the upper coefficients of the plane before stay in LDS (18 registers fewer)
+  __device__ __forceinline__ void keep() {}
+  __device__ __forceinline__ double kept(const double *hs, int s, int t, int par) const { return hs[plane(s, 1 - par) + t]; }
+};
+template <>
+struct PairCoeffs<float> {
+  typedef unsigned E;
+  static constexpr int kRegs = 7;
+  unsigned h[7];
+  __device__ __forceinline__ void load(const void *H, long n, long row, unsigned i)
+  {
+#pragma unroll
+    for (int j = 0; j < 7; j++) h[j] = at((const unsigned *)H, j * n + row, i);
+  }
+  static constexpr int kPlanes = 7;
+  unsigned k[5] = {};
+  __device__ __forceinline__ void store(unsigned *hs, int t, int) const
+  {
+#pragma unroll
+    for (int j = 0; j < 7; j++) hs[j * pair_threads<float>() + t] = h[j];
+  }
+  __device__ __forceinline__ float up(int s) const { return half16_value(h[(s - 14) >> 1], (s - 14) & 1); }
+  __device__ __forceinline__ void keep()
+  {
+#pragma unroll
+    for (int j = 0; j < 5; j++) k[j] = h[j + 2];
+  }
+  __device__ __forceinline__ float kept(const unsigned *, int s, int, int) const
+  {
+    return half16_value(k[(s - 18) >> 1], (s - 14) & 1);
+  }
+  static __device__ __forceinline__ float lo(const unsigned *hs, int s, int t, int)
+  {
+    return half16_value(hs[((s - 14) >> 1) * pair_threads<float>() + t], (s - 14) & 1);
+  }
+};
+
+template <typename T>
+struct PairArgs {
+  Box bx, cb;
+  PairTiles g;
+  const void *H;
+  const T *dinv, *f, *s;  // FP64: D^-1, null, null.  FP16: e, f, s of half16_sweep_kernel
+  const T *b, *x, *xc;
+  T *out, *r, *bs;
+  T c1, a, c;             // first step's factor, the second one's
+  int raw, unscale;
+  const double *inv;
+  double *part;
+};
+template <typename T>
+constexpr int pair_lds()
+{
+  return pair_threads<T>() * (PairCoeffs<T>::kPlanes * (int)sizeof(typename PairCoeffs<T>::E) + 3 * (int)sizeof(T)) +
+         8 * kPairPad * (int)sizeof(T);
+}
+
+template <typename T, int MODE>
+__device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *lds)
+{
+  typedef PairCoeffs<T> C;
+  constexpr bool F16 = sizeof(T) == 4;
+  const PairTiles &g = A.g;
+  const Box &bx = A.bx;
+  typename C::E *Hs = (typename C::E *)lds + kPairPad;
+  T *V = (T *)(Hs + C::kPlanes * pair_threads<T>()) + kPairPad, *Y = V + 2 * pair_threads<T>() + 2 * kPairPad;
+  const int t = threadIdx.x, tk = g.tk;
+  const int kt = blk % g.nk, rest = blk / g.nk, jt = rest % g.nj, it = rest / g.nj;
+  const int ia = it * g.chunk, ib = min(bx.nx, ia + g.chunk);
+  const int tj = (int)((t + 0.5f) * (1.f / tk)), J = jt * (g.tj - 4) - 2 + tj, K = kt * (tk - 4) - 2 + t - tj * tk;
+  const bool live = tj < g.tj && J >= 0 && J < bx.ny && K >= 0 && K < bx.nz;
+  const bool mine = live && tj >= 2 && tj < g.tj - 2 && t - tj * tk >= 2 && t - tj * tk < tk - 2;
+  const unsigned o = live ? (unsigned)J * bx.nz + K : 0u;
+  const long n = bx.n(), sx = (long)bx.ny * bx.nz;
+  // coarse plane's in-plane sum at (J, K): the first four terms of coarse_value
+  const int j1 = J >> 1, k1 = K >> 1, j0 = j1 - 1 + (J & 1), k0 = k1 - 1 + (K & 1);
+  const auto plane_sum = [&](int ci) -> T {
+    if (!live || ci < 0 || ci >= A.cb.nx) return T(0);
+    const T *p = A.xc + (long)ci * A.cb.ny * A.cb.nz;
+    const auto v = [&](int j, int k) {
+      const bool in = j >= 0 && j < A.cb.ny && k >= 0 && k < A.cb.nz;
+      const T y = p[in ? j * A.cb.nz + k : 0];
+      return in ? y : T(0);
+    };
+    return (v(j0, k0) + v(j0, k1)) + (v(j1, k0) + v(j1, k1));
+  };
+  struct Row {
+    T b, d, s, v;  // right-hand side, D^-1 (FP64) or e (FP16), row scale, v0
+  };
+  // v0 and the vectors on plane i (zero outside the box); planes come in order from ia - 2 on
+  T sum0 = 0, sum1 = 0;
+  int have = -2;  // (the coarse plane that sum1 holds)
+  const T inv = MODE == PAIR_POWER ? (T)*A.inv : T(0);
+  const auto load_row = [&](int i, Row &w) {
+    const long row = (long)min(max(i, 0), bx.nx - 1) * sx;
+    const bool in = live && i >= 0 && i < bx.nx;
+    w.d = at(A.dinv, row, o);
+    w.s = F16 ? at(A.s, row, o) : T(1);
+    T v;
+    if constexpr (MODE == PAIR_POWER) {
+      w.b = T(0);
+      v = inv * at(A.x, row, o);
+    } else if constexpr (MODE == PAIR_PRE) {
+      w.b = at(A.b, row, o);
+      v = A.c1 * (F16 ? at(A.f, row, o) : w.d) * w.b;
+      if (F16 && A.raw) w.b /= w.s;
+    } else {
+      w.b = at(A.b, row, o);
+      const int hi = i >> 1, lo = hi - 1 + (i & 1);  // parents of plane i
+      if (i >= 0 && have != hi) {
+        sum0 = have == hi - 1 ? sum1 : plane_sum(hi - 1);
+        sum1 = plane_sum(hi);
+        have = hi;
+      }
+      const T pro = T(0.125) * ((lo == hi ? sum1 : sum0) + sum1);
+      v = F16 ? at(A.x, row, o) + w.s * pro : at(A.x, row, o) + pro;
+    }
+    w.v = in ? v : T(0);
+  };
+  const int i0 = max(ia - 2, 0), ilast = min(ib, bx.nx);  // (plane nx has no rows: its y1 is zero)
+  C h, hn;
+  Row w0, w1, w2;
+  load_row(i0, w0);
+  load_row(i0 + 1, w1);
+  h.load(A.H, n, (long)i0 * sx, o);
+  __syncthreads();  // (the last use of LDS by the caller)
+  V[(i0 & 1) * pair_threads<T>() + t] = w0.v;
+  V[((i0 + 1) & 1) * pair_threads<T>() + t] = w1.v;
+  T p1 = 0, p2 = 0, q = 0, pb = 0, pd = 1, ps = 1, py = 0, pstep = 0;
+  double sum = 0;
+  for (int i = i0; i <= ilast; i++) {
+    const bool inside_i = i < bx.nx;
+    h.store(Hs, t, i & 1);
+    load_row(i + 2, w2);
+    if (i + 1 < bx.nx) hn.load(A.H, n, (long)(i + 1) * sx, o);
+    __syncthreads();
+    const T *V0 = V + (i & 1) * pair_threads<T>() + t, *V1 = V + ((i + 1) & 1) * pair_threads<T>() + t;
+    // first sweep on plane i
+    T acc = (F16 ? w0.d : h.up(13)) * V0[0] + p1;
+    p1 = T(0);
+#pragma unroll
+    for (int s = 14; s < 27; s++) {
+      const int off = ((s / 3) % 3 - 1) * tk + s % 3 - 1;
+      const T lo = C::lo(Hs, s, t - off, i & 1) * V0[-off];
+      if (s < 18) {
+        acc += h.up(s) * V0[off];
+        acc += lo;
+      } else {
+        acc += h.up(s) * V1[off];
+        p1 += lo;
+      }
+    }
+    const T y0 = w0.v;
+    T y1, step = T(0);
+    if constexpr (MODE == PAIR_POWER) {
+      y1 = w0.d * acc;
+    } else {
+      const T res = w0.b - acc;
+      const T cc = MODE == PAIR_PRE ? A.c : A.c1;
+      step = F16 ? cc * res / w0.d : cc * w0.d * res;
+      if (MODE == PAIR_PRE) step = A.a * y0 + step;
+      y1 = y0 + step;
+    }
+    if (!live || !inside_i) y1 = T(0);
+    Y[t] = y1;
+    if (MODE == PAIR_PRE && mine && i >= ia && i < ib) {
+      at(A.out, i * sx, o) = y1;
+      if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
+    }
+    __syncthreads();
+    // second sweep: plane i - 1 is complete with y1 on plane i
+    T z = q;
+    const T *Yt = Y + t;
+#pragma unroll
+    for (int s = 18; s < 27; s++) z += h.kept(Hs, s, t, i & 1) * Yt[((s / 3) % 3 - 1) * tk + s % 3 - 1];
+    if (mine && i > ia && i <= ib) {
+      const long row = (i - 1) * sx;
+      if constexpr (MODE == PAIR_POWER) {
+        const T y2 = pd * z;
+        at(A.out, row, o) = y2;
+        sum += (double)y2 * (double)y2;
+      } else if constexpr (MODE == PAIR_PRE) {
+        at(A.r, row, o) = F16 ? ps * (pb - z) : pb - z;
+      } else {
+        const T dn = A.a * pstep + (F16 ? A.c * (pb - z) / pd : A.c * pd * (pb - z));
+        at(A.out, row, o) = F16 && A.unscale ? (py + dn) / ps : py + dn;
+      }
+    }
+    q = (F16 ? w0.d : h.up(13)) * y1 + p2;
+    p2 = T(0);
+#pragma unroll
+    for (int s = 14; s < 27; s++) {
+      const int off = ((s / 3) % 3 - 1) * tk + s % 3 - 1;
+      const T lo = C::lo(Hs, s, t - off, i & 1) * Yt[-off];
+      if (s < 18) {
+        q += h.up(s) * Yt[off];
+        q += lo;
+      } else {
+        p2 += lo;
+      }
+    }
+    pb = w0.b;
+    pd = w0.d;
+    ps = w0.s;
+    py = y1;
+    pstep = step;
+    V[(i & 1) * pair_threads<T>() + t] = w2.v;
+    h.keep();
+#pragma unroll
+    for (int j = 0; j < C::kRegs; j++) h.h[j] = hn.h[j];
+    w0 = w1;
+    w1 = w2;
+    __syncthreads();
+  }
+  if constexpr (MODE == PAIR_POWER) {
+    const double tot = block_sum<pair_threads<T>()>(sum, t, (double *)lds);
+    if (t == 0) A.part[blk] = tot;
+  }
+}
+
+// Workgroups of one XCD take consecutive faces (K, then J, then I), whose borders meet in its L2.
+template <typename T, int MODE>
+__global__ void __launch_bounds__(pair_threads<T>()) pair_kernel(PairArgs<T> A)
+{
+  extern __shared__ double pair_smem[];
+  const int total = A.g.nk * A.g.nj * A.g.ni, per = (total + 7) / 8, blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if (blk >= total) return;
+  pair_body<T, MODE>(A, blk, (char *)pair_smem);
+}
+
+template <typename T, int MODE>
+void pair_sweep(const PairArgs<T> &A, hipStream_t st)
+{
+  hipLaunchKernelGGL((pair_kernel<T, MODE>), dim3((unsigned)((A.g.blocks() + 7) / 8 * 8)), dim3(pair_threads<T>()),
+                     pair_lds<T>(), st, A);
+}
+
 // The half stencil alone (the coarsest level, which is solved directly).
 __global__ void half_from_full_kernel(long n, const double *__restrict__ A, double *__restrict__ H,
                                       float *__restrict__ H32)
@@ -1001,6 +1322,8 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
   PowerArgs g{};
   g.nl = nl;
   unsigned blocks = 0;
+  int nb = 0;
+  unsigned blocks_small = 0;
   size_t parts = 2 * kMaxLevels;  // norms and their inverses, then the levels' block sums
   for (int k = 0; k < nl; k++) {
     MGLevel &lv = mg->L[k];
@@ -1019,6 +1342,7 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     l.first = blocks;
     blocks += (l.blocks + 7) / 8 * 8;
     parts += std::max(256, l.blocks);
+    if (pair_level<double>(lv.box)) nb = k + 1;  // (levels shrink: the first ones)
   }
   if (!mg->part.holds(parts)) DOHP_CALL(mg->part.alloc(parts));
   double *norm = mg->part.ptr, *inv = norm + kMaxLevels, *at = inv + kMaxLevels;
@@ -1028,7 +1352,44 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
   }
   hipLaunchKernelGGL(power_start_kernel, dim3(256, nl), dim3(256), 0, st, g);
   hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 1, norm, inv);
-  for (int k = 0; k < its; k++) {
+  // large levels take two iterations a pass, the others one by one beside them; the last iteration, whose growth is the
+  // estimate, is a single one everywhere
+  const int pairs = nb ? (its - 1) / 2 : 0;
+  PowerArgs gs = g, gb = g;  // the small levels alone; the large ones with their pairs' block counts
+  if (pairs) {
+    gs.nl = nl - nb;
+    unsigned first = 0;
+    for (int k = nb; k < nl; k++) {
+      gs.l[k - nb] = g.l[k];
+      gs.l[k - nb].first = first;
+      first += (g.l[k].blocks + 7) / 8 * 8;
+    }
+    blocks_small = first;
+  }
+  for (int q = 0; q < pairs; q++) {
+    for (int k = 0; k < nb; k++) {
+      PowerLevel &l = gb.l[k];
+      PairArgs<double> pa{};
+      pa.bx = l.bx;
+      pa.g = pair_tiles<double>(l.bx, kPairSlots);
+      pa.H = l.H;
+      pa.dinv = l.dinv;
+      pa.x = l.v[q & 1];
+      pa.out = l.v[1 - (q & 1)];
+      pa.inv = inv + k;
+      pa.part = l.part;
+      l.blocks = pa.g.blocks();
+      pair_sweep<double, PAIR_POWER>(pa, st);
+    }
+    for (int k = 0; k < 2 && gs.nl; k++) {
+      hipLaunchKernelGGL(power_step_kernel, dim3(blocks_small), dim3(kPowerThreads), 0, st, gs, k, inv + nb);
+      hipLaunchKernelGGL(power_norm_kernel, dim3(gs.nl), dim3(1024), 0, st, gs, 0, norm + nb, inv + nb);
+    }
+    hipLaunchKernelGGL(power_norm_kernel, dim3(nb), dim3(1024), 0, st, gb, 0, norm, inv);
+  }
+  if (pairs & 1)
+    for (int k = 0; k < nb; k++) std::swap(g.l[k].v[0], g.l[k].v[1]);
+  for (int k = 0; k < its - 2 * pairs; k++) {
     hipLaunchKernelGGL(power_step_kernel, dim3(blocks), dim3(kPowerThreads), 0, st, g, k & 1, inv);
     hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 0, norm, inv);
   }
@@ -1126,7 +1487,14 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
   double a, c, c1;
   ChebCoeffs pre(mg, lv);
   pre.step(0, a, c1);
-  if (mg->degree == 1) {
+  const bool pair = sizeof(T) == 8 && mg->degree == 2 && pair_level<double>(lv.box);
+  PairArgs<double> pa{};
+  if (pair) {
+    pre.step(1, a, c);
+    pa = PairArgs<double>{lv.box, cv.box, pair_tiles<double>(lv.box, kPairSlots), lv.H, lv.dinv64.ptr, nullptr, nullptr,
+                          (const double *)b, nullptr, cv.x64.ptr, lv.d64.ptr, lv.r64.ptr, nullptr, c1, a, c};
+    pair_sweep<double, PAIR_PRE>(pa, st);
+  } else if (mg->degree == 1) {
     sweep<T, SW_FIRST_RESID>(lv.box, H, dinv, b, nullptr, other, nullptr, cur, T(0), T(0), (T)c1, 0, st);
   } else {
     for (int k = 1; k < mg->degree; k++) {
@@ -1145,6 +1513,17 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
                      nullptr);
   vcycle<T>(mg, l + 1, P::b(cv), P::x(cv), st);
   ChebCoeffs post(mg, lv);
+  if (pair) {
+    post.step(0, a, c1);
+    post.step(1, a, c);
+    pa.x = lv.d64.ptr;
+    pa.out = (double *)x;
+    pa.c1 = c1;
+    pa.a = a;
+    pa.c = c;
+    pair_sweep<double, PAIR_POST>(pa, st);
+    return;
+  }
   for (int k = 0; k < mg->degree; k++) {
     post.step(k, a, c);
     const int keep_d = k + 1 < mg->degree;
@@ -1194,7 +1573,15 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
   double a, c, c1;
   ChebCoeffs pre(mg, lv);
   pre.step(0, a, c1);
-  if (mg->degree == 1) {
+  const bool pair = mg->degree == 2 && pair_level<float>(lv.box);
+  PairArgs<float> pa{};
+  if (pair) {
+    pre.step(1, a, c);
+    pa = PairArgs<float>{lv.box, cv.box, pair_tiles<float>(lv.box, kPairSlots), lv.H16.ptr, lv.e16.ptr, lv.f16.ptr,
+                         lv.sc16.ptr, b, nullptr, cv.x32.ptr, lv.d32.ptr, lv.r32.ptr, lv.t32.ptr, (float)c1, (float)a,
+                         (float)c, raw, 1};
+    pair_sweep<float, PAIR_PRE>(pa, st);
+  } else if (mg->degree == 1) {
     sweep16<SW_FIRST_RESID>(lv, b, nullptr, other, cur, 0, 0, c1, 0, raw, 0, st);
   } else {
     for (int k = 1; k < mg->degree; k++) {
@@ -1213,6 +1600,18 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
                      l + 2 < mg->L.size() ? cv.sc16.ptr : nullptr);
   vcycle16(mg, l + 1, cv.b32.ptr, cv.x32.ptr, st);
   ChebCoeffs post(mg, lv);
+  if (pair) {
+    post.step(0, a, c1);
+    post.step(1, a, c);
+    pa.b = bs;
+    pa.x = lv.d32.ptr;
+    pa.out = x;
+    pa.c1 = (float)c1;
+    pa.a = (float)a;
+    pa.c = (float)c;
+    pair_sweep<float, PAIR_POST>(pa, st);
+    return;
+  }
   for (int k = 0; k < mg->degree; k++) {
     post.step(k, a, c);
     const int last = k + 1 == mg->degree;
@@ -1325,6 +1724,14 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
     if (!err && l + 1 < mg->L.size()) err = lv.e16.alloc(n);
     if (!err && l + 1 < mg->L.size()) err = lv.f16.alloc(n);
     if (!err && l == 0 && mg->L.size() > 1) err = lv.t32.alloc(n);
+  }
+  if (!err && pair_level<double>(mg->L[0].box)) {
+    for (const void *k : {(const void *)pair_kernel<double, PAIR_POWER>, (const void *)pair_kernel<double, PAIR_PRE>,
+                          (const void *)pair_kernel<double, PAIR_POST>})
+      if (!err && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds<double>()) != hipSuccess) {
+        set_error("multigrid: the sweeps' LDS is not available");
+        err = dohpERR_HIP;
+      }
   }
   if (!err) err = mg_fill(mg, st);
   if (err) {

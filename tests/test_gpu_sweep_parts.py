@@ -36,15 +36,10 @@ def rounded(st):
     return out
 
 
-# Owned boxes (M p - 1 rows a side): lines along J 47 (one part), 49 and 51 (64 x 4 tiles split, the last part empty or
-# nearly), 113 and 119 lines (64 x 8 tiles split), the last two from 1024 tiles on.  What separates the two sides is FP32
-# rounding: about 30 roundings of 6e-8 per row and sweep, a dozen sweeps on each of up to five levels: 5e-5.
-@pytest.mark.parametrize("degree", [1, 2])
-@pytest.mark.parametrize("M", [(3, 12, 5), (2, 25, 9), (5, 26, 3), (48, 57, 34), (27, 60, 65)])
-def test_fp16_vcycle_on_the_rounded_operators(C, M, degree):  # noqa: F811
-    p = 4 if M[1] == 12 else 2
+def check(C, M, p, degree):  # noqa: F811
     print(f"FP16 V-cycle M={M} p={p} degree={degree}", flush=True)
     op, q1, mg, L = setup(C, M, p, 7, degree)
+    assert abs(mg.lmax - L[0][1]) <= 1e-12 * L[0][1]
     g = torch.Generator(device="cuda").manual_seed(5)
     r = (torch.rand(q1.nrows, dtype=torch.float64, device="cuda", generator=g) * 2 - 1).float()
     shape = L[0][0].shape[1:]
@@ -56,7 +51,26 @@ def test_fp16_vcycle_on_the_rounded_operators(C, M, degree):  # noqa: F811
     R = [(rounded(st) if l + 1 < len(L) else st, lmax) for l, (st, lmax) in enumerate(L)]
     ref = vcycle(R, 0, degree, r.double().reshape(shape)).reshape(-1)
     mg.set_coefficients(True)
-    mg.apply_f32(r, z)
+    for _ in range(3):  # eager, captured, replayed
+        z.fill_(float("nan"))
+        mg.apply_f32(r, z)
     err = z.double() - ref
     assert float(torch.linalg.norm(err)) <= 5e-5 * float(torch.linalg.norm(ref))
     assert float(err.abs().max()) <= 5e-5 * float(ref.abs().max())  # (no single row off, edges of the box included)
+
+
+# Owned boxes (M p - 1 rows a side): lines along J 47 (one part), 49 and 51 (64 x 4 tiles split, the last part empty or
+# nearly), 113 and 119 lines (64 x 8 tiles split), the last two from 1024 tiles on.  What separates the two sides is FP32
+# rounding: about 30 roundings of 6e-8 per row and sweep, a dozen sweeps on each of up to five levels: 5e-5.
+@pytest.mark.parametrize("degree", [1, 2])
+@pytest.mark.parametrize("M", [(3, 12, 5), (2, 25, 9), (5, 26, 3), (48, 57, 34), (27, 60, 65)])
+def test_fp16_vcycle_on_the_rounded_operators(C, M, degree):  # noqa: F811
+    check(C, M, 4 if M[1] == 12 else 2, degree)
+
+
+# Two sweeps in one pass (FP64 from 600 k rows, FP16 from 800 k, degree 2; power iterations): faces that end inside a
+# workgroup's, one workgroup's face larger than the box's, few planes, columns from 49 to 68 and 129 rows; 67 x 95 x 95 =
+# 604,675 rows takes FP64 pairs only.  Tolerances as above, lmax as the power iteration's in FP64.
+@pytest.mark.parametrize("M", [(8, 120, 120), (120, 8, 120), (120, 120, 8), (34, 48, 48), (25, 65, 65), (128, 65, 13)])
+def test_paired_sweeps(C, M):  # noqa: F811
+    check(C, M, 2, 2)
