@@ -643,7 +643,11 @@ __global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, Split sp,
 // 295 against 476.
 // PAIR_POWER: w = (D^-1 A)^2 (v / ||v||) and its sum of squares.  PAIR_PRE: the first two smoothing steps from zero and
 // their residual.  PAIR_POST: prolongation and the last two smoothing steps.
-enum { PAIR_POWER, PAIR_PRE, PAIR_POST };
+// PAIR_PRE1 and PAIR_POST1 march with one product, for one smoothing step: the first step from zero and its residual, or
+// prolongation and the step (FP16 only: the coefficients come in 7 aligned dwords per row instead of 20, 159^3 rows 70 ->
+// 58 and 76 -> 51 us; in FP64 the sweeps are at the rate of memory).
+enum { PAIR_POWER, PAIR_PRE, PAIR_POST, PAIR_PRE1, PAIR_POST1 };
+constexpr bool pair_two(int mode) { return mode <= PAIR_POST; }
 constexpr int kPairPad = 80;  // LDS entries around the face: border threads read past it, values that nothing uses
 constexpr int kPairSlots = 256;
 template <typename T>
@@ -661,23 +665,25 @@ struct PairTiles {
   int tk, tj, nk, nj, ni, chunk;  // columns and lines of a face, workgroups along K, J and I, planes of one
   int blocks() const { return nk * nj * ni; }
 };
-// Levels that take pairs.  Below, a face's border and the few planes of a chunk cost more than the second read of the
+// Levels that take them.  Below, a face's border and the few planes of a chunk cost more than the second read of the
 // coefficients, which then comes from the 256 MB cache: V-cycles of 79^3 rows take 153 us with pairs against 151 (FP64) and
-// 126 against 116 (FP16), of 89^3 159 against 211 and 126 against 122, of 99^3 134 against 148 (FP16).
+// 126 against 116 (FP16), of 89^3 159 against 211 and 126 against 122, of 99^3 132 against 148 (FP16).  One step a level
+// (FP16): 99^3 92 against 91 us, 119^3 96 against 100, 159^3 180 against 202.
 template <typename T>
-inline bool pair_level(const Box &b)
+inline bool pair_level(const Box &b, int degree)
 {
-  return b.n() >= (sizeof(T) == 8 ? 600000 : 800000);
+  return degree <= 2 && b.n() >= (sizeof(T) == 8 ? 600000 : degree == 2 ? 800000 : 1200000);
 }
 // Faces as wide as the box divides into at most 64 columns, and as many chunks along I as fill `slots` workgroups.
 template <typename T>
-PairTiles pair_tiles(const Box &b, int slots)
+PairTiles pair_tiles(const Box &b, int slots, bool two = true)
 {
   PairTiles g;
+  const int e = two ? 4 : 2;
   g.nk = (b.nz + pair_width<T>() - 1) / pair_width<T>();
-  g.tk = (b.nz + g.nk - 1) / g.nk + 4;
-  g.tj = std::min(pair_threads<T>() / g.tk, b.ny + 4);
-  g.nj = (b.ny + g.tj - 5) / (g.tj - 4);
+  g.tk = (b.nz + g.nk - 1) / g.nk + e;
+  g.tj = std::min(pair_threads<T>() / g.tk, b.ny + e);
+  g.nj = (b.ny + g.tj - e - 1) / (g.tj - e);
   const int ni = std::max(1, std::min(slots / (g.nk * g.nj), b.nx / 8));
   g.chunk = (b.nx + ni - 1) / ni;
   g.ni = (b.nx + g.chunk - 1) / g.chunk;
@@ -769,7 +775,9 @@ template <typename T, int MODE>
 __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *lds)
 {
   typedef PairCoeffs<T> C;
-  constexpr bool F16 = sizeof(T) == 4;
+  constexpr bool F16 = sizeof(T) == 4, TWO = pair_two(MODE);
+  constexpr bool PRE = MODE == PAIR_PRE || MODE == PAIR_PRE1, POST = MODE == PAIR_POST || MODE == PAIR_POST1;
+  constexpr int B = TWO ? 2 : 1;  // border of the face
   const PairTiles &g = A.g;
   const Box &bx = A.bx;
   typename C::E *Hs = (typename C::E *)lds + kPairPad;
@@ -777,9 +785,9 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
   const int t = threadIdx.x, tk = g.tk;
   const int kt = blk % g.nk, rest = blk / g.nk, jt = rest % g.nj, it = rest / g.nj;
   const int ia = it * g.chunk, ib = min(bx.nx, ia + g.chunk);
-  const int tj = (int)((t + 0.5f) * (1.f / tk)), J = jt * (g.tj - 4) - 2 + tj, K = kt * (tk - 4) - 2 + t - tj * tk;
+  const int tj = (int)((t + 0.5f) * (1.f / tk)), J = jt * (g.tj - 2 * B) - B + tj, K = kt * (tk - 2 * B) - B + t - tj * tk;
   const bool live = tj < g.tj && J >= 0 && J < bx.ny && K >= 0 && K < bx.nz;
-  const bool mine = live && tj >= 2 && tj < g.tj - 2 && t - tj * tk >= 2 && t - tj * tk < tk - 2;
+  const bool mine = live && tj >= B && tj < g.tj - B && t - tj * tk >= B && t - tj * tk < tk - B;
   const unsigned o = live ? (unsigned)J * bx.nz + K : 0u;
   const long n = bx.n(), sx = (long)bx.ny * bx.nz;
   // coarse plane's in-plane sum at (J, K): the first four terms of coarse_value
@@ -810,7 +818,7 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
     if constexpr (MODE == PAIR_POWER) {
       w.b = T(0);
       v = inv * at(A.x, row, o);
-    } else if constexpr (MODE == PAIR_PRE) {
+    } else if constexpr (PRE) {
       w.b = at(A.b, row, o);
       v = A.c1 * (F16 ? at(A.f, row, o) : w.d) * w.b;
       if (F16 && A.raw) w.b /= w.s;
@@ -823,11 +831,13 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
         have = hi;
       }
       const T pro = T(0.125) * ((lo == hi ? sum1 : sum0) + sum1);
-      v = F16 ? at(A.x, row, o) + w.s * pro : at(A.x, row, o) + pro;
+      // (after one step from zero the iterate is c1 b' / e again, neither stored nor read)
+      const T x = MODE == PAIR_POST1 ? A.c1 * w.b / w.d : at(A.x, row, o);
+      v = F16 ? x + w.s * pro : x + pro;
     }
     w.v = in ? v : T(0);
   };
-  const int i0 = max(ia - 2, 0), ilast = min(ib, bx.nx);  // (plane nx has no rows: its y1 is zero)
+  const int i0 = max(ia - B, 0), ilast = TWO ? ib : ib - 1;  // (plane nx has no rows: its y1 is zero)
   C h, hn;
   Row w0, w1, w2;
   load_row(i0, w0);
@@ -870,50 +880,62 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
       step = F16 ? cc * res / w0.d : cc * w0.d * res;
       if (MODE == PAIR_PRE) step = A.a * y0 + step;
       y1 = y0 + step;
-    }
-    if (!live || !inside_i) y1 = T(0);
-    Y[t] = y1;
-    if (MODE == PAIR_PRE && mine && i >= ia && i < ib) {
-      at(A.out, i * sx, o) = y1;
-      if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
-    }
-    __syncthreads();
-    // second sweep: plane i - 1 is complete with y1 on plane i
-    T z = q;
-    const T *Yt = Y + t;
-#pragma unroll
-    for (int s = 18; s < 27; s++) z += h.kept(Hs, s, t, i & 1) * Yt[((s / 3) % 3 - 1) * tk + s % 3 - 1];
-    if (mine && i > ia && i <= ib) {
-      const long row = (i - 1) * sx;
-      if constexpr (MODE == PAIR_POWER) {
-        const T y2 = pd * z;
-        at(A.out, row, o) = y2;
-        sum += (double)y2 * (double)y2;
-      } else if constexpr (MODE == PAIR_PRE) {
-        at(A.r, row, o) = F16 ? ps * (pb - z) : pb - z;
-      } else {
-        const T dn = A.a * pstep + (F16 ? A.c * (pb - z) / pd : A.c * pd * (pb - z));
-        at(A.out, row, o) = F16 && A.unscale ? (py + dn) / ps : py + dn;
+      if (!TWO && mine && i >= ia) {
+        if (PRE) {
+          at(A.r, i * sx, o) = F16 ? w0.s * res : res;
+          if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
+        } else {
+          at(A.out, i * sx, o) = F16 && A.unscale ? y1 / w0.s : y1;
+        }
       }
     }
-    q = (F16 ? w0.d : h.up(13)) * y1 + p2;
-    p2 = T(0);
-#pragma unroll
-    for (int s = 14; s < 27; s++) {
-      const int off = ((s / 3) % 3 - 1) * tk + s % 3 - 1;
-      const T lo = C::lo(Hs, s, t - off, i & 1) * Yt[-off];
-      if (s < 18) {
-        q += h.up(s) * Yt[off];
-        q += lo;
-      } else {
-        p2 += lo;
+    if constexpr (TWO) {
+      if (!live || !inside_i) y1 = T(0);
+      Y[t] = y1;
+      if (MODE == PAIR_PRE && mine && i >= ia && i < ib) {
+        at(A.out, i * sx, o) = y1;
+        if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
       }
+      __syncthreads();
+      // second sweep: plane i - 1 is complete with y1 on plane i
+      T z = q;
+      const T *Yt = Y + t;
+#pragma unroll
+      for (int s = 18; s < 27; s++) z += h.kept(Hs, s, t, i & 1) * Yt[((s / 3) % 3 - 1) * tk + s % 3 - 1];
+      if (mine && i > ia && i <= ib) {
+        const long row = (i - 1) * sx;
+        if constexpr (MODE == PAIR_POWER) {
+          const T y2 = pd * z;
+          at(A.out, row, o) = y2;
+          sum += (double)y2 * (double)y2;
+        } else if constexpr (MODE == PAIR_PRE) {
+          at(A.r, row, o) = F16 ? ps * (pb - z) : pb - z;
+        } else {
+          const T dn = A.a * pstep + (F16 ? A.c * (pb - z) / pd : A.c * pd * (pb - z));
+          at(A.out, row, o) = F16 && A.unscale ? (py + dn) / ps : py + dn;
+        }
+      }
+      q = (F16 ? w0.d : h.up(13)) * y1 + p2;
+      p2 = T(0);
+#pragma unroll
+      for (int s = 14; s < 27; s++) {
+        const int off = ((s / 3) % 3 - 1) * tk + s % 3 - 1;
+        const T lo = C::lo(Hs, s, t - off, i & 1) * Yt[-off];
+        if (s < 18) {
+          q += h.up(s) * Yt[off];
+          q += lo;
+        } else {
+          p2 += lo;
+        }
+      }
+      pb = w0.b;
+      pd = w0.d;
+      ps = w0.s;
+      py = y1;
+      pstep = step;
+    } else {
+      __syncthreads();
     }
-    pb = w0.b;
-    pd = w0.d;
-    ps = w0.s;
-    py = y1;
-    pstep = step;
     V[(i & 1) * pair_threads<T>() + t] = w2.v;
     h.keep();
 #pragma unroll
@@ -1342,7 +1364,7 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     l.first = blocks;
     blocks += (l.blocks + 7) / 8 * 8;
     parts += std::max(256, l.blocks);
-    if (pair_level<double>(lv.box)) nb = k + 1;  // (levels shrink: the first ones)
+    if (pair_level<double>(lv.box, 2)) nb = k + 1;  // (levels shrink: the first ones)
   }
   if (!mg->part.holds(parts)) DOHP_CALL(mg->part.alloc(parts));
   double *norm = mg->part.ptr, *inv = norm + kMaxLevels, *at = inv + kMaxLevels;
@@ -1487,7 +1509,7 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
   double a, c, c1;
   ChebCoeffs pre(mg, lv);
   pre.step(0, a, c1);
-  const bool pair = sizeof(T) == 8 && mg->degree == 2 && pair_level<double>(lv.box);
+  const bool pair = sizeof(T) == 8 && mg->degree == 2 && pair_level<double>(lv.box, 2);
   PairArgs<double> pa{};
   if (pair) {
     pre.step(1, a, c);
@@ -1573,14 +1595,17 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
   double a, c, c1;
   ChebCoeffs pre(mg, lv);
   pre.step(0, a, c1);
-  const bool pair = mg->degree == 2 && pair_level<float>(lv.box);
+  const bool two = mg->degree == 2, pair = pair_level<float>(lv.box, mg->degree);
   PairArgs<float> pa{};
   if (pair) {
-    pre.step(1, a, c);
-    pa = PairArgs<float>{lv.box, cv.box, pair_tiles<float>(lv.box, kPairSlots), lv.H16.ptr, lv.e16.ptr, lv.f16.ptr,
+    if (two) pre.step(1, a, c);
+    else a = c = 0;
+    other = lv.r32.ptr;
+    pa = PairArgs<float>{lv.box, cv.box, pair_tiles<float>(lv.box, kPairSlots, two), lv.H16.ptr, lv.e16.ptr, lv.f16.ptr,
                          lv.sc16.ptr, b, nullptr, cv.x32.ptr, lv.d32.ptr, lv.r32.ptr, lv.t32.ptr, (float)c1, (float)a,
                          (float)c, raw, 1};
-    pair_sweep<float, PAIR_PRE>(pa, st);
+    if (two) pair_sweep<float, PAIR_PRE>(pa, st);
+    else pair_sweep<float, PAIR_PRE1>(pa, st);
   } else if (mg->degree == 1) {
     sweep16<SW_FIRST_RESID>(lv, b, nullptr, other, cur, 0, 0, c1, 0, raw, 0, st);
   } else {
@@ -1602,14 +1627,15 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
   ChebCoeffs post(mg, lv);
   if (pair) {
     post.step(0, a, c1);
-    post.step(1, a, c);
+    if (two) post.step(1, a, c);
     pa.b = bs;
     pa.x = lv.d32.ptr;
     pa.out = x;
     pa.c1 = (float)c1;
     pa.a = (float)a;
     pa.c = (float)c;
-    pair_sweep<float, PAIR_POST>(pa, st);
+    if (two) pair_sweep<float, PAIR_POST>(pa, st);
+    else pair_sweep<float, PAIR_POST1>(pa, st);
     return;
   }
   for (int k = 0; k < mg->degree; k++) {
@@ -1725,7 +1751,7 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
     if (!err && l + 1 < mg->L.size()) err = lv.f16.alloc(n);
     if (!err && l == 0 && mg->L.size() > 1) err = lv.t32.alloc(n);
   }
-  if (!err && pair_level<double>(mg->L[0].box)) {
+  if (!err && pair_level<double>(mg->L[0].box, 2)) {
     for (const void *k : {(const void *)pair_kernel<double, PAIR_POWER>, (const void *)pair_kernel<double, PAIR_PRE>,
                           (const void *)pair_kernel<double, PAIR_POST>})
       if (!err && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds<double>()) != hipSuccess) {

@@ -68,9 +68,12 @@ def test_fp16_vcycle_on_the_rounded_operators(C, M, degree):  # noqa: F811
     check(C, M, 4 if M[1] == 12 else 2, degree)
 
 
-# Two sweeps in one pass (FP64 from 600 k rows, FP16 from 800 k, degree 2; power iterations): faces that end inside a
-# workgroup's, one workgroup's face larger than the box's, few planes, columns from 49 to 68 and 129 rows; 67 x 95 x 95 =
-# 604,675 rows takes FP64 pairs only.  Tolerances as above, lmax as the power iteration's in FP64.
-@pytest.mark.parametrize("M", [(8, 120, 120), (120, 8, 120), (120, 120, 8), (34, 48, 48), (25, 65, 65), (128, 65, 13)])
-def test_paired_sweeps(C, M):  # noqa: F811
-    check(C, M, 2, 2)
+# Two sweeps in one pass (FP64 from 600 k rows, FP16 from 800 k, degree 2; power iterations), or one FP16 sweep at degree 1
+# (from 1.2 M): faces that end inside a workgroup's, one workgroup's face larger than the box's, few planes, columns from
+# 49 to 68 and 129 rows; 67 x 95 x 95 = 604,675 rows takes FP64 pairs only.  Tolerances as above, lmax as the power
+# iteration's in FP64.
+@pytest.mark.parametrize("M,degree", [((8, 120, 120), 2), ((120, 8, 120), 2), ((120, 120, 8), 2), ((34, 48, 48), 2),
+                                      ((25, 65, 65), 2), ((128, 65, 13), 2), ((54, 54, 54), 1), ((8, 150, 150), 1),
+                                      ((150, 150, 8), 1)])
+def test_paired_sweeps(C, M, degree):  # noqa: F811
+    check(C, M, 2, degree)
