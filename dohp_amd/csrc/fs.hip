@@ -258,7 +258,8 @@ __global__ void __launch_bounds__(256) fs_gather_kernel(const int *__restrict__ 
                                                         const double *__restrict__ g, const double *__restrict__ dcache,
                                                         long nowned, int inhom, int add, double *__restrict__ x)
 {
-  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
+  // each XCD takes a run of elements, whose shared faces and partly used lines of g stay in its L2
+  const long blk = (long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), i = (blk * 256 + threadIdx.x) * 4;
   if (i >= nexp) return;
   const int m = (int)min(4L, nexp - i);
   int c[4];
@@ -305,8 +306,10 @@ __global__ void __launch_bounds__(256) fs_scatter_block_kernel(int p, int M0, in
                                                                int nx, int ny, int nz, const double *__restrict__ x,
                                                                int add, double *__restrict__ g)
 {
-  const int k = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y, i = blockIdx.z;
-  if (k >= nz || j >= ny) return;
+  // (each XCD takes a run of planes: the lines of x that hold an element's neighbouring rows and planes stay in its L2)
+  const int k = (blockIdx.x >> 3) * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  const int i = (int)(blockIdx.x & 7) * gridDim.z + blockIdx.z;
+  if (k >= nz || j >= ny || i >= nx) return;
   // (i and j are the same over a wavefront: its branches on them are uniform)
   const int n = p + 1, I[3] = {i + I0, __builtin_amdgcn_readfirstlane(j) + J0, k + K0}, M[3] = {M0, M1, M2};
   int e[3][2], a[3][2], m[3];  // per direction: the elements of the node and its index in them, even element first
@@ -365,7 +368,7 @@ extern "C" dErr dFSGlobalToExpanded(dohpFS fs, const double *g, double *x, int h
   DOHP_CHECK(hmode == dFS_HOMOGENEOUS || hmode == dFS_INHOMOGENEOUS, dohpERR_ARG, "invalid homogeneous mode");
   const long nexp = (long)fs->nelem * fs->n * fs->n * fs->n;
   const int bs = 256;
-  hipLaunchKernelGGL(fs_gather_kernel, dim3((unsigned)((nexp + 4 * bs - 1) / (4 * bs))), dim3(bs), 0, (hipStream_t)stream,
+  hipLaunchKernelGGL(fs_gather_kernel, dim3((unsigned)((nexp + 32 * bs - 1) / (32 * bs) * 8)), dim3(bs), 0, (hipStream_t)stream,
                      fs->d_elem_nodes.ptr, nexp, g, fs->d_dcache.ptr, fs->nowned, hmode == dFS_INHOMOGENEOUS,
                      imode == dADD_VALUES, x);
   DOHP_HIP(hipGetLastError());
@@ -383,7 +386,7 @@ extern "C" dErr dFSExpandedToGlobal(dohpFS fs, const double *x, double *g, int h
     const int w = fs->dirichlet_mask & 1, top = (fs->dirichlet_mask >> 1) & 1, bot = (fs->dirichlet_mask >> 2) & 1;
     const int nx = fs->p * fs->M[0] + 1 - 2 * w, ny = fs->p * fs->M[1] + 1 - 2 * w, nz = fs->p * fs->M[2] + 1 - top - bot;
     if (fs->nowned > 0)
-      hipLaunchKernelGGL(fs_scatter_block_kernel, dim3((nz + 63) / 64, (ny + 3) / 4, nx), dim3(64, 4), 0, st, fs->p,
+      hipLaunchKernelGGL(fs_scatter_block_kernel, dim3(8 * ((nz + 63) / 64), (ny + 3) / 4, (nx + 7) / 8), dim3(64, 4), 0, st, fs->p,
                          fs->M[0], fs->M[1], fs->M[2], w, w, bot, nx, ny, nz, x, imode == dADD_VALUES, g);
     DOHP_HIP(hipGetLastError());
     return 0;
