@@ -150,7 +150,7 @@ inline bool sweep_big(const Box &b)
 // the Galerkin product 3.7 times, and ran at the rate of that traffic.  A box's lines are therefore split into eight
 // parts along J, one per XCD (blockIdx.x & 7), each traversed x, y, z in order, so that a part's last plane is still in
 // its L2 (191^3: 36 k entries of 112 bytes a plane over eight caches of 4 MB).  At 239^3 the FP16 sweeps fetch 0.63 GB and
-// take 158 to 195 instead of 170 to 221 us, the Galerkin product 1.37 instead of 1.62 ms, the half stencils 1.10 instead
+// take 158 to 195 instead of 170 to 221 us, the Galerkin product (with a load a fine node) 1.37 instead of 1.62 ms, the half stencils 1.10 instead
 // of 1.44 ms; a power iteration at 191^3 231 instead of 244 us.  Boxes with fewer than two tiles of lines per part are not
 // split (47^3, all of it in every L2: no difference).
 struct Split {
@@ -1018,9 +1018,11 @@ __host__ __device__ constexpr double pweight(int e, int t)
 // and are summed into 3 x 3 partial sums in registers (every load unconditional: a support node outside the fine box
 // reads entry 0 with weight 0).  The partial sums meet the x weights through LDS, three of the 27 entries per wavefront.
 // With one thread per row the nine parts followed one another, 729 loads at 13 wavefronts per SIMD in all: latency
-// bound, 1.90 ms at 95^3 coarse rows and 0.11 ms at 5^3; this takes 0.71 and 0.01 ms.  Entries toward coarse nodes
-// outside the box are zero, as the assembly leaves them on the finest level.
-__global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const double *__restrict__ Af, double *__restrict__ Ac)
+// bound, 1.90 ms at 95^3 coarse rows and 0.11 ms at 5^3; this takes 0.46 and 0.01 ms (0.71 with a load for each of the
+// three fine nodes along k, whose lanes are two rows apart: two of them come in one).  Entries toward coarse nodes outside
+// the box are zero, as the assembly leaves them on the finest level.
+__global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const double *__restrict__ Af,
+                                                  double *__restrict__ Ac)
 {
   __shared__ double psum[9][9][64];  // [x part][3 x 3 sum][row]
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, a = w / 3 - 1, si = w % 3 - 1;
@@ -1036,28 +1038,42 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const 
   double T[9];
 #pragma unroll
   for (int u = 0; u < 9; u++) T[u] = 0.0;
+  const bool ini = fi < f.nx, ink = 2 * K + 2 < f.nz;
 #pragma unroll
-  for (int b = -1; b <= 1; b++)
+  for (int b = -1; b <= 1; b++) {
+    const int fj = 2 * J + 1 + b;
+    const bool in = ini && fj < f.ny;
+    const long fr = in ? fi * sx + fj * sy + 2 * K : 0;  // the fine node at d = -1 (inside along k, as that at d = 0)
+    double v[3][9];
+#pragma unroll
+    for (int s = 0; s < 9; s++) {
+      const double *p = Af + ((si + 1) * 9 + s) * nf + fr;
+      struct __attribute__((packed, aligned(8))) Two {
+        double lo, hi;
+      };
+      const Two q = *(const Two *)p;
+      v[0][s] = q.lo;
+      v[1][s] = q.hi;
+      v[2][s] = p[ink ? 2 : 0];
+    }
 #pragma unroll
     for (int d = -1; d <= 1; d++) {
-      const int fj = 2 * J + 1 + b, fk = 2 * K + 1 + d;
-      const bool in = fi < f.nx && fj < f.ny && fk < f.nz;
-      const long fr = in ? fi * sx + fj * sy + fk : 0;
-      const double w0 = in ? pweight(b, 0) * pweight(d, 0) : 0.0;
+      const double w0 = in && (d < 1 || ink) ? pweight(b, 0) * pweight(d, 0) : 0.0;
 #pragma unroll
       for (int sj = -1; sj <= 1; sj++)
 #pragma unroll
         for (int sk = -1; sk <= 1; sk++) {
-          const double v = w0 * Af[((si + 1) * 9 + (sj + 1) * 3 + (sk + 1)) * nf + fr];
+          const double vs = w0 * v[d + 1][(sj + 1) * 3 + sk + 1];
 #pragma unroll
           for (int tj = -1; tj <= 1; tj++)
 #pragma unroll
             for (int tk = -1; tk <= 1; tk++) {
               const double q = pweight(b + sj, tj) * pweight(d + sk, tk);
-              if (q != 0.0) T[(tj + 1) * 3 + (tk + 1)] = fma(v, q, T[(tj + 1) * 3 + (tk + 1)]);
+              if (q != 0.0) T[(tj + 1) * 3 + (tk + 1)] = fma(vs, q, T[(tj + 1) * 3 + (tk + 1)]);
             }
         }
     }
+  }
 #pragma unroll
   for (int u = 0; u < 9; u++) psum[w][u][lane] = T[u];
   __syncthreads();
@@ -1377,7 +1393,7 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
   // large levels take two iterations a pass, the others one by one beside them; the last iteration, whose growth is the
   // estimate, is a single one everywhere
   const int pairs = nb ? (its - 1) / 2 : 0;
-  PowerArgs gs = g, gb = g;  // the small levels alone; the large ones with their pairs' block counts
+  PowerArgs gs = g, gb = g;  // the small levels alone; all levels, the large ones with their pairs' block counts
   if (pairs) {
     gs.nl = nl - nb;
     unsigned first = 0;
@@ -1405,9 +1421,9 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     }
     for (int k = 0; k < 2 && gs.nl; k++) {
       hipLaunchKernelGGL(power_step_kernel, dim3(blocks_small), dim3(kPowerThreads), 0, st, gs, k, inv + nb);
-      hipLaunchKernelGGL(power_norm_kernel, dim3(gs.nl), dim3(1024), 0, st, gs, 0, norm + nb, inv + nb);
+      if (k == 0) hipLaunchKernelGGL(power_norm_kernel, dim3(gs.nl), dim3(1024), 0, st, gs, 0, norm + nb, inv + nb);
     }
-    hipLaunchKernelGGL(power_norm_kernel, dim3(nb), dim3(1024), 0, st, gb, 0, norm, inv);
+    hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, gb, 0, norm, inv);
   }
   if (pairs & 1)
     for (int k = 0; k < nb; k++) std::swap(g.l[k].v[0], g.l[k].v[1]);
