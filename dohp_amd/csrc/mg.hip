@@ -362,8 +362,8 @@ void residual(const Box &bx, const T *H, const T *b, const T *x, T *r, hipStream
 
 // Power iterations for the largest eigenvalue of D^-1 A, on all smoothed levels at once: an iteration is one launch
 // over the blocks of every level (the coarse ones ride along with the finest), w = D^-1 A (v / ||v||) with the scaling
-// applied in the staging and the sums of squares of w reduced per block, and one that sums each level's block sums in
-// order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3 rows and their coarse
+// applied in the staging and the sums of squares of w reduced per block; where a norm is wanted, one more sums each
+// level's block sums in order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3 rows and their coarse
 // levels, 15 iterations, 6.5 -> 3.5 ms (4.7 TB/s on the 17 values a row cannot do without).
 constexpr int kMaxLevels = 16, kPowerThreads = kBX * 8;
 struct PowerLevel {
@@ -638,14 +638,14 @@ __global__ void __launch_bounds__(kBX *BY) half16_sweep_kernel(Box bx, Split sp,
 //  - Faces: one workgroup per compute unit.  FP16 coefficients: 1024 threads, 64 columns wide (32: 252 instead of 221 us
 //    at 239^3).  FP64: 768 threads, whose 168 registers hold a plane ahead (1024 threads: 128, and 176 bytes spilled; 915
 //    us a pair of power iterations at 191^3 against 256), 48 columns (32: 269 us).
-// 239^3 rows, FP16: both pre-smoothing steps and the residual 221 us against 353 in two sweeps, both post-smoothing steps
+// 239^3 rows, FP16: both pre-smoothing steps and the residual 204 us against 353 in two sweeps, both post-smoothing steps
 // 235 against 370.  191^3, FP64: two power iterations 256 us against 462, pre-smoothing 264 against 392, post-smoothing
 // 295 against 476.
 // PAIR_POWER: w = (D^-1 A)^2 (v / ||v||) and its sum of squares.  PAIR_PRE: the first two smoothing steps from zero and
 // their residual.  PAIR_POST: prolongation and the last two smoothing steps.
 // PAIR_PRE1 and PAIR_POST1 march with one product, for one smoothing step: the first step from zero and its residual, or
 // prolongation and the step (FP16 only: the coefficients come in 7 aligned dwords per row instead of 20, 159^3 rows 70 ->
-// 58 and 76 -> 51 us; in FP64 the sweeps are at the rate of memory).
+// 50 and 76 -> 53 us; in FP64 the sweeps are at the rate of memory).
 enum { PAIR_POWER, PAIR_PRE, PAIR_POST, PAIR_PRE1, PAIR_POST1 };
 constexpr bool pair_two(int mode) { return mode <= PAIR_POST; }
 constexpr int kPairPad = 80;  // LDS entries around the face: border threads read past it, values that nothing uses
@@ -756,9 +756,9 @@ struct PairArgs {
   Box bx, cb;
   PairTiles g;
   const void *H;
-  const T *dinv, *f, *s;  // FP64: D^-1, null, null.  FP16: e, f, s of half16_sweep_kernel
+  const T *dinv, *s;      // FP64: D^-1, null.  FP16: e, s of half16_sweep_kernel
   const T *b, *x, *xc;
-  T *out, *r, *bs;
+  T *out, *r;
   T c1, a, c;             // first step's factor, the second one's
   int raw, unscale;
   const double *inv;
@@ -820,10 +820,11 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
       v = inv * at(A.x, row, o);
     } else if constexpr (PRE) {
       w.b = at(A.b, row, o);
-      v = A.c1 * (F16 ? at(A.f, row, o) : w.d) * w.b;
       if (F16 && A.raw) w.b /= w.s;
+      v = F16 ? A.c1 * w.b / w.d : A.c1 * w.d * w.b;
     } else {
       w.b = at(A.b, row, o);
+      if (F16 && A.raw) w.b /= w.s;
       const int hi = i >> 1, lo = hi - 1 + (i & 1);  // parents of plane i
       if (i >= 0 && have != hi) {
         sum0 = have == hi - 1 ? sum1 : plane_sum(hi - 1);
@@ -831,7 +832,7 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
         have = hi;
       }
       const T pro = T(0.125) * ((lo == hi ? sum1 : sum0) + sum1);
-      // (after one step from zero the iterate is c1 b' / e again, neither stored nor read)
+      // (after one step from zero the iterate is c1 b' / e again, neither stored nor read; on the finest level b' from b too)
       const T x = MODE == PAIR_POST1 ? A.c1 * w.b / w.d : at(A.x, row, o);
       v = F16 ? x + w.s * pro : x + pro;
     }
@@ -883,7 +884,6 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
       if (!TWO && mine && i >= ia) {
         if (PRE) {
           at(A.r, i * sx, o) = F16 ? w0.s * res : res;
-          if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
         } else {
           at(A.out, i * sx, o) = F16 && A.unscale ? y1 / w0.s : y1;
         }
@@ -892,10 +892,7 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
     if constexpr (TWO) {
       if (!live || !inside_i) y1 = T(0);
       Y[t] = y1;
-      if (MODE == PAIR_PRE && mine && i >= ia && i < ib) {
-        at(A.out, i * sx, o) = y1;
-        if (F16 && A.raw) at(A.bs, i * sx, o) = w0.b;
-      }
+      if (MODE == PAIR_PRE && mine && i >= ia && i < ib) at(A.out, i * sx, o) = y1;
       __syncthreads();
       // second sweep: plane i - 1 is complete with y1 on plane i
       T z = q;
@@ -979,29 +976,46 @@ __global__ void half_from_full_kernel(long n, const double *__restrict__ A, doub
   }
 }
 
-// bc = P^T rf, divided by the coarse level's row scales s (null: not)
+// Two neighbouring entries in one load.
 template <typename T>
-__global__ void restrict_kernel(Box f, Box c, const T *__restrict__ rf, T *__restrict__ bc, const T *__restrict__ s)
+struct __attribute__((packed, aligned(sizeof(T)))) Two {
+  T lo, hi;
+};
+
+// bc = P^T rf, divided by the coarse level's row scales s (null: not).  Split over the L2 caches as the sweeps are, and two
+// of the three fine rows along k in one load: 119^3 coarse rows in FP32 33 -> 26 us, 79^3 15 -> 11.6.
+template <typename T>
+__global__ void restrict_kernel(Box f, Box c, Split sp, const T *__restrict__ rf, T *__restrict__ bc,
+                                const T *__restrict__ s)
 {
-  int I, J, K;
-  long C;
-  if (!box_index(c, I, J, K, C)) return;
+  const int I = blockIdx.z, J = sp.j0(blockIdx.x, blockIdx.y, kBY) + threadIdx.y, K = sp.k0(blockIdx.x) + threadIdx.x;
+  if (J >= sp.j1(blockIdx.x, c.ny) || K >= c.nz) return;
+  const long C = ((long)I * c.ny + J) * c.nz + K;
   const long sy = f.nz, sx = (long)f.ny * f.nz;
   const int F0 = 2 * I + 1, F1 = 2 * J + 1, F2 = 2 * K + 1;
   const long base = F0 * sx + F1 * sy + F2;  // (F0, F1, F2) is inside the fine box; its upper neighbours may not be
+  const bool ink = F2 + 1 < f.nz;
   T acc = 0;
 #pragma unroll
   for (int a = -1; a <= 1; a++)
 #pragma unroll
-    for (int b = -1; b <= 1; b++)
-#pragma unroll
-      for (int d = -1; d <= 1; d++) {
-        const bool in = F0 + a < f.nx && F1 + b < f.ny && F2 + d < f.nz;
-        const T w = T((a ? 0.5 : 1.0) * (b ? 0.5 : 1.0) * (d ? 0.5 : 1.0));
-        const T v = w * rf[in ? base + a * sx + b * sy + d : base];  // unconditional load, dropped by a select
-        acc += in ? v : T(0);
-      }
+    for (int b = -1; b <= 1; b++) {
+      const bool in = F0 + a < f.nx && F1 + b < f.ny;
+      const T w = T((a ? 0.5 : 1.0) * (b ? 0.5 : 1.0));
+      const T *p = rf + (in ? base + a * sx + b * sy : base);  // unconditional loads, dropped by a select
+      const Two<T> q = *(const Two<T> *)(p - 1);
+      const T v = p[ink ? 1 : 0];
+      acc += in ? T(0.5) * w * q.lo : T(0);
+      acc += in ? w * q.hi : T(0);
+      acc += in && ink ? T(0.5) * w * v : T(0);
+    }
   bc[C] = s ? acc / s[C] : acc;
+}
+template <typename T>
+void restrict_to(const Box &f, const Box &c, const T *rf, T *bc, const T *s, hipStream_t st)
+{
+  const Split sp = split_of(c, kBY);
+  hipLaunchKernelGGL(restrict_kernel<T>, split_grid(c, sp, kBY, 1), box_block(), 0, st, f, c, sp, rf, bc, s);
 }
 
 // 1-D prolongation weight of the coarse node at offset t (in -1..1) from coarse node c at the fine node at offset e
@@ -1048,10 +1062,7 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const 
 #pragma unroll
     for (int s = 0; s < 9; s++) {
       const double *p = Af + ((si + 1) * 9 + s) * nf + fr;
-      struct __attribute__((packed, aligned(8))) Two {
-        double lo, hi;
-      };
-      const Two q = *(const Two *)p;
+      const Two<double> q = *(const Two<double> *)p;
       v[0][s] = q.lo;
       v[1][s] = q.hi;
       v[2][s] = p[ink ? 2 : 0];
@@ -1390,8 +1401,10 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
   }
   hipLaunchKernelGGL(power_start_kernel, dim3(256, nl), dim3(256), 0, st, g);
   hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 1, norm, inv);
-  // large levels take two iterations a pass, the others one by one beside them; the last iteration, whose growth is the
-  // estimate, is a single one everywhere
+  // The vectors are normalised before the last iteration; until then every iteration scales by the start's 1 / ||v||, which
+  // leaves them between 1e-66 and 1e22 times the start after fifteen (a norm a launch: 5 us an iteration, 60 of the 560 us
+  // of a Newton step at 25 k rows).  Large levels take two iterations a pass, the others one by one beside them; the last
+  // iteration, whose growth is the estimate, is a single one everywhere.
   const int pairs = nb ? (its - 1) / 2 : 0;
   PowerArgs gs = g, gb = g;  // the small levels alone; all levels, the large ones with their pairs' block counts
   if (pairs) {
@@ -1419,17 +1432,16 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
       l.blocks = pa.g.blocks();
       pair_sweep<double, PAIR_POWER>(pa, st);
     }
-    for (int k = 0; k < 2 && gs.nl; k++) {
+    for (int k = 0; k < 2 && gs.nl; k++)
       hipLaunchKernelGGL(power_step_kernel, dim3(blocks_small), dim3(kPowerThreads), 0, st, gs, k, inv + nb);
-      if (k == 0) hipLaunchKernelGGL(power_norm_kernel, dim3(gs.nl), dim3(1024), 0, st, gs, 0, norm + nb, inv + nb);
-    }
-    hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, gb, 0, norm, inv);
   }
+  const int singles = its - 2 * pairs;
+  if (pairs && singles == 1) hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, gb, 0, norm, inv);
   if (pairs & 1)
     for (int k = 0; k < nb; k++) std::swap(g.l[k].v[0], g.l[k].v[1]);
-  for (int k = 0; k < its - 2 * pairs; k++) {
+  for (int k = 0; k < singles; k++) {
     hipLaunchKernelGGL(power_step_kernel, dim3(blocks), dim3(kPowerThreads), 0, st, g, k & 1, inv);
-    hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 0, norm, inv);
+    if (k >= singles - 2) hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 0, norm, inv);
   }
   DOHP_HIP(hipGetLastError());
   return 0;
@@ -1529,8 +1541,8 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
   PairArgs<double> pa{};
   if (pair) {
     pre.step(1, a, c);
-    pa = PairArgs<double>{lv.box, cv.box, pair_tiles<double>(lv.box, kPairSlots), lv.H, lv.dinv64.ptr, nullptr, nullptr,
-                          (const double *)b, nullptr, cv.x64.ptr, lv.d64.ptr, lv.r64.ptr, nullptr, c1, a, c};
+    pa = PairArgs<double>{lv.box, cv.box, pair_tiles<double>(lv.box, kPairSlots), lv.H, lv.dinv64.ptr, nullptr,
+                          (const double *)b, nullptr, cv.x64.ptr, lv.d64.ptr, lv.r64.ptr, c1, a, c};
     pair_sweep<double, PAIR_PRE>(pa, st);
   } else if (mg->degree == 1) {
     sweep<T, SW_FIRST_RESID>(lv.box, H, dinv, b, nullptr, other, nullptr, cur, T(0), T(0), (T)c1, 0, st);
@@ -1547,8 +1559,7 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
     }
     residual<T>(lv.box, H, b, cur, other, st);
   }
-  hipLaunchKernelGGL(restrict_kernel<T>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, P::b(cv),
-                     nullptr);
+  restrict_to<T>(lv.box, cv.box, other, P::b(cv), nullptr, st);
   vcycle<T>(mg, l + 1, P::b(cv), P::x(cv), st);
   ChebCoeffs post(mg, lv);
   if (pair) {
@@ -1617,9 +1628,9 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
     if (two) pre.step(1, a, c);
     else a = c = 0;
     other = lv.r32.ptr;
-    pa = PairArgs<float>{lv.box, cv.box, pair_tiles<float>(lv.box, kPairSlots, two), lv.H16.ptr, lv.e16.ptr, lv.f16.ptr,
-                         lv.sc16.ptr, b, nullptr, cv.x32.ptr, lv.d32.ptr, lv.r32.ptr, lv.t32.ptr, (float)c1, (float)a,
-                         (float)c, raw, 1};
+    pa = PairArgs<float>{lv.box, cv.box, pair_tiles<float>(lv.box, kPairSlots, two), lv.H16.ptr, lv.e16.ptr,
+                         lv.sc16.ptr, b, nullptr, cv.x32.ptr, lv.d32.ptr, lv.r32.ptr, (float)c1, (float)a, (float)c,
+                         raw, 1};
     if (two) pair_sweep<float, PAIR_PRE>(pa, st);
     else pair_sweep<float, PAIR_PRE1>(pa, st);
   } else if (mg->degree == 1) {
@@ -1637,14 +1648,12 @@ void vcycle16(_p_dohpMG *mg, size_t l, const float *b, float *x, hipStream_t st)
     }
     sweep16<SW_RESID>(lv, bs, cur, other, nullptr, 0, 0, 0, 0, 0, 0, st);
   }
-  hipLaunchKernelGGL(restrict_kernel<float>, box_grid(cv.box), box_block(), 0, st, lv.box, cv.box, other, cv.b32.ptr,
-                     l + 2 < mg->L.size() ? cv.sc16.ptr : nullptr);
+  restrict_to<float>(lv.box, cv.box, other, cv.b32.ptr, l + 2 < mg->L.size() ? cv.sc16.ptr : nullptr, st);
   vcycle16(mg, l + 1, cv.b32.ptr, cv.x32.ptr, st);
   ChebCoeffs post(mg, lv);
   if (pair) {
     post.step(0, a, c1);
     if (two) post.step(1, a, c);
-    pa.b = bs;
     pa.x = lv.d32.ptr;
     pa.out = x;
     pa.c1 = (float)c1;
