@@ -1105,8 +1105,8 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const 
 // Explicit inverse of the (symmetric positive definite) coarsest matrix, in place, by Gauss-Jordan elimination on
 // 32 x 32 blocks without pivoting.  A step k takes two launches: the panel kernel inverts the diagonal block (every
 // workgroup for itself, in LDS), forms its part of R = D A_k: and copies its part of the block column A_:k; the update
-// kernel writes A_ij -= A_ik R_j, R in block row k, -A_ik D in block column k and D itself: 31 us a
-// step.  A hierarchy's whole set-up at 47 x 47 x 47 rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343
+// kernel writes A_ij -= A_ik R_j, R in block row k, -A_ik D in block column k and D itself: 30 -> 18 us a step at 504
+// rows since a pivot pair waits at one barrier and no load waits for another.  A hierarchy's whole set-up at 47 x 47 x 47 rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343
 // 13.4 -> 0.72 ms, at 65^3 over 512 46 -> 0.94 ms: scalar host code between two copies did the elimination before.
 constexpr int kCB = 32;
 __global__ void dense_fill_kernel(Box b, const double *__restrict__ st, double *__restrict__ A)
@@ -1126,41 +1126,68 @@ __global__ void __launch_bounds__(256) dense_panel_kernel(int n, int k0, const d
                                                           double *__restrict__ R, double *__restrict__ Cc,
                                                           double *__restrict__ D, double *__restrict__ bad)
 {
-  __shared__ double d[kCB][kCB + 1];
+  // the pivots read one copy of the block and write the other (a thread keeps its own entries in registers), and the block row's part that R needs is loaded ahead of the pivots
+  __shared__ double d[2][kCB][kCB + 1], ak[kCB][kCB + 1];
   const int t = threadIdx.x, m = min(kCB, n - k0);
-  for (int q = t; q < kCB * kCB; q += 256) {
-    const int r = q / kCB, c = q % kCB;
-    d[r][c] = r < m && c < m ? A[(long)(k0 + r) * n + k0 + c] : r == c ? 1.0 : 0.0;
-  }
-  __syncthreads();
   const int c = t % kCB, r0 = t / kCB;  // this thread's column and rows r0, r0 + 8, ...
-  for (int p = 0; p < m; p++) {
-    const double piv = d[p][p];
-    if (t == 0 && blockIdx.x == 0 && !(piv > 0.0)) *bad = 1.0;
-    const double ip = 1.0 / piv, rowc = (c == p ? 1.0 : d[p][c]) * ip;
-    double colr[4];
+  const int j0 = blockIdx.x * kCB, j = j0 + c;  // columns (of R) and rows (of the copied panel) of this workgroup
+  // (every load unconditional, here and below: behind branches a thread's loads follow one another, 17 instead of 12 us)
+  double v[4], w[4];
 #pragma unroll
-    for (int u = 0; u < 4; u++) colr[u] = d[r0 + 8 * u][p];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = r0 + 8 * u;
-      d[r][c] = r == p ? rowc : (c == p ? 0.0 : d[r][c]) - colr[u] * rowc;
-    }
-    __syncthreads();
+  for (int u = 0; u < 4; u++) {
+    const long row = (long)min(k0 + r0 + 8 * u, n - 1) * n;
+    v[u] = A[row + min(k0 + c, n - 1)];
+    w[u] = A[row + min(j, n - 1)];
   }
-  if (blockIdx.x == 0)
-    for (int q = t; q < kCB * kCB; q += 256) D[q] = d[q / kCB][q % kCB];
-  // columns (of R) and rows (of the copied panel) j0 .. j0 + 31 of this workgroup
-  const int j0 = blockIdx.x * kCB, j = j0 + c;
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int r = r0 + 8 * u;
-    if (j < n && r < m) {
-      double s = 0.0;
-      for (int q = 0; q < m; q++) s += d[r][q] * A[(long)(k0 + q) * n + j];
-      R[(long)r * n + j] = s;
+    v[u] = r < m && c < m ? v[u] : r == c ? 1.0 : 0.0;
+    ak[r][c] = r < m && j < n ? w[u] : 0.0;
+    d[0][r][c] = v[u];
+  }
+  __syncthreads();
+  // (two pivots a barrier: the second one's row and column after the first come from the same copy; past m the block is
+  // the identity, on which a pivot changes nothing)
+  for (int p = 0; p < m; p += 2) {
+    const double(&s)[kCB][kCB + 1] = d[(p >> 1) & 1];
+    const double a0 = s[p][p], a0q = s[p][p + 1], b1 = s[p + 1][p], b1q = s[p + 1][p + 1], s0 = s[p][c], s1 = s[p + 1][c];
+    double cp[4], cq[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      cp[u] = s[r0 + 8 * u][p];
+      cq[u] = s[r0 + 8 * u][p + 1];
     }
+    const double i0 = 1.0 / a0, row0 = (c == p ? 1.0 : s0) * i0, row0q = a0q * i0;
+    const double x1 = (c == p ? 0.0 : s1) - b1 * row0, a1 = b1q - b1 * row0q;
+    const double row1 = (c == p + 1 ? 1.0 : x1) * (1.0 / a1);
+    if (t == 0 && blockIdx.x == 0 && !(a0 > 0.0 && a1 > 0.0)) *bad = 1.0;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int r = r0 + 8 * u;
+      const double e0 = (c == p ? 0.0 : v[u]) - cp[u] * row0, e = r == p ? row0 : e0;
+      const double q0 = cq[u] - cp[u] * row0q, q = r == p ? row0q : q0;
+      const double x = (c == p + 1 ? 0.0 : e) - q * row1;
+      v[u] = r == p + 1 ? row1 : x;
+      d[1 - ((p >> 1) & 1)][r][c] = v[u];
+    }
+    __syncthreads();
+  }
+  const double(&f)[kCB][kCB + 1] = d[((m + 1) >> 1) & 1];
+  if (blockIdx.x == 0)
+#pragma unroll
+    for (int u = 0; u < 4; u++) D[(r0 + 8 * u) * kCB + c] = v[u];
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+  for (int q = 0; q < kCB; q++) {  // (past m the rows of ak are zero)
+    const double a = ak[q][c];
+#pragma unroll
+    for (int u = 0; u < 4; u++) sum[u] += f[r0 + 8 * u][q] * a;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + 8 * u;
+    if (j < n && r < m) R[(long)r * n + j] = sum[u];
     if (j0 + r < n && c < m) Cc[(long)(j0 + r) * kCB + c] = A[(long)(j0 + r) * n + k0 + c];
   }
 }
@@ -1173,22 +1200,34 @@ __global__ void __launch_bounds__(256) dense_update_kernel(int n, int k0, double
   __shared__ double cs[kCB][kCB + 1], rs[kCB][kCB + 1];
   const int t = threadIdx.x, m = min(kCB, n - k0), i0 = blockIdx.y * kCB, j0 = blockIdx.x * kCB, c = t % kCB, r0 = t / kCB;
   const bool row = i0 == k0, col = j0 == k0;
+  double vc[4], vr[4], va[4];  // (unconditional loads, as in the panel kernel)
+  const int j = min(j0 + c, n - 1);
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = r0 + 8 * u, i = min(i0 + r, n - 1);
+    vc[u] = Cc[(long)i * kCB + c];
+    vr[u] = col ? D[r * kCB + c] : R[(long)min(r, m - 1) * n + j];
+    va[u] = A[(long)i * n + j];
+  }
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int r = r0 + 8 * u;
-    cs[r][c] = i0 + r < n && c < m ? Cc[(long)(i0 + r) * kCB + c] : 0.0;
-    rs[r][c] = r < m && j0 + c < n ? (col ? D[r * kCB + c] : R[(long)r * n + j0 + c]) : 0.0;
+    cs[r][c] = i0 + r < n && c < m ? vc[u] : 0.0;
+    rs[r][c] = r < m && j0 + c < n ? vr[u] : 0.0;
   }
   __syncthreads();
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+  for (int q = 0; q < kCB; q++) {  // (past m both are zero)
+    const double x = rs[q][c];
+#pragma unroll
+    for (int u = 0; u < 4; u++) sum[u] += cs[r0 + 8 * u][q] * x;
+  }
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int r = r0 + 8 * u;
-    if (i0 + r >= n || j0 + c >= n) continue;
-    double *a = &A[(long)(i0 + r) * n + j0 + c];
-    double s = 0.0;
-    if (!row)
-      for (int q = 0; q < m; q++) s += cs[r][q] * rs[q][c];
-    *a = row ? rs[r][c] : (col ? 0.0 : *a) - s;
+    if (i0 + r < n && j0 + c < n)
+      A[(long)(i0 + r) * n + j0 + c] = row ? rs[r][c] : (col ? 0.0 : va[u]) - sum[u];
   }
 }
 
