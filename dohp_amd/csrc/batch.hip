@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "common.h"
+#define DOHP_PITCH_N4 4
 #include "element.h"
 
 using namespace dohp;

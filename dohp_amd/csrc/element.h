@@ -213,9 +213,12 @@ enum { DIR_X = 0, DIR_Y = 1, DIR_Z = 2 };
 // At n = 4 a line of the tile is followed by an unused slot: at a pitch of 4 the 16 lanes of an element start on a
 // quarter of the banks in the z phase (conflicts a third of the compute units' cycles; A x at degree 3, 250 k elements
 // 185 -> 177 us, the residual 255 -> 250).  At the other even orders the larger tiles cost more than the conflicts (n = 6:
-// A x 154 -> 187 us; the batched mixed orders 393 -> 485).  Point t (i n^2 + j n + k, over all elements of the workgroup)
-// is at tile_slot(t).
-constexpr int line_pitch(int N) { return N == 4 ? 5 : N; }
+// A x 154 -> 187 us; the batched mixed orders 393 -> 485).  The batch keeps n = 4 at 4 as well (0.5 % faster).  Point t
+// (i n^2 + j n + k, over all elements of the workgroup) is at tile_slot(t).
+#ifndef DOHP_PITCH_N4
+#define DOHP_PITCH_N4 5
+#endif
+constexpr int line_pitch(int N) { return N == 4 ? DOHP_PITCH_N4 : N; }
 constexpr int tile_len(int N) { return N * N * line_pitch(N); }
 template <int N>
 __device__ __forceinline__ int tile_slot(int t)
