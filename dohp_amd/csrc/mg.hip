@@ -150,9 +150,9 @@ inline bool sweep_big(const Box &b)
 // the Galerkin product 3.7 times, and ran at the rate of that traffic.  A box's lines are therefore split into eight
 // parts along J, one per XCD (blockIdx.x & 7), each traversed x, y, z in order, so that a part's last plane is still in
 // its L2 (191^3: 36 k entries of 112 bytes a plane over eight caches of 4 MB).  At 239^3 the FP16 sweeps fetch 0.63 GB and
-// take 158 to 195 instead of 170 to 221 us, the Galerkin product (with a load a fine node) 1.37 instead of 1.62 ms, the half stencils 1.10 instead
-// of 1.44 ms; a power iteration at 191^3 231 instead of 244 us.  Boxes with fewer than two tiles of lines per part are not
-// split (47^3, all of it in every L2: no difference).
+// take 158 to 195 instead of 170 to 221 us, the Galerkin product (with a load a fine node) 1.37 instead of 1.62 ms, the
+// half stencils 1.10 instead of 1.44 ms; a power iteration at 191^3 231 instead of 244 us.  Boxes with fewer than two
+// tiles of lines per part are not split (47^3, all of it in every L2: no difference).
 struct Split {
   int lg, lines;  // log2 of the number of parts, lines of a part
   __device__ __forceinline__ int j0(unsigned bx, unsigned by, int BY) const
@@ -309,7 +309,8 @@ __global__ void __launch_bounds__(kBX *BY, 4) half_sweep_kernel(Box bx, Split sp
   const int J1 = sp.j1(blockIdx.x, bx.ny);
   if (J0 >= J1) return;
   if constexpr (PRO) stage_coarse<BY, NR>(cb, xc, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, ct);
-  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, unsigned i, int gi, int gj, int gk) {
+  stage_tile<BY, NR>(bx, I0, J0, K0, threadIdx.y * kBX + threadIdx.x, tile,
+                     [&](long g, unsigned i, int gi, int gj, int gk) {
     if constexpr (FIRST) return c1 * at(dinv, g, i) * at(b, g, i);
     else if constexpr (PRO) return at(x, g, i) + coarse_value<BY, NR>(ct, I0, J0, K0, gi, gj, gk);
     else return at(x, g, i);
@@ -363,8 +364,9 @@ void residual(const Box &bx, const T *H, const T *b, const T *x, T *r, hipStream
 // Power iterations for the largest eigenvalue of D^-1 A, on all smoothed levels at once: an iteration is one launch
 // over the blocks of every level (the coarse ones ride along with the finest), w = D^-1 A (v / ||v||) with the scaling
 // applied in the staging and the sums of squares of w reduced per block; where a norm is wanted, one more sums each
-// level's block sums in order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3 rows and their coarse
-// levels, 15 iterations, 6.5 -> 3.5 ms (4.7 TB/s on the 17 values a row cannot do without).
+// level's block sums in order.  Against a residual, a scaling, a sum and a normalisation per level and iteration: 191^3
+// rows and their coarse levels, 15 iterations, 6.5 -> 3.5 ms (4.7 TB/s on the 17 values a row cannot do without); 2.3 ms
+// with the largest levels in pairs (pair_kernel).
 constexpr int kMaxLevels = 16, kPowerThreads = kBX * 8;
 struct PowerLevel {
   Box bx;
