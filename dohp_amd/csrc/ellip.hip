@@ -365,16 +365,21 @@ __global__ void zero_kernel(T *__restrict__ y, long n)
 }
 
 // Linearization state in lattice order (closure order for a space from element maps, lat2clo = null): owned
-// values from u, Dirichlet values from the cache.  If f is not null it also gets its first value on every owned node:
-// the forcing term, or zero.
+// values from u, Dirichlet values from the cache.  The FP32 copy is written here, by every residual, and not by the first
+// application that reads it: applications only read the state, so a replayed graph of one, a replayed residual and
+// applications on several streams all see the last state.  If f is not null it also gets its first value on every owned
+// node: the forcing term, or zero.
 __global__ void lattice_state_kernel(const double *__restrict__ u, const double *__restrict__ dcache,
                                      const int *__restrict__ lat2clo, long nowned, long nlat, double *__restrict__ st,
-                                     const double *__restrict__ forcing, double *__restrict__ f)
+                                     float *__restrict__ st32, const double *__restrict__ forcing,
+                                     double *__restrict__ f)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nlat) return;
   const long c = lat2clo ? lat2clo[i] : i;
-  st[i] = c < nowned ? u[c] : dcache[c - nowned];
+  const double v = c < nowned ? u[c] : dcache[c - nowned];
+  st[i] = v;
+  st32[i] = (float)v;
   if (f && c < nowned) f[c] = forcing ? forcing[c] : 0.0;
 }
 
@@ -403,7 +408,6 @@ struct _p_dohpEllip {
   DevBuf<double> forcing;                     // assembled forcing term -(f, phi) on the owned nodes
   bool has_forcing = false;
   DevBuf<float> state32, tab32;
-  bool state32_ok = false;  // state32 is the rounded state (formed by the first FP32 application that reads it)
   // Set by the element kernels when a scattered contribution is not finite (a NaN or Inf in the input vector or the
   // state).  The checked entry points clear a flag in pinned host memory, launch with it, wait for their stream and read
   // it: no clearing kernel and no copy.  Unchecked launches set a flag on the device that nobody reads, so that one still
@@ -850,10 +854,9 @@ dErr set_state(_p_dohpEllip *op, const double *u, double *f, hipStream_t st)
 {
   const dohpFS fs = op->fs;
   hipLaunchKernelGGL(lattice_state_kernel, dim3((fs->nclosure + 255) / 256), dim3(256), 0, st, u, fs->d_dcache.ptr,
-                     fs->d_lat2clo.ptr, fs->nowned, fs->nclosure, op->state.ptr, op->has_forcing ? op->forcing.ptr : nullptr,
-                     f);
+                     fs->d_lat2clo.ptr, fs->nowned, fs->nclosure, op->state.ptr, op->state32.ptr,
+                     op->has_forcing ? op->forcing.ptr : nullptr, f);
   op->has_state = true;
-  op->state32_ok = false;
   drop_qd(op);
   DOHP_HIP(hipGetLastError());
   return 0;
@@ -936,26 +939,10 @@ struct Prec<float> {
   static const float *state(const _p_dohpEllip *op) { return op->state32.ptr; }
 };
 
-// The FP32 state, rounded once per linearization (in a captured graph: by every replay, and by the next eager
-// application, since the capture itself runs nothing).
-dErr ensure_state32(_p_dohpEllip *op, hipStream_t st)
-{
-  if (op->state32_ok) return 0;
-  const long n = op->fs->nclosure;
-  hipLaunchKernelGGL(round_f32_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, op->state.ptr,
-                     op->state32.ptr, n);
-  DOHP_HIP(hipGetLastError());
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  DOHP_HIP(hipStreamIsCapturing(st, &cap));
-  op->state32_ok = cap == hipStreamCaptureStatusNone;
-  return 0;
-}
-
 template <typename T>
 dErr apply_recomputed(_p_dohpEllip *op, const T *x, T *y, hipStream_t st)
 {
   if (is_linear(op)) return launch<T, MODE_LIN>(op, nullptr, x, y, st);
-  if (sizeof(T) == 4) DOHP_CALL(ensure_state32(op, st));
   return launch<T, MODE_JAC>(op, Prec<T>::state(op), x, y, st);
 }
 
