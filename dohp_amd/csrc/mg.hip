@@ -1111,6 +1111,7 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const 
 // rows since a pivot pair waits at one barrier and no load waits for another.  A hierarchy's whole set-up at 47 x 47 x 47 rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343
 // 13.4 -> 0.72 ms, at 65^3 over 512 46 -> 0.94 ms: scalar host code between two copies did the elimination before.
 constexpr int kCB = 32;
+constexpr long kMaxCoarse = 4096;
 __global__ void dense_fill_kernel(Box b, const double *__restrict__ st, double *__restrict__ A)
 {
   const long n = b.n(), t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1402,6 +1403,17 @@ struct _p_dohpMG {
 
 namespace {
 
+// The sweep's grid of a level in a power iteration, and the block sums that the level's launches write: 256 of the start
+// vector, one per workgroup of a sweep, or one per workgroup of a pair.  Neither of the last two bounds the other: on a
+// box of two planes the faces of a pair can be more (2 x 800 x 800 rows: 1360 workgroups against 1352).
+dim3 power_grid(const Box &b) { return split_grid(b, split_of(b, 8), 8, sweep_big(b) ? 2 : 1); }
+long power_sums(const Box &b)
+{
+  const dim3 g = power_grid(b);
+  const long single = (long)g.x * g.y * g.z, pair = pair_level<double>(b, 2) ? pair_tiles<double>(b, kPairSlots).blocks() : 0;
+  return std::max({256L, single, pair});
+}
+
 // lmax of D^-1 A on every smoothed level by power iteration, in the levels' work vectors (free outside a V-cycle).  The
 // iterations stay on the device and leave the last norms at the start of mg->part.
 dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
@@ -1415,6 +1427,7 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
   int nb = 0;
   unsigned blocks_small = 0;
   size_t parts = 2 * kMaxLevels;  // norms and their inverses, then the levels' block sums
+  long sums[kMaxLevels];
   for (int k = 0; k < nl; k++) {
     MGLevel &lv = mg->L[k];
     PowerLevel &l = g.l[k];
@@ -1425,20 +1438,20 @@ dErr estimate_lmax(_p_dohpMG *mg, hipStream_t st, int its)
     l.v[1] = lv.d64.ptr;
     l.big = sweep_big(lv.box);
     l.sp = split_of(lv.box, 8);
-    const dim3 grid = split_grid(lv.box, l.sp, 8, l.big ? 2 : 1);
+    const dim3 grid = power_grid(lv.box);
     l.gx = grid.x;
     l.gy = grid.y;
     l.blocks = (int)(grid.x * grid.y * grid.z);
     l.first = blocks;
     blocks += (l.blocks + 7) / 8 * 8;
-    parts += std::max(256, l.blocks);
+    parts += sums[k] = power_sums(lv.box);
     if (pair_level<double>(lv.box, 2)) nb = k + 1;  // (levels shrink: the first ones)
   }
   if (!mg->part.holds(parts)) DOHP_CALL(mg->part.alloc(parts));
   double *norm = mg->part.ptr, *inv = norm + kMaxLevels, *at = inv + kMaxLevels;
   for (int k = 0; k < nl; k++) {
     g.l[k].part = at;
-    at += std::max(256, g.l[k].blocks);
+    at += sums[k];
   }
   hipLaunchKernelGGL(power_start_kernel, dim3(256, nl), dim3(256), 0, st, g);
   hipLaunchKernelGGL(power_norm_kernel, dim3(nl), dim3(1024), 0, st, g, 1, norm, inv);
@@ -1493,7 +1506,6 @@ dErr coarse_inverse(_p_dohpMG *mg, hipStream_t st)
 {
   const MGLevel &lv = mg->L.back();
   const int n = (int)lv.n;
-  DOHP_CHECK(lv.n <= 4096, dohpERR_ARG, "multigrid: the coarsest level is too large for a direct solve");
   const size_t nn = (size_t)n * n, nw = 1 + kCB * kCB + 2 * (size_t)kCB * n;
   if (!mg->cinv64.holds(nn)) DOHP_CALL(mg->cinv64.alloc(nn));
   if (!mg->cinv32.holds(nn)) DOHP_CALL(mg->cinv32.alloc(nn));
@@ -1765,6 +1777,18 @@ dErr mg_fill(_p_dohpMG *mg, hipStream_t st)
 
 }  // namespace
 
+// The places for block sums that the power iterations keep for a level of nx x ny x nz rows, and the sums that a sweep and
+// a pair of sweeps write (0: the level takes no pairs).
+extern "C" dErr dohpMGPowerSums_Private(int nx, int ny, int nz, long *places, long *single, long *pair)
+{
+  const Box b{nx, ny, nz};
+  const dim3 g = power_grid(b);
+  *places = power_sums(b);
+  *single = (long)g.x * g.y * g.z;
+  *pair = pair_level<double>(b, 2) ? pair_tiles<double>(b, kPairSlots).blocks() : 0;
+  return 0;
+}
+
 extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohpMG *out, void *stream)
 {
   DOHP_CHECK(q1 && out, dohpERR_ARG, "null argument");
@@ -1794,6 +1818,10 @@ extern "C" dErr dohpMGCreate(dohpMat q1, int smooth_degree, int max_coarse, dohp
     if (err) break;
     c.A64 = c.own64.ptr;
     mg->L.push_back(std::move(c));
+  }
+  if (!err && mg->L.back().n > kMaxCoarse) {  // (a plate: refused before anything is launched)
+    set_error("multigrid: the coarsest level is too large for a direct solve");
+    err = dohpERR_ARG;
   }
   for (size_t l = 0; !err && l < mg->L.size(); l++) {
     MGLevel &lv = mg->L[l];
