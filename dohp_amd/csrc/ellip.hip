@@ -842,7 +842,11 @@ dErr checked(_p_dohpEllip *op, hipStream_t st, const char *what, F f)
   op->flag = op->nan_dev;
   const dErr err = f();
   op->flag = op->nanflag.ptr;
-  if (err) return err;
+  if (err) {  // kernels that were launched before the error hold the pinned flag: they end before the next checked call
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;  // (in a capture nothing has run)
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) (void)hipStreamSynchronize(st);
+    return err;
+  }
   DOHP_HIP(hipStreamSynchronize(st));
   DOHP_CHECK(*(volatile int *)op->nan_host == 0, dohpERR_NAN,
              std::string(what) + ": non-finite value met on the device (NaN or Inf in the input vector or the state)");
