@@ -382,9 +382,10 @@ extern "C" dErr dFSExpandedToGlobal(dohpFS fs, const double *x, double *g, int h
   (void)hmode;  // Dirichlet entries of the closure are discarded either way (fs.c:592-640)
   const int bs = 256, n3 = fs->n * fs->n * fs->n;
   hipStream_t st = (hipStream_t)stream;
-  if (fs->is_block()) {
-    const int w = fs->dirichlet_mask & 1, top = (fs->dirichlet_mask >> 1) & 1, bot = (fs->dirichlet_mask >> 2) & 1;
-    const int nx = fs->p * fs->M[0] + 1 - 2 * w, ny = fs->p * fs->M[1] + 1 - 2 * w, nz = fs->p * fs->M[2] + 1 - top - bot;
+  const int w = fs->dirichlet_mask & 1, top = (fs->dirichlet_mask >> 1) & 1, bot = (fs->dirichlet_mask >> 2) & 1;
+  const int nx = fs->p * fs->M[0] + 1 - 2 * w, ny = fs->p * fs->M[1] + 1 - 2 * w, nz = fs->p * fs->M[2] + 1 - top - bot;
+  // (a grid has at most 65536 blocks along y and z: longer boxes go colour by colour, whose grid is one-dimensional)
+  if (fs->is_block() && (ny + 3) / 4 <= 65535 && (nx + 7) / 8 <= 65535) {
     if (fs->nowned > 0)
       hipLaunchKernelGGL(fs_scatter_block_kernel, dim3(8 * ((nz + 63) / 64), (ny + 3) / 4, (nx + 7) / 8), dim3(64, 4), 0, st, fs->p,
                          fs->M[0], fs->M[1], fs->M[2], w, w, bot, nx, ny, nz, x, imode == dADD_VALUES, g);
