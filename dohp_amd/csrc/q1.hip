@@ -386,12 +386,12 @@ __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per
 // Rows of the 27-point stencil st[27][n] on node planes plane0 .. of the lattice, from the sub-cell matrices of the
 // sub-cells around them: a thread adds the diagonal and the 13 upper entries of its row (36 values, each sub-cell entry
 // read once) and also stores each upper entry as the lower one of that neighbour's row; entries toward nodes that are not
-// owned are zero.  I0, J0, K0: first owned node of the lattice; G: sub-cells per direction.
-__global__ void __launch_bounds__(256) q1_gather_kernel(int plane0, int slots, int I0, int J0, int K0, int nx, int ny,
+// owned are zero.  I0, J0, K0: first owned node of the lattice; line0: first line of this launch; G: sub-cells per direction.
+__global__ void __launch_bounds__(256) q1_gather_kernel(int plane0, int line0, int slots, int I0, int J0, int K0, int nx, int ny,
                                                         int nz, int G0, int G1, int G2, const double *__restrict__ KC,
                                                         double *__restrict__ st)
 {
-  const int K = blockIdx.x * 64 + threadIdx.x, J = blockIdx.y * 4 + threadIdx.y, I = plane0 + blockIdx.z - I0;
+  const int K = blockIdx.x * 64 + threadIdx.x, J = line0 + blockIdx.y * 4 + threadIdx.y, I = plane0 + blockIdx.z - I0;
   if (K >= nz || J >= ny || I < 0 || I >= nx) return;
   const long n = (long)nx * ny * nz, i = ((long)I * ny + J) * nz + K, ring = (long)slots * G1 * G2;
   // sub-cell (node - r) for each corner r of it that this node is (clamped: one outside the block adds nothing)
@@ -713,6 +713,7 @@ namespace {
 // Ring of sub-cell matrices of an assembly: as many layers of elements per pass as keep it in the 256 MB cache, so that
 // the gather does not read them from HBM (32^3 elements, p = 6: 96 MB 2.61 ms, 192 MB 2.31, 512 MB 2.64, one pass 3.02).
 constexpr size_t kQ1RingBytes = (size_t)192 << 20;
+constexpr int kQ1MaxGrid = 65535;  // blocks of a launch along y and z
 
 template <typename F>
 dErr q1_dispatch(int n, F f)
@@ -791,7 +792,9 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   // before it are kept in a ring of layers.
   const int G[3] = {fs->M[0] * fs->p, fs->M[1] * fs->p, fs->M[2] * fs->p};
   const size_t layer = (size_t)G[1] * G[2] * 36;
-  int lx = (int)std::min<size_t>(fs->M[0], std::max<size_t>(1, kQ1RingBytes / (8 * layer * fs->p)));
+  // (and as many as leave the gather's planes and blocks of lines within a grid's 65536)
+  int lx = (int)std::min<size_t>({(size_t)fs->M[0], (size_t)(kQ1MaxGrid / fs->p - 1),
+                                  std::max<size_t>(1, kQ1RingBytes / (8 * layer * fs->p))});
   int slots = 0;
   for (;; lx = (lx + 1) / 2) {
     slots = lx * fs->p + 1;
@@ -801,7 +804,6 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
     if (err != dohpERR_OOM || lx == 1) return err;
   }
   const int m = fs->dirichlet_mask, I0 = m & 1, K0 = (m >> 2) & 1;
-  const dim3 gg((A->box[2] + 63) / 64, (A->box[1] + 3) / 4);
   for (int x0 = 0; x0 < fs->M[0]; x0 += lx) {
     const int x1 = std::min(fs->M[0], x0 + lx);
     const long first = (long)x0 * fs->M[1] * fs->M[2], nel = (long)(x1 - x0) * fs->M[1] * fs->M[2];
@@ -823,8 +825,11 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
     }));
     // node planes whose sub-cells are all there: up to the pass's last layer of sub-cells, and the block's last plane
     const int p0 = x0 * fs->p, p1 = x1 == fs->M[0] ? G[0] + 1 : x1 * fs->p;
-    hipLaunchKernelGGL(q1_gather_kernel, dim3(gg.x, gg.y, p1 - p0), dim3(64, 4), 0, st, p0, slots, I0, I0, K0, A->box[0],
-                       A->box[1], A->box[2], G[0], G[1], G[2], A->q1ring.ptr, A->st64.ptr);
+    for (int line0 = 0; line0 < A->box[1]; line0 += 4 * kQ1MaxGrid) {
+      const dim3 grid((A->box[2] + 63) / 64, std::min(kQ1MaxGrid, (A->box[1] - line0 + 3) / 4), p1 - p0);
+      hipLaunchKernelGGL(q1_gather_kernel, grid, dim3(64, 4), 0, st, p0, line0, slots, I0, I0, K0, A->box[0], A->box[1],
+                         A->box[2], G[0], G[1], G[2], A->q1ring.ptr, A->st64.ptr);
+    }
     DOHP_HIP(hipGetLastError());
   }
   return 0;

@@ -36,3 +36,27 @@ def test_scatter(C, M):
         g = dev(g0)
         fs.expanded_to_global(dev(xe), g, C.INHOMOGENEOUS, imode)
         np.testing.assert_array_equal(g.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("M,p", [((65540, 1, 1), 1), ((32770, 1, 1), 2), ((1, 262200, 1), 1), ((1, 131100, 1), 2)])
+def test_q1_assembly(C, M, p):
+    """A uniform bar, corrected matrix: symmetric, and with free boundaries every row sums to zero; away from the ends the
+    rows repeat with the degree."""
+    print(f"long bar M={M} p={p}", flush=True)
+    fs = C.FS(M, p, block_vertices(M, box=(0, M[0], 0, M[1], 0, M[2])), dirichlet_mask=0)
+    op = C.Ellip(fs, p=2.0)
+    op.set_q1_mode(1)
+    A = op.assemble_q1().to_scipy()
+    big = abs(A).max()
+    # a row adds up to 27 entries of at most eight terms each: some hundred roundings of 1.1e-16
+    assert np.abs(A.sum(axis=1)).max() <= 1e-13 * big
+    assert (A != A.T).nnz == 0
+    d = A.diagonal()
+    cross = (p + 1) ** 2  # rows of a plane across a bar along x
+    if M[0] > 1:
+        d = d.reshape(-1, cross)
+    else:  # node (i, j, k) of a bar along y
+        d = d.reshape(p + 1, -1, p + 1).transpose(1, 0, 2).reshape(-1, cross)
+    assert d.min() > 0
+    inner = d[p:-p]
+    assert np.abs(inner[p:] - inner[:-p]).max() <= 1e-13 * big
