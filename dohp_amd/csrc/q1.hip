@@ -749,6 +749,11 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   DOHP_CHECK(fs->is_block(), dohpERR_ARG, "the embedded-Q1 matrix needs a block space (dFSCreateBlock)");
   const float *cscale = dohpEllipGetQ1CellScales_Private(op);
   hipStream_t st = (hipStream_t)stream;
+  // Not in a capture: a replay would change the stencil behind the flags that say which of the matrix's other forms, and of
+  // its hierarchy, still have to follow.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  DOHP_HIP(hipStreamIsCapturing(st, &cap));
+  DOHP_CHECK(cap == hipStreamCaptureStatusNone, dohpERR_HIP, "the embedded-Q1 assembly cannot be captured in a graph");
   if (u) DOHP_CALL(dohpEllipFunctionState_Private(op, u, st));
   _p_dohpMat *A = *out;
   if (A) A->mg_stale = true;  // new values: the cached hierarchy is recomputed, in its own buffers, when next used
