@@ -754,7 +754,10 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   DOHP_HIP(hipStreamIsCapturing(st, &cap));
   DOHP_CHECK(cap == hipStreamCaptureStatusNone, dohpERR_HIP, "the embedded-Q1 assembly cannot be captured in a graph");
-  if (u) DOHP_CALL(dohpEllipFunctionState_Private(op, u, st));
+  if (u) {
+    DOHP_CALL(dohpEllipFunctionState_Private(op, u, st));
+    DOHP_HIP(hipStreamSynchronize(st));  // (u has been read when the call returns; its kernels go on)
+  }
   _p_dohpMat *A = *out;
   if (A) A->mg_stale = true;  // new values: the cached hierarchy is recomputed, in its own buffers, when next used
   if (!A) {
