@@ -441,12 +441,14 @@ dErr pcg(Ctx &c, dohpEllip op, Prec<Z> &M, Budget &bud, const T *b, T *x, double
   int k = 0, ns = 0;
   bool restart = false;
   auto switches = [&](int used) { return M.learned_on && bud.fallback_its > 0 && used >= bud.fallback_its; };
+  auto fall_back = [&]() {
+    if (!switches(bud.used)) return;
+    M.learned_on = false;
+    bud.fell_back = 1;
+    restart = true;
+  };
   auto precondition = [&]() -> dErr {
-    if (switches(bud.used)) {
-      M.learned_on = false;
-      bud.fell_back = 1;
-      restart = true;
-    }
+    fall_back();
     if constexpr (LOW) return M.apply(c, lr.ptr, z.ptr);
     else return M.apply(c, r.ptr, z.ptr);
   };
@@ -484,7 +486,11 @@ dErr pcg(Ctx &c, dohpEllip op, Prec<Z> &M, Budget &bud, const T *b, T *x, double
       DOHP_HIP(hipMemcpyAsync(snap + (long)ns * c.n, x, sizeof(T) * c.n, hipMemcpyDeviceToDevice, c.st));
       ns++;
     }
-    if (std::sqrt(rr) <= tol || k >= max_it) break;
+    if (std::sqrt(rr) <= tol) break;
+    if (k >= max_it) {  // (a budget used up by the last iteration is reported)
+      fall_back();
+      break;
+    }
     if (!ahead) DOHP_CALL(precondition());
     // (a preconditioner that changed starts a new Krylov sequence)
     DOHP_CALL(direction(restart ? KB_FIRST : flexible ? KB_FLEXIBLE : KB_STANDARD));
