@@ -174,6 +174,33 @@ struct PoolBuf {
   ~PoolBuf() { release(); }
 };
 
+// A workspace of one object that its calls take in turn, on whatever streams: a call's kernels wait for those of the call
+// before.  It is kept until the object goes or gives it back when memory runs out.
+struct SharedScratch {
+  DevBuf<double> buf;
+  hipEvent_t done = nullptr;  // end of the last call's kernels
+  SharedScratch() = default;
+  SharedScratch(const SharedScratch &) = delete;
+  SharedScratch &operator=(const SharedScratch &) = delete;
+  ~SharedScratch()
+  {
+    if (done) (void)hipEventDestroy(done);
+  }
+  dErr begin(hipStream_t st)
+  {
+    if (done)
+      DOHP_HIP(hipStreamWaitEvent(st, done, 0));
+    else
+      DOHP_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    return 0;
+  }
+  dErr end(hipStream_t st)
+  {
+    DOHP_HIP(hipEventRecord(done, st));
+    return 0;
+  }
+};
+
 // Current device and its compute-unit count (the properties are read once per device).
 inline dErr current_device_cus(int &dev, int &cus)
 {
@@ -211,6 +238,8 @@ dErr dohpEllipMatMultAdd_Private(dohpEllip op, const float *x, float *y, hipStre
 dErr dohpEllipPinned_Private(dohpEllip op, double **host, double **dev);
 // The operator's pool of solver work vectors.
 dohp::Pool *dohpEllipPool_Private(dohpEllip op);
+// The operator's ring of sub-cell matrices (the workspace of its Q1 assemblies).
+dohp::SharedScratch *dohpEllipQ1Ring_Private(dohpEllip op);
 
 // Sparse matrix on the owned nodes.  CSR is the assembled form; on a block space the owned nodes
 // form a box of the node lattice (nx * ny * nz, lexicographic, last index fastest) and every row
@@ -235,7 +264,6 @@ struct _p_dohpMat {
   bool mg_stale = false;   // refilled since the cached hierarchy was computed (refreshed in place on its next use)
   dohp::DevBuf<double> q1tab;   // the assembly kernel's 1-D tables, of degree q1tab_degree
   int q1tab_degree = 0;
-  dohp::DevBuf<double> q1ring;  // sub-cell matrices of a few layers (the assembly's workspace)
   ~_p_dohpMat() { dohpMGDestroy(&mg); }
 };
 // Sets the box of a block-space matrix and allocates its stencil form (*box = false: not a box, CSR only).

@@ -387,6 +387,7 @@ __global__ void lattice_state_kernel(const double *__restrict__ u, const double 
 
 struct _p_dohpEllip {
   dohp::Pool pool;  // work vectors of the solves on this operator (freed with it)
+  dohp::SharedScratch q1ring;  // sub-cell matrices of a few layers: the workspace of its Q1 assemblies
   dohpFS fs = nullptr;
   dohpEllipParam prm{};
   int scatter = 1;  // 0 = colours (deterministic), 1 = atomics
@@ -895,6 +896,7 @@ extern "C" dErr dohpEllipFunctionState_Private(dohpEllip op, const double *u, hi
 }
 
 dohp::Pool *dohpEllipPool_Private(dohpEllip op) { return &op->pool; }
+dohp::SharedScratch *dohpEllipQ1Ring_Private(dohpEllip op) { return &op->q1ring; }
 
 extern "C" dErr dohpEllipGetQ1Context_Private(dohpEllip op, dohpFS *fs, dohpEllipParam *prm, const double **kvert,
                                               const double **state, int *q1mode)

@@ -735,6 +735,44 @@ dErr q1_dispatch(int n, F f)
   return 0;
 }
 
+// The passes of an assembly: sub-cell matrices of lx layers of elements into the ring of `slots` layers of sub-cells, and
+// the node planes that they complete into the matrix's stencil.
+dErr q1_passes(dohpFS fs, const dohpEllipParam &prm, const Q1Phys &ph, _p_dohpMat *A, const double *kvert,
+               const double *state, int q1mode, const float *cscale, int lx, int slots, double *ring, hipStream_t st)
+{
+  const int G[3] = {fs->M[0] * fs->p, fs->M[1] * fs->p, fs->M[2] * fs->p};
+  const int m = fs->dirichlet_mask, I0 = m & 1, K0 = (m >> 2) & 1;
+  for (int x0 = 0; x0 < fs->M[0]; x0 += lx) {
+    const int x1 = std::min(fs->M[0], x0 + lx);
+    const long first = (long)x0 * fs->M[1] * fs->M[2], nel = (long)(x1 - x0) * fs->M[1] * fs->M[2];
+    DOHP_CALL(q1_dispatch(fs->n, [&](auto NN) {
+      constexpr int N = decltype(NN)::value;
+      const bool has_u = state && (prm.p != 2.0 || prm.lambda != 0.0);
+      const size_t lds = has_u ? sizeof(double) * q1_epb(N) * (q1_lds_z(N) + q1_lds_y(N)) : 0;
+      const dim3 grid((unsigned)((nel + q1_epb(N) - 1) / q1_epb(N)));
+      auto go = [&](auto kernel) {
+        if (lds > 65536)
+          (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipLaunchKernelGGL(kernel, grid, dim3(q1_threads(N)), lds, st, first, nel, slots, fs->d_elem_verts.ptr,
+                           fs->d_vcoords.ptr, kvert, state, q1mode, A->q1tab.ptr, ph, cscale, ring);
+      };
+      if (prm.lambda != 0.0)
+        go(q1_cell_kernel<N, true>);
+      else
+        go(q1_cell_kernel<N, false>);
+    }));
+    // node planes whose sub-cells are all there: up to the pass's last layer of sub-cells, and the block's last plane
+    const int p0 = x0 * fs->p, p1 = x1 == fs->M[0] ? G[0] + 1 : x1 * fs->p;
+    for (int line0 = 0; line0 < A->box[1]; line0 += 4 * kQ1MaxGrid) {
+      const dim3 grid((A->box[2] + 63) / 64, std::min(kQ1MaxGrid, (A->box[1] - line0 + 3) / 4), p1 - p0);
+      hipLaunchKernelGGL(q1_gather_kernel, grid, dim3(64, 4), 0, st, p0, line0, slots, I0, I0, K0, A->box[0], A->box[1],
+                         A->box[2], G[0], G[1], G[2], ring, A->st64.ptr);
+    }
+    DOHP_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
 }  // namespace
 
 extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out, void *stream)
@@ -760,9 +798,16 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   }
   _p_dohpMat *A = *out;
   if (A) A->mg_stale = true;  // new values: the cached hierarchy is recomputed, in its own buffers, when next used
+  SharedScratch &ring = *dohpEllipQ1Ring_Private(op);
+  const auto with_room = [&](auto alloc) -> dErr {  // (the ring of an earlier assembly makes room for a matrix)
+    const dErr err = alloc();
+    if (err != dohpERR_OOM || !ring.buf.ptr) return err;
+    ring.buf.release();
+    return alloc();
+  };
   if (!A) {
     A = new _p_dohpMat;
-    dErr err = build_pattern(fs, A);
+    dErr err = with_room([&]() { return build_pattern(fs, A); });
     if (err) {
       delete A;
       return err;
@@ -793,7 +838,7 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   // On a block space the owned nodes form a box and the matrix is a 27-point stencil (without owned nodes there is
   // nothing to assemble); the CSR values are read back from it on demand.
   bool box = false;
-  DOHP_CALL(dohpMatPrepareStencil_Private(A, fs, &box, st));
+  DOHP_CALL(with_room([&]() { return dohpMatPrepareStencil_Private(A, fs, &box, st); }));
   A->csr_stale = box;
   if (!box) return 0;
   // Layers of elements per pass: the sub-cell matrices of a pass (288 bytes per sub-cell) and of the layer of sub-cells
@@ -806,41 +851,15 @@ extern "C" dErr dohpEllipAssembleQ1(dohpEllip op, const double *u, dohpMat *out,
   int slots = 0;
   for (;; lx = (lx + 1) / 2) {
     slots = lx * fs->p + 1;
-    if (A->q1ring.n >= slots * layer) break;
-    const dErr err = A->q1ring.alloc(slots * layer);
+    if (ring.buf.n >= slots * layer) break;
+    const dErr err = ring.buf.alloc(slots * layer);
     if (!err) break;
     if (err != dohpERR_OOM || lx == 1) return err;
   }
-  const int m = fs->dirichlet_mask, I0 = m & 1, K0 = (m >> 2) & 1;
-  for (int x0 = 0; x0 < fs->M[0]; x0 += lx) {
-    const int x1 = std::min(fs->M[0], x0 + lx);
-    const long first = (long)x0 * fs->M[1] * fs->M[2], nel = (long)(x1 - x0) * fs->M[1] * fs->M[2];
-    DOHP_CALL(q1_dispatch(fs->n, [&](auto NN) {
-      constexpr int N = decltype(NN)::value;
-      const bool has_u = state && (prm.p != 2.0 || prm.lambda != 0.0);
-      const size_t lds = has_u ? sizeof(double) * q1_epb(N) * (q1_lds_z(N) + q1_lds_y(N)) : 0;
-      const dim3 grid((unsigned)((nel + q1_epb(N) - 1) / q1_epb(N)));
-      auto go = [&](auto kernel) {
-        if (lds > 65536)
-          (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        hipLaunchKernelGGL(kernel, grid, dim3(q1_threads(N)), lds, st, first, nel, slots, fs->d_elem_verts.ptr,
-                           fs->d_vcoords.ptr, kvert, state, q1mode, A->q1tab.ptr, ph, cscale, A->q1ring.ptr);
-      };
-      if (prm.lambda != 0.0)
-        go(q1_cell_kernel<N, true>);
-      else
-        go(q1_cell_kernel<N, false>);
-    }));
-    // node planes whose sub-cells are all there: up to the pass's last layer of sub-cells, and the block's last plane
-    const int p0 = x0 * fs->p, p1 = x1 == fs->M[0] ? G[0] + 1 : x1 * fs->p;
-    for (int line0 = 0; line0 < A->box[1]; line0 += 4 * kQ1MaxGrid) {
-      const dim3 grid((A->box[2] + 63) / 64, std::min(kQ1MaxGrid, (A->box[1] - line0 + 3) / 4), p1 - p0);
-      hipLaunchKernelGGL(q1_gather_kernel, grid, dim3(64, 4), 0, st, p0, line0, slots, I0, I0, K0, A->box[0], A->box[1],
-                         A->box[2], G[0], G[1], G[2], A->q1ring.ptr, A->st64.ptr);
-    }
-    DOHP_HIP(hipGetLastError());
-  }
-  return 0;
+  DOHP_CALL(ring.begin(st));
+  const dErr err = q1_passes(fs, prm, ph, A, kvert, state, q1mode, cscale, lx, slots, ring.buf.ptr, st);
+  DOHP_CALL(ring.end(st));  // (also after an error: what was launched still uses the ring)
+  return err;
 }
 
 extern "C" dErr dohpMatGetSizes(dohpMat A, long *nrows, long *nnz)

@@ -239,7 +239,10 @@ typedef struct _p_dohpMat *dohpMat;
  * (owned vector, Dirichlet values from the cache; NULL = the state of the last function
  * evaluation) into a device CSR over owned nodes.  *mat == NULL creates the matrix (pattern:
  * 27 lattice neighbours, dFSCreateMatrix, src/fs/interface/fs.c:770-813); otherwise it is
- * refilled in place (SAME_NONZERO_PATTERN). */
+ * refilled in place (SAME_NONZERO_PATTERN).  u has been read when the call returns; the assembly goes on in stream
+ * order.  Not in a graph capture.  The operator keeps a workspace of 288 bytes per sub-cell of a few layers of
+ * elements: at most 192 MiB, or one layer of elements and one of sub-cells where those take more.  The matrices
+ * assembled from one operator share it; assemblies on several streams take it in turn. */
 dErr dohpEllipAssembleQ1(dohpEllip op, const double *u_dev, dohpMat *mat, void *stream);
 /* Arithmetic of later Q1 assemblies (no reference counterpart): 0 = the reference's (default; sub-cell
  * derivatives +-1 per element-reference unit, efstopo.c:665-706, and the element-natural inverse
