@@ -27,7 +27,6 @@
 #include <vector>
 
 #include "common.h"
-#define DOHP_PITCH_N4 4
 #include "element.h"
 
 using namespace dohp;
@@ -66,7 +65,7 @@ inline bool pack_valid(int N, int pack, int tsize, int mfma)
 inline size_t cfg_lds(int N, int pack, int tsize)
 {
   const size_t E = item_elems(N, pack), N3 = (size_t)N * N * N;
-  return E * 32 * sizeof(double) + 3 * E * tile_len(N) * tsize + E * N3 * sizeof(int);
+  return E * 32 * sizeof(double) + 3 * E * N3 * tsize + E * N3 * sizeof(int);
 }
 
 struct BArgs {
@@ -114,12 +113,12 @@ template <int N, int DIR, bool ACC, int E>
 __device__ __forceinline__ void mfma_contract(const float *in, float *out, bf16x4 oh, bf16x4 ol, int passes,
                                               int wave, int lane)
 {
-  constexpr int NN = N * N, NB = (NN + 15) / 16;
+  constexpr int NN = N * N, N3 = NN * N, NB = (NN + 15) / 16;
   const int r16 = lane & 15, kg = lane >> 4;
   for (int p = wave; p < E * NB; p += 4) {
     const int e = p / NB, rb = p - e * NB;
-    const float *ti = in + e * tile_len(N);
-    float *to = out + e * tile_len(N);
+    const float *ti = in + e * N3;
+    float *to = out + e * N3;
     const int r = rb * 16 + r16, ra = r / N, rr = r - ra * N;
     bf16x4 xh, xl;
 #pragma unroll
@@ -156,8 +155,8 @@ __device__ __forceinline__ void batch_item(const BArgs &g, const int4 it, const 
   constexpr bool WS = PACK == PACK_WAVE;
   constexpr int EW = WS ? E / 4 : E, GT = WS ? 64 : kBT, NS = (EW * N3 + GT - 1) / GT;
   double *VX = (double *)smem;
-  T *TA = (T *)(VX + E * 32), *TGX = TA + E * tile_len(N), *TGY = TGX + E * tile_len(N);
-  int *IDX = (int *)(TGY + E * tile_len(N));
+  T *TA = (T *)(VX + E * 32), *TGX = TA + E * N3, *TGY = TGX + E * N3;
+  int *IDX = (int *)(TGY + E * N3);
   // the thread index is laundered so that nothing derived from it is hoisted out of the item loop
   // (each order would keep its own copies live across every other order's code)
   int tid = threadIdx.x;
@@ -175,7 +174,7 @@ __device__ __forceinline__ void batch_item(const BArgs &g, const int4 it, const 
       const int ts = e0 * N3 + t, l = ts / N3;
       const int c = l < count ? gidx[ts] : -1;
       IDX[ts] = c;
-      TA[tile_slot<N>(ts)] = c >= 0 ? x[c] : T(0);
+      TA[ts] = c >= 0 ? x[c] : T(0);
     }
   }
   for (int t = gt; t < EW * 8; t += GT) {
@@ -208,7 +207,7 @@ __device__ __forceinline__ void batch_item(const BArgs &g, const int4 it, const 
   int lb = line;  // derived values are formed here, not hoisted above the gather
   asm volatile("" : "+v"(lb));
   const int le = lb / NN, ab = lb - le * NN, a = ab / N, b = ab - a * N;
-  T *A = &TA[le * tile_len(N)], *GX = &TGX[le * tile_len(N)], *GY = &TGY[le * tile_len(N)];
+  T *A = &TA[le * N3], *GX = &TGX[le * N3], *GY = &TGY[le * N3];
   typedef const __attribute__((address_space(4))) double ConstD;
   const double *wl = g.wphi + wphi_off(N);
   const ConstD *wq = (const ConstD *)sgpr_fence(wl), *phq = wq + N;
@@ -298,7 +297,7 @@ __device__ __forceinline__ void batch_item(const BArgs &g, const int4 it, const 
         const int le2 = e0 + t / NN, ab2 = t % NN, top = le2 * N3 + ab2 * N + N - 1, bot = top + N3 - N + 1;
         const int ct = IDX[top];
         if (ct >= 0 && ct == IDX[bot]) {
-          TA[tile_slot<N>(bot)] += TA[tile_slot<N>(top)];
+          TA[bot] += TA[top];
           IDX[top] = -2;
         }
       }
@@ -311,7 +310,7 @@ __device__ __forceinline__ void batch_item(const BArgs &g, const int4 it, const 
     if (t < EW * N3) {
       const int ts = e0 * N3 + brick_slot<N, EW>(t), c = IDX[ts];
       if (c >= 0) {
-        const T v = TA[tile_slot<N>(ts)];
+        const T v = TA[ts];
         if (excl) y[c] = v;
         else atomicAdd(&y[c], v);
       }

@@ -200,7 +200,7 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ tab, int op, cons
   }
 }
 
-// Element tiles [i][j][k] (k fastest, the reference's node order; lines of n values at a pitch of line_pitch(n)).  A thread (a, b) of an
+// Element tiles [i][j][k] (k fastest, the reference's node order).  A thread (a, b) of an
 // element owns one line per phase: a z line (i, j) = (a, b), a y line (i, k) = (a, b) or an
 // x line (j, k) = (a, b).  No register value crosses from one phase to the next, so any one-to-one
 // assignment of lines to threads within a phase is valid.  At n = 7 the y lines are dealt out as
@@ -210,39 +210,31 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ tab, int op, cons
 // residual and recomputing kernels at degree 6 run 1.3-1.9 % faster).  At the other orders no
 // permutation of this kind measured faster, and (a, b) is kept.
 enum { DIR_X = 0, DIR_Y = 1, DIR_Z = 2 };
-// At n = 4 a line of the tile is followed by an unused slot: at a pitch of 4 the 16 lanes of an element start on a
-// quarter of the banks in the z phase (conflicts a third of the compute units' cycles; A x at degree 3, 250 k elements
-// 185 -> 177 us, the residual 255 -> 250).  At the other even orders the larger tiles cost more than the conflicts (n = 6:
-// A x 154 -> 187 us; the batched mixed orders 393 -> 485).  The batch keeps n = 4 at 4 as well (0.5 % faster).  Point t
-// (i n^2 + j n + k, over all elements of the workgroup) is at tile_slot(t).
-#ifndef DOHP_PITCH_N4
-#define DOHP_PITCH_N4 5
-#endif
-constexpr int line_pitch(int N) { return N == 4 ? DOHP_PITCH_N4 : N; }
-constexpr int tile_len(int N) { return N * N * line_pitch(N); }
-template <int N>
+// Lines lie P >= n values apart (the kernels choose P, see tile_pitch in ellip.hip); point t (i n^2 + j n + k, over all
+// elements of the workgroup) is at tile_slot(t).
+template <int N, int P>
 __device__ __forceinline__ int tile_slot(int t)
 {
-  return line_pitch(N) == N ? t : t + t / N;
+  return P == N ? t : t + t / N * (P - N);
 }
-template <int N, int DIR>
+template <int N, int DIR, int P = N>
 __device__ __forceinline__ int line_at(int a, int b, int s)
 {
+  static_assert(P == N || N != 7, "the permuted lines have no padding");
   if constexpr (DIR == DIR_Y && N == 7) return (b * N + s) * N + (a == 0 ? 0 : N - a);
-  constexpr int P = line_pitch(N);
   return DIR == DIR_Z ? (a * N + b) * P + s : DIR == DIR_Y ? (a * N + s) * P + b : (s * N + a) * P + b;
 }
-template <int N, int DIR, typename T>
+template <int N, int DIR, int P = N, typename T>
 __device__ __forceinline__ void ld_line(const T *tile, int a, int b, T (&v)[N])
 {
 #pragma unroll
-  for (int s = 0; s < N; s++) v[s] = tile[line_at<N, DIR>(a, b, s)];
+  for (int s = 0; s < N; s++) v[s] = tile[line_at<N, DIR, P>(a, b, s)];
 }
-template <int N, int DIR, typename T>
+template <int N, int DIR, int P = N, typename T>
 __device__ __forceinline__ void st_line(T *tile, int a, int b, const T (&v)[N])
 {
 #pragma unroll
-  for (int s = 0; s < N; s++) tile[line_at<N, DIR>(a, b, s)] = v[s];
+  for (int s = 0; s < N; s++) tile[line_at<N, DIR, P>(a, b, s)] = v[s];
 }
 
 // Barrier between line phases: the whole workgroup (WS = false), or only the wavefront when every
@@ -265,41 +257,41 @@ __device__ __forceinline__ void tile_sync()
 // overwritten; GX and GY are scratch.  Every thread of the workgroup must call it.  Three line
 // phases: z (B); y (B, and Dh B into GY); x (B and Dh B into GX, B of GY); the z derivative stays
 // in registers.
-template <int N, typename T, bool WS = false>
+template <int N, typename T, bool WS = false, int P = N>
 __device__ __forceinline__ void forward(const T *tab, T *A, T *GX, T *GY, int a, int b, T (&q)[N], T (&gx)[N],
                                         T (&gy)[N], T (&gz)[N])
 {
   T in[N], out[N];
-  ld_line<N, DIR_Z>(A, a, b, in);
+  ld_line<N, DIR_Z, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_B, in, out);
-  st_line<N, DIR_Z>(A, a, b, out);
+  st_line<N, DIR_Z, P>(A, a, b, out);
   tile_sync<WS>();
-  ld_line<N, DIR_Y>(A, a, b, in);
+  ld_line<N, DIR_Y, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_B, in, out);
-  st_line<N, DIR_Y>(A, a, b, out);
+  st_line<N, DIR_Y, P>(A, a, b, out);
   eo_apply<N, -1>(tab, OP_DB, in, out);
-  st_line<N, DIR_Y>(GY, a, b, out);
+  st_line<N, DIR_Y, P>(GY, a, b, out);
   tile_sync<WS>();
-  ld_line<N, DIR_X>(A, a, b, in);
+  ld_line<N, DIR_X, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_B, in, out);
-  st_line<N, DIR_X>(A, a, b, out);
+  st_line<N, DIR_X, P>(A, a, b, out);
   eo_apply<N, -1>(tab, OP_DB, in, out);
-  st_line<N, DIR_X>(GX, a, b, out);
-  ld_line<N, DIR_X>(GY, a, b, in);
+  st_line<N, DIR_X, P>(GX, a, b, out);
+  ld_line<N, DIR_X, P>(GY, a, b, in);
   eo_apply<N, 1>(tab, OP_B, in, out);
-  st_line<N, DIR_X>(GY, a, b, out);
+  st_line<N, DIR_X, P>(GY, a, b, out);
   tile_sync<WS>();
-  ld_line<N, DIR_Z>(A, a, b, q);
+  ld_line<N, DIR_Z, P>(A, a, b, q);
   eo_apply<N, -1>(tab, OP_D, q, gz);
-  ld_line<N, DIR_Z>(GX, a, b, gx);
-  ld_line<N, DIR_Z>(GY, a, b, gy);
+  ld_line<N, DIR_Z, P>(GX, a, b, gx);
+  ld_line<N, DIR_Z, P>(GY, a, b, gy);
 }
 
 // Transposed applies: from the pointwise values v and the mapped fluxes d0, d1, d2 along the
 // thread's z line, the element's nodal contributions B^T (v + Dh_x^T d0 + Dh_y^T d1 + Dh_z^T d2)
 // land in tile A.  Three line phases after the z one: x (B^T of the sum, plus (Dh B)^T of d0; B^T
 // of d1), y (B^T, plus (Dh B)^T of d1), z (B^T).  Ends with a barrier.
-template <int N, typename T, bool WS = false>
+template <int N, typename T, bool WS = false, int P = N>
 __device__ __forceinline__ void backward(const T *tab, T *A, T *GX, T *GY, int a, int b, const T (&v)[N],
                                          const T (&d0)[N], const T (&d1)[N], const T (&d2)[N])
 {
@@ -307,32 +299,32 @@ __device__ __forceinline__ void backward(const T *tab, T *A, T *GX, T *GY, int a
   eo_apply<N, -1>(tab, OP_DT, d2, w);
 #pragma unroll
   for (int s = 0; s < N; s++) w[s] += v[s];
-  st_line<N, DIR_Z>(A, a, b, w);
-  st_line<N, DIR_Z>(GY, a, b, d1);
-  st_line<N, DIR_Z>(GX, a, b, d0);
+  st_line<N, DIR_Z, P>(A, a, b, w);
+  st_line<N, DIR_Z, P>(GY, a, b, d1);
+  st_line<N, DIR_Z, P>(GX, a, b, d0);
   tile_sync<WS>();
-  ld_line<N, DIR_X>(A, a, b, in);
+  ld_line<N, DIR_X, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_BT, in, w);
-  ld_line<N, DIR_X>(GX, a, b, in);
+  ld_line<N, DIR_X, P>(GX, a, b, in);
   eo_apply<N, -1>(tab, OP_DBT, in, out);
 #pragma unroll
   for (int s = 0; s < N; s++) w[s] += out[s];
-  st_line<N, DIR_X>(A, a, b, w);
-  ld_line<N, DIR_X>(GY, a, b, in);
+  st_line<N, DIR_X, P>(A, a, b, w);
+  ld_line<N, DIR_X, P>(GY, a, b, in);
   eo_apply<N, 1>(tab, OP_BT, in, out);
-  st_line<N, DIR_X>(GY, a, b, out);
+  st_line<N, DIR_X, P>(GY, a, b, out);
   tile_sync<WS>();
-  ld_line<N, DIR_Y>(A, a, b, in);
+  ld_line<N, DIR_Y, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_BT, in, w);
-  ld_line<N, DIR_Y>(GY, a, b, in);
+  ld_line<N, DIR_Y, P>(GY, a, b, in);
   eo_apply<N, -1>(tab, OP_DBT, in, out);
 #pragma unroll
   for (int s = 0; s < N; s++) w[s] += out[s];
-  st_line<N, DIR_Y>(A, a, b, w);
+  st_line<N, DIR_Y, P>(A, a, b, w);
   tile_sync<WS>();
-  ld_line<N, DIR_Z>(A, a, b, in);
+  ld_line<N, DIR_Z, P>(A, a, b, in);
   eo_apply<N, 1>(tab, OP_BT, in, out);
-  st_line<N, DIR_Z>(A, a, b, out);
+  st_line<N, DIR_Z, P>(A, a, b, out);
   tile_sync<WS>();
 }
 
@@ -344,8 +336,8 @@ __device__ __forceinline__ void backward(const T *tab, T *A, T *GX, T *GY, int a
 // K step (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64, the precision of the kernel, so nothing is
 // rounded below it).  Operand layout of the 16x16x4 products: lane l holds A[l % 16][l / 16] of the
 // operator, B[l / 16][l % 16] of the lines and, after the product, C[row(l / 16, r)][l % 16],
-// r = 0..3, with row = 4 (l / 16) + r in FP32 and l / 16 + 4 r in FP64 (measured on gfx950).  Line inputs are one or two fields (K = 8 per field: positions s = 0..n-1 along the
-// line, the rest zero), outputs one or two fields (rows 0..7 into the first, 8..15 into the
+// r = 0..3, with row = 4 (l / 16) + r in FP32 and l / 16 + 4 r in FP64 (measured on gfx950).  Line inputs are one or two
+// fields (K = 8 per field: positions s = 0..n-1 along the line, the rest zero), outputs one or two fields (rows 0..7 into the first, 8..15 into the
 // second).  A pass reads and writes only its own lines, so it can update a field in place; passes
 // in different directions are separated by workgroup barriers.  Every lane of the wavefront must
 // be active (the workgroup has 256 threads, one per line; lines past the elements are a pad tile).
@@ -377,12 +369,12 @@ struct Mfma16<double> {
 // in the tiles (the line of its lane's column in block j is lane 16 j + l % 16's own line), frag = the
 // operator's fragments.  (Issuing the four blocks' reads together, then four independent product
 // chains, measured slower: more registers, the same matrix-pipe time.)
-template <int N, int DIR, typename T, int NIN, int NOUT>
+template <int N, int DIR, typename T, int NIN, int NOUT, int P>
 __device__ __forceinline__ void mfma_lines(const T *__restrict__ frag, const T *in0, const T *in1, T *out0, T *out1,
                                            int own, int lane)
 {
   static_assert(N <= kMfmaMaxN, "the line pass holds at most 8 points per field");
-  constexpr int STR = DIR == DIR_Z ? 1 : DIR == DIR_Y ? line_pitch(N) : N * line_pitch(N), KS = 2 * NIN;
+  constexpr int STR = DIR == DIR_Z ? 1 : DIR == DIR_Y ? P : N * P, KS = 2 * NIN;
   typedef typename Mfma16<T>::acc acc;
   const int kq = lane >> 4;
   T op[KS];
@@ -411,51 +403,51 @@ __device__ __forceinline__ void mfma_lines(const T *__restrict__ frag, const T *
 // forward() on the matrix cores: z (B), y (B and Dh B), x (B and Dh B; B of GY); the z derivative
 // of the thread's own line stays on the vector units.  TA, TGX, TGY are the workgroup's tiles, le the
 // thread's tile.  Called by all 256 threads.
-template <int N, typename T>
+template <int N, typename T, int P>
 __device__ __forceinline__ void forward_mfma(const T *tab, const T *frag, T *TA, T *TGX, T *TGY, int le, int a,
                                              int b, T (&q)[N], T (&gx)[N], T (&gy)[N], T (&gz)[N])
 {
-  const int lane = threadIdx.x & 63, e0 = le * tile_len(N);
-  const int bz = e0 + line_at<N, DIR_Z>(a, b, 0), by = e0 + line_at<N, DIR_Y>(a, b, 0),
-            bx = e0 + line_at<N, DIR_X>(a, b, 0);
-  mfma_lines<N, DIR_Z, T, 1, 1>(frag + MF_B, TA, TA, TA, TA, bz, lane);
+  const int lane = threadIdx.x & 63, e0 = le * N * N * P;
+  const int bz = e0 + line_at<N, DIR_Z, P>(a, b, 0), by = e0 + line_at<N, DIR_Y, P>(a, b, 0),
+            bx = e0 + line_at<N, DIR_X, P>(a, b, 0);
+  mfma_lines<N, DIR_Z, T, 1, 1, P>(frag + MF_B, TA, TA, TA, TA, bz, lane);
   __syncthreads();
-  mfma_lines<N, DIR_Y, T, 1, 2>(frag + MF_BDB, TA, TA, TA, TGY, by, lane);
+  mfma_lines<N, DIR_Y, T, 1, 2, P>(frag + MF_BDB, TA, TA, TA, TGY, by, lane);
   __syncthreads();
-  mfma_lines<N, DIR_X, T, 1, 2>(frag + MF_BDB, TA, TA, TA, TGX, bx, lane);
-  mfma_lines<N, DIR_X, T, 1, 1>(frag + MF_B, TGY, TGY, TGY, TGY, bx, lane);
+  mfma_lines<N, DIR_X, T, 1, 2, P>(frag + MF_BDB, TA, TA, TA, TGX, bx, lane);
+  mfma_lines<N, DIR_X, T, 1, 1, P>(frag + MF_B, TGY, TGY, TGY, TGY, bx, lane);
   __syncthreads();
-  ld_line<N, DIR_Z>(&TA[e0], a, b, q);
+  ld_line<N, DIR_Z, P>(&TA[e0], a, b, q);
   eo_apply<N, -1>(tab, OP_D, q, gz);
-  ld_line<N, DIR_Z>(&TGX[e0], a, b, gx);
-  ld_line<N, DIR_Z>(&TGY[e0], a, b, gy);
+  ld_line<N, DIR_Z, P>(&TGX[e0], a, b, gx);
+  ld_line<N, DIR_Z, P>(&TGY[e0], a, b, gy);
 }
 
 // backward() on the matrix cores: the z transposed derivative of the thread's own line on the
 // vector units, then x (B^T of the sum plus (Dh B)^T of d0; B^T of d1), y (B^T plus (Dh B)^T of
 // d1), z (B^T).  Ends with a barrier; the result is in TA.
-template <int N, typename T>
+template <int N, typename T, int P>
 __device__ __forceinline__ void backward_mfma(const T *tab, const T *frag, T *TA, T *TGX, T *TGY, int le, int a,
                                               int b, const T (&v)[N], const T (&d0)[N], const T (&d1)[N],
                                               const T (&d2)[N])
 {
-  const int lane = threadIdx.x & 63, e0 = le * tile_len(N);
-  const int bz = e0 + line_at<N, DIR_Z>(a, b, 0), by = e0 + line_at<N, DIR_Y>(a, b, 0),
-            bx = e0 + line_at<N, DIR_X>(a, b, 0);
+  const int lane = threadIdx.x & 63, e0 = le * N * N * P;
+  const int bz = e0 + line_at<N, DIR_Z, P>(a, b, 0), by = e0 + line_at<N, DIR_Y, P>(a, b, 0),
+            bx = e0 + line_at<N, DIR_X, P>(a, b, 0);
   T w[N];
   eo_apply<N, -1>(tab, OP_DT, d2, w);
 #pragma unroll
   for (int s = 0; s < N; s++) w[s] += v[s];
-  st_line<N, DIR_Z>(&TA[e0], a, b, w);
-  st_line<N, DIR_Z>(&TGY[e0], a, b, d1);
-  st_line<N, DIR_Z>(&TGX[e0], a, b, d0);
+  st_line<N, DIR_Z, P>(&TA[e0], a, b, w);
+  st_line<N, DIR_Z, P>(&TGY[e0], a, b, d1);
+  st_line<N, DIR_Z, P>(&TGX[e0], a, b, d0);
   __syncthreads();
-  mfma_lines<N, DIR_X, T, 2, 1>(frag + MF_BTDBT, TA, TGX, TA, TA, bx, lane);
-  mfma_lines<N, DIR_X, T, 1, 1>(frag + MF_BT, TGY, TGY, TGY, TGY, bx, lane);
+  mfma_lines<N, DIR_X, T, 2, 1, P>(frag + MF_BTDBT, TA, TGX, TA, TA, bx, lane);
+  mfma_lines<N, DIR_X, T, 1, 1, P>(frag + MF_BT, TGY, TGY, TGY, TGY, bx, lane);
   __syncthreads();
-  mfma_lines<N, DIR_Y, T, 2, 1>(frag + MF_BTDBT, TA, TGY, TA, TA, by, lane);
+  mfma_lines<N, DIR_Y, T, 2, 1, P>(frag + MF_BTDBT, TA, TGY, TA, TA, by, lane);
   __syncthreads();
-  mfma_lines<N, DIR_Z, T, 1, 1>(frag + MF_BT, TA, TA, TA, TA, bz, lane);
+  mfma_lines<N, DIR_Z, T, 1, 1, P>(frag + MF_BT, TA, TA, TA, TA, bz, lane);
   __syncthreads();
 }
 

@@ -68,11 +68,20 @@ constexpr bool jac_state_first()
   return sizeof(T) == 4 || N >= 9;
 }
 
+// Pitch of the element tiles' lines.  At n = 4 a line is followed by an unused slot: at a pitch of 4 the 16 lanes of an
+// element start on a quarter of the banks in the z phase (conflicts a third of the compute units' cycles).  250 k elements
+// of degree 3, pitch 4 -> 5, fastest shape: A x 168 -> 159 us (FP32 128 -> 126), residual 260 -> 248, recomputing J v
+// 346 -> 335 (FP32 179 -> 176).  From stored data, whose kernel waits for memory and contracts one field, the larger tiles
+// cost more: J v with the Bratu term 231 -> 234 us, on the matrix cores 324 -> 364 (FP32 180 -> 194); it keeps 4.  At the
+// other even orders they do in every mode (n = 6: A x 154 -> 187 us).
+constexpr int tile_pitch(int N, int mode) { return N == 4 && mode != MODE_JQD ? 5 : N; }
+
 // MF: the contractions as line passes on the matrix cores (n <= 8; 256 threads, one per line of the
 // workgroup's tiles, lines past the elements in a pad tile).
 template <int N, typename T, int MODE, int EPB, bool MF = false>
 __global__ void __launch_bounds__(MF ? 256 : wg_threads(N, EPB))
-__attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <= 7 ? 3 : 1))) ellip_kernel(const int *__restrict__ elist, long ne, BoxMap bm,
+__attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <= 7 ? 3 : 1))) ellip_kernel(
+                                                    const int *__restrict__ elist, long ne, BoxMap bm,
                                                     const int *__restrict__ enodes, const int *__restrict__ everts,
                                                     const double *__restrict__ vxyz, const double *__restrict__ kv,
                                                     const T *__restrict__ ustate, const T *__restrict__ xdir,
@@ -84,7 +93,8 @@ __attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <=
                 "matrix-core passes: n <= 8, one line per thread, modes that scatter");
   constexpr int NN = N * N, N3 = NN * N, NT = MF ? 256 : wg_threads(N, EPB), NS = (EPB * N3 + NT - 1) / NT;
   constexpr int ET = EPB + (MF ? 1 : 0);  // element tiles (the pad tile last)
-  __shared__ T TA[ET * tile_len(N)], TGX[ET * tile_len(N)], TGY[ET * tile_len(N)];
+  constexpr int P = tile_pitch(N, MODE);
+  __shared__ T TA[ET * NN * P], TGX[ET * NN * P], TGY[ET * NN * P];
   __shared__ int IDX[EPB * N3];
   __shared__ double VX[ET * 8 * 4];
   __shared__ int EB[ET * 4];  // per element slot: first lattice point, 1 if the slot holds an element
@@ -180,7 +190,7 @@ __attribute__((amdgpu_waves_per_eu((MODE == MODE_FUN || MODE == MODE_QD) && N <=
       if (t < EPB * N3) {
         const T v = own[s] >= 0 ? xv[s] : T(0), u = lat[s] >= 0 ? uv[s] : T(0);
         IDX[t] = own[s];
-        TA[tile_slot<N>(t)] = STATE_FIRST ? u : v;
+        TA[tile_slot<N, P>(t)] = STATE_FIRST ? u : v;
         if (MODE == MODE_JAC) pre2[s] = STATE_FIRST ? v : u;
       }
     }
@@ -227,7 +237,8 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
   constexpr bool PREFETCH_VALUES = MODE != MODE_JAC || sizeof(T) == 4;
   constexpr bool GATHER_X = MODE == MODE_LIN || MODE == MODE_JQD;  // else the state
   constexpr bool PREFETCH_STATE = MODE == MODE_JAC && PREFETCH_VALUES;
-  __shared__ T TA[EPB * tile_len(N)], TGX[EPB * tile_len(N)], TGY[EPB * tile_len(N)];
+  constexpr int P = tile_pitch(N, MODE);
+  __shared__ T TA[EPB * NN * P], TGX[EPB * NN * P], TGY[EPB * NN * P];
   __shared__ int IDX[EPB * N3];
   __shared__ double VX[EPB * 8 * 4];
   const int tid = threadIdx.x;
@@ -299,7 +310,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
         const int t = s * NT + tid;
         if (t < EPB * N3) {
           IDX[t] = pidx[s];
-          TA[tile_slot<N>(t)] = pval[s];
+          TA[tile_slot<N, P>(t)] = pval[s];
         }
       }
     }
@@ -322,7 +333,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && MODE == MODE_LIN ? 3 : 1)))
         if (t < EPB * N3) {
           IDX[t] = own;
           const T xv = own >= 0 ? xdir[own] : T(0), uv = lat >= 0 ? ustate[lat] : T(0);
-          TA[tile_slot<N>(t)] = jac_state_first<N, T>() ? uv : xv;
+          TA[tile_slot<N, P>(t)] = jac_state_first<N, T>() ? uv : xv;
           pre2[s] = jac_state_first<N, T>() ? xv : uv;
         }
       }
