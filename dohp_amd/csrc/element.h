@@ -336,9 +336,9 @@ __device__ __forceinline__ void backward(const T *tab, T *A, T *GX, T *GY, int a
 // K step (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64, the precision of the kernel, so nothing is
 // rounded below it).  Operand layout of the 16x16x4 products: lane l holds A[l % 16][l / 16] of the
 // operator, B[l / 16][l % 16] of the lines and, after the product, C[row(l / 16, r)][l % 16],
-// r = 0..3, with row = 4 (l / 16) + r in FP32 and l / 16 + 4 r in FP64 (measured on gfx950).  Line inputs are one or two
-// fields (K = 8 per field: positions s = 0..n-1 along the line, the rest zero), outputs one or two fields (rows 0..7 into the first, 8..15 into the
-// second).  A pass reads and writes only its own lines, so it can update a field in place; passes
+// r = 0..3, with row = 4 (l / 16) + r in FP32 and l / 16 + 4 r in FP64 (measured on gfx950).  Line
+// inputs are one or two fields (K = 8 per field: positions s = 0..n-1 along the line, the rest
+// zero), outputs one or two fields (rows 0..7 into the first, 8..15 into the second).  A pass reads and writes only its own lines, so it can update a field in place; passes
 // in different directions are separated by workgroup barriers.  Every lane of the wavefront must
 // be active (the workgroup has 256 threads, one per line; lines past the elements are a pad tile).
 constexpr int kMfmaMaxN = 8;

@@ -368,9 +368,9 @@ extern "C" dErr dFSGlobalToExpanded(dohpFS fs, const double *g, double *x, int h
   DOHP_CHECK(hmode == dFS_HOMOGENEOUS || hmode == dFS_INHOMOGENEOUS, dohpERR_ARG, "invalid homogeneous mode");
   const long nexp = (long)fs->nelem * fs->n * fs->n * fs->n;
   const int bs = 256;
-  hipLaunchKernelGGL(fs_gather_kernel, dim3((unsigned)((nexp + 32 * bs - 1) / (32 * bs) * 8)), dim3(bs), 0, (hipStream_t)stream,
-                     fs->d_elem_nodes.ptr, nexp, g, fs->d_dcache.ptr, fs->nowned, hmode == dFS_INHOMOGENEOUS,
-                     imode == dADD_VALUES, x);
+  hipLaunchKernelGGL(fs_gather_kernel, dim3((unsigned)((nexp + 32 * bs - 1) / (32 * bs) * 8)), dim3(bs), 0,
+                     (hipStream_t)stream, fs->d_elem_nodes.ptr, nexp, g, fs->d_dcache.ptr, fs->nowned,
+                     hmode == dFS_INHOMOGENEOUS, imode == dADD_VALUES, x);
   DOHP_HIP(hipGetLastError());
   return 0;
 }
@@ -387,8 +387,8 @@ extern "C" dErr dFSExpandedToGlobal(dohpFS fs, const double *x, double *g, int h
   // (a grid has at most 65536 blocks along y and z: longer boxes go colour by colour, whose grid is one-dimensional)
   if (fs->is_block() && (ny + 3) / 4 <= 65535 && (nx + 7) / 8 <= 65535) {
     if (fs->nowned > 0)
-      hipLaunchKernelGGL(fs_scatter_block_kernel, dim3(8 * ((nz + 63) / 64), (ny + 3) / 4, (nx + 7) / 8), dim3(64, 4), 0, st, fs->p,
-                         fs->M[0], fs->M[1], fs->M[2], w, w, bot, nx, ny, nz, x, imode == dADD_VALUES, g);
+      hipLaunchKernelGGL(fs_scatter_block_kernel, dim3(8 * ((nz + 63) / 64), (ny + 3) / 4, (nx + 7) / 8), dim3(64, 4), 0,
+                         st, fs->p, fs->M[0], fs->M[1], fs->M[2], w, w, bot, nx, ny, nz, x, imode == dADD_VALUES, g);
     DOHP_HIP(hipGetLastError());
     return 0;
   }

@@ -468,10 +468,11 @@ __global__ void diag_kernel(long n, const double *__restrict__ A, double *__rest
 // The half stencil of a level in FP64 (H, null where the level's own stencil serves), FP32 and FP16 in one pass over its
 // 27-point stencil A: a row's 13 upper entries are read once for all three, the row scales of its neighbours come from
 // a staged tile, and its lower neighbours' entries (which those rows round) are read for the diagonal's compensation.
-// 112 bytes read and 112 + 56 + 48 written per row and 27 FP64 divisions: 191^3 rows 0.95 -> 0.51 ms against a copy of the half
-// stencil and an FP16 pass that took 52 square roots per row.
-__global__ void __launch_bounds__(256) half_setup_kernel(Box bx, Split sp, const double *__restrict__ A, double *__restrict__ H,
-                                                         float *__restrict__ H32, _Float16 *__restrict__ H16,
+// 112 bytes read and 112 + 56 + 48 written per row and 27 FP64 divisions: 191^3 rows 0.95 -> 0.51 ms against a copy of the
+// half stencil and an FP16 pass that took 52 square roots per row.
+__global__ void __launch_bounds__(256) half_setup_kernel(Box bx, Split sp, const double *__restrict__ A,
+                                                         double *__restrict__ H, float *__restrict__ H32,
+                                                         _Float16 *__restrict__ H16,
                                                          float *__restrict__ dg, const float *__restrict__ sc,
                                                          float *__restrict__ eg, float *__restrict__ fg, int scaled_in)
 {
@@ -560,7 +561,8 @@ __global__ void __launch_bounds__(256) half16_residual_kernel(Box bx, const _Flo
 {
   __shared__ float tile[SweepTile<kBY, 1>::N];
   const int I = blockIdx.z, J0 = blockIdx.y * kBY, K0 = blockIdx.x * kBX;
-  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile, [&](long g, unsigned i, int, int, int) { return at(sc, g, i) * at(x, g, i); });
+  stage_tile<kBY, 1>(bx, I, J0, K0, threadIdx.y * kBX + threadIdx.x, tile,
+                     [&](long g, unsigned i, int, int, int) { return at(sc, g, i) * at(x, g, i); });
   const int J = J0 + threadIdx.y, K = K0 + threadIdx.x;
   if (K >= bx.nz || J >= bx.ny) return;
   const long row = ((long)I * bx.ny + J0) * bx.nz + K0;
@@ -834,7 +836,7 @@ __device__ __forceinline__ void pair_body(const PairArgs<T> &A, int blk, char *l
         have = hi;
       }
       const T pro = T(0.125) * ((lo == hi ? sum1 : sum0) + sum1);
-      // (after one step from zero the iterate is c1 b' / e again, neither stored nor read; on the finest level b' from b too)
+      // (after one step from zero the iterate is c1 b' / e again, neither stored nor read; on the finest level b' from b)
       const T x = MODE == PAIR_POST1 ? A.c1 * w.b / w.d : at(A.x, row, o);
       v = F16 ? x + w.s * pro : x + pro;
     }
@@ -954,7 +956,8 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(pair_threads<T>()) pair_kernel(PairArgs<T> A)
 {
   extern __shared__ double pair_smem[];
-  const int total = A.g.nk * A.g.nj * A.g.ni, per = (total + 7) / 8, blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  const int total = A.g.nk * A.g.nj * A.g.ni, per = (total + 7) / 8;
+  const int blk = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if (blk >= total) return;
   pair_body<T, MODE>(A, blk, (char *)pair_smem);
 }
@@ -1108,8 +1111,9 @@ __global__ void __launch_bounds__(576) rap_kernel(Box f, Box c, int part, const 
 // 32 x 32 blocks without pivoting.  A step k takes two launches: the panel kernel inverts the diagonal block (every
 // workgroup for itself, in LDS), forms its part of R = D A_k: and copies its part of the block column A_:k; the update
 // kernel writes A_ij -= A_ik R_j, R in block row k, -A_ik D in block column k and D itself: 30 -> 18 us a step at 504
-// rows since a pivot pair waits at one barrier and no load waits for another.  A hierarchy's whole set-up at 47 x 47 x 47 rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343
-// 13.4 -> 0.72 ms, at 65^3 over 512 46 -> 0.94 ms: scalar host code between two copies did the elimination before.
+// rows since a pivot pair waits at one barrier and no load waits for another.  A hierarchy's whole set-up at 47 x 47 x 47
+// rows over 125 coarsest ones 2.1 -> 0.44 ms, at 63^3 over 343 13.4 -> 0.72 ms, at 65^3 over 512 46 -> 0.94 ms: scalar
+// host code between two copies did the elimination before.
 constexpr int kCB = 32;
 constexpr long kMaxCoarse = 4096;
 __global__ void dense_fill_kernel(Box b, const double *__restrict__ st, double *__restrict__ A)
@@ -1129,7 +1133,8 @@ __global__ void __launch_bounds__(256) dense_panel_kernel(int n, int k0, const d
                                                           double *__restrict__ R, double *__restrict__ Cc,
                                                           double *__restrict__ D, double *__restrict__ bad)
 {
-  // the pivots read one copy of the block and write the other (a thread keeps its own entries in registers), and the block row's part that R needs is loaded ahead of the pivots
+  // the pivots read one copy of the block and write the other (a thread keeps its own entries in registers), and the
+  // block row's part that R needs is loaded ahead of the pivots
   __shared__ double d[2][kCB][kCB + 1], ak[kCB][kCB + 1];
   const int t = threadIdx.x, m = min(kCB, n - k0);
   const int c = t % kCB, r0 = t / kCB;  // this thread's column and rows r0, r0 + 8, ...
@@ -1360,7 +1365,7 @@ struct MGLevel {
   DevBuf<float> H32, dinv32, b32, x32, r32, d32;
   DevBuf<_Float16> H16;        // FP16 upper off-diagonals, pairs of directions per row [7][n][2] (half16_row)
   DevBuf<float> dg16, sc16;    // their diagonal d and row scales s
-  DevBuf<float> e16, f16;      // d / s^2; the first smoothing step's factor (half16_setup_kernel)
+  DevBuf<float> e16, f16;      // d / s^2; the first smoothing step's factor (half_setup_kernel)
   DevBuf<float> t32;           // finest level: the scaled right-hand side
   double lmax = 0;
 };
@@ -1410,7 +1415,8 @@ dim3 power_grid(const Box &b) { return split_grid(b, split_of(b, 8), 8, sweep_bi
 long power_sums(const Box &b)
 {
   const dim3 g = power_grid(b);
-  const long single = (long)g.x * g.y * g.z, pair = pair_level<double>(b, 2) ? pair_tiles<double>(b, kPairSlots).blocks() : 0;
+  const long single = (long)g.x * g.y * g.z;
+  const long pair = pair_level<double>(b, 2) ? pair_tiles<double>(b, kPairSlots).blocks() : 0;
   return std::max({256L, single, pair});
 }
 
@@ -1638,8 +1644,9 @@ void vcycle(_p_dohpMG *mg, size_t l, const T *b, T *x, hipStream_t st)
 }
 
 // The tile of the FP16 sweeps: two planes of 64 x 4 rows from 8 million rows on, where the level's 48 bytes a row
-// (384 MB) stream from HBM and the fewer staged loads show (239^3: 162 against 166 us, 207^3: 115 against 118), one plane
-// below, where the level lives in the 256 MB cache (191^3: 78 against 82 us, 95^3: 15.0 against 15.6).
+// (384 MB) stream from HBM and the fewer staged loads show (a sweep of 239^3 rows 162 against 166 us, 207^3: 115 against
+// 118), one plane below, where the level lives in the 256 MB cache (191^3: 78 against 82 us, 95^3: 15.0 against 15.6).
+// Levels of that size come here at smoothing degrees of 3 and more; at 1 and 2 they march (pair_level).
 template <int MODE>
 void sweep16(const MGLevel &lv, const float *b, const float *y, float *out, float *y1, double a, double c, double c1,
              int keep_d, int raw, int unscale, hipStream_t st, const Box &cb = Box{}, const float *xc = nullptr)

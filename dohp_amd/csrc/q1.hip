@@ -145,7 +145,11 @@ __device__ inline void q1_geo(const double *__restrict__ vxyz, const double *__r
     g.Gk[c] = 0.125 * s;
   }
 }
-// Rows J[m] = dX/dx_m of the Jacobian's transpose at (x0, x1, x2); its inverse rows c[m] = grad x_m and determinant.
+// Rows J[m] = dX/dx_m of the Jacobian's transpose at (x0, x1, x2); its inverse rows c[m] = grad x_m and determinant.  This
+// reciprocal, the powers and the roots below are the operator's (element.h: hardware estimates refined by two Newton steps
+// in FP64).  Matrix entries against 80-bit arithmetic, nine cases of p = 1.25 to 2 and degree 1 to 6: 1.8e-16 to 4.9e-16 in
+// the Frobenius norm, and the same to 15 % with pow, sqrt and divisions, which take a Newton step at 32^3, p = 6 from 7.67
+// to 7.91 ms.
 __device__ __forceinline__ double q1_inverse(const Q1Geo &g, double x0, double x1, double x2, double (&c)[3][3])
 {
   double J[3][3];
@@ -183,7 +187,8 @@ __device__ __forceinline__ double q1_inverse(const Q1Geo &g, double x0, double x
 // Eight coloured launches that added 64 entries per sub-cell into the stencil, and its clearing, took 6.2 ms at 32^3
 // elements, p = 6 (7.1 M sub-cells); this and the gather below take 2.3 ms (1.5 and 0.7).
 template <int N, bool LAM>
-__global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per_eu(2))) q1_cell_kernel(long first, long nel, int slots,
+__global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per_eu(2))) q1_cell_kernel(
+                                                                long first, long nel, int slots,
                                                                 const int *__restrict__ everts,
                                                                 const double *__restrict__ vxyz,
                                                                 const double *__restrict__ kv,
@@ -202,7 +207,8 @@ __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per
   const long e0 = first + (long)blockIdx.x * EPB;
   const int ne = (int)min((long)EPB, first + nel - e0);
   for (int t = tid; t < 2 * NQ + P + 2 * NQ * N; t += NT) tb[t] = tab[t];
-  for (int t = tid; t < ne * 17; t += NT) q1_geo(vxyz, ph.has_k ? kv : nullptr, everts + (e0 + t / 17) * 8, t % 17, geo[t / 17]);
+  for (int t = tid; t < ne * 17; t += NT)
+    q1_geo(vxyz, ph.has_k ? kv : nullptr, everts + (e0 + t / 17) * 8, t % 17, geo[t / 17]);
   // the state enters the block only through eta(grad u) and s (p != 2) and lambda e^u: for the linear operator
   // (p = 2, lambda = 0) eta = 1 and s = 0 whatever the state, and its interpolation is skipped
   const bool has_u = ustate && (ph.p != 2.0 || LAM);
@@ -386,10 +392,11 @@ __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per
 // Rows of the 27-point stencil st[27][n] on node planes plane0 .. of the lattice, from the sub-cell matrices of the
 // sub-cells around them: a thread adds the diagonal and the 13 upper entries of its row (36 values, each sub-cell entry
 // read once) and also stores each upper entry as the lower one of that neighbour's row; entries toward nodes that are not
-// owned are zero.  I0, J0, K0: first owned node of the lattice; line0: first line of this launch; G: sub-cells per direction.
-__global__ void __launch_bounds__(256) q1_gather_kernel(int plane0, int line0, int slots, int I0, int J0, int K0, int nx, int ny,
-                                                        int nz, int G0, int G1, int G2, const double *__restrict__ KC,
-                                                        double *__restrict__ st)
+// owned are zero.  I0, J0, K0: first owned node of the lattice; line0: first line of this launch; G: sub-cells per
+// direction.
+__global__ void __launch_bounds__(256) q1_gather_kernel(int plane0, int line0, int slots, int I0, int J0, int K0, int nx,
+                                                        int ny, int nz, int G0, int G1, int G2,
+                                                        const double *__restrict__ KC, double *__restrict__ st)
 {
   const int K = blockIdx.x * 64 + threadIdx.x, J = line0 + blockIdx.y * 4 + threadIdx.y, I = plane0 + blockIdx.z - I0;
   if (K >= nz || J >= ny || I < 0 || I >= nx) return;

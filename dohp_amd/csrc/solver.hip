@@ -274,13 +274,19 @@ struct Ops;
 template <>
 struct Ops<double> {
   static dErr A(dohpEllip op, const double *x, double *y, hipStream_t s) { return dohpEllipMatMult_Private(op, x, y, s); }
-  static dErr A_add(dohpEllip op, const double *x, double *y, hipStream_t s) { return dohpEllipMatMultAdd_Private(op, x, y, s); }
+  static dErr A_add(dohpEllip op, const double *x, double *y, hipStream_t s)
+  {
+    return dohpEllipMatMultAdd_Private(op, x, y, s);
+  }
   static dErr Q(dohpMat m, const double *x, double *y, hipStream_t s) { return dohpMatMult(m, x, y, s); }
 };
 template <>
 struct Ops<float> {
   static dErr A(dohpEllip op, const float *x, float *y, hipStream_t s) { return dohpEllipMatMult_Private(op, x, y, s); }
-  static dErr A_add(dohpEllip op, const float *x, float *y, hipStream_t s) { return dohpEllipMatMultAdd_Private(op, x, y, s); }
+  static dErr A_add(dohpEllip op, const float *x, float *y, hipStream_t s)
+  {
+    return dohpEllipMatMultAdd_Private(op, x, y, s);
+  }
   static dErr Q(dohpMat m, const float *x, float *y, hipStream_t s) { return dohpMatMultF32(m, x, y, s); }
 };
 
