@@ -881,7 +881,13 @@ dErr set_state(_p_dohpEllip *op, const double *u, double *f, hipStream_t st)
 dErr ellip_function(_p_dohpEllip *op, const double *u, double *f, hipStream_t st)
 {
   if (op->prm.exact >= 0 && !op->has_forcing) DOHP_CALL(assemble_forcing(op, st));
-  DOHP_CALL(set_state(op, u, f, st));
+  // The state kernel also sets f, one launch less.  Where f is cleared and what that kernel writes (20 bytes a node) passes
+  // the 256 MB cache, f is cleared behind it instead and so is in the cache for the scatter: p = 6, together and apart 201
+  // and 201 us at 7 M nodes, 291 and 293 at 10 M, 1524 and 1493 at 56 M; p = 3 520 and 501 at 14 M, 270 and 274 at 7 M.
+  // A forcing term would have to be read again: together at every size (1572 and 1589 us at 56 M).
+  const bool apart = !op->has_forcing && op->fs->nclosure > 12000000;
+  DOHP_CALL(set_state(op, u, apart ? nullptr : f, st));
+  if (apart) DOHP_CALL(zero(f, op->fs->nowned, st));
   return launch<double, MODE_FUN>(op, op->state.ptr, nullptr, f, st);
 }
 
