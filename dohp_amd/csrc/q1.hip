@@ -99,13 +99,15 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F f
 // exp out of line: its registers do not constrain the allocation of the sub-cell block
 __device__ __noinline__ double q1_exp(double x) { return exp(x); }
 
-// Elements per workgroup and LDS (doubles per element: the state contracted along z, then along z and y; the node values
-// share the latter's space) of the sub-cell kernel.
+// LDS (doubles per element: the state contracted along z, then along z and y; the node values share the latter's space)
+// and elements per workgroup of the sub-cell kernel: as many as fill two lanes a sub-cell of its 256 threads and fit.  At
+// degree 1 with a state 112 instead of 128 leave LDS for a second workgroup on the compute unit: 8 M sub-cells 5.61 ->
+// 3.96 ms an assembly (without a state 3.19 with 128, 3.27 with 112).
 constexpr int q1_lds_z(int N) { return 2 * N * N * 2 * (N - 1); }
 constexpr int q1_lds_y(int N) { return 3 * N * 4 * (N - 1) * (N - 1); }
-constexpr int q1_epb(int N)
+constexpr int q1_epb(int N, bool has_u)
 {
-  const int P3 = (N - 1) * (N - 1) * (N - 1), want = P3 >= 216 ? 1 : P3 == 1 ? 128 : 256 / P3;
+  const int P3 = (N - 1) * (N - 1) * (N - 1), want = P3 >= 216 ? 1 : P3 == 1 ? (has_u ? 112 : 128) : 256 / P3;
   const int fit = 8000 / (q1_lds_z(N) + q1_lds_y(N));
   return want < fit ? want : fit < 1 ? 1 : fit;
 }
@@ -186,7 +188,7 @@ __device__ __forceinline__ double q1_inverse(const Q1Geo &g, double x0, double x
 //    overlap the other's points (seven wavefronts in one round: 190 us a pass of 663,000 sub-cells against 148).
 // Eight coloured launches that added 64 entries per sub-cell into the stencil, and its clearing, took 6.2 ms at 32^3
 // elements, p = 6 (7.1 M sub-cells); this and the gather below take 2.3 ms (1.5 and 0.7).
-template <int N, bool LAM>
+template <int N, bool STATE, bool LAM>
 __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per_eu(2))) q1_cell_kernel(
                                                                 long first, long nel, int slots,
                                                                 const int *__restrict__ everts,
@@ -197,27 +199,36 @@ __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per
                                                                 const float *__restrict__ cscale,
                                                                 double *__restrict__ KC)
 {
-  constexpr int P = N - 1, NP3 = P * P * P, NQ = 2 * P, NN = N * N, EPB = q1_epb(N), NT = q1_threads(N);
+  constexpr int P = N - 1, NP3 = P * P * P, NQ = 2 * P, NN = N * N, EPB = q1_epb(N, STATE), NT = q1_threads(N);
   constexpr int LZ = q1_lds_z(N), LY = q1_lds_y(N);
   extern __shared__ double lds[];  // [EPB][LZ], [EPB][LY] (with a state)
   __shared__ Q1Geo geo[EPB];
+  __shared__ int el[EPB][3];  // the elements' places in the block (their divisions once an element, not a point or sub-cell)
   __shared__ double tb[2 * NQ + P + 2 * NQ * N];  // zq, wq, hsub, B, D
   const double *zq = tb, *wq = tb + NQ, *hsub = tb + 2 * NQ, *Bs = tb + 2 * NQ + P, *Ds = Bs + NQ * N;
   const int tid = threadIdx.x;
   const long e0 = first + (long)blockIdx.x * EPB;
   const int ne = (int)min((long)EPB, first + nel - e0);
   for (int t = tid; t < 2 * NQ + P + 2 * NQ * N; t += NT) tb[t] = tab[t];
+  for (int t = tid; t < ne; t += NT) {  // (nelem is an int)
+    const int e = (int)e0 + t, col = e / ph.M2, ex = col / ph.M1;
+    el[t][0] = ex;
+    el[t][1] = col - ex * ph.M1;
+    el[t][2] = e - col * ph.M2;
+  }
   for (int t = tid; t < ne * 17; t += NT)
     q1_geo(vxyz, ph.has_k ? kv : nullptr, everts + (e0 + t / 17) * 8, t % 17, geo[t / 17]);
-  // the state enters the block only through eta(grad u) and s (p != 2) and lambda e^u: for the linear operator
-  // (p = 2, lambda = 0) eta = 1 and s = 0 whatever the state, and its interpolation is skipped
-  const bool has_u = ustate && (ph.p != 2.0 || LAM);
+  // (a branch on the pointer, not on STATE alone: without it the compiler forms several points' states at once and spills,
+  // 4.7 -> 8.0 ms at 40^3 elements, p = 6)
+  const bool has_u = STATE && ustate;
   double *Z = lds, *Y = lds + EPB * LZ;
   if (has_u) {
+    __syncthreads();
     for (int t = tid; t < ne * NN * N; t += NT) {
       const int l = t / (NN * N), r = t - l * NN * N, a = r / NN, b = (r / N) % N, c = r % N;
-      const long e = e0 + l, ex = e / ((long)ph.M1 * ph.M2), ey = (e / ph.M2) % ph.M1, ez = e % ph.M2;
-      Y[l * LY + r] = ustate[((ex * P + a) * ph.Ly + ey * P + b) * ph.Lz + ez * P + c];
+      const long I = (long)el[l][0] * P + a;
+      const int J = el[l][1] * P + b, K = el[l][2] * P + c;
+      Y[l * LY + r] = ustate[(I * ph.Ly + J) * ph.Lz + K];
     }
     __syncthreads();
     for (int t = tid; t < ne * NN * NQ; t += NT) {  // along z: values, derivatives
@@ -376,7 +387,7 @@ __global__ void __launch_bounds__(q1_threads(N)) __attribute__((amdgpu_waves_per
              h[r2] * (sg(r0, c2) * B02[c0][y] + sg(r1, c2) * B12[x][c1]) +
              h[c2] * (sg(r2, c0) * B02[r0][y] + sg(r2, c1) * B12[x][r1]);
     };
-    const int ex = (int)(e / ((long)ph.M1 * ph.M2)), ey = (int)((e / ph.M2) % ph.M1), ez = (int)(e % ph.M2);
+    const int ex = el[l][0], ey = el[l][1], ez = el[l][2];
     const long G1 = (long)ph.M1 * P, G2 = (long)ph.M2 * P, ring = slots * G1 * G2;
     double *out = KC + (kk ? 18 * ring : 0) + ((long)((ex * P + pa) % slots) * G1 + ey * P + pb) * G2 + ez * P + pc;
     // lane 0 of the pair stores the first 18 entries, lane 1 the others, each with the other lane's point added
@@ -754,19 +765,22 @@ dErr q1_passes(dohpFS fs, const dohpEllipParam &prm, const Q1Phys &ph, _p_dohpMa
     const long first = (long)x0 * fs->M[1] * fs->M[2], nel = (long)(x1 - x0) * fs->M[1] * fs->M[2];
     DOHP_CALL(q1_dispatch(fs->n, [&](auto NN) {
       constexpr int N = decltype(NN)::value;
-      const bool has_u = state && (prm.p != 2.0 || prm.lambda != 0.0);
-      const size_t lds = has_u ? sizeof(double) * q1_epb(N) * (q1_lds_z(N) + q1_lds_y(N)) : 0;
-      const dim3 grid((unsigned)((nel + q1_epb(N) - 1) / q1_epb(N)));
-      auto go = [&](auto kernel) {
+      const auto go = [&](auto kernel, bool with_state) {
+        const int epb = q1_epb(N, with_state);
+        const size_t lds = with_state ? sizeof(double) * epb * (q1_lds_z(N) + q1_lds_y(N)) : 0;
         if (lds > 65536)
           (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        hipLaunchKernelGGL(kernel, grid, dim3(q1_threads(N)), lds, st, first, nel, slots, fs->d_elem_verts.ptr,
-                           fs->d_vcoords.ptr, kvert, state, q1mode, A->q1tab.ptr, ph, cscale, ring);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((nel + epb - 1) / epb)), dim3(q1_threads(N)), lds, st, first, nel, slots,
+                           fs->d_elem_verts.ptr, fs->d_vcoords.ptr, kvert, state, q1mode, A->q1tab.ptr, ph, cscale, ring);
       };
+      // the state enters a sub-cell only through eta(grad u) and s (p != 2) and lambda e^u: for the linear operator
+      // (p = 2, lambda = 0) eta = 1 and s = 0 whatever the state, and its interpolation is left out
       if (prm.lambda != 0.0)
-        go(q1_cell_kernel<N, true>);
+        go(q1_cell_kernel<N, true, true>, true);
+      else if (prm.p != 2.0)
+        go(q1_cell_kernel<N, true, false>, true);
       else
-        go(q1_cell_kernel<N, false>);
+        go(q1_cell_kernel<N, false, false>, false);
     }));
     // node planes whose sub-cells are all there: up to the pass's last layer of sub-cells, and the block's last plane
     const int p0 = x0 * fs->p, p1 = x1 == fs->M[0] ? G[0] + 1 : x1 * fs->p;
