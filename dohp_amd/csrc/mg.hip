@@ -152,7 +152,10 @@ inline bool sweep_big(const Box &b)
 // its L2 (191^3: 36 k entries of 112 bytes a plane over eight caches of 4 MB).  At 239^3 the FP16 sweeps fetch 0.63 GB and
 // take 158 to 195 instead of 170 to 221 us, the Galerkin product (with a load a fine node) 1.37 instead of 1.62 ms, the
 // half stencils 1.10 instead of 1.44 ms; a power iteration at 191^3 231 instead of 244 us.  Boxes with fewer than two
-// tiles of lines per part are not split (47^3, all of it in every L2: no difference).
+// tiles of lines per part are not split (47^3, all of it in every L2: no difference), nor are boxes with short lines, whose
+// blocks are many and touch little: V-cycles of three steps on 399 x 399 x 15 rows 2580 (FP64), 917 (FP16) and 699 us
+// split, 2311, 871 and 626 not, on 359 x 359 x 35 1781, 819, 758 and 1711, 779, 726, but on 59 x 449 x 59 449, 235, 232 and
+// 478, 247, 262.
 struct Split {
   int lg, lines;  // log2 of the number of parts, lines of a part
   __device__ __forceinline__ int j0(unsigned bx, unsigned by, int BY) const
@@ -168,7 +171,7 @@ struct Split {
 inline Split split_of(const Box &b, int BY)
 {
   const int l = (b.ny + 15) / 16 * 2;  // (even: the coarse tiles start at half the first line)
-  return l >= 2 * BY ? Split{3, l} : Split{0, b.ny};
+  return l >= 2 * BY && b.nz >= 48 ? Split{3, l} : Split{0, b.ny};
 }
 inline dim3 split_grid(const Box &b, const Split &s, int BY, int NR)
 {
@@ -192,8 +195,8 @@ __device__ __forceinline__ T &at(T *p, long row, unsigned i)
 
 // Fills the tile of the block at (I0, J0, K0) with load(row, i, gi, gj, gk), row + i the row of the tile entry at
 // (gi, gj, gk) (every load unconditional: entries outside the box load a row inside it and are zero).  A wavefront takes
-// whole lines of 64 columns, whose line numbers are scalars; the two columns beside them go to the first threads.  Ends
-// with a barrier.
+// whole lines of 64 columns, whose line numbers are scalars; the two columns beside them go to the first threads (zero
+// without a load where one tile covers the lines).  Ends with a barrier.
 template <int BY, int NR, typename T, typename Load>
 __device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0, int tid, T *tile, Load load)
 {
@@ -212,7 +215,7 @@ __device__ __forceinline__ void stage_tile(const Box &bx, int I0, int J0, int K0
     const T y = load(in ? gi * sx + gj * sy + K0 : (long)K0, kl, gi, gj, K0 + lane);
     v[u] = in && ink ? y : T(0);
   }
-  if (tid < 2 * L) {
+  if (bx.nz > kBX && tid < 2 * L) {
     const int l = tid >> 1, gi = I0 + l / S::TY - 1, gj = J0 + l % S::TY - 1, gk = tid & 1 ? K0 + kBX : K0 - 1;
     const bool in = inside(bx, gi, gj, gk);
     const T y = load(in ? gi * sx + gj * sy + gk : 0L, 0u, gi, gj, gk);
