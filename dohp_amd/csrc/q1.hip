@@ -184,7 +184,7 @@ __device__ __forceinline__ double q1_inverse(const Q1Geo &g, double x0, double x
 //    against 36 x 8 x 8 and the gradients.
 //  - A pair of lanes shares a sub-cell, one for each point of the last direction, and exchanges halves of the entries at
 //    the end: one thread with the entries and all partial sums live needs 360 registers (one wavefront per SIMD).
-//  - Four wavefronts a workgroup in two rounds at 249 registers: two workgroups per compute unit, so one's contractions
+//  - Four wavefronts a workgroup in two rounds at 245 registers: two workgroups per compute unit, so one's contractions
 //    overlap the other's points (seven wavefronts in one round: 190 us a pass of 663,000 sub-cells against 148).
 // Eight coloured launches that added 64 entries per sub-cell into the stencil, and its clearing, took 6.2 ms at 32^3
 // elements, p = 6 (7.1 M sub-cells); this and the gather below take 2.3 ms (1.5 and 0.7).
